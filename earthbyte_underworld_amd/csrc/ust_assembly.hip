@@ -284,13 +284,6 @@ __device__ __forceinline__ void element_nodes_of(const GridDev &g, int ie, int j
 // ------------------------------------------------------------------------------------------
 #define PW_WAVES 2
 #define PW_CH 11
-// a wavefront's own LDS rows: its LDS operations complete in order, so a wave-level barrier (no compiler
-// reordering across it) is all the reduction needs between a wave's writes and its reads
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 template <int DIM, int S, bool NEED_T, bool NEED_VEL, bool SW>
 __global__ __launch_bounds__(64 * PW_WAVES, (DIM == 2 ? 2 : 1)) void k_particle_weights(
     GridDev g, const int *__restrict__ cell_off, const double *__restrict__ xi0, const double *__restrict__ xi1,

@@ -154,6 +154,14 @@ static inline GridDev grid_dev(const ust_grid *g, long long wg_target = UST_COL_
     return d;
 }
 
+// A wavefront's own LDS: its LDS operations complete in order, so a wave-level barrier (no compiler reordering across
+// it) is all that one wave needs between its lanes' writes and reads of each other's values.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // bfloat16 is the upper half of an FP32: widened by a shift, narrowed with round-to-nearest-even
 __device__ __forceinline__ float bf16_to_f32(unsigned short b) { return __uint_as_float(((unsigned)b) << 16); }
 __device__ __forceinline__ unsigned short f32_to_bf16(float f) {

@@ -9,13 +9,15 @@
 // its cells and weighs their volume (_GetCentroids :203-231, _Calculate3D/2D :763-925).
 //
 // Within one particle's turn every boundary cell is decided on its own (owner and distances only), and the next
-// boundary is a set, so the reference's lists can be held as sets: one bit per sub-cell.  Only the particle
-// order is sequential.  One 64-lane wave owns one element and a sub-cell set is 64-bit words, word j covering
-// sub-cells 64 j .. 64 j + 63.  In a turn, lane L decides sub-cell 64 j + L of every boundary word j that holds
-// cells, one ballot per word, which leaves the claimed set one word per lane; the next boundary is that set
-// dilated by whole-word shifts across lanes (+-1, +-nx, +-nx*ny sub-cells, masked at the sub-grid's x and y
-// faces), less the cells the particle owns.  The boundary sets of all particles of the element, the owner grid
-// and the particle coordinates stay in LDS.
+// boundary is a set, so the reference's lists can be held in any order.  Only the particle order is sequential.
+//
+// k_dvc_grow: a group of G lanes owns one element, 64/G elements to a wave.  All boundary sets of an element sit
+// in one ring of sub-cell indices in LDS: the particles take their turns in the same order every round, so a
+// turn reads its set at the head and appends its next one at the tail.  In a turn lane t decides boundary cell t;
+// the claimed cells are compacted in place, and then lane t takes neighbour t % (2 dim) of claimed cell t / (2 dim),
+// with one bit per sub-cell to take each neighbour once.
+// k_dvc_spill: the elements whose sets outgrew the ring (marked by a negative weight), one element to a wave with the
+// sets as 64-bit words, which no element accepted by the launcher outgrows.
 #include "ust_common.h"
 
 namespace {
@@ -28,6 +30,7 @@ struct DvcShape {
     int words;    // 64-bit words of a sub-cell set
     int max_np;   // particles per element the LDS layout holds
     float inv[2]; // 1 / n[0], 1 / n[1]
+    int ring;     // k_dvc_grow: sub-cell indices the ring of boundary sets holds (even)
 };
 
 // floor(c / n) for 0 <= c < 4096 and 1 <= n <= 64: (c + 1/2) / n is at least 1/128 away from an integer and the
@@ -76,22 +79,15 @@ __device__ __forceinline__ unsigned long long set_down(unsigned long long x, int
     return r ? (a >> r) | (lane_word(x, lane + q + 1) << (64 - r)) : a;
 }
 
-// flag bits: 1 element without particles, 2 more particles than the LDS layout holds, 4 round limit reached.
+// Region growth of one element by one wave, a boundary set as 64-bit words, word j covering sub-cells 64 j .. 64 j + 63:
+// in a turn lane L decides sub-cell 64 j + L of every boundary word j that holds cells, one ballot per word, which
+// leaves the claimed set one word per lane; the next boundary is that set dilated by whole-word shifts across lanes
+// (+-1, +-nx, +-nx*ny sub-cells, masked at the sub-grid's x and y faces), less the cells the particle owns.
 // OT: the owner grid's type, signed char when at most 127 particles share an element (less LDS, more waves)
 template <int DIM, typename OT>
-__global__ __launch_bounds__(DVC_LANES) void k_dvc_weights(DvcShape s, const int *cell_off, int nel, double *xi0,
-                                                           double *xi1, double *xi2, double *w, int set_centroids,
-                                                           int *flag) {
-    extern __shared__ __align__(16) unsigned char dvc_lds[];
-    const int e = blockIdx.x;
+__device__ void dvc_element_words(const DvcShape &s, unsigned char *dvc_lds, int off, int np, double *xi0, double *xi1,
+                                  double *xi2, double *w, int set_centroids, int *flag) {
     const int lane = threadIdx.x;
-    if (e >= nel) return;
-    const int off = cell_off[e];
-    const int np = cell_off[e + 1] - off;
-    if (np <= 0 || np > s.max_np) {
-        if (lane == 0) atomicOr(flag, np <= 0 ? 1 : 2);
-        return;
-    }
     const int W = s.words, ncell = s.ncell;
     // LDS: centres per axis | particle coordinates (np x DIM) | boundary sets (np x W) | owner
     double *axc = (double *)dvc_lds;                                  // n[0] + n[1] + n[2]
@@ -250,6 +246,315 @@ __global__ __launch_bounds__(DVC_LANES) void k_dvc_weights(DvcShape s, const int
     }
 }
 
+// per > 1: the elements whose boundary sets outgrew k_dvc_grow's ring (it left a negative weight on their first particle);
+// a wave looks at `per` elements and redoes the marked ones.  per = 1: every element, where particles so many that
+// k_dvc_grow's LDS does not fit share one.
+template <int DIM, typename OT>
+__global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, int nel, double *xi0,
+                                                         double *xi1, double *xi2, double *w, int set_centroids,
+                                                         int *flag, int per) {
+    extern __shared__ __align__(16) unsigned char dvc_lds[];
+    const int el = blockIdx.x * per + (int)threadIdx.x;
+    const bool mine = (int)threadIdx.x < per && el < nel;
+    int off = 0, np = 0;
+    if (mine) {
+        off = cell_off[el];
+        np = cell_off[el + 1] - off;
+    }
+    const bool holds = mine && np > 0 && np <= s.max_np;
+    if (per == 1 && mine && !holds) atomicOr(flag, np <= 0 ? 1 : 2);
+    unsigned long long todo = __ballot(holds && (per == 1 || w[off] < 0.0));
+    while (todo) {
+        const int j = __builtin_ctzll(todo);
+        todo &= todo - 1ull;
+        dvc_element_words<DIM, OT>(s, dvc_lds, __shfl(off, j), __shfl(np, j), xi0, xi1, xi2, w, set_centroids, flag);
+        __syncthreads();  // the next element reuses the LDS
+    }
+}
+
+// bytes of one element's LDS in k_dvc_grow: coordinates in FP32 | ring | one bit per sub-cell | set sizes | owner
+__host__ __device__ inline size_t grow_lds_element(const DvcShape &s, size_t ot) {
+    return ((size_t)s.max_np * 16 + (size_t)s.ring * 2 + (size_t)((s.ncell + 31) / 32) * 4 + (size_t)s.max_np * 2 +
+            (size_t)s.ncell * ot + 15) & ~(size_t)15;
+}
+// and of the tables all elements of a workgroup share: centres per axis | the neighbours every sub-cell has
+__host__ __device__ inline size_t grow_lds_shared(const DvcShape &s) {
+    return ((size_t)(s.n[0] + s.n[1] + s.n[2]) * 8 + (size_t)s.ncell + 15) & ~(size_t)15;
+}
+
+// Bound: the latency of the sequential turns (about 200 in 3D at 30 particles, some 200 VALU and 14 LDS instructions
+// each), so what counts is the elements in flight, which LDS limits (40 per CU at 30 particles), and the length of a
+// turn: the claim test reads FP32 coordinates in one 16-byte access, and a lane per neighbour expands five claimed
+// cells a pass.  96^3 elements x 30 particles: 178 ms with one element to a wave and the sets as words, 43 ms here; its
+// bytes (1.5 GB) would take 0.3 ms.
+constexpr int GROW_WAVES = 2;
+constexpr int DVC_WIDE_2D = 16384;  // 2D swarms of fewer elements give an element 32 lanes
+
+template <int DIM, int G, typename OT>
+__global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const int *__restrict__ cell_off, int nel,
+                                                              double *xi0, double *xi1, double *xi2, double *w,
+                                                              int set_centroids, int *flag) {
+    static_assert(G == 16 || G == 32, "group votes are 32-bit");
+    extern __shared__ __align__(16) unsigned char dvc_lds[];
+    constexpr int ND = 2 * DIM;      // neighbours of a sub-cell
+    constexpr int CP = G / ND;       // claimed cells expanded per pass, one lane per neighbour
+    const int ncell = s.ncell, nbw = (ncell + 31) / 32;
+    const unsigned R = (unsigned)s.ring;
+    const int nx = s.n[0], nxy = s.n[0] * s.n[1];
+    const double d[3] = {2.0 / s.n[0], 2.0 / s.n[1], 2.0 / s.n[2]};
+    double *axc = (double *)dvc_lds;                                           // n[0] + n[1] + n[2]
+    unsigned char *nbv = (unsigned char *)(axc + (s.n[0] + s.n[1] + s.n[2]));  // ncell: bit q = neighbour q exists
+    {
+        const int t = threadIdx.x;
+        if (t < DIM) {  // centres accumulated as the grid constructor does: -1 - d/2, then + d per cell
+            const int n = t == 0 ? s.n[0] : (t == 1 ? s.n[1] : s.n[2]);
+            const double dl = t == 0 ? d[0] : (t == 1 ? d[1] : d[2]);
+            double *a = axc + (t == 0 ? 0 : (t == 1 ? s.n[0] : s.n[0] + s.n[1]));
+            double x = -1.0 - dl / 2.0;
+            for (int i = 0; i < n; i++) {
+                x = x + dl;
+                a[i] = x;
+            }
+        }
+        for (int c = t; c < ncell; c += 64 * GROW_WAVES) {
+            const CellWalk q(s, c);
+            nbv[c] = (unsigned char)((q.i > 0) | (q.i < nx - 1) << 1 | (q.j > 0) << 2 | (q.j < s.n[1] - 1) << 3 |
+                                     (q.k > 0) << 4 | (q.k < s.n[2] - 1) << 5);
+        }
+    }
+    const int lane = threadIdx.x & 63, gl = lane % G, grp = threadIdx.x / G;
+    const int e = blockIdx.x * (64 * GROW_WAVES / G) + grp;
+    int off = 0, np = 0;
+    if (e < nel) {
+        off = cell_off[e];
+        np = cell_off[e + 1] - off;
+        if ((np <= 0 || np > s.max_np) && gl == 0) atomicOr(flag, np <= 0 ? 1 : 2);
+    }
+    __syncthreads();  // the tables; from here on every wave works in its own LDS
+    if (np <= 0 || np > s.max_np) return;
+    float4 *pf = (float4 *)(dvc_lds + grow_lds_shared(s) + grp * grow_lds_element(s, sizeof(OT)));
+    unsigned short *ring = (unsigned short *)(pf + s.max_np);
+    unsigned *seen = (unsigned *)(ring + R);
+    unsigned short *cnt = (unsigned short *)(seen + nbw);
+    OT *owner = (OT *)(cnt + s.max_np);
+
+    // the group's lanes with pred set, and this lane's rank among them
+    auto vote = [&](bool pred) -> unsigned {
+        const unsigned long long b = __ballot(pred);
+        if (G == 32) return lane & 32 ? (unsigned)(b >> 32) : (unsigned)b;
+        return (unsigned)(b >> (lane - gl)) & 0xffffu;
+    };
+    const unsigned below = (1u << gl) - 1u;
+    auto rank = [&](unsigned b) -> unsigned { return (unsigned)__popc(b & below); };
+    auto wrap = [&](unsigned x) -> unsigned { return min(x, x - R); };  // x < 2 R: below R the difference wraps high
+
+    // owner grid unowned, no cell seen; the particles' FP32 coordinates, and their seed cells in the set sizes' place
+    for (int c = gl; c < ncell; c += G) owner[c] = -1;
+    for (int c = gl; c < nbw; c += G) seen[c] = 0u;
+    bool tame = true;
+    for (int p = gl; p < np; p += G) {
+        const double x[3] = {xi0[off + p], xi1[off + p], DIM == 3 ? xi2[off + p] : 0.0};
+        int idx[3] = {0, 0, 0};
+#pragma unroll
+        for (int a = 0; a < DIM; a++) {
+            const double t = (x[a] - (-1.0)) / d[a];
+            // C truncation toward zero; k == n moves to n - 1; outside [-1, 1] (and NaN): the nearest cell
+            idx[a] = (t >= 0.0) ? (t < (double)s.n[a] ? (int)t : s.n[a] - 1) : 0;
+            tame = tame && fabs(x[a]) <= 1.5;
+        }
+        pf[p] = make_float4((float)x[0], (float)x[1], (float)x[2], 0.0f);
+        cnt[p] = (unsigned short)(idx[0] + idx[1] * nx + (DIM == 3 ? idx[2] * nxy : 0));
+    }
+    // The claim test in FP32 first.  With |coordinates| <= 1.5 its error against the FP64 one is below 2.5e-5: centre and
+    // coordinates are within 2e-7, so a factor po + pp - 2 c (at most 5) within 1.8e-6, po - pp (at most 3) within
+    // 3.6e-7, each of at most three products within 8e-6.  Inside 3e-5 of zero the FP64 test decides.
+    const float tol = vote(!tame) ? INFINITY : 3e-5f;
+    const float fnx = (float)s.n[0], fny = (float)s.n[1];
+    const float fd[3] = {(float)d[0], (float)d[1], (float)d[2]};
+    const float f0[3] = {(float)(-1.0 + 0.5 * d[0]), (float)(-1.0 + 0.5 * d[1]), (float)(-1.0 + 0.5 * d[2])};
+    wave_sync();
+
+    // this lane's neighbour in the expansion of claimed cells
+    const int dir = gl % ND, slot = gl / ND;
+    const int step = (dir & 1 ? 1 : -1) * (dir < 2 ? 1 : (dir < 4 ? nx : nxy));
+    const bool expand = gl < CP * ND;
+
+    // seeds in particle order (a later particle seeded in the same cell takes it), each with its neighbours
+    // (DVCWeights.c:676-696); none of them can be the particle's own
+    unsigned head = 0, tail = 0, live = 0;
+    bool spill = false;
+    for (int p = 0; p < np; p++) {
+        const int seed = cnt[p];
+        const bool ok = gl < ND && ((nbv[seed] >> dir) & 1);
+        const unsigned b = vote(ok), n = (unsigned)__popc(b);
+        wave_sync();
+        if (gl == 0) {
+            owner[seed] = (OT)p;
+            cnt[p] = (unsigned short)n;
+        }
+        if (ok) ring[tail + rank(b)] = (unsigned short)(seed + step);  // the ring holds more than 2 dim per particle
+        tail += n;
+    }
+    live = tail;
+    wave_sync();
+
+    // rounds over the particles in order until every boundary is empty (DVCWeights.c:698-710).  Every claim changes an
+    // owner and an owner only changes to a strictly nearer particle, so the rounds are bounded; the limit below
+    // keeps the loop finite whatever the rounding does.
+    const long long max_rounds = (long long)ncell * np + 2;
+    long long rounds = 0;
+    while (live > 0 && !spill) {
+        if (++rounds > max_rounds) {
+            if (gl == 0) atomicOr(flag, 4);
+            break;
+        }
+        for (int p0 = 0; p0 < np && !spill; p0 += G) {
+            unsigned turns = vote(p0 + gl < np && cnt[p0 + gl < np ? p0 + gl : 0] != 0);
+            while (turns && !spill) {
+                const int p = p0 + __builtin_ctz(turns);
+                turns &= turns - 1u;
+                const unsigned n = cnt[p];
+                const float4 pp = pf[p];
+                // claims, compacted in place at the head
+                unsigned nc = 0;
+                for (unsigned b0 = 0; b0 < n; b0 += G) {
+                    bool win = false;
+                    int c = 0;
+                    if (b0 + gl < n) {
+                        c = ring[wrap(head + b0 + gl)];
+                        const int o = owner[c];
+                        win = o == -1;
+                        if (o >= 0 && o != p) {
+                            const float4 po = pf[o];
+                            // (i, j, k) as small_div takes them, in floats
+                            const float fc = (float)c, ft = floorf((fc + 0.5f) * s.inv[0]);
+                            const float fi = fc - ft * fnx, fk = DIM == 3 ? floorf((ft + 0.5f) * s.inv[1]) : 0.0f;
+                            const float cx = f0[0] + fd[0] * fi, cy = f0[1] + fd[1] * (ft - fk * fny);
+                            float t = (po.x + pp.x - 2.0f * cx) * (po.x - pp.x) + (po.y + pp.y - 2.0f * cy) * (po.y - pp.y);
+                            if (DIM == 3) t += (po.z + pp.z - 2.0f * (f0[2] + fd[2] * fk)) * (po.z - pp.z);
+                            win = t > tol;
+                            if (!(t > tol || t < -tol)) {
+                                const CellWalk cw(s, c);
+                                const double cc[3] = {axc[cw.i], axc[s.n[0] + cw.j],
+                                                      DIM == 3 ? axc[s.n[0] + s.n[1] + cw.k] : 0.0};
+                                const double xo[3] = {xi0[off + o], xi1[off + o], DIM == 3 ? xi2[off + o] : 0.0};
+                                const double xp[3] = {xi0[off + p], xi1[off + p], DIM == 3 ? xi2[off + p] : 0.0};
+                                win = dvc_distance_test<DIM>(cc, xo, xp) > 0.0;
+                            }
+                        }
+                    }
+                    const unsigned b = vote(win);
+                    wave_sync();
+                    if (win) {
+                        owner[c] = (OT)p;
+                        ring[wrap(head + nc + rank(b))] = (unsigned short)c;
+                    }
+                    nc += (unsigned)__popc(b);
+                    wave_sync();
+                }
+                // the neighbours of the claimed cells that p does not own, each once
+                unsigned nn = 0;
+                for (unsigned b0 = 0; b0 < nc; b0 += CP) {
+                    bool ok = false;
+                    int c1 = 0;
+                    if (expand && b0 + slot < nc) {
+                        const int c = ring[wrap(head + b0 + slot)];
+                        c1 = c + step;
+                        if (((nbv[c] >> dir) & 1) && owner[c1] != (OT)p) {
+                            const unsigned bit = 1u << (c1 & 31);
+                            ok = !(atomicOr(&seen[c1 >> 5], bit) & bit);
+                        }
+                    }
+                    const unsigned b = vote(ok), m = (unsigned)__popc(b);
+                    if (live + nn + m > R) {  // the claimed cells and the sets still to come stay until their turn
+                        spill = true;
+                        break;
+                    }
+                    if (ok) ring[wrap(tail + nn + rank(b))] = (unsigned short)c1;
+                    nn += m;
+                }
+                if (spill) break;
+                wave_sync();
+                for (unsigned i = gl; i < nn; i += G) seen[ring[wrap(tail + i)] >> 5] = 0u;
+                if (gl == 0) cnt[p] = (unsigned short)nn;
+                head = wrap(head + n);
+                tail = wrap(tail + nn);
+                live += nn - n;
+                wave_sync();
+            }
+        }
+    }
+    if (spill) {
+        if (gl == 0) w[off] = -1.0;  // for k_dvc_spill, which starts from the same particles
+        return;
+    }
+
+    // centroids summed in sub-cell order, weight = count * cell volume (DVCWeights.c:203-231): the owner grid turned
+    // into one set of sub-cells per particle, `wc` words of 32 at a time in the ring's memory (an odd number, against
+    // bank conflicts), which lane q walks for particle p0 + q
+    const double vol = DIM == 3 ? d[0] * d[1] * d[2] : d[0] * d[1];
+    const double *cys = axc + s.n[0], *czs = cys + s.n[1];
+    unsigned *set = (unsigned *)ring;
+    const int nq = np < G ? np : G;
+    int wc = (int)R / 2 / nq;
+    wc = wc >= nbw ? nbw | 1 : (wc - 1) | 1;
+    if (wc * nq * 2 > (int)R) wc -= 2;
+    for (int p0 = 0; p0 < np; p0 += G) {
+        double sx = 0.0, sy = 0.0, sz = 0.0;
+        int count = 0;
+        for (int w0 = 0; w0 < nbw; w0 += wc) {
+            const int w1 = w0 + wc < nbw ? w0 + wc : nbw, c1 = 32 * w1 < ncell ? 32 * w1 : ncell;
+            for (int t = gl; t < nq * wc; t += G) set[t] = 0u;
+            wave_sync();
+            for (int c = 32 * w0 + gl; c < c1; c += G) {
+                const int q = (int)owner[c] - p0;
+                if (q >= 0 && q < nq) atomicOr(&set[q * wc + (c >> 5) - w0], 1u << (c & 31));
+            }
+            wave_sync();
+            if (gl < nq) {
+                int t = w0;
+                unsigned bits = set[gl * wc];
+                while (true) {
+                    while (!bits && ++t < w1) bits = set[gl * wc + t - w0];
+                    if (!bits) break;
+                    const CellWalk cw(s, 32 * t + __builtin_ctz(bits));
+                    bits &= bits - 1u;
+                    count++;
+                    sx += axc[cw.i];
+                    sy += cys[cw.j];
+                    if (DIM == 3) sz += czs[cw.k];
+                }
+            }
+            wave_sync();
+        }
+        if (gl < nq && p0 + gl < np) {
+            const int p = off + p0 + gl;
+            w[p] = (double)count * vol;
+            if (set_centroids) {
+                xi0[p] = count ? sx / count : 0.0;
+                xi1[p] = count ? sy / count : 0.0;
+                if (DIM == 3) xi2[p] = count ? sz / count : 0.0;
+            }
+        }
+    }
+}
+
+template <int DIM, int G, typename OT>
+static int launch_dvc(const DvcShape &s, size_t lds_words, const int *cell_off, int nel, double *xi0, double *xi1,
+                      double *xi2, double *w, int set_centroids, int *flag, hipStream_t st) {
+    constexpr int EPB = 64 * GROW_WAVES / G;
+    const size_t lds = grow_lds_shared(s) + EPB * grow_lds_element(s, sizeof(OT));
+    const bool grow = lds <= 65536;
+    if (grow)
+        hipLaunchKernelGGL((k_dvc_grow<DIM, G, OT>), dim3((nel + EPB - 1) / EPB), dim3(64 * GROW_WAVES), lds, st, s,
+                           cell_off, nel, xi0, xi1, xi2, w, set_centroids, flag);
+    const int per = grow ? DVC_LANES : 1;
+    hipLaunchKernelGGL((k_dvc_spill<DIM, OT>), dim3((nel + per - 1) / per), dim3(DVC_LANES), lds_words, st, s, cell_off,
+                       nel, xi0, xi1, xi2, w, set_centroids, flag, per);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -285,20 +590,23 @@ int ust_k_dvc_weights(int dim, const int *res, int nel, const int *cell_off, int
     if (nel == 0) return UST_OK;
     hipStream_t st = ust_stream(stream);
     const bool narrow = max_np <= 127;
-    if (dim == 3 && narrow)
-        hipLaunchKernelGGL((k_dvc_weights<3, signed char>), dim3(nel), dim3(DVC_LANES), lds, st, s, cell_off, nel,
-                           xi0, xi1, xi2, w, set_centroids, flag);
-    else if (dim == 3)
-        hipLaunchKernelGGL((k_dvc_weights<3, short>), dim3(nel), dim3(DVC_LANES), lds, st, s, cell_off, nel, xi0,
-                           xi1, xi2, w, set_centroids, flag);
-    else if (narrow)
-        hipLaunchKernelGGL((k_dvc_weights<2, signed char>), dim3(nel), dim3(DVC_LANES), lds, st, s, cell_off, nel,
-                           xi0, xi1, xi2, w, set_centroids, flag);
-    else
-        hipLaunchKernelGGL((k_dvc_weights<2, short>), dim3(nel), dim3(DVC_LANES), lds, st, s, cell_off, nel, xi0,
-                           xi1, xi2, w, set_centroids, flag);
-    UST_LAUNCH_CHECK();
-    return UST_OK;
+    // the ring, from the most entries that 10^dim sub-cells and random particles needed: 930 for 30 particles in 3D (1,016
+    // given), 1,356 for 60 (1,406), 1,755 for 100 (1,700: a few elements spill); 123 for 20 in 2D (240).  Longer
+    // rings cost waves, since LDS limits the elements in flight: 64^3 x 30 particles took 16.6 ms with 1,980 entries,
+    // 14.9 ms with 1,210, 12.8 ms with 1,016.
+    const int by_cell = s.ncell + 7 * max_np, by_np = 5 * s.ncell / 8 + 13 * max_np;
+    s.ring = ((by_cell < by_np ? by_cell : by_np) + 1) & ~1;
+#define DVC(D, G, OT) return launch_dvc<D, G, OT>(s, lds, cell_off, nel, xi0, xi1, xi2, w, set_centroids, flag, st)
+    // 3D boundaries hold 10 to 20 sub-cells on average: 32 lanes (64^3 x 30 particles: 12.8 ms, with 16 lanes 20.1 ms).
+    // 2D ones hold 4: 16 lanes (512^2 x 20: 1.33 ms, with 32 lanes 2.05 ms), unless the elements are too few to fill
+    // the GPU, where the shorter turns count (64^2 x 20: 0.126 ms with 32 lanes, 0.144 ms with 16).
+    if (dim == 3 && narrow) DVC(3, 32, signed char);
+    if (dim == 3) DVC(3, 32, short);
+    if (nel < DVC_WIDE_2D && narrow) DVC(2, 32, signed char);
+    if (nel < DVC_WIDE_2D) DVC(2, 32, short);
+    if (narrow) DVC(2, 16, signed char);
+    DVC(2, 16, short);
+#undef DVC
 }
 
 }  // extern "C"

@@ -317,3 +317,53 @@ def test_pcdvc_advected_96cube_keeps_elements_populated():
     sums = np.add.reduceat(w, off[:-1])
     assert np.max(np.abs(sums - 8.0)) < 1e-9
     s.close()
+
+
+def _dvc_edge_points(kind, rng):
+    """(dim, res, particles per element) of the cases where the growth kernel's rules change."""
+    if kind == "spill":  # particles on the cells of a tiling by 7-cell crosses: the longest boundaries per particle, more
+        # than the ring holds, and every tie there is; the elements beside it fit
+        k, j, i = np.meshgrid(*[np.arange(9)] * 3, indexing="ij")
+        on = (i + 2 * j + 3 * k + 4) % 7 == 0
+        cross = np.stack([(a[on] + 0.5) * 2.0 / 9.0 - 1.0 for a in (i, j, k)], axis=1)
+        return 3, (9, 9, 9), [rng.uniform(-1, 1, (20, 3)), cross, rng.uniform(-1, 1, (1, 3)), cross[::-1]]
+    if kind == "outside":  # coordinates beyond the FP32 test's range, on the faces, and coincident
+        a = rng.uniform(-1.7, 1.7, (25, 3))
+        b = np.repeat(rng.uniform(-1, 1, (5, 3)), 6, axis=0)
+        c = rng.choice([-1.0, -0.2, 0.0, 0.2, 1.0], (33, 3))
+        return 3, (10, 10, 10), [a, b, c, rng.uniform(0.0, 0.1, (40, 3))]
+    if kind == "many":  # so many that the growth kernel's LDS does not fit
+        return 3, (4, 4, 4), [rng.uniform(-1, 1, (n, 3)) for n in (400, 3, 399)]
+    return 2, (12, 5), [rng.uniform(-1, 1, (n, 2)) for n in (1, 2, 31, 32, 33, 64, 65, 100)]  # "passes"
+
+
+@pytest.mark.parametrize("kind", ["spill", "outside", "many", "passes"])
+def test_dvc_growth_edges(kind):
+    """Bit-equal to the oracle where the sets outgrow the ring, where the FP32 claim test is not allowed to decide, where
+    the LDS of the growth kernel does not suffice and at the edges of a group's lanes."""
+    from oracle import dvc_oracle as D
+    dim, res, pts = _dvc_edge_points(kind, np.random.default_rng(77))
+    s = _system(dim, (len(pts),) + (1,) * (dim - 1))
+    off = np.concatenate([[0], np.cumsum([len(p) for p in pts])]).astype(np.int32)
+    xi = np.zeros((off[-1], 3))
+    xi[:, :dim] = np.concatenate(pts)
+    s.upload_swarm(off, xi, np.ones(off[-1]))
+    s.dvc_weights(res)
+    xi1, w1 = s.integration_points()
+    xi_ref, w_ref = D.dvc_swarm(dim, off, xi, res)
+    assert np.array_equal(w1, w_ref)
+    assert np.array_equal(xi1[:, :dim], xi_ref[:, :dim])
+    s.close()
+
+
+def test_dvc_2d_lane_groups_agree(oracle):
+    """2D swarms below and from 16,384 elements give an element 32 or 16 lanes: both bit-equal to the C oracle."""
+    for nel in ((127, 129), (128, 128)):
+        s = _system(2, nel)
+        s.random_particle_layout(particlesPerCell=7, seed=5)
+        off, xi, _, _ = s.swarm()
+        s.dvc_weights(10)
+        xi1, w1 = s.integration_points()
+        xi_ref, w_ref = oracle.dvc_swarm(2, (10, 10), off, xi)
+        assert np.array_equal(w1, w_ref) and np.array_equal(xi1[:, :2], xi_ref[:, :2])
+        s.close()
