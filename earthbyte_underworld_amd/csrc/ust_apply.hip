@@ -4,8 +4,7 @@
 //
 // 3D: one 256-thread workgroup owns a 16x16 column of elements, one element per thread, and streams a
 // chunk of element layers along z.  Node planes are staged in LDS once each; per layer every thread applies
-// its element with sum factorisation (gradients at the Lagrange points from edge differences, stress, and
-// the transposed interpolation back to the vertices, ~0.8 kflop per element) and leaves its 8 vertex
+// its element (element_apply3 below, about 460 operations) and leaves its 8 vertex
 // results in LDS; each node of the plane below the layer then sums, in a fixed order, the contributions of
 // the (up to) four elements above it and the four below it (carried in registers from the previous layer),
 // and is finished: written to y through the epilogue, unless it lies on the ring of the column (shared with
@@ -23,122 +22,132 @@
 // axes orthogonal to k, in increasing order
 __host__ __device__ constexpr int P1(int k) { return k == 0 ? 1 : 0; }
 __host__ __device__ constexpr int P2(int k) { return k == 2 ? 1 : 2; }
-__host__ __device__ constexpr int bit_on(int axis, int k, int bk, int b1, int b2) {
-    return axis == k ? bk : (axis == P1(k) ? b1 : b2);
-}
-// vertex index a = bx + 2 by + 4 bz with bit bk on axis k and (b1, b2) on the orthogonal axes
-__host__ __device__ constexpr int node3(int k, int bk, int b1, int b2) {
-    return bit_on(0, k, bk, b1, b2) + 2 * bit_on(1, k, bk, b1, b2) + 4 * bit_on(2, k, bk, b1, b2);
-}
+__host__ __device__ constexpr int pow3(int k) { return k == 0 ? 1 : (k == 1 ? 3 : 9); }
 
-// 2x2 vertex values -> 3x3 Lagrange points {-1, 0, 1}^2 (bilinear interpolation)
+// ------------------------------------------------------------------------------------------
+// Element action y = K_e u in 3D, in monomials.  A velocity component is trilinear, u_i = sum c_i[m] xi^m over the
+// 8 exponents m in {0,1}^3 (a bit mask, bit 0 for x); its gradients are bilinear with the same coefficients,
+//   d u_i / d x_k = s_k sum_{m has bit k} c_i[m] xi^(m without k),
+// and the vertex functions tested with are trilinear in the same way.  The particle sums therefore enter through the 27
+// moments M[a,b,c] = sum_q W_q xi_q^a eta_q^b zeta_q^c, a, b, c <= 2, which three passes of sums and differences make from
+// the weights at {-1,0,1}^3: a normal strain meets its 4 test functions in a symmetric 4 x 4 product of moments, a shear
+// strain (6 monomials, shared by its two test functions) in a symmetric 6 x 6 one.  Per element 81 operations for the
+// moments, 81 and 66 to and from the coefficients, 72 scalings, 156 multiply-adds: 456, where interpolating gradients to
+// and stresses from the 27 points took about 750.
+// ------------------------------------------------------------------------------------------
+// weights at {-1, 0, 1}^3 -> moments, in place
 template <typename T>
-__device__ __forceinline__ void interp22(const T D[2][2], T G[3][3]) {
-    const T h = (T)0.5;
-    G[0][0] = D[0][0];
-    G[0][2] = D[0][1];
-    G[2][0] = D[1][0];
-    G[2][2] = D[1][1];
-    G[1][0] = h * (D[0][0] + D[1][0]);
-    G[1][2] = h * (D[0][1] + D[1][1]);
-    G[0][1] = h * (D[0][0] + D[0][1]);
-    G[2][1] = h * (D[1][0] + D[1][1]);
-    G[1][1] = (T)0.25 * (D[0][0] + D[0][1] + D[1][0] + D[1][1]);
-}
-
-// transpose of interp22
-template <typename T>
-__device__ __forceinline__ void interp22T(const T R[3][3], T O[2][2]) {
-    const T h = (T)0.5, c = (T)0.25 * R[1][1];
-    O[0][0] = R[0][0] + h * (R[1][0] + R[0][1]) + c;
-    O[1][0] = R[2][0] + h * (R[1][0] + R[2][1]) + c;
-    O[0][1] = R[0][2] + h * (R[0][1] + R[1][2]) + c;
-    O[1][1] = R[2][2] + h * (R[2][1] + R[1][2]) + c;
-}
-
-// physical gradient d u_i / d x_k at the 9 points orthogonal to k (constant along k):
-// gp[q1][q2] = (s_k / 2) * interp22(u(k=1) - u(k=0))
-template <typename T, int I, int K, typename U>
-__device__ __forceinline__ void grad3(const U &u, T sk, T gp[3][3]) {
-    T D[2][2];
+__device__ __forceinline__ void moments3(T M[27]) {
 #pragma unroll
-    for (int b1 = 0; b1 < 2; b1++)
+    for (int k = 0; k < 3; k++)
 #pragma unroll
-        for (int b2 = 0; b2 < 2; b2++)
-            D[b1][b2] = (T)0.5 * sk * (u(node3(K, 1, b1, b2), I) - u(node3(K, 0, b1, b2), I));
-    interp22<T>(D, gp);
-}
-
-// y[.][I] += (s_K/2) sgn(a_K) interp22T(R)  for derivative direction K
-template <typename T, int I, int K>
-__device__ __forceinline__ void scatter3(const T R[3][3], T sk, T y[8][3]) {
-    T O[2][2];
-    interp22T<T>(R, O);
-#pragma unroll
-    for (int b1 = 0; b1 < 2; b1++)
-#pragma unroll
-        for (int b2 = 0; b2 < 2; b2++) {
-            const T v = (T)0.5 * sk * O[b1][b2];
-            y[node3(K, 1, b1, b2)][I] += v;
-            y[node3(K, 0, b1, b2)][I] -= v;
+        for (int l = 0; l < 9; l++) {
+            const int i = (l % 3) * pow3(P1(k)) + (l / 3) * pow3(P2(k)), d = pow3(k);
+            const T t = M[i] + M[i + 2 * d], df = M[i + 2 * d] - M[i];
+            M[i] = t + M[i + d];
+            M[i + d] = df;
+            M[i + 2 * d] = t;
         }
 }
 
+// 8 times the coefficients of component I (index: the bit mask; [0] is not needed).  Differences are taken before sums,
+// so a smooth field loses no digits to its mean.
 template <typename T, int I, typename U>
-__device__ __forceinline__ void diag3(const U &u, const T W[27], const T s[3], T y[8][3]) {
-    T gp[3][3], R[3][3];
-    grad3<T, I, I>(u, s[I], gp);
+__device__ __forceinline__ void coefficients3(const U &u, T c[8]) {
+    T v[8];
 #pragma unroll
-    for (int q1 = 0; q1 < 3; q1++)
-#pragma unroll
-        for (int q2 = 0; q2 < 3; q2++) {
-            T ws = (T)0;
-#pragma unroll
-            for (int qk = 0; qk < 3; qk++) {
-                int qs[3];
-                qs[I] = qk;
-                qs[P1(I)] = q1;
-                qs[P2(I)] = q2;
-                ws += W[qs[0] + 3 * qs[1] + 9 * qs[2]];
-            }
-            R[q1][q2] = (T)2 * gp[q1][q2] * ws;
-        }
-    scatter3<T, I, I>(R, s[I], y);
+    for (int a = 0; a < 8; a++) v[a] = u(a, I);
+    const T x0 = v[1] - v[0], x1 = v[3] - v[2], x2 = v[5] - v[4], x3 = v[7] - v[6];  // along x at (y, z)
+    const T p0 = x0 + x1, p1 = x2 + x3, m0 = x1 - x0, m1 = x3 - x2;
+    c[1] = p0 + p1;
+    c[5] = p1 - p0;
+    c[3] = m0 + m1;
+    c[7] = m1 - m0;
+    const T y0 = (v[2] - v[0]) + (v[3] - v[1]), y1 = (v[6] - v[4]) + (v[7] - v[5]);  // along y, summed over x
+    c[2] = y0 + y1;
+    c[6] = y1 - y0;
+    c[4] = ((v[4] - v[0]) + (v[5] - v[1])) + ((v[6] - v[2]) + (v[7] - v[3]));
 }
 
-template <typename T, int I, int K, typename U>
-__device__ __forceinline__ void pair3(const U &u, const T W[27], const T s[3], T y[8][3]) {
-    T gik[3][3], gki[3][3], Rik[3][3], Rki[3][3];
-    grad3<T, I, K>(u, s[K], gik);  // d u_I / d x_K : indexed by the axes orthogonal to K
-    grad3<T, K, I>(u, s[I], gki);  // d u_K / d x_I : indexed by the axes orthogonal to I
+// the transpose: y[a][I] = sum over the masks of z times the vertex's signs
+template <typename T, int I>
+__device__ __forceinline__ void vertices3(const T z[8], T y[8][3]) {
+    const T p0 = z[1] + z[3], m0 = z[1] - z[3], p1 = z[5] + z[7], m1 = z[5] - z[7];
+    const T f0 = z[2] - z[6], f1 = z[2] + z[6];
+    // x part e and the rest h at (y, z)
+    const T e[4] = {m0 - m1, p0 - p1, m0 + m1, p0 + p1};
+    const T h[4] = {-f0 - z[4], f0 - z[4], z[4] - f1, f1 + z[4]};
 #pragma unroll
-    for (int a = 0; a < 3; a++)
-#pragma unroll
-        for (int b = 0; b < 3; b++) {
-            Rik[a][b] = (T)0;
-            Rki[a][b] = (T)0;
-        }
-#pragma unroll
-    for (int q = 0; q < 27; q++) {
-        const int qs[3] = {q % 3, (q / 3) % 3, q / 9};
-        const T t = W[q] * (gik[qs[P1(K)]][qs[P2(K)]] + gki[qs[P1(I)]][qs[P2(I)]]);
-        Rik[qs[P1(K)]][qs[P2(K)]] += t;
-        Rki[qs[P1(I)]][qs[P2(I)]] += t;
+    for (int b = 0; b < 4; b++) {
+        y[2 * b][I] = h[b] - e[b];
+        y[2 * b + 1][I] = h[b] + e[b];
     }
-    scatter3<T, I, K>(Rik, s[K], y);
-    scatter3<T, K, I>(Rki, s[I], y);
 }
 
-// u(a, i): component i of the element's vertex a (read where needed, so that the velocities need not all be
-// held in registers at once)
+// stress of the normal strain I against its test functions
+template <typename T, int I>
+__device__ __forceinline__ void normal3(const T c[3][8], const T M[27], const T s[3], T z[3][8]) {
+    T g[4];
+#pragma unroll
+    for (int m = 0; m < 4; m++) g[m] = (T)2 * s[I] * c[I][(1 << I) | (m & 1) << P1(I) | (m >> 1) << P2(I)];
+#pragma unroll
+    for (int n = 0; n < 4; n++) {
+        T r = (T)0;
+#pragma unroll
+        for (int m = 0; m < 4; m++)
+            r += M[((m & 1) + (n & 1)) * pow3(P1(I)) + ((m >> 1) + (n >> 1)) * pow3(P2(I))] * g[m];
+        z[I][(1 << I) | (n & 1) << P1(I) | (n >> 1) << P2(I)] += s[I] * r;
+    }
+}
+
+// stress of the shear strain d u_I / d x_K + d u_K / d x_I: monomials {1, xi_I, xi_K} x {1, xi_J}
+template <typename T, int I, int K>
+__device__ __forceinline__ void shear3(const T c[3][8], const T M[27], const T s[3], T z[3][8]) {
+    constexpr int J = 3 - I - K;
+    T t[3][2];
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        t[0][j] = s[K] * c[I][(1 << K) | j << J] + s[I] * c[K][(1 << I) | j << J];
+        t[1][j] = s[K] * c[I][(1 << K) | (1 << I) | j << J];
+        t[2][j] = s[I] * c[K][(1 << I) | (1 << K) | j << J];
+    }
+#pragma unroll
+    for (int n = 0; n < 3; n++)
+#pragma unroll
+        for (int l = 0; l < 2; l++) {
+            T r = (T)0;
+#pragma unroll
+            for (int m = 0; m < 3; m++)
+#pragma unroll
+                for (int j = 0; j < 2; j++)
+                    r += M[((m == 1) + (n == 1)) * pow3(I) + ((m == 2) + (n == 2)) * pow3(K) + (j + l) * pow3(J)] * t[m][j];
+            if (n != 2) z[I][(1 << K) | (n == 1) << I | l << J] += s[K] * r;
+            if (n != 1) z[K][(1 << I) | (n == 2) << K | l << J] += s[I] * r;
+        }
+}
+
+// u(a, i): component i of the element's vertex a; W: the element's weights (made into its moments); s: 2 / h
 template <typename T, typename U>
-__device__ __forceinline__ void element_apply3(const U &u, const T W[27], const T s[3], T y[8][3]) {
-    diag3<T, 0>(u, W, s, y);
-    diag3<T, 1>(u, W, s, y);
-    diag3<T, 2>(u, W, s, y);
-    pair3<T, 0, 1>(u, W, s, y);
-    pair3<T, 0, 2>(u, W, s, y);
-    pair3<T, 1, 2>(u, W, s, y);
+__device__ __forceinline__ void element_apply3(const U &u, T W[27], const T h2[3], T y[8][3]) {
+    T c[3][8], z[3][8];
+    const T s[3] = {(T)0.125 * h2[0], (T)0.125 * h2[1], (T)0.125 * h2[2]};
+    coefficients3<T, 0>(u, c[0]);
+    coefficients3<T, 1>(u, c[1]);
+    coefficients3<T, 2>(u, c[2]);
+    moments3<T>(W);
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int m = 0; m < 8; m++) z[i][m] = (T)0;
+    normal3<T, 0>(c, W, s, z);
+    normal3<T, 1>(c, W, s, z);
+    normal3<T, 2>(c, W, s, z);
+    shear3<T, 0, 1>(c, W, s, z);
+    shear3<T, 0, 2>(c, W, s, z);
+    shear3<T, 1, 2>(c, W, s, z);
+    vertices3<T, 0>(z[0], y);
+    vertices3<T, 1>(z[1], y);
+    vertices3<T, 2>(z[2], y);
 }
 
 // ---------------------------------------- 2D ----------------------------------------------
@@ -357,7 +366,7 @@ __global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(
     static_assert(NCP <= UST_TILE, "one coarse value per thread");
     __shared__ T sc[MODE == EPI_PCHEBY0 ? 2 * NCP : 1];
     const int ntxy = g.tnx * g.tny;
-    const int tile = blockIdx.x;
+    const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int txy = tile % ntxy, chunk = tile / ntxy;
     const int x0 = (txy % g.tnx) * UST_TX3, y0 = (txy / g.tnx) * UST_TY3;
     const int z0 = chunk * g.tz, z1 = min(z0 + g.tz, g.nz);
@@ -518,10 +527,6 @@ __global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(
                 for (int q = 0; q < 27; q++) wq[q] = wload<T, WT>(W, wbase + ((size_t)k * 27 + q) * UST_TILE);
             }
             T ye[8][3];
-#pragma unroll
-            for (int a = 0; a < 8; a++)
-#pragma unroll
-                for (int i = 0; i < 3; i++) ye[a][i] = (T)0;
             const T *sb = &su[cur][(lx + CPX * ly) * 3], *st = &su[nxt][(lx + CPX * ly) * 3];
             auto ue = [&](int a, int i) -> T {
                 return (a >> 2 ? st : sb)[((a & 1) + CPX * ((a >> 1) & 1)) * 3 + i];
@@ -589,7 +594,7 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, const WT *_
     constexpr int CX = TX / 2 + 1, CY = TY / 2 + 1, CZ = TZ / 2 + 1, NC = CX * CY * CZ * 3;
     static_assert(NC <= UST_TILE, "one coarse value per thread");
     __shared__ T sc[MODE == EPI_PCHEBY0 ? NC : 1];
-    const int tile = blockIdx.x;
+    const int tile = xcd_block(blockIdx.x, gridDim.x);
     const int tx0 = (tile % g.tnx) * TX, ty0 = ((tile / g.tnx) % g.tny) * TY, tz0 = (tile / (g.tnx * g.tny)) * TZ;
     T cv = (T)0;
     if (MODE == EPI_PCHEBY0) {
@@ -664,10 +669,7 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, const WT *_
         for (int a = 0; a < 8; a++) {
             const int ln = (lx + (a & 1)) + NX * ((ly + ((a >> 1) & 1)) + NY * (lz + (a >> 2)));
 #pragma unroll
-            for (int i = 0; i < 3; i++) {
-                ue[a][i] = su[ln * 3 + i];
-                ye[a][i] = (T)0;
-            }
+            for (int i = 0; i < 3; i++) ue[a][i] = su[ln * 3 + i];
         }
         const T s[3] = {(T)(2.0 / g.hx), (T)(2.0 / g.hy), (T)(2.0 / g.hz)};
         element_apply3<T>([&](int a, int i) -> T { return ue[a][i]; }, wq, s, ye);
@@ -746,7 +748,7 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
     __shared__ T su[HNN * 3];   // staged node block, origin (nx0 - 1, ny0 - 1, nz0 - 1)
     __shared__ T eb[24 * HNE];  // element results: eb[(a*3 + i) * HNE + slot] (HNE odd: rows shift banks)
     const int hnx = (g.nnx + HOX - 1) / HOX, hny = (g.nny + HOY - 1) / HOY;
-    const int tile = blockIdx.x, tid = threadIdx.x;
+    const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
     const int nx0 = (tile % hnx) * HOX, ny0 = ((tile / hnx) % hny) * HOY, nz0 = (tile / (hnx * hny)) * HOZ;
     const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1;  // EPI_PCHEBY0: the coarse grid
     // staging: value t of the block is node n = t / 3, component c = t % 3; nodes outside the grid stage 0
@@ -791,10 +793,6 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
     __syncthreads();
     if (tid < HNE) {
         T ye[8][3];
-#pragma unroll
-        for (int a = 0; a < 8; a++)
-#pragma unroll
-            for (int i = 0; i < 3; i++) ye[a][i] = (T)0;
         const T s[3] = {(T)(2.0 / g.hx), (T)(2.0 / g.hy), (T)(2.0 / g.hz)};
         const T *sb = &su[(lx + HNX * (ly + HNY * lz)) * 3];
         element_apply3<T>([&](int a, int i) -> T {

@@ -154,6 +154,14 @@ static inline GridDev grid_dev(const ust_grid *g, long long wg_target = UST_COL_
     return d;
 }
 
+// Workgroups go to the 8 XCDs in turn, and each XCD has its own L2.  xcd_block turns the block index into a position such
+// that one XCD takes a contiguous run of positions, so tiles that share nodes and cache lines share an L2.
+#define UST_XCDS 8
+__device__ __forceinline__ int xcd_block(int b, int n) {
+    const int x = b % UST_XCDS, q = n / UST_XCDS, r = n % UST_XCDS;
+    return x * q + (x < r ? x : r) + b / UST_XCDS;
+}
+
 // A wavefront's own LDS: its LDS operations complete in order, so a wave-level barrier (no compiler reordering across
 // it) is all that one wave needs between its lanes' writes and reads of each other's values.
 __device__ __forceinline__ void wave_sync() {

@@ -586,3 +586,30 @@ def test_column_kernel_against_element_reference(nel):
             a.free()
     for a in [dm, W64, W32, W16, work, du] + ([W16f] if W16f else []):
         a.free()
+
+
+@pytest.mark.parametrize("nel", [(17, 9, 5), (40, 30, 20), (80, 70, 60)])
+def test_fp32_product_of_a_field_with_a_large_mean(nel):
+    """The FP32 product (halo, tile and column kernels) of u = 1000 + N(0, 1) against FP64 on the same floats.  Velocity
+    differences of neighbours are exact in FP32 here, so with differences taken before sums each element's result
+    carries about 60 roundings of its own size, 60 x 6e-8 = 4e-6; sums taken first would round the mean away: 1e-4."""
+    import ctypes as C
+    import earthbyte_underworld_amd as ust  # noqa: F401  (loads the library)
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    g = _grid(3, nel)
+    n = int(np.prod([k + 1 for k in nel])) * 3
+    wl = lib.ust_k_weights_len(C.byref(g))
+    rng = np.random.default_rng(4)
+    W = rng.uniform(0.1, 1.0, wl).astype(np.float32)
+    u = (1000.0 + rng.normal(size=n)).astype(np.float32)
+    W32, W64 = _Dev(lib, W), _Dev(lib, W.astype(np.float64))
+    dm, d32, d64 = _Dev(lib, np.zeros(n, np.uint8)), _Dev(lib, u), _Dev(lib, u.astype(np.float64))
+    y32, y64 = _Dev(lib, np.zeros(n, np.float32)), _Dev(lib, np.zeros(n))
+    work = _Dev(lib, np.zeros(lib.ust_k_apply_work_len(C.byref(g))))
+    assert lib.ust_k_apply_K_f32(C.byref(g), W32.p, dm.p, d32.p, y32.p, work.p, None) == 0
+    a = y32.get().astype(np.float64)
+    assert lib.ust_k_apply_K_f64(C.byref(g), W64.p, dm.p, d64.p, y64.p, work.p, None) == 0
+    assert rel_err(a, y64.get()) < 4e-6
+    for x in (W32, W64, dm, d32, d64, y32, y64, work):
+        x.free()
