@@ -24,26 +24,82 @@ struct YieldDev {
     double softening_strain, healing_rate;
 };
 
+// Q1 interpolation at the local coordinates xi, one axis after the other (a difference and one multiply-add per pair: a
+// third of the operations of summing shape functions, and few values live at once).  v(a): the value at vertex a.
+template <int DIM, typename V>
+__device__ __forceinline__ double q1_value(const double *xi, V v) {
+    const double fx = 0.5 * (1.0 + xi[0]), fy = 0.5 * (1.0 + xi[1]);
+    double z[2] = {0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < (DIM == 3 ? 2 : 1); c++) {
+        const double u0 = v(4 * c), u1 = v(4 * c + 1), u2 = v(4 * c + 2), u3 = v(4 * c + 3);
+        const double m0 = u0 + fx * (u1 - u0), m1 = u2 + fx * (u3 - u2);
+        z[c] = m0 + fy * (m1 - m0);
+    }
+    return DIM == 3 ? z[0] + 0.5 * (1.0 + xi[2]) * (z[1] - z[0]) : z[0];
+}
+// and its derivatives g along the element's axes over [0, 1]
+template <int DIM, typename V>
+__device__ __forceinline__ void q1_gradient(const double *xi, V v, double *g) {
+    const double fx = 0.5 * (1.0 + xi[0]), fy = 0.5 * (1.0 + xi[1]);
+    double gx[2] = {0.0, 0.0}, gy[2] = {0.0, 0.0}, z[2] = {0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < (DIM == 3 ? 2 : 1); c++) {
+        const double u0 = v(4 * c), u1 = v(4 * c + 1), u2 = v(4 * c + 2), u3 = v(4 * c + 3);
+        const double d0 = u1 - u0, d1 = u3 - u2, m0 = u0 + fx * d0, m1 = u2 + fx * d1;
+        gx[c] = d0 + fy * (d1 - d0);
+        gy[c] = m1 - m0;
+        z[c] = m0 + fy * gy[c];
+    }
+    const double fz = DIM == 3 ? 0.5 * (1.0 + xi[2]) : 0.0;
+    g[0] = DIM == 3 ? gx[0] + fz * (gx[1] - gx[0]) : gx[0];
+    g[1] = DIM == 3 ? gy[0] + fz * (gy[1] - gy[0]) : gy[0];
+    if (DIM == 3) g[2] = z[1] - z[0];
+}
+
+// nodal values around an element: the values of vertex a start NC doubles per node after those of its first node.  Four row
+// pointers and immediate offsets: the loads need no address of their own.
+template <int DIM, int NC>
+struct VertexRows {
+    const double *r[DIM == 3 ? 4 : 2];
+    __device__ __forceinline__ VertexRows(const GridDev &g, const double *v, size_t n0) {
+        r[0] = v + n0 * NC;
+        r[1] = r[0] + (size_t)g.nnx * NC;
+        if (DIM == 3) {
+            r[2] = r[0] + (size_t)g.nnx * g.nny * NC;
+            r[3] = r[2] + (size_t)g.nnx * NC;
+        }
+    }
+    __device__ __forceinline__ double operator()(int a, int c) const { return r[a >> 1][(a & 1) * NC + c]; }
+};
+
+// what DruckerPrager takes from its friction angle: criterion = k p + 6 C cosphi f in 3D, k p + C cosphi in 2D
+struct FrictionDev {
+    double k, cosphi, f;
+};
+template <int DIM>
+__device__ __forceinline__ FrictionDev friction_of(double friction) {
+    const double phi = atan(friction), sinphi = sin(phi);
+    FrictionDev d;
+    d.cosphi = cos(phi);
+    d.f = DIM == 3 ? 1.0 / (sqrt(3.0) * (3.0 - sinphi)) : 1.0;
+    d.k = DIM == 3 ? 6.0 * sinphi * d.f : sinphi;
+    return d;
+}
+
+// fric: friction_of the unsoftened coefficient of each of the material's rheologies
 template <int DIM, bool NEED_T, bool NEED_VEL, bool SW>
-__device__ double particle_viscosity(const GridDev &g, const ust_material &M, const int *nodes, const double *xi,
-                                     const double *T, const double *vel, const double *pres, int e, float coh,
-                                     int prev, const YieldDev &ys, int pi, int *yflag) {
-    constexpr int NV = 1 << DIM;
+__device__ double particle_viscosity(const GridDev &g, const ust_material &M, const FrictionDev *fric, size_t n0,
+                                     const double *xi, const double *T, const double *vel, const double *pres, int e,
+                                     float coh, int prev, const YieldDev &ys, int pi, int *yflag) {
     double eta = 0.0;
     for (int r = 0; r < M.nrh; r++) {
         const ust_rheology &rh = M.rh[r];
         if (rh.type == UST_RH_MATERIALVISCOSITY) {
             eta = rh.p[0];
         } else if (NEED_T && rh.type == UST_RH_ARRHENIUS) {
-            double Tp = 0.0, y = 0.0;
-#pragma unroll
-            for (int a = 0; a < NV; a++) {
-                double N = 1.0;
-#pragma unroll
-                for (int d = 0; d < DIM; d++) N *= 0.5 * (1.0 + sgn((a >> d) & 1) * xi[d]);
-                Tp += N * T[nodes[a]];
-                y += N * ((a >> 1) & 1);
-            }
+            const VertexRows<DIM, 1> tv(g, T, n0);
+            const double Tp = q1_value<DIM>(xi, [&](int a) { return tv(a, 0); }), y = 0.5 * (1.0 + xi[1]);
             if (rh.p[2] > (0.0 + 1e-12)) {
                 // y(xi) on a rectilinear element: ymin + (j + local fraction) * hy
                 int j = (e / g.nx) % g.ny;
@@ -61,26 +117,17 @@ __device__ double particle_viscosity(const GridDev &g, const ust_material &M, co
             const double minVisc = dp ? rh.p[3] : rh.p[1];
             const int srSoft = (int)(dp ? rh.p[4] : rh.p[2]);
             if (!prev) continue;
-            // velocity gradient at xi: L[i][k] = sum_a GNx[k][a] u[a][i]
+            // velocity gradient at xi: L[i][k] = d u_i / d x_k
             double L[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
-            const double s[3] = {2.0 / g.hx, 2.0 / g.hy, 2.0 / g.hz};
+            const double rh3[3] = {1.0 / g.hx, 1.0 / g.hy, 1.0 / g.hz};
+            const VertexRows<DIM, DIM> uv(g, vel, n0);
 #pragma unroll
-            for (int a = 0; a < NV; a++) {
-                double dN[3];
+            for (int i = 0; i < DIM; i++) {
+                q1_gradient<DIM>(xi, [&](int a) { return uv(a, i); }, L[i]);
 #pragma unroll
-                for (int k = 0; k < DIM; k++) {
-                    double v = 0.5 * sgn((a >> k) & 1);
-#pragma unroll
-                    for (int d = 0; d < DIM; d++)
-                        if (d != k) v *= 0.5 * (1.0 + sgn((a >> d) & 1) * xi[d]);
-                    dN[k] = s[k] * v;
-                }
-#pragma unroll
-                for (int i = 0; i < DIM; i++) {
-                    double ui = vel[(size_t)nodes[a] * DIM + i];
-#pragma unroll
-                    for (int k = 0; k < DIM; k++) L[i][k] += dN[k] * ui;
-                }
+                for (int k = 0; k < DIM; k++) L[i][k] *= rh3[k];
+                // 3D: a component's 8 values at a time (all 24 at once cost a wave per SIMD)
+                if (DIM == 3) asm volatile("" ::: "memory");
             }
             double inv;
             if (DIM == 3) {
@@ -112,17 +159,9 @@ __device__ double particle_viscosity(const GridDev &g, const ust_material &M, co
             if (!dp) {
                 criterion = cohesion;
             } else {
-                const double friction = rh.p[1] * (1.0 - ratio) + rh.p[6] * ratio;
-                double pressure = pres[e], phi = atan(friction), k, c;
-                if (DIM == 3) {
-                    double sinphi = sin(phi), oneOver = 1.0 / (sqrt(3.0) * (3.0 - sinphi));
-                    k = 6.0 * sinphi * oneOver;
-                    c = 6.0 * cohesion * cos(phi) * oneOver;
-                } else {
-                    c = cohesion * cos(phi);
-                    k = sin(phi);
-                }
-                criterion = k * pressure + c;
+                const FrictionDev fr = sw ? friction_of<DIM>(rh.p[1] * (1.0 - ratio) + rh.p[6] * ratio) : fric[r];
+                const double c = DIM == 3 ? 6.0 * cohesion * fr.cosphi * fr.f : cohesion * fr.cosphi;
+                criterion = fr.k * pres[e] + c;
                 if (ys.tensile) ys.tensile[pi] = criterion <= 0.0;
                 if (criterion < rh.p[2]) criterion = rh.p[2];
             }
@@ -186,23 +225,21 @@ __device__ __forceinline__ double hydrostatic_density(const ust_buoyancy &b, dou
 }
 
 template <int DIM, bool NEED_T>
-__device__ double particle_density(const GridDev &g, const BuoyDev &bd, const ust_material &M, const int *nodes,
+__device__ double particle_density(const GridDev &g, const BuoyDev &bd, const ust_material &M, size_t n0,
                                    const double *xi, const double *T, int e) {
     if (!bd.full) return M.density;
     const int idx[3] = {e % g.nx, (e / g.nx) % g.ny, e / (g.nx * g.ny)};
     const double mn[3] = {g.xmin, g.ymin, g.zmin}, h[3] = {g.hx, g.hy, g.hz};
     const int va = bd.b.vertical_axis;
-    const double cv = mn[va] + ((double)idx[va] + 0.5 * (xi[va] + 1.0)) * h[va];
+    double cv = 0.0;
+#pragma unroll
+    for (int d = 0; d < DIM; d++)  // no indexing by va: the arrays stay in registers
+        if (d == va) cv = mn[d] + ((double)idx[d] + 0.5 * (xi[d] + 1.0)) * h[d];
     const double depth = fabs(bd.top - cv);
     double temperature = 0.0;
     if (NEED_T) {
-#pragma unroll
-        for (int a = 0; a < (1 << DIM); a++) {
-            double N = 1.0;
-#pragma unroll
-            for (int d = 0; d < DIM; d++) N *= 0.5 * (1.0 + sgn((a >> d) & 1) * xi[d]);
-            temperature += N * T[nodes[a]];
-        }
+        const VertexRows<DIM, 1> tv(g, T, n0);
+        temperature = q1_value<DIM>(xi, [&](int a) { return tv(a, 0); });
     }
     double background = 0.0;
     if (bd.b.hydrostatic) background = hydrostatic_density(bd.b, mn[1] + ((double)idx[1] + 0.5 * (xi[1] + 1.0)) * h[1]);
@@ -212,165 +249,260 @@ __device__ double particle_density(const GridDev &g, const BuoyDev &bd, const us
 }
 
 // ------------------------------------------------------------------------------------------
-// One particle's contributions to its element's 43 (3D) weight sums: the Lagrange weights of K
-// (w detJ eta L_q), the vertex weights of G (w detJ N_b) and of f (w detJ rho N_b).  Shared by both
-// particle-weight kernels; the viscosity and yield flag go to eta_out / yield_out.
+// particles -> weights on the matrix cores.  An element's sums are products over its particles,
+//   WK[qx,qy,qz] = sum_p (Lx Ly)_p[qx,qy] (w detJ eta Lz)_p[qz],   WG, WF[bx,by,bz] = sum_p (Nx Ny)_p (w detJ {1, rho} Nz)_p,
+// which are exactly the four 4 x 4 blocks of v_mfma_f64_4x4x4_4b: blocks 0-2 hold the 9 x 3 products of WK, block 3 the
+// 4 x 4 of WG and WF; a step takes 4 particles.  (2D: two blocks, 3 x 3 and 2 x 4, twice, so a step takes 8.)  A wave owns
+// `epw` consecutive elements and reads their particles 64 at a time, one per lane: rheology, density and the 20 (2D: 12)
+// factors, left in the wave's LDS (32 particles, then the other 32: LDS sets the waves in flight), where the matrix steps
+// read one factor of each side per lane.  The next 64 particles are loaded while the matrix steps run.  A lane ends with
+// one of the element's 43 sums, so nothing is reduced; the sums of 8 elements are written together, in 64-byte runs.
+//
+// Bound: latency, with 16 waves per CU for plain rheology (LDS) and 8 where stresses are looked up (registers: 207 in 3D).
+// 21 M particles on 128x128x64, 61 materials: 842 -> 400 us (1.2 GB, 3 TB/s) against lanes that accumulate the 43 sums in
+// registers and reduce them through LDS, 8 waves per CU.  Arrhenius + DruckerPrager with cohesion noise, 4.6 M particles
+// on 95x51x47: 685 -> 280 us; 3.3 M on 512x256: 228 -> 105 us (the friction terms once per material; 3 waves per SIMD for
+// the 3D one, with 20 to 27 spilled registers, were slower: 437 against 392 us for the whole assembly).
+//
+// NEED_T / NEED_VEL / SW compile the temperature and strain-rate lookups (Arrhenius, yield) and the strain-weakening state
+// in only when a material uses them.  Without them a material's chain is one number, taken once per workgroup.
 // ------------------------------------------------------------------------------------------
+#define PW_EPW 16
+// waves wanted before a wave takes more elements: 2,048 and 32,768 measured the same within 1%
+#define PW_MIN_WAVES 8192
+// waves per workgroup (with lookups the material table, up to 28 KB, goes beside them into 64 KB of LDS) and the waves per
+// SIMD the register budget must allow
+__host__ __device__ constexpr int pw_waves(bool lookups) { return lookups ? 2 : 4; }
+__host__ __device__ constexpr int pw_minb(bool lookups) { return lookups ? 2 : 4; }
+__host__ __device__ constexpr int pw_factors(int dim) { return dim == 3 ? 20 : 12; }
+// doubles between the rows of two particles: odd, so that the lanes' row writes spread over the LDS banks
+__host__ __device__ constexpr int pw_row(int dim) { return pw_factors(dim) + 1; }
+constexpr int PW_HALF = 32, PW_OUT = 8;
+__host__ __device__ constexpr int pw_sums(int dim) { return dim == 3 ? 43 : 17; }
+// doubles of one wave's LDS: the factors of PW_HALF particles, a row of zeros, and the sums of PW_OUT elements
+__host__ __device__ constexpr int pw_wave_lds(int dim) { return (PW_HALF + 1) * pw_row(dim) + pw_sums(dim) * (PW_OUT + 1); }
+// bytes of the per-workgroup material table
+__host__ __device__ constexpr size_t pw_table(bool lookups, int nmat) {
+    return lookups ? (size_t)nmat * (sizeof(ust_material) + UST_MAX_RHEOLOGIES * sizeof(FrictionDev))
+                   : (size_t)nmat * 2 * sizeof(double);
+}
+
+struct ParticleArrays {
+    const double *xi0, *xi1, *xi2, *w;
+    const unsigned char *mat;
+    const float *coh;
+};
+template <int DIM>
+struct ParticleIn {
+    double x[3], w;
+    int m;
+    float coh;
+    __device__ __forceinline__ void load(const ParticleArrays &a, int p, int nmat) {
+        x[0] = a.xi0[p];
+        x[1] = a.xi1[p];
+        x[2] = DIM == 3 ? a.xi2[p] : 0.0;
+        w = a.w[p];
+        m = a.mat ? (int)a.mat[p] : 0;
+        m = m < nmat ? m : 0;
+        coh = a.coh ? a.coh[p] : 1.0f;
+    }
+};
+
 template <int DIM, bool NEED_T, bool NEED_VEL, bool SW>
-__device__ __forceinline__ void particle_contrib(
-    const GridDev &g, int e, int pi, const int *nodes, double detJ, const double *__restrict__ xi0,
-    const double *__restrict__ xi1, const double *__restrict__ xi2, const double *__restrict__ w,
-    const unsigned char *__restrict__ mat, const float *__restrict__ coh, const ust_material *__restrict__ mats,
-    int nmat, const double *__restrict__ T, const double *__restrict__ vel, const double *__restrict__ pres, int prev,
-    const YieldDev &ys, const BuoyDev &bd, double *__restrict__ eta_out, unsigned char *__restrict__ yield_out,
-    double *acc) {
-    constexpr int NQ = DIM == 3 ? 27 : 9;
-    constexpr int NV = 1 << DIM;
-    double xi[3];
-    xi[0] = xi0[pi];
-    xi[1] = xi1[pi];
-    xi[2] = DIM == 3 ? xi2[pi] : 0.0;
-    const int m = mat ? (int)mat[pi] : 0;
-    const ust_material &M = mats[m < nmat ? m : 0];
-    int yf = -1;
-    const double eta = particle_viscosity<DIM, NEED_T, NEED_VEL, SW>(g, M, nodes, xi, T, vel, pres, e,
-                                                                 coh ? coh[pi] : 1.0f, prev, ys, pi, &yf);
-    if (eta_out) eta_out[pi] = eta;
-    if (NEED_VEL && yield_out && yf >= 0) yield_out[pi] = (unsigned char)yf;
-    const double wd = w[pi] * detJ;
-    const double et = wd * eta;
-    const double wr = wd * particle_density<DIM, NEED_T>(g, bd, M, nodes, xi, T, e);
-    double Lx[3], Ly[3], Lz[3];
-    lagrange3(xi[0], Lx);
-    lagrange3(xi[1], Ly);
-    if (DIM == 3) lagrange3(xi[2], Lz);
-#pragma unroll
-    for (int qz = 0; qz < (DIM == 3 ? 3 : 1); qz++)
-#pragma unroll
-        for (int qy = 0; qy < 3; qy++) {
-            const double eyz = et * Ly[qy] * (DIM == 3 ? Lz[qz] : 1.0);
-#pragma unroll
-            for (int qx = 0; qx < 3; qx++) acc[qx + 3 * qy + 9 * qz] += eyz * Lx[qx];
-        }
-    const double Nx[2] = {0.5 * (1.0 - xi[0]), 0.5 * (1.0 + xi[0])};
-    const double Ny[2] = {0.5 * (1.0 - xi[1]), 0.5 * (1.0 + xi[1])};
-    const double Nz[2] = {0.5 * (1.0 - xi[2]), 0.5 * (1.0 + xi[2])};
-#pragma unroll
-    for (int b = 0; b < NV; b++) {
-        double N = Nx[b & 1] * Ny[(b >> 1) & 1];
-        if (DIM == 3) N *= Nz[(b >> 2) & 1];
-        acc[NQ + b] += wd * N;
-        acc[NQ + NV + b] += wr * N;
-    }
-}
-
-__device__ __forceinline__ void element_nodes_of(const GridDev &g, int ie, int je, int ke, int dim, int *nodes) {
-    const int n0 = ie + g.nnx * (je + g.nny * ke);
-    for (int a = 0; a < (1 << dim); a++)
-        nodes[a] = n0 + (a & 1) + g.nnx * ((a >> 1) & 1) + (dim == 3 ? g.nnx * g.nny * ((a >> 2) & 1) : 0);
-}
-
-// ------------------------------------------------------------------------------------------
-// particles -> weights.  A wavefront covers 64/S consecutive elements (S chosen near the mean particle
-// count, so few lanes idle); lane k of a segment takes particles k, k+S, ... of its element (coalesced:
-// particles are cell-sorted) and accumulates its 43 (3D) partial sums in registers.  The partials are
-// then reduced through LDS in chunks of PW_CH columns: every lane writes its chunk, and lane t sums
-// column t of one segment; the odd row length keeps the 64-bit row writes of a wavefront free of bank
-// conflicts, and each wave reduces in its own LDS rows, so waves never wait for each other.  Workgroups
-// are persistent (grid-stride over element groups) and copy the material table
-// (at most UST_MAX_MATERIALS entries) into LDS once, so the per-particle rheology chain reads LDS instead
-// of making dependent global loads.  NEED_T / NEED_VEL / SW compile the temperature and strain-rate lookups
-// (Arrhenius, yield) and the strain-weakening state in only when a material uses them.
-// ------------------------------------------------------------------------------------------
-#define PW_WAVES 2
-#define PW_CH 11
-template <int DIM, int S, bool NEED_T, bool NEED_VEL, bool SW>
-__global__ __launch_bounds__(64 * PW_WAVES, (DIM == 2 ? 2 : 1)) void k_particle_weights(
-    GridDev g, const int *__restrict__ cell_off, const double *__restrict__ xi0, const double *__restrict__ xi1,
-    const double *__restrict__ xi2, const double *__restrict__ w, const unsigned char *__restrict__ mat,
-    const float *__restrict__ coh, const ust_material *__restrict__ mats, int nmat, const double *__restrict__ T,
-    const double *__restrict__ vel, const double *__restrict__ pres, int prev, YieldDev ys, BuoyDev bd,
-    double *__restrict__ eta_out, unsigned char *__restrict__ yield_out, double *__restrict__ WK,
+__global__ __launch_bounds__(64 * pw_waves(NEED_T || NEED_VEL), pw_minb(NEED_T || NEED_VEL)) void k_particle_weights(
+    GridDev g, const int *__restrict__ cell_off, ParticleArrays in, const ust_material *__restrict__ mats, int nmat,
+    const double *__restrict__ T, const double *__restrict__ vel, const double *__restrict__ pres, int prev, YieldDev ys,
+    BuoyDev bd, double *__restrict__ eta_out, unsigned char *__restrict__ yield_out, int epw, double *__restrict__ WK,
     double *__restrict__ WG, double *__restrict__ WF) {
-    constexpr int NQ = DIM == 3 ? 27 : 9;
-    constexpr int NV = 1 << DIM;
-    constexpr int NA = NQ + 2 * NV;  // accumulators per lane
-    constexpr int LD = PW_CH;        // odd row length (in doubles)
-    constexpr int nseg = 64 / S;
-    __shared__ double red[PW_WAVES][64 * LD];
-    __shared__ size_t sbase[PW_WAVES][nseg];
-    __shared__ ust_material smat[UST_MAX_MATERIALS];
-    {
+    constexpr bool LOOKUPS = NEED_T || NEED_VEL;
+    constexpr int PW_WAVES = pw_waves(LOOKUPS);
+    constexpr int NF = pw_factors(DIM), ROW = pw_row(DIM);
+    constexpr int STEP = DIM == 3 ? 4 : 8;  // particles per matrix step
+    constexpr int NQ = DIM == 3 ? 27 : 9, NV = 1 << DIM, NS = pw_sums(DIM);
+    extern __shared__ __align__(16) unsigned char pw_lds[];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double *buf = (double *)pw_lds + (size_t)wv * pw_wave_lds(DIM);
+    double *osum = buf + (PW_HALF + 1) * ROW;  // osum[sum * (PW_OUT + 1) + element % PW_OUT]
+    double *tab = (double *)pw_lds + (size_t)PW_WAVES * pw_wave_lds(DIM);
+    // the material table: {viscosity, density}, or the materials and their friction terms
+    const ust_material *smat = (const ust_material *)tab;
+    const FrictionDev *sfric = (const FrictionDev *)(smat + nmat);
+    if (LOOKUPS) {
         const int nw = nmat * (int)(sizeof(ust_material) / sizeof(int));
-        const int *src = (const int *)mats;
-        int *dst = (int *)smat;
-        for (int i = threadIdx.x; i < nw; i += blockDim.x) dst[i] = src[i];
-    }
-    __syncthreads();
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int seg = lane / S, k = lane % S;
-    const int ngroups = (g.nel + PW_WAVES * nseg - 1) / (PW_WAVES * nseg);
-    const double detJ = (DIM == 3) ? 0.125 * g.hx * g.hy * g.hz : 0.25 * g.hx * g.hy;
-    double *r = red[wv];
-    // the next group's particle range is loaded one group ahead, while this group is reduced
-    int grp = blockIdx.x;
-    int p0 = 0, p1 = 0;
-    {
-        const int e = (grp * PW_WAVES + wv) * nseg + seg;
-        if (grp < ngroups && seg < nseg && e < g.nel) {
-            p0 = cell_off[e];
-            p1 = cell_off[e + 1];
+        for (int i = threadIdx.x; i < nw; i += blockDim.x) ((int *)tab)[i] = ((const int *)mats)[i];
+        for (int i = threadIdx.x; i < nmat * UST_MAX_RHEOLOGIES; i += blockDim.x) {
+            const ust_material &M = mats[i / UST_MAX_RHEOLOGIES];
+            const int r = i % UST_MAX_RHEOLOGIES;
+            FrictionDev f = {0.0, 0.0, 0.0};
+            if (NEED_VEL && r < M.nrh && M.rh[r].type == UST_RH_DRUCKERPRAGER)
+                f = friction_of<DIM>(M.rh[r].p[1] * (1.0 - 0.0) + M.rh[r].p[6] * 0.0);
+            ((FrictionDev *)sfric)[i] = f;
+        }
+    } else {
+        for (int i = threadIdx.x; i < nmat; i += blockDim.x) {
+            int yf = -1;
+            tab[2 * i] = particle_viscosity<DIM, false, false, false>(g, mats[i], nullptr, 0, nullptr, nullptr, nullptr,
+                                                                       nullptr, 0, 1.0f, prev, ys, 0, &yf);
+            tab[2 * i + 1] = mats[i].density;
         }
     }
-    for (; grp < ngroups; grp += gridDim.x) {
-        const int ebase = (grp * PW_WAVES + wv) * nseg;
-        const int e = ebase + seg;
-        const int pbeg = p0, pend = p1;
-        {
-            const int en = ebase + gridDim.x * PW_WAVES * nseg + seg;
-            if (grp + (int)gridDim.x < ngroups && seg < nseg && en < g.nel) {
-                p0 = cell_off[en];
-                p1 = cell_off[en + 1];
+    if (lane < NF) buf[PW_HALF * ROW + lane] = 0.0;
+    __syncthreads();
+    const int e0 = (blockIdx.x * PW_WAVES + wv) * epw;
+    if (e0 >= g.nel) return;
+    const int ne = min(epw, g.nel - e0);
+    // lane t: the first particle of element e0 + t (t <= ne)
+    const int offs = cell_off[e0 + (lane < ne ? lane : ne)];
+    const int pbeg = __builtin_amdgcn_readlane(offs, 0), pend = __builtin_amdgcn_readlane(offs, ne);
+
+    // this lane's part of a matrix step: it feeds A[i][k] and B[k][j] (i = j = lane % 4) of block b and ends with
+    // D[lane / 16][lane % 4]
+    const int li = lane & 3, lb = (lane >> 2) & 3, lk = lane >> 4;
+    int fa, fb, sub;
+    if (DIM == 3) {
+        fa = lb < 3 ? min(4 * lb + li, 8) : 9 + li;
+        fb = lb < 3 ? 13 + min(li, 2) : 16 + li;
+        sub = lk;
+    } else {
+        fa = lb & 1 ? 3 + min(li, 1) : min(li, 2);
+        fb = lb & 1 ? 8 + li : 5 + min(li, 2);
+        sub = lk + 4 * (lb >> 1);
+    }
+    // which sum D is: WK's NQ, then WG's and WF's NV; -1 none
+    int col = -1;
+    if (DIM == 3) {
+        if (lb == 3) col = NQ + (li & 2 ? NV : 0) + lk + 4 * (li & 1);
+        else if (4 * lb + lk < 9 && li < 3) col = 4 * lb + lk + 9 * li;
+    } else if (lb == 0) {
+        if (lk < 3 && li < 3) col = lk + 3 * li;
+    } else if (lb == 1 && lk < 2) {
+        col = NQ + (li & 2 ? NV : 0) + lk + 2 * (li & 1);
+    }
+    // lane t: the slot of weight 0 of element e0 + t (t < ne <= 16)
+    const unsigned long long slots = widx(g, e0 + (lane < ne ? lane : 0), 0);
+    const double detJ = (DIM == 3) ? 0.125 * g.hx * g.hy * g.hz : 0.25 * g.hx * g.hy;
+    double D = 0.0;
+    int e = 0, elo = pbeg, ehi = __builtin_amdgcn_readlane(offs, 1);
+    auto finish = [&]() {
+        if (DIM == 2) D += __shfl_xor(D, 8);  // the two halves of a step
+        if (col >= 0) osum[col * (PW_OUT + 1) + e % PW_OUT] = D;
+        D = 0.0;
+        e++;
+        elo = ehi;
+        ehi = __builtin_amdgcn_readlane(offs, e < ne ? e + 1 : ne);
+        if (e % PW_OUT != 0 && e != ne) return;
+        wave_sync();
+        const int ef = (e - 1) / PW_OUT * PW_OUT, n = e - ef;
+        const int k = lane % PW_OUT;
+        const unsigned lo = __shfl((int)(unsigned)slots, ef + k), hi = __shfl((int)(slots >> 32), ef + k);
+        if (k < n) {
+            double *const wk = WK + (size_t)(((unsigned long long)hi << 32) | lo);
+            const size_t el = (size_t)(e0 + ef + k);
+#pragma unroll
+            for (int t = 0; t < (NS + 64 / PW_OUT - 1) / (64 / PW_OUT); t++) {
+                const int sum = lane / PW_OUT + t * (64 / PW_OUT);
+                if (sum >= NS) continue;
+                const double v = osum[sum * (PW_OUT + 1) + k];
+                if (sum < NQ) wk[sum * UST_TILE] = v;
+                else if (sum < NQ + NV) WG[(size_t)(sum - NQ) * g.nel + el] = v;
+                else WF[(size_t)(sum - NQ - NV) * g.nel + el] = v;
             }
         }
-        double acc[NA];
-#pragma unroll
-        for (int t = 0; t < NA; t++) acc[t] = 0.0;
-        // slot of K weight 0 of each segment's element (weight q sits q * UST_TILE further on in every layout),
-        // left in LDS for the reduction threads instead of recomputing the layout index per store
-        if (seg < nseg && e < g.nel) {
-            if (k == 0) sbase[wv][seg] = widx(g, e, 0);
-            const int ie = e % g.nx, je = (e / g.nx) % g.ny, ke = e / (g.nx * g.ny);
-            int nodes[NV];
-            element_nodes_of(g, ie, je, ke, DIM, nodes);
-            for (int pi = pbeg + k; pi < pend; pi += S)
-                particle_contrib<DIM, NEED_T, NEED_VEL, SW>(g, e, pi, nodes, detJ, xi0, xi1, xi2, w, mat, coh, smat,
-                                                            nmat, T, vel, pres, prev, ys, bd, eta_out, yield_out,
-                                                            acc);
+        wave_sync();
+    };
+    ParticleIn<DIM> nxt;
+    if (!LOOKUPS && pbeg < pend) nxt.load(in, min(pbeg + lane, pend - 1), nmat);
+    for (int b0 = pbeg; b0 < pend; b0 += 64) {
+        const int bend = min(b0 + 64, pend), p = min(b0 + lane, pend - 1);
+        ParticleIn<DIM> q = nxt;
+        if (LOOKUPS) q.load(in, p, nmat);  // the registers of a load ahead would cost a wave
+        else if (bend < pend) nxt.load(in, min(bend + lane, pend - 1), nmat);
+        // lanes past the last particle repeat it; their rows are not read
+        double eta, rho;
+        const ust_material &M = LOOKUPS ? smat[q.m] : mats[q.m];
+        if (LOOKUPS || bd.full) {
+            int pe = 0;
+            for (int t = 1; t < ne; t++) pe += p >= __builtin_amdgcn_readlane(offs, t);
+            pe += e0;
+            const int ie = pe % g.nx, je = (pe / g.nx) % g.ny, ke = pe / (g.nx * g.ny);
+            const size_t n0 = (size_t)ie + (size_t)g.nnx * ((size_t)je + (size_t)g.nny * ke);  // the element's first node
+            int yf = -1;
+            if (LOOKUPS) {
+                eta = particle_viscosity<DIM, NEED_T, NEED_VEL, SW>(g, M, sfric + q.m * UST_MAX_RHEOLOGIES, n0, q.x, T,
+                                                                    vel, pres, pe, q.coh, prev, ys, p, &yf);
+                if (NEED_VEL && yield_out && yf >= 0) yield_out[p] = (unsigned char)yf;
+            } else {
+                eta = tab[2 * q.m];
+            }
+            rho = particle_density<DIM, NEED_T>(g, bd, M, n0, q.x, T, pe);
+        } else {
+            eta = tab[2 * q.m];
+            rho = tab[2 * q.m + 1];
         }
+        if (eta_out) eta_out[p] = eta;
+        const double wd = q.w * detJ, et = wd * eta, wr = wd * rho;
+        for (int h0 = b0; h0 < bend; h0 += PW_HALF) {
+            const int hend = min(h0 + PW_HALF, bend);
+            if (lane / PW_HALF == (h0 - b0) / PW_HALF) {
+                double *r = buf + (lane % PW_HALF) * ROW;
+                // taken anew in each half: the factors, hoisted out of the loop, would hold 40 registers through it
+                double x0 = q.x[0], x1 = q.x[1], x2 = q.x[2];
+                asm volatile("" : "+v"(x0), "+v"(x1), "+v"(x2));
+                double Lx[3], Ly[3], Lz[3];
+                lagrange3(x0, Lx);
+                lagrange3(x1, Ly);
+                if (DIM == 3) lagrange3(x2, Lz);
+                const double Nx[2] = {0.5 * (1.0 - x0), 0.5 * (1.0 + x0)};
+                const double Ny[2] = {0.5 * (1.0 - x1), 0.5 * (1.0 + x1)};
+                const double Nz[2] = {0.5 * (1.0 - x2), 0.5 * (1.0 + x2)};
+                if (DIM == 3) {
 #pragma unroll
-        for (int c0 = 0; c0 < NA; c0 += PW_CH) {
+                    for (int t = 0; t < 9; t++) r[t] = Lx[t % 3] * Ly[t / 3];
 #pragma unroll
-            for (int t = 0; t < PW_CH; t++)
-                if (c0 + t < NA) r[lane * LD + t] = acc[c0 + t];
-            wave_sync();
-            const int nc = NA - c0 < PW_CH ? NA - c0 : PW_CH;
-            for (int t = lane; t < nseg * nc; t += 64) {
-                const int sg = t / nc, col = c0 + t % nc, el = ebase + sg;
-                if (el < g.nel) {
-                    // S independent LDS reads into four partial sums (S is a compile-time constant)
-                    double ps[4] = {0.0, 0.0, 0.0, 0.0};
+                    for (int t = 0; t < 4; t++) r[9 + t] = Nx[t & 1] * Ny[t >> 1];
 #pragma unroll
-                    for (int row = 0; row < S; row++) ps[row & 3] += r[(sg * S + row) * LD + (col - c0)];
-                    const double sum = (ps[0] + ps[1]) + (ps[2] + ps[3]);
-                    if (col < NQ) WK[sbase[wv][sg] + (size_t)col * UST_TILE] = sum;
-                    else if (col < NQ + NV) WG[(size_t)(col - NQ) * g.nel + el] = sum;
-                    else WF[(size_t)(col - NQ - NV) * g.nel + el] = sum;
+                    for (int t = 0; t < 3; t++) r[13 + t] = et * Lz[t];
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        r[16 + t] = wd * Nz[t];
+                        r[18 + t] = wr * Nz[t];
+                    }
+                } else {
+#pragma unroll
+                    for (int t = 0; t < 3; t++) {
+                        r[t] = Lx[t];
+                        r[5 + t] = et * Ly[t];
+                    }
+#pragma unroll
+                    for (int t = 0; t < 2; t++) {
+                        r[3 + t] = Nx[t];
+                        r[8 + t] = wd * Ny[t];
+                        r[10 + t] = wr * Ny[t];
+                    }
                 }
             }
             wave_sync();
+            while (e < ne) {
+                const int lo = max(elo, h0) - h0, hi = min(ehi, hend) - h0;
+                if (lo < hi) {  // the next step's factors are read while this one multiplies
+                    int row = lo + sub < hi ? lo + sub : PW_HALF;
+                    double a = buf[row * ROW + fa], b = buf[row * ROW + fb];
+                    for (int st = lo + STEP; st < hi; st += STEP) {
+                        row = st + sub < hi ? st + sub : PW_HALF;
+                        const double an = buf[row * ROW + fa], bn = buf[row * ROW + fb];
+                        D = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, D, 0, 0, 0);
+                        a = an;
+                        b = bn;
+                    }
+                    D = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, D, 0, 0, 0);
+                }
+                if (ehi > hend) break;  // the element goes on in the next particles
+                finish();
+            }
+            wave_sync();
         }
     }
+    while (e < ne) finish();  // elements without particles
 }
 
 // ------------------------------------------------------------------------------------------
@@ -583,63 +715,32 @@ extern "C" int ust_k_particle_weights(const ust_grid *gr, const int *cell_off, i
     // otherwise)
     const bool needT = temperature != nullptr, needV = velocity != nullptr && pressure != nullptr;
     hipStream_t st = ust_stream(stream);
-    // segment width: the smallest candidate >= the caller's particles-per-cell hint (the mean count; a cell
-    // with more particles than S loops), so few lanes idle; segments never straddle a wavefront
-    int S = 64;
-    const int cands[6] = {8, 12, 16, 21, 32, 64};
-    for (int c = 0; c < 6; c++)
-        if (cands[c] >= ppc_hint) {
-            S = cands[c];
-            break;
-        }
-    const int ngroups = (g.nel + PW_WAVES * (64 / S) - 1) / (PW_WAVES * (64 / S));
-    // persistent workgroups: as many as fit on the device at once (at least one per compute unit)
-    static int n_cu = 0;
-    if (n_cu == 0) {
-        int dev = 0, v = 0;
-        if (hipGetDevice(&dev) == hipSuccess &&
-            hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && v > 0)
-            n_cu = v;
-        else
-            n_cu = 256;
-    }
-#define LAUNCH_PW(D, SS, NT, NVL, SWK)                                                                         \
-    do {                                                                                                       \
-        int per_cu = 0;                                                                                        \
-        if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_particle_weights<D, SS, NT, NVL, SWK>,     \
-                                                         64 * PW_WAVES, 0) != hipSuccess || per_cu < 1)        \
-            per_cu = 1;                                                                                        \
-        const int nb = ngroups < n_cu * per_cu ? ngroups : n_cu * per_cu;                                      \
-        hipLaunchKernelGGL((k_particle_weights<D, SS, NT, NVL, SWK>), dim3(nb), dim3(64 * PW_WAVES), 0, st, g, \
-                           cell_off, xi0, xi1, xi2, w, mat, coh_scale, materials_dev, nmat, temperature,       \
-                           velocity, pressure, prev_solution, ys, bd, eta_out, yield_out, WK, WG, WF);         \
-    } while (0)
-#define LAUNCH_S(D, NT, NVL, SWK)                                  \
-    do {                                                           \
-        switch (S) {                                               \
-            case 8: LAUNCH_PW(D, 8, NT, NVL, SWK); break;          \
-            case 12: LAUNCH_PW(D, 12, NT, NVL, SWK); break;        \
-            case 16: LAUNCH_PW(D, 16, NT, NVL, SWK); break;        \
-            case 21: LAUNCH_PW(D, 21, NT, NVL, SWK); break;        \
-            case 32: LAUNCH_PW(D, 32, NT, NVL, SWK); break;        \
-            default: LAUNCH_PW(D, 64, NT, NVL, SWK); break;        \
-        }                                                          \
-    } while (0)
-    // strain weakening is compiled in only when the yield state carries it (it costs registers)
-    const bool sw = needV && ys.pfw != nullptr;
-#define LAUNCH_F(D)                                                  \
-    do {                                                             \
-        if (needT && needV && sw) LAUNCH_S(D, true, true, true);     \
-        else if (needT && needV) LAUNCH_S(D, true, true, false);     \
-        else if (needT) LAUNCH_S(D, true, false, false);             \
-        else if (needV && sw) LAUNCH_S(D, false, true, true);        \
-        else if (needV) LAUNCH_S(D, false, true, false);             \
-        else LAUNCH_S(D, false, false, false);                       \
+    (void)ppc_hint;
+    // elements per wave: 16 (a row of a weight tile, whose stores fill cache lines) once that leaves enough waves to fill
+    // the GPU several times over, fewer on smaller grids
+    int epw = PW_EPW;
+    while (epw > 1 && g.nel / epw < PW_MIN_WAVES) epw /= 2;
+    const int waves = pw_waves(needT || needV);
+    const unsigned grid = ust_grid_size((size_t)g.nel, waves * epw);
+    const bool sw = needV && ys.pfw != nullptr;  // compiled in only when the yield state carries it (it costs registers)
+    const ParticleArrays in = {xi0, xi1, xi2, w, mat, coh_scale};
+    const size_t lds = (size_t)waves * pw_wave_lds(g.dim) * sizeof(double) + pw_table(needT || needV, nmat);
+#define LAUNCH_PW(D, NT, NVL, SWK)                                                                                      \
+    hipLaunchKernelGGL((k_particle_weights<D, NT, NVL, SWK>), dim3(grid), dim3(64 * waves), lds, st, g, cell_off, in, \
+                       materials_dev, nmat, temperature, velocity, pressure, prev_solution, ys, bd, eta_out, yield_out,  \
+                       epw, WK, WG, WF)
+#define LAUNCH_F(D)                                              \
+    do {                                                         \
+        if (needT && needV && sw) LAUNCH_PW(D, true, true, true); \
+        else if (needT && needV) LAUNCH_PW(D, true, true, false); \
+        else if (needT) LAUNCH_PW(D, true, false, false);         \
+        else if (needV && sw) LAUNCH_PW(D, false, true, true);    \
+        else if (needV) LAUNCH_PW(D, false, true, false);         \
+        else LAUNCH_PW(D, false, false, false);                   \
     } while (0)
     if (g.dim == 3) LAUNCH_F(3);
     else LAUNCH_F(2);
 #undef LAUNCH_F
-#undef LAUNCH_S
 #undef LAUNCH_PW
     UST_LAUNCH_CHECK();
     return UST_OK;

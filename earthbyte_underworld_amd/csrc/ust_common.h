@@ -80,9 +80,8 @@ struct GridDev {
     double ymax;
 };
 
-// index of quadrature weight q of element e in the tile-blocked layout
-__host__ __device__ __forceinline__ size_t widx(const GridDev &g, int e, int q) {
-    const int ex = e % g.nx, ey = (e / g.nx) % g.ny, ez = e / (g.nx * g.ny);
+// index of quadrature weight q of element (ex, ey, ez) in the tile-blocked layout
+__host__ __device__ __forceinline__ size_t widx_at(const GridDev &g, int ex, int ey, int ez, int q) {
     if (g.dim == 3 && g.col) {
         const int txy = ex / UST_TX3 + g.tnx * (ey / UST_TY3);
         const int l = ex % UST_TX3 + UST_TX3 * (ey % UST_TY3);
@@ -96,6 +95,10 @@ __host__ __device__ __forceinline__ size_t widx(const GridDev &g, int e, int q) 
     const int t = ex / UST_TX2 + g.tnx * (ey / UST_TY2);
     const int l = ex % UST_TX2 + UST_TX2 * (ey % UST_TY2);
     return ((size_t)t * 9 + q) * UST_TILE + l;
+}
+
+__host__ __device__ __forceinline__ size_t widx(const GridDev &g, int e, int q) {
+    return widx_at(g, e % g.nx, (e / g.nx) % g.ny, e / (g.nx * g.ny), q);
 }
 
 // wg_target: the workgroups a column launch aims at (the z-chunk length follows)

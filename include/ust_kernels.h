@@ -182,7 +182,7 @@ const char *ust_dev_error_string(void);
 /* eta_out/yield_out (np) may be NULL.  temperature (nodal), velocity (nodal, interleaved dim),
  * pressure (per element), coh_scale (per particle) may be NULL when no rheology needs them.
  * WK (nq per element, tile-blocked), WG (nv*nel), WF (nv*nel): nq = 3^dim, nv = 2^dim.  ppc_hint: the
- * mean particle count per cell (sizes the lane segment of an element; any count is handled).  yield_state
+ * mean particle count per cell (unused: the particles are read as one run).  yield_state
  * may be NULL (no strain weakening, no tensile flags). */
 int ust_k_particle_weights(const ust_grid *g, const int *cell_off, int ppc_hint, const double *xi0,
                            const double *xi1, const double *xi2, const double *w,

@@ -447,3 +447,58 @@ def test_strain_weakening_initial_damage(oracle):
                                                initialDamageWavenumberCosI=0.75))
     s.strain_weakening_initialise()
     assert np.allclose(s.strain_weakening()[0], plain * np.cos(np.pi * x[:, 0] * 0.75) ** 2, rtol=1e-14, atol=0)
+
+
+# counts at the edges of a matrix step (4 particles, 8 in 2D), of the 32 staged at a time and of the 64 loaded at a time
+EDGE_COUNTS = [1, 3, 4, 5, 7, 8, 9, 31, 32, 33, 63, 64, 65, 1, 1, 130, 2, 96]
+
+
+@pytest.mark.parametrize("dim,nel", [(2, (6, 3)), (3, (3, 3, 2)), (2, (18, 1)), (3, (1, 1, 18))])
+def test_particle_weights_step_edges(oracle, dim, nel):
+    import earthbyte_underworld_amd as ust
+    s = ust.StokesSystem(dim, nel)
+    s.random_particle_layout(seed=23, cell_counts=EDGE_COUNTS)
+    s.set_materials([ust.RheologyMaterial([ust.MaterialViscosity(eta0=2.0)], density=1.5),
+                     ust.RheologyMaterial([ust.MaterialViscosity(eta0=300.0),
+                                           ust.ViscosityLimiter(maxViscosity=70.0, minViscosity=1.0)], density=0.5)])
+    s.assign_materials([ust.Everywhere(0), ust.Box(1, (0.3,) * dim, (0.8,) * dim)])
+    s.assemble()
+    o = OracleProblem(s)
+    eta, _ = s.particle_viscosity()
+    assert rel_err(eta, o.eta) < 1e-13
+    assert max_rel_err(s.element_matrices(), o.Ke) < TOL
+    assert max_rel_err(s.element_G(), o.Ge) < TOL
+    assert max_rel_err(s.element_f(), o.fe) < TOL
+
+
+@pytest.mark.parametrize("dim,nel", [(2, (40, 3)), (3, (20, 3, 2)), (3, (64, 64, 33))])
+def test_particle_weights_of_empty_elements(dim, nel):
+    """Elements without particles get zero weights, at every place of a wave's 1 to 16 elements, and the others weights that
+    add up to their particles'."""
+    import earthbyte_underworld_amd as ust
+    from tests.test_gpu_operators import _Dev
+    rng = np.random.default_rng(3)
+    ne = int(np.prod(nel))
+    counts = rng.integers(0, 12, ne) * (rng.random(ne) < 0.6)
+    counts[:3] = 0
+    counts[-2:] = 0
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    xi = rng.uniform(-1, 1, (3, off[-1]))
+    w = rng.uniform(0.1, 1.0, off[-1])
+    s = ust.StokesSystem(dim, nel)
+    s.set_materials([ust.RheologyMaterial([ust.MaterialViscosity(eta0=3.0)], density=2.0)])
+    d = [_Dev(s.lib, a) for a in (off, xi[0], xi[1], xi[2], w)]
+    assert s.lib.ust_swarm_upload_dev(s.ctx, int(off[-1]), *[a.p for a in d], None, None, int(counts.max())) == 0
+    s.assemble()
+    WK, WG, WF = s.weights()
+    empty = counts == 0
+    assert np.all(WK[:, empty] == 0) and np.all(WG[:, empty] == 0) and np.all(WF[:, empty] == 0)
+    e = np.repeat(np.arange(ne), counts)
+    detJ = float(np.prod([0.5 * (s.max[k] - s.min[k]) / nel[k] for k in range(dim)]))
+    mass = np.bincount(e, weights=w * detJ, minlength=ne)
+    # sums of the vertex and Lagrange functions are 1: each element's weights add to its particles' (5 roundings each)
+    assert np.max(np.abs(WG.sum(0) - mass)) < 1e-14 * mass.max() * 5
+    assert np.max(np.abs(WK.sum(0) - 3.0 * mass)) < 1e-14 * mass.max() * 50
+    assert np.max(np.abs(WF.sum(0) - 2.0 * mass)) < 1e-14 * mass.max() * 10
+    for a in d:
+        a.free()
