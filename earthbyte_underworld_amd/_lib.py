@@ -223,6 +223,8 @@ _SIGS = {
     "ust_k_prolong_add_f32": (I, [C.POINTER(Grid), vp, vp, vp, vp]),
     "ust_k_particle_weights": (I, [C.POINTER(Grid), vp, I, vp, vp, vp, vp, vp, vp, vp, I, vp, vp, vp, I, vp, vp,
                                    vp, vp, vp, vp, vp, vp]),
+    "ust_k_derive": (I, [C.POINTER(Grid), vp, vp, vp, D, vp, vp, vp, vp, vp, vp, vp, vp]),
+    "ust_k_uzawa_diag": (I, [C.POINTER(Grid), vp, vp, vp, vp]),
     "ust_k_strain_weakening_step": (I, [vp, vp, I, C.c_double, vp]),
     "ust_k_permute_f64": (I, [vp, vp, vp, I, vp]),
     "ust_k_pcdvc_plan": (I, [C.POINTER(Grid), vp, vp, vp, C.POINTER(PcdvcOpts), vp, vp, vp, vp]),

@@ -642,42 +642,173 @@ __global__ void k_adjust_force(GridDev g, const double *__restrict__ WG, double 
     for (int b = 0; b < NV; b++) WF[(size_t)b * g.nel + e] *= f;
 }
 
-// diag of K_e: sum_q W_q (sum_k GNx_k(a)^2 + GNx_i(a)^2)
+// diag of K_e: sum_q W_q (sum_k GNx_k(a)^2 + GNx_i(a)^2), with GNx_k(a)^2 = s_k^2 / 4^DIM prod_{d != k} cfac^2.  Per
+// direction k the weights are summed along k, then taken against cfac^2 = {4, 1, 0} or {0, 1, 4} along the others.
 template <int DIM>
-__device__ __forceinline__ void element_K_diag(const GridDev &g, const double *WK, int e, double *dg) {
+__device__ __forceinline__ void element_K_diag(const GridDev &g, const double *__restrict__ WK, int e, double *dg) {
     constexpr int NQ = DIM == 3 ? 27 : 9, NV = 1 << DIM;
     const double s[3] = {2.0 / g.hx, 2.0 / g.hy, 2.0 / g.hz};
+    const double *w = WK + widx(g, e, 0);
+    double W[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; q++) W[q] = w[q * UST_TILE];
 #pragma unroll
     for (int v = 0; v < NV * DIM; v++) dg[v] = 0.0;
-    for (int q = 0; q < NQ; q++) {
-        const double wq = WK[widx(g, e, q)];
+#pragma unroll
+    for (int k = 0; k < DIM; k++) {
+        constexpr int p3[3] = {1, 3, 9};
+        const int u = k == 0 ? 1 : 0, v = k == 2 ? 1 : 2;  // the other axes (v: 3D only)
+        const double t = s[k] * s[k] / (double)(1 << (2 * DIM));
+        double c[2][3];  // [bit on u][point on v]
+#pragma unroll
+        for (int qv = 0; qv < (DIM == 3 ? 3 : 1); qv++) {
+            double l[3];
+#pragma unroll
+            for (int qu = 0; qu < 3; qu++) {
+                const int i = qu * p3[u] + (DIM == 3 ? qv * p3[v] : 0);
+                l[qu] = W[i] + W[i + p3[k]] + W[i + 2 * p3[k]];
+            }
+            c[0][qv] = 4.0 * l[0] + l[1];
+            c[1][qv] = l[1] + 4.0 * l[2];
+        }
 #pragma unroll
         for (int a = 0; a < NV; a++) {
-            double gk[3], s2 = 0.0;
+            const double *cu = c[(a >> u) & 1];
+            const double d = t * (DIM == 3 ? ((a >> v) & 1 ? cu[1] + 4.0 * cu[2] : 4.0 * cu[0] + cu[1]) : cu[0]);
 #pragma unroll
-            for (int k = 0; k < DIM; k++) {
-                gk[k] = gnx_at<DIM>(a, k, q, s);
-                s2 += gk[k] * gk[k];
-            }
-#pragma unroll
-            for (int i = 0; i < DIM; i++) dg[a * DIM + i] += wq * (s2 + gk[i] * gk[i]);
+            for (int i = 0; i < DIM; i++) dg[a * DIM + i] += i == k ? 2.0 * d : d;
         }
     }
 }
 
+// approxS = g^T diag(K_e)^-1 g (UzawaPreconditionerTerm.c:195-212)
 template <int DIM>
-__global__ void k_uzawa_diag(GridDev g, const double *__restrict__ WK, const double *__restrict__ WG,
-                             double *__restrict__ approxS) {
+__device__ __forceinline__ double uzawa_diag(const GridDev &g, const double *__restrict__ WK,
+                                             const double *__restrict__ WG, int e, double *ge) {
     constexpr int ND = (1 << DIM) * DIM;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= g.nel) return;
-    double dg[ND], ge[ND];
+    double dg[ND];
     element_K_diag<DIM>(g, WK, e, dg);
     element_G<DIM>(g, WG, e, ge);
     double s = 0.0;
 #pragma unroll
     for (int v = 0; v < ND; v++) s += ge[v] * (ge[v] / dg[v]);
-    approxS[e] = s;
+    return s;
+}
+
+template <int DIM>
+__global__ __launch_bounds__(256, 4) void k_uzawa_diag(GridDev g, const double *__restrict__ WK,
+                                                    const double *__restrict__ WG, double *__restrict__ approxS) {
+    const int e = blockIdx.x * blockDim.x + threadIdx.x;
+    if (e >= g.nel) return;
+    double ge[(1 << DIM) * DIM];
+    approxS[e] = uzawa_diag<DIM>(g, WK, WG, e, ge);
+}
+
+// ------------------------------------------------------------------------------------------
+// What an assembly derives from the weights, in one pass over the elements and one over the nodes, with the two norms of
+// the null-space test on the way (ksp_pressure_nullspace.c:139-158): a third launch leaves them in host memory.  Before,
+// thirteen launches and two copies with a wait each: 45 of the 72 us of a 64x64 assembly, 270 of 671 us at 128x128x64.
+// ------------------------------------------------------------------------------------------
+constexpr int DERIVE_BLOCKS = 1024;  // partial results per pass
+
+// approxS, h = 0 and per block the largest row sum of |D| over the free dofs
+template <int DIM>
+__global__ __launch_bounds__(256, 4) void k_derive_elements(GridDev g, const double *__restrict__ WK,
+                                                         const double *__restrict__ WG,
+                                                         const unsigned char *__restrict__ mask,
+                                                         double *__restrict__ approxS, double *__restrict__ h,
+                                                         double *__restrict__ partial) {
+    constexpr int NV = 1 << DIM;
+    __shared__ double sh[4];
+    double m = 0.0;
+    for (int e = blockIdx.x * 256 + threadIdx.x; e < g.nel; e += gridDim.x * 256) {
+        const int ex = e % g.nx, ey = (e / g.nx) % g.ny, ez = e / (g.nx * g.ny);
+        const unsigned char *mk = mask + ((size_t)ex + (size_t)g.nnx * ((size_t)ey + (size_t)g.nny * ez)) * DIM;
+        unsigned char bc[NV * DIM];
+#pragma unroll
+        for (int a = 0; a < NV; a++)
+#pragma unroll
+            for (int i = 0; i < DIM; i++)
+                bc[a * DIM + i] = mk[((size_t)(a & 1) + (size_t)g.nnx * ((a >> 1) & 1) +
+                                      (DIM == 3 ? (size_t)g.nnx * g.nny * (a >> 2) : 0)) * DIM + i];
+        double ge[NV * DIM];
+        approxS[e] = uzawa_diag<DIM>(g, WK, WG, e, ge);
+        h[e] = 0.0;
+        double s = 0.0;
+#pragma unroll
+        for (int v = 0; v < NV * DIM; v++) s += bc[v] ? 0.0 : fabs(ge[v]);
+        m = fmax(m, s);
+    }
+    for (int off = 32; off > 0; off >>= 1) m = fmax(m, __shfl_xor(m, off, 64));
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[blockIdx.x] = fmax(fmax(sh[0], sh[1]), fmax(sh[2], sh[3]));
+}
+
+// f = gravity dir sum of WF around the node (0 on Dirichlet dofs) and per block the sum of squares of G 1
+template <int DIM>
+__global__ __launch_bounds__(256) void k_derive_nodes(GridDev g, const double *__restrict__ WG,
+                                                      const double *__restrict__ WF, double gravity, FDir dir,
+                                                      const unsigned char *__restrict__ mask, double *__restrict__ f,
+                                                      double *__restrict__ partial) {
+    constexpr int NV = 1 << DIM;
+    __shared__ double sh[4];
+    const double hr[3] = {1.0 / g.hx, 1.0 / g.hy, 1.0 / g.hz};
+    const int nnodes = g.nnx * g.nny * g.nnz;
+    double s = 0.0;
+    for (int n = blockIdx.x * 256 + threadIdx.x; n < nnodes; n += gridDim.x * 256) {
+        const int gx = n % g.nnx, gy = (n / g.nnx) % g.nny, gz = n / (g.nnx * g.nny);
+        double fn = 0.0, gn[DIM];
+#pragma unroll
+        for (int i = 0; i < DIM; i++) gn[i] = 0.0;
+#pragma unroll
+        for (int a = 0; a < NV; a++) {
+            const int ex = gx - (a & 1), ey = gy - ((a >> 1) & 1), ez = DIM == 3 ? gz - (a >> 2) : 0;
+            const bool in = ex >= 0 && ey >= 0 && ez >= 0 && ex < g.nx && ey < g.ny && ez < g.nz;
+            const size_t e = in ? (size_t)ex + (size_t)g.nx * ((size_t)ey + (size_t)g.ny * ez) : 0;
+            const double wa = WG[(size_t)a * g.nel + e], wf = WF[(size_t)a * g.nel + e];
+            double wi[DIM];
+#pragma unroll
+            for (int i = 0; i < DIM; i++) wi[i] = WG[(size_t)(a ^ (1 << i)) * g.nel + e];
+            if (!in) continue;
+            fn += wf;
+#pragma unroll
+            for (int i = 0; i < DIM; i++) gn[i] -= (double)sgn((a >> i) & 1) * hr[i] * (wa + wi[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < DIM; i++) {
+            const size_t dof = (size_t)n * DIM + i;
+            const bool bc = mask[dof] != 0;
+            f[dof] = bc || dir.d[i] == 0.0 ? 0.0 : gravity * dir.d[i] * fn;
+            s += bc ? 0.0 : gn[i] * gn[i];
+        }
+    }
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) partial[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+}
+
+// out[0] = the sum of the first ns partials, out[1] = the largest of the nm at DERIVE_BLOCKS
+__global__ __launch_bounds__(256) void k_derive_norms(const double *__restrict__ partial, int ns, int nm,
+                                                      double *__restrict__ out) {
+    __shared__ double sh[2][4];
+    double s = 0.0, m = 0.0;
+    for (int i = threadIdx.x; i < ns; i += 256) s += partial[i];
+    for (int i = threadIdx.x; i < nm; i += 256) m = fmax(m, partial[DERIVE_BLOCKS + i]);
+    for (int off = 32; off > 0; off >>= 1) {
+        s += __shfl_xor(s, off, 64);
+        m = fmax(m, __shfl_xor(m, off, 64));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sh[0][threadIdx.x >> 6] = s;
+        sh[1][threadIdx.x >> 6] = m;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        out[0] = (sh[0][0] + sh[0][1]) + (sh[0][2] + sh[0][3]);
+        out[1] = fmax(fmax(sh[1][0], sh[1][1]), fmax(sh[1][2], sh[1][3]));
+    }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -824,6 +955,30 @@ extern "C" int ust_k_uzawa_diag(const ust_grid *gr, const double *WK, const doub
     else
         hipLaunchKernelGGL(k_uzawa_diag<2>, dim3(ust_grid_size(g.nel, UST_BLOCK)), dim3(UST_BLOCK), 0,
                            ust_stream(stream), g, WK, WG, approxS);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+
+extern "C" int ust_k_derive(const ust_grid *gr, const double *WK, const double *WG, const double *WF, double gravity,
+                            const double *dir, const unsigned char *mask, double *approxS, double *f, double *h,
+                            double *partial, double *norms, void *stream) {
+    if (!gr || !WK || !WG || !WF || !dir || !mask || !approxS || !f || !h || !partial || !norms) return UST_EINVAL;
+    GridDev g = grid_dev(gr);
+    if (g.nel <= 0) return UST_EINVAL;
+    const FDir d = {{dir[0], dir[1], g.dim == 3 ? dir[2] : 0.0}};
+    hipStream_t st = ust_stream(stream);
+    const unsigned be = ust_grid_size((size_t)g.nel, 256), bn = ust_grid_size((size_t)g.nnx * g.nny * g.nnz, 256);
+    const int ne = (int)(be < DERIVE_BLOCKS ? be : DERIVE_BLOCKS), nn = (int)(bn < DERIVE_BLOCKS ? bn : DERIVE_BLOCKS);
+    if (g.dim == 3) {
+        hipLaunchKernelGGL(k_derive_elements<3>, dim3(ne), dim3(256), 0, st, g, WK, WG, mask, approxS, h,
+                           partial + DERIVE_BLOCKS);
+        hipLaunchKernelGGL(k_derive_nodes<3>, dim3(nn), dim3(256), 0, st, g, WG, WF, gravity, d, mask, f, partial);
+    } else {
+        hipLaunchKernelGGL(k_derive_elements<2>, dim3(ne), dim3(256), 0, st, g, WK, WG, mask, approxS, h,
+                           partial + DERIVE_BLOCKS);
+        hipLaunchKernelGGL(k_derive_nodes<2>, dim3(nn), dim3(256), 0, st, g, WG, WF, gravity, d, mask, f, partial);
+    }
+    hipLaunchKernelGGL(k_derive_norms, dim3(1), dim3(256), 0, st, partial, nn, ne, norms);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }

@@ -59,7 +59,7 @@ int ust_create(ust_context **out, int device) {
         free(ctx);
         return rc;
     }
-    rc = ust_dev_malloc((void **)&ctx->partial, 1024 * sizeof(double));
+    rc = ust_dev_malloc((void **)&ctx->partial, 2048 * sizeof(double));
     if (rc == UST_OK) rc = ust_dev_malloc((void **)&ctx->scal, SC_COUNT * sizeof(double));
     if (rc == UST_OK) rc = ust_host_malloc_pinned((void **)&ctx->scal_h, SC_COUNT * sizeof(double));
     if (rc == UST_OK) rc = ust_dev_malloc((void **)&ctx->mats_d, UST_MAX_MATERIALS * sizeof(ust_material));
@@ -91,7 +91,6 @@ static void free_mesh_data(ust_context *ctx) {
     DFREE(ctx->f);
     DFREE(ctx->h);
     DFREE(ctx->tmpv);
-    DFREE(ctx->tmpp);
     DFREE(ctx->kwork);
     DFREE(ctx->WK32_0);
     ctx->wk32_0_valid = 0;
@@ -184,7 +183,6 @@ int ust_set_mesh(ust_context *ctx, int dim, const int nel[3], const double xmin[
     DALLOC(ctx, ctx->f, nd * sizeof(double));
     DALLOC(ctx, ctx->h, ne * sizeof(double));
     DALLOC(ctx, ctx->tmpv, nd * sizeof(double));
-    DALLOC(ctx, ctx->tmpp, ne * sizeof(double));
     ctx->kwork_len = ust_k_apply_work_len(&ctx->grid);
     DALLOC(ctx, ctx->kwork, ctx->kwork_len * sizeof(double));
     ctx->has_mesh = 1;
@@ -575,7 +573,6 @@ int ust_assemble(ust_context *ctx, double gravity) {
         free(m0);
         if (rc) return rc;
     }
-    size_t nd = (size_t)ctx->ndof, ne = (size_t)ctx->nel;
     /* the temperature and strain-rate/pressure lookups are compiled into the particle kernel only when a
      * material's rheology chain or density reads them; the density law runs only when a material has a
      * thermal or depth coefficient or a hydrostatic background is set (else rho = the material density) */
@@ -608,30 +605,23 @@ int ust_assemble(ust_context *ctx, double gravity) {
                                     fullDensity ? &ctx->buoy : NULL, ctx->eta, ctx->yielded, ctx->WK, ctx->WG,
                                     ctx->WF, ctx->stream));
     if (ctx->buoy.adjust) CKD(ctx, ust_k_adjust_force_weights(&ctx->grid, ctx->WG, ctx->WF, ctx->stream));
-    CKD(ctx, ust_k_uzawa_diag(&ctx->grid, ctx->WK, ctx->WG, ctx->approxS, ctx->stream));
-    /* f = buoyancy - K_{free,bc} u_bc ; h = -G_bc^T u_bc */
-    CKD(ctx, ust_k_fill_f64(ctx->f, 0.0, nd, ctx->stream));
+    /* approxS, f = buoyancy, h = 0, and the norms of the null-space test: ||G t|| / ||t|| < nstol ||D||_inf for the
+     * constant pressure t, nstol = 1e-7 (KSPRemovePressureNullspace_BSSCR, ksp_pressure_nullspace.c:139-158;
+     * BSSCR.c:391).  With particle quadrature G t is usually not zero, and the constant is then part of the
+     * solution. */
     double dir[3];
     ust_buoyancy_direction(ctx, dir);
-    CKD(ctx, ust_k_force_dir(&ctx->grid, ctx->WF, gravity, dir, ctx->mask_d, ctx->f, ctx->stream));
-    CKD(ctx, ust_k_fill_f64(ctx->h, 0.0, ne, ctx->stream));
+    CKD(ctx, ust_k_derive(&ctx->grid, ctx->WK, ctx->WG, ctx->WF, gravity, dir, ctx->mask_d, ctx->approxS, ctx->f, ctx->h,
+                          ctx->partial, ctx->scal_h + SC_T0, ctx->stream));
+    /* f = buoyancy - K_{free,bc} u_bc ; h = -G_bc^T u_bc */
     if (ctx->bc_nonzero) { /* homogeneous Dirichlet values lift nothing */
         CKD(ctx, ust_k_lift_K(&ctx->grid, ctx->WK, ctx->mask_d, ctx->bcval_d, ctx->f, ctx->stream));
         CKD(ctx, ust_k_apply_Gt(&ctx->grid, ctx->WG, ctx->mask_d, ctx->bcval_d, ctx->h, 1, ctx->stream));
     }
-    /* is the constant pressure t in the null space of G?  ||G t|| / ||t|| < nstol ||D||_inf, nstol = 1e-7
-     * (KSPRemovePressureNullspace_BSSCR, ksp_pressure_nullspace.c:139-158; BSSCR.c:391).  With particle
-     * quadrature G t is usually not zero, and the constant is then part of the solution. */
+    CKD(ctx, ust_stream_sync(ctx->stream));
     {
-        double g1, gnorm;
-        CKD(ctx, ust_k_fill_f64(ctx->tmpp, 1.0, ne, ctx->stream));
-        CKD(ctx, ust_k_apply_G(&ctx->grid, ctx->WG, ctx->mask_d, ctx->tmpp, ctx->tmpv, ctx->stream));
-        CKD(ctx, ust_k_dot_f64(ctx->tmpv, ctx->tmpv, nd, ctx->partial, ctx->scal + SC_T0, ctx->stream));
-        CKD(ctx, ust_read_scalar(ctx, SC_T0, &g1));
-        CKD(ctx, ust_k_apply_Gt(&ctx->grid, ctx->WG, ctx->mask_d, ctx->tmpv, ctx->tmpp, 2, ctx->stream));
-        CKD(ctx, ust_k_absmax_f64(ctx->tmpp, ne, ctx->partial, ctx->scal + SC_T0, ctx->stream));
-        CKD(ctx, ust_read_scalar(ctx, SC_T0, &gnorm));
-        ctx->ns_ratio = gnorm > 0 ? sqrt(g1) / sqrt((double)ne) / gnorm : 0.0;
+        const double g1 = ctx->scal_h[SC_T0], gnorm = ctx->scal_h[SC_T0 + 1];
+        ctx->ns_ratio = gnorm > 0 ? sqrt(g1) / sqrt((double)ctx->nel) / gnorm : 0.0;
         ctx->nullspace = ctx->ns_ratio < 1e-7;
     }
     ctx->gravity = gravity;

@@ -84,7 +84,7 @@ struct ust_context {
     double *bcval_d, *bcval_h;
     int nullspace; /* constant pressure found in the null space of G (ksp_pressure_nullspace.c:139-158 test) */
     double ns_ratio; /* ||G 1|| / ||1|| / ||D||_inf of the last assembly */
-    double *tmpv, *tmpp; /* velocity- and pressure-sized scratch of the assembly */
+    double *tmpv; /* velocity-sized scratch */
     void *kwork;         /* K u workspace (per-tile node partials) in FP64 elements, for every level's grid */
     size_t kwork_len;
     /* assembly */

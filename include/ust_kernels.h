@@ -228,6 +228,12 @@ int ust_k_element_f_dir(const ust_grid *g, const double *WF, double gravity, con
                         int count, double *fe, void *stream);
 /* approxS_e = sum_v G_e[v]^2 / K_e[v][v] (UzawaPreconditionerTerm.c:200-212) */
 int ust_k_uzawa_diag(const ust_grid *g, const double *WK, const double *WG, double *approxS, void *stream);
+/* What an assembly derives from the weights: approxS as ust_k_uzawa_diag, f as ust_k_force_dir from zero, h = 0, and
+ * norms[0] = ||G 1||^2 over the free dofs, norms[1] = the largest row sum of |G^T| over them.  partial: 2048 doubles;
+ * norms: 2 doubles the device can write (pinned host memory: valid after a stream synchronisation). */
+int ust_k_derive(const ust_grid *g, const double *WK, const double *WG, const double *WF, double gravity,
+                 const double *dir, const unsigned char *mask, double *approxS, double *f, double *h, double *partial,
+                 double *norms, void *stream);
 
 /* --- swarm advection and re-sort (SwarmAdvector.c:288-313, TimeIntegrand.c:221-330) --- */
 /* Per particle: position from (cell, xi), Euler (order 1) or midpoint (order 2) step through the Q1 velocity

@@ -502,3 +502,51 @@ def test_particle_weights_of_empty_elements(dim, nel):
     assert np.max(np.abs(WF.sum(0) - 2.0 * mass)) < 1e-14 * mass.max() * 10
     for a in d:
         a.free()
+
+
+# fewer elements than a block, partial blocks, and more than the passes' blocks take at once (1024 x 256)
+@pytest.mark.parametrize("dim,nel", [(2, (5, 3)), (2, (600, 500)), (3, (3, 2, 5)), (3, (70, 65, 60))])
+def test_derived_terms_of_an_assembly(dim, nel):
+    """ust_k_derive on random weights and masks: approxS as ust_k_uzawa_diag (the same device code: bit-equal), h = 0, and
+    f, ||G 1||^2 and the largest row sum of |G^T| against NumPy sums (up to a few hundred roundings: 1e-13)."""
+    import ctypes as C
+    import earthbyte_underworld_amd as ust  # noqa: F401  (loads the library)
+    from earthbyte_underworld_amd import _lib as L
+    from tests.test_gpu_operators import _Dev, _grid
+    lib = L.load()
+    g = _grid(dim, nel)
+    ne, nv = int(np.prod(nel)), 1 << dim
+    nn = [k + 1 for k in nel]
+    n = int(np.prod(nn))
+    rng = np.random.default_rng(8)
+    wl = lib.ust_k_weights_len(C.byref(g))
+    WG, WF = rng.uniform(0.5, 1.0, (nv, ne)), rng.normal(size=(nv, ne))
+    mask = (rng.random((n, dim)) < 0.2).astype(np.uint8)
+    dirn = np.array([0.0, -1.0, 0.3])
+    dW, dG, dF = _Dev(lib, rng.uniform(0.1, 1.0, wl)), _Dev(lib, WG), _Dev(lib, WF)
+    dm, da, da2 = _Dev(lib, mask), _Dev(lib, np.full(ne, np.nan)), _Dev(lib, np.zeros(ne))
+    df, dh = _Dev(lib, np.full(n * dim, np.nan)), _Dev(lib, np.full(ne, np.nan))
+    dp, dn = _Dev(lib, np.zeros(2048)), _Dev(lib, np.zeros(2))
+    assert lib.ust_k_derive(C.byref(g), dW.p, dG.p, dF.p, 2.5, dirn.ctypes.data_as(C.c_void_p), dm.p, da.p, df.p, dh.p,
+                            dp.p, dn.p, None) == 0
+    assert lib.ust_k_uzawa_diag(C.byref(g), dW.p, dG.p, da2.p, None) == 0
+    assert np.array_equal(da.get(), da2.get()) and np.all(dh.get() == 0.0)
+    e = np.arange(ne)
+    ijk = [e % nel[0], (e // nel[0]) % nel[1]] + ([e // (nel[0] * nel[1])] if dim == 3 else [])
+    f, g1, rows = np.zeros((n, dim)), np.zeros((n, dim)), np.zeros(ne)
+    for a in range(nv):
+        node = np.zeros(ne, np.int64)
+        for k in reversed(range(dim)):
+            node = node * nn[k] + ijk[k] + ((a >> k) & 1)
+        for i in range(dim):
+            Ge = -(2 * ((a >> i) & 1) - 1) / g.h[i] * (WG[a] + WG[a ^ (1 << i)])
+            np.add.at(g1[:, i], node, Ge)
+            rows += np.where(mask[node, i], 0.0, np.abs(Ge))
+            np.add.at(f[:, i], node, 2.5 * dirn[i] * WF[a])
+    f[mask != 0] = 0.0
+    norms = dn.get()
+    assert rel_err(df.get(), f.reshape(-1)) < 1e-13
+    assert abs(norms[0] - np.sum(g1[mask == 0] ** 2)) < 1e-13 * norms[0]
+    assert abs(norms[1] - rows.max()) < 1e-14 * norms[1]
+    for x in (dW, dG, dF, dm, da, da2, df, dh, dp, dn):
+        x.free()
