@@ -209,6 +209,20 @@ _SIGS = {
     "ust_k_dot_f32": (I, [vp, vp, C.c_size_t, vp, vp, vp]),
     "ust_k_cg_p_guarded_f32": (I, [vp, vp, vp, C.c_size_t, vp]),
     "ust_k_cg_xr_rr_guarded_f32": (I, [vp, vp, vp, vp, vp, vp, vp, C.c_size_t, vp, vp, vp]),
+    "ust_k_cg_parts": (I, [C.c_size_t]),
+    "ust_k_cg_begin_f64": (I, [vp, vp, vp, C.c_size_t, D, vp, vp, vp]),
+    "ust_k_cg_begin_f32": (I, [vp, D, vp, vp, C.c_size_t, D, vp, vp, vp]),
+    "ust_k_cg_dot_rz_f64": (I, [vp, vp, C.c_size_t, vp, vp]),
+    "ust_k_cg_dot_rz_zf": (I, [vp, vp, C.c_size_t, vp, vp]),
+    "ust_k_cg_dot_rz_f32": (I, [vp, vp, C.c_size_t, vp, vp]),
+    "ust_k_cg_dot_pq_f64": (I, [vp, vp, C.c_size_t, vp, vp]),
+    "ust_k_cg_dot_pq_f32": (I, [vp, vp, C.c_size_t, vp, vp]),
+    "ust_k_cg_dir_f64": (I, [vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_dir_zf": (I, [vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_dir_f32": (I, [vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_step_f64": (I, [vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_step_f32": (I, [vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_state": (I, [vp, vp, C.c_size_t, vp, vp]),
     "ust_k_apply_K_f32_bf16w": (I, [C.POINTER(Grid), vp, vp, vp, vp, vp, vp]),
     "ust_k_apply_K_residual_f32_bf16w": (I, [C.POINTER(Grid), vp, vp, vp, vp, vp, vp, vp]),
     "ust_k_apply_K_cheby_f32_bf16w": (I, [C.POINTER(Grid), vp, vp, vp, vp, vp, vp, C.c_float, C.c_float, I, vp,

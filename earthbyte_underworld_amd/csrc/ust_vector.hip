@@ -85,18 +85,6 @@ __global__ __launch_bounds__(256) void kv_dot_stage1(const T *x, const T *y, siz
     }
 }
 
-// x . y with x in FP64 and y in FP32 (the PCG's r . z with the FP32 V-cycle output z)
-__global__ __launch_bounds__(256) void kv_dot_mixed_stage1(const double *x, const float *y, size_t n,
-                                                           double *partial) {
-    __shared__ double sh[256 / 64];
-    double s = 0.0;
-    GRID_STRIDE(i, n) s += x[i] * (double)y[i];
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
-}
-
 // sum of the stage-1 partials (one 256-thread block); the total is valid in thread 0
 __device__ __forceinline__ double block_sum_partials(const double *partial, int np) {
     __shared__ double sh[4];
@@ -113,18 +101,7 @@ __global__ __launch_bounds__(256) void kv_reduce_stage2(const double *partial, i
     if (threadIdx.x == 0) out[0] = s;
 }
 
-// stage 2 of r . z fused with the CG beta update (kv_cg_beta)
-__global__ __launch_bounds__(256) void kv_reduce_beta(const double *partial, int np, double *rz, double *rz_old,
-                                                      double *c) {
-    const double s = block_sum_partials(partial, np);
-    if (threadIdx.x != 0) return;
-    rz[0] = s;
-    if (c[1] != 0.0) return;
-    c[3] = s / rz_old[0];
-    rz_old[0] = s;
-}
-
-// stage 2 of r . r fused with the CG convergence check (kv_cg_check)
+// stage 2 of r . r fused with the CG convergence check
 __global__ __launch_bounds__(256) void kv_reduce_check(const double *partial, int np, double *rr, double *c) {
     const double s = block_sum_partials(partial, np);
     if (threadIdx.x != 0) return;
@@ -185,69 +162,8 @@ __global__ void kv_cg_xr(T *x, T *r, const T *p, const T *q, const double *num, 
     }
 }
 
-// Device-side CG control block c: c[0] = stopping threshold on r.r, c[1] = state (0 running,
-// 1 converged, 2 NaN), c[2] = iterations taken, c[3] = beta.  Once the state leaves 0 every update
-// kernel below returns at once, so iterations launched past convergence change nothing.
-__global__ void kv_cg_start(const double *bb, double rtol2, double *c, double *rz_old) {
-    c[0] = rtol2 * bb[0];
-    c[1] = bb[0] > 0.0 ? 0.0 : 1.0;
-    c[2] = 0.0;
-    c[3] = 0.0;
-    rz_old[0] = 1.0;
-}
-
-__global__ void kv_cg_beta(const double *rz, double *rz_old, double *c) {
-    if (c[1] != 0.0) return;
-    c[3] = rz[0] / rz_old[0];
-    rz_old[0] = rz[0];
-}
-
-__global__ void kv_cg_p_guarded(const double *z, double *p, const double *c, size_t n) {
-    if (c[1] != 0.0) return;
-    const double beta = c[3];
-    GRID_STRIDE(i, n) p[i] = z[i] + beta * p[i];
-}
-
-__global__ void kv_cg_xr_guarded(double *x, double *r, const double *p, const double *q, const double *rz,
-                                 const double *pq, const double *c, size_t n) {
-    if (c[1] != 0.0) return;
-    const double a = rz[0] / pq[0];
-    GRID_STRIDE(i, n) {
-        x[i] += a * p[i];
-        r[i] -= a * q[i];
-    }
-}
-
-__global__ void kv_cg_p_guarded_zf(const float *z, double *p, const double *c, size_t n) {
-    if (c[1] != 0.0) return;
-    const double beta = c[3];
-    GRID_STRIDE(i, n) p[i] = (double)z[i] + beta * p[i];
-}
-
-// x += a p, r -= a q and the block partials of r . r (zero partials once converged, so the stage-2 sum is 0
-// and the check kernel ignores it)
-__global__ __launch_bounds__(256) void kv_cg_xr_rr_guarded(double *x, double *r, const double *p, const double *q,
-                                                           const double *rz, const double *pq, const double *c,
-                                                           size_t n, double *partial) {
-    __shared__ double sh[256 / 64];
-    double s = 0.0;
-    if (c[1] == 0.0) {
-        const double a = rz[0] / pq[0];
-        GRID_STRIDE(i, n) {
-            x[i] += a * p[i];
-            const double ri = r[i] - a * q[i];
-            r[i] = ri;
-            s += ri * ri;
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
-    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) partial[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
-}
-
-// The FP32 velocity PCG inside FP64 iterative refinement: p = z + beta p, and x += a p, r -= a q with the
-// block partials of r . r accumulated in FP64
+// p = z + beta p, and x += a p, r -= a q with the block partials of r . r accumulated in FP64, as separate kernels
+// guarded by a control block c (c[0] threshold on r.r, c[1] state, c[2] iterations, c[3] beta)
 __global__ void kv_cg_p_guarded_f32(const float *z, float *p, const double *c, size_t n) {
     if (c[1] != 0.0) return;
     const float beta = (float)c[3];
@@ -362,23 +278,216 @@ __global__ __launch_bounds__(256) void kv4_cg_p_guarded_f32(const float *__restr
     for (size_t i = 4 * n4 + gid(); i < n; i += gstride()) p[i] = z[i] + beta * p[i];
 }
 
-static inline bool al16(const void *a) { return ((uintptr_t)a & 15u) == 0; }
+// ------------------------------------------------------------------------------------------
+// The inner CG with its scalars on the device, three vector kernels per iteration and no reduction kernels between them:
+// every dot product leaves one partial sum per workgroup (at most UST_CG_PARTS), and the kernel that needs the scalar
+// sums them in each of its workgroups, in one fixed order, so all of them hold the same value.  A separate one-workgroup
+// reduction cost a launch of 4-5 us in a chain where most kernels take 3-6 us; reading 8 KB of partials from L2 in every
+// workgroup costs about 1 us, and starting a solve takes one kernel instead of six.  Whole solves with reduction kernels
+// and now: 2D 64x64 FP64 136.0 -> 129.6 ms, 3D 24x16x16 FP64 699 -> 661 ms, 64x64x32 with FP32 PCG 371 -> 351 ms.
+//
+// Control block c: c[0] = rtol^2, c[1] = state (0 running, 1 converged, 2 NaN), c[2] = iterations taken when the state
+// was last decided, c[3] = r.z of this iteration, c[4] = iterations done, c[5] = r.z of the previous one, c[6] = the
+// threshold on r.r.  The direction kernel decides the state of the iterations before it: its workgroup 0 writes c[1],
+// c[2], c[3] and c[6] while the others may still read them, which is safe since each workgroup decides from the same
+// sums, and c[1] only changes to the state that they all find (a workgroup reading the new state stops as it would have
+// done by itself).  c[4] and c[5] are written by the step kernel, which reads neither.  Once the state has left 0 both
+// kernels return, so iterations launched past convergence change nothing.
+// ------------------------------------------------------------------------------------------
+#define CG_RZ 0
+#define CG_PQ UST_CG_PARTS
+#define CG_RR (2 * UST_CG_PARTS)
 
-// y = (float)(s x): the FP64 residual scaled to unit norm for the FP32 correction solve
-__global__ void kv_d2f_scaled(const double *x, float *y, double s, size_t n) {
-    GRID_STRIDE(i, n) y[i] = (float)(s * x[i]);
+// four consecutive values, one or two 16-byte accesses
+template <typename T>
+struct alignas(16) V4 {
+    T v[4];
+};
+
+__device__ __forceinline__ void block_partial(double s, double *out) {
+    __shared__ double sh[4];
+    for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
+
+// sums of na partials at a and nb at b, and the control block, the same in every thread of every workgroup
+struct CgSums {
+    double a, b, c[7];
+};
+__device__ __forceinline__ CgSums cg_sums(const double *a, int na, const double *b, int nb, const double *c) {
+    __shared__ double sh[8 + 7];
+    double sa = 0.0, sb = 0.0;
+    if (threadIdx.x < 7) sh[8 + threadIdx.x] = c[threadIdx.x];
+#pragma unroll
+    for (int r = 0; r < UST_CG_PARTS / 256; r++) {
+        const int i = threadIdx.x + 256 * r;
+        if (i < na) sa += a[i];
+        if (i < nb) sb += b[i];
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        sa += __shfl_xor(sa, off, 64);
+        sb += __shfl_xor(sb, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        sh[threadIdx.x >> 6] = sa;
+        sh[4 + (threadIdx.x >> 6)] = sb;
+    }
+    __syncthreads();
+    CgSums o;
+    o.a = (sh[0] + sh[1]) + (sh[2] + sh[3]);
+    o.b = (sh[4] + sh[5]) + (sh[6] + sh[7]);
+    for (int k = 0; k < 7; k++) o.c[k] = sh[8 + k];
+    return o;
+}
+
+// the state that the sums decide, with the threshold: before the first iteration rr is b.b
+__device__ __forceinline__ double cg_state(const CgSums &s, double rr, double *thr) {
+    if (s.c[1] != 0.0) return s.c[1];
+    if (s.c[4] == 0.0) {
+        *thr = s.c[0] * rr;
+        return rr > 0.0 ? 0.0 : 1.0;
+    }
+    *thr = s.c[6];
+    return !(rr == rr) ? 2.0 : rr <= s.c[6] ? 1.0 : 0.0;
+}
+
+// x = 0, r = s b (in r's type), partials of r.r, the control block
+template <typename T>
+__global__ __launch_bounds__(256) void kv_cg_begin(const double *__restrict__ b, double s, T *__restrict__ x,
+                                                   T *__restrict__ r, size_t n, double rtol2, double *c, double *part) {
+    double acc = 0.0;
+    for (size_t i = gid(); i < n; i += gstride()) {
+        const T v = (T)(s * b[i]);
+        x[i] = (T)0;
+        r[i] = v;
+        acc += (double)v * (double)v;
+    }
+    if (blockIdx.x == 0 && threadIdx.x < 7) c[threadIdx.x] = threadIdx.x == 0 ? rtol2 : threadIdx.x == 5 ? 1.0 : 0.0;
+    block_partial(acc, part + CG_RR);
+}
+
+// partials of x . y
+template <typename TX, typename TY>
+__global__ __launch_bounds__(256) void kv_dot_part(const TX *__restrict__ x, const TY *__restrict__ y, size_t n,
+                                                   double *part) {
+    double s = 0.0;
+    const size_t n4 = n / 4;
+    for (size_t i = gid(); i < n4; i += gstride()) {
+        const V4<TX> a = ((const V4<TX> *)x)[i];
+        const V4<TY> b = ((const V4<TY> *)y)[i];
+#pragma unroll
+        for (int k = 0; k < 4; k++) s += (double)a.v[k] * (double)b.v[k];
+    }
+    for (size_t i = 4 * n4 + gid(); i < n; i += gstride()) s += (double)x[i] * (double)y[i];
+    block_partial(s, part);
+}
+
+// direction: p = z + (r.z / previous r.z) p, p = z in the first iteration (p is not read)
+template <typename TZ, typename TP>
+__global__ __launch_bounds__(256) void kv_cg_dir(const TZ *__restrict__ z, TP *__restrict__ p, double *c,
+                                                 const double *part, int nrz, int nrr, size_t n) {
+    const size_t n4 = n / 4;
+    size_t i = gid();
+    V4<TZ> zv = {};
+    V4<TP> pv = {};
+    if (i < n4) { /* the first vectors are on their way while the sums are formed */
+        zv = ((const V4<TZ> *)z)[i];
+        pv = ((const V4<TP> *)p)[i];
+    }
+    const CgSums s = cg_sums(part + CG_RZ, nrz, part + CG_RR, nrr, c);
+    double thr = 0.0;
+    const double state = cg_state(s, s.b, &thr);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && s.c[1] == 0.0) {
+        c[1] = state;
+        c[2] = s.c[4];
+        c[3] = s.a;
+        c[6] = thr;
+    }
+    if (state != 0.0) return;
+    const bool first = s.c[4] == 0.0;
+    const TP beta = (TP)(s.a / s.c[5]);
+    while (i < n4) {
+        V4<TP> o;
+#pragma unroll
+        for (int k = 0; k < 4; k++) o.v[k] = first ? (TP)zv.v[k] : (TP)zv.v[k] + beta * pv.v[k];
+        ((V4<TP> *)p)[i] = o;
+        i += gstride();
+        if (i < n4) {
+            zv = ((const V4<TZ> *)z)[i];
+            pv = ((const V4<TP> *)p)[i];
+        }
+    }
+    for (size_t j = 4 * n4 + gid(); j < n; j += gstride()) p[j] = first ? (TP)z[j] : (TP)z[j] + beta * p[j];
+}
+
+// step: a = r.z / p.q, x += a p, r -= a q, partials of r.r
+template <typename T>
+__global__ __launch_bounds__(256) void kv_cg_step(T *__restrict__ x, T *__restrict__ r, const T *__restrict__ p,
+                                                  const T *__restrict__ q, double *c, double *part, int npq, size_t n) {
+    const size_t n4 = n / 4;
+    size_t i = gid();
+    V4<T> xv = {}, rv = {}, pv = {}, qv = {};
+    if (i < n4) {
+        xv = ((const V4<T> *)x)[i];
+        rv = ((const V4<T> *)r)[i];
+        pv = ((const V4<T> *)p)[i];
+        qv = ((const V4<T> *)q)[i];
+    }
+    const CgSums s = cg_sums(part + CG_PQ, npq, nullptr, 0, c);
+    if (s.c[1] != 0.0) return;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        c[4] = s.c[4] + 1.0;
+        c[5] = s.c[3];
+    }
+    const T a = (T)(s.c[3] / s.a);
+    double acc = 0.0;
+    while (i < n4) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            xv.v[k] += a * pv.v[k];
+            rv.v[k] -= a * qv.v[k];
+            acc += (double)rv.v[k] * (double)rv.v[k];
+        }
+        ((V4<T> *)x)[i] = xv;
+        ((V4<T> *)r)[i] = rv;
+        i += gstride();
+        if (i < n4) {
+            xv = ((const V4<T> *)x)[i];
+            rv = ((const V4<T> *)r)[i];
+            pv = ((const V4<T> *)p)[i];
+            qv = ((const V4<T> *)q)[i];
+        }
+    }
+    for (size_t j = 4 * n4 + gid(); j < n; j += gstride()) {
+        x[j] += a * p[j];
+        const T ri = r[j] - a * q[j];
+        r[j] = ri;
+        acc += (double)ri * (double)ri;
+    }
+    block_partial(acc, part + CG_RR);
+}
+
+// the state after the iterations so far, for the host (pinned memory)
+__global__ __launch_bounds__(256) void kv_cg_state(double *c, const double *part, int nrr, double *host) {
+    const CgSums s = cg_sums(part + CG_RR, nrr, nullptr, 0, c);
+    if (threadIdx.x != 0) return;
+    double thr = 0.0;
+    const double state = cg_state(s, s.a, &thr);
+    if (s.c[1] == 0.0 && s.c[4] != 0.0) {
+        c[1] = state;
+        c[2] = s.c[4];
+    }
+    host[0] = state;
+    host[1] = s.c[1] != 0.0 ? s.c[2] : s.c[4];
+}
+
+static inline bool al16(const void *a) { return ((uintptr_t)a & 15u) == 0; }
 
 // y += s x with x in FP32: the correction of a refinement step
 __global__ void kv_axpy_f32_to_f64(double s, const float *x, double *y, size_t n) {
     GRID_STRIDE(i, n) y[i] += s * (double)x[i];
-}
-
-__global__ void kv_cg_check(const double *rr, double *c) {
-    if (c[1] != 0.0) return;
-    c[2] += 1.0;
-    if (!(rr[0] == rr[0])) c[1] = 2.0;
-    else if (rr[0] <= c[0]) c[1] = 1.0;
 }
 
 template <typename T>
@@ -425,6 +534,33 @@ __global__ void kv_residual(const T *b, const T *Ax, T *r, size_t n) {
         return UST_OK;                                                                                 \
     } while (0)
 
+// vectors of the device-controlled CG: 16-byte aligned
+template <typename... P>
+static inline bool cg_vectors(size_t n, P... p) {
+    return n > 0 && ((p && al16(p)) && ...);
+}
+template <typename TX, typename TY>
+static int cg_dot(const TX *x, const TY *y, size_t n, double *part, void *stream) {
+    if (!cg_vectors(n, x, y)) return UST_EINVAL;
+    hipLaunchKernelGGL((kv_dot_part<TX, TY>), dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), x, y, n, part);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+template <typename TZ, typename TP>
+static int cg_dir(const TZ *z, TP *p, double *c, double *part, int nrz, size_t n, void *stream) {
+    if (!cg_vectors(n, z, p) || nrz < 1 || nrz > UST_CG_PARTS) return UST_EINVAL;
+    hipLaunchKernelGGL((kv_cg_dir<TZ, TP>), dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), z, p, c, part, nrz,
+                       (int)rgrid(n), n);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+template <typename T>
+static int cg_step(T *x, T *r, const T *p, const T *q, double *c, double *part, int npq, size_t n, void *stream) {
+    if (!cg_vectors(n, x, r, p, q) || npq < 1 || npq > UST_CG_PARTS) return UST_EINVAL;
+    hipLaunchKernelGGL(kv_cg_step<T>, dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), x, r, p, q, c, part, npq, n);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
 extern "C" {
 
 int ust_k_fill_f64(double *x, double v, size_t n, void *stream) { LV(kv_fill<double>, n, x, v, n); }
@@ -517,59 +653,61 @@ int ust_k_cg_update_xr_f32(float *x, float *r, const float *p, const float *q, c
     LV(kv_cg_xr<float>, n, x, r, p, q, num, den, n);
 }
 
-int ust_k_cg_start(const double *bb, double rtol2, double *ctl, double *rz_old, void *stream) {
-    hipLaunchKernelGGL(kv_cg_start, dim3(1), dim3(1), 0, ust_stream(stream), bb, rtol2, ctl, rz_old);
+int ust_k_cg_parts(size_t n) { return (int)rgrid(n); }
+int ust_k_cg_begin_f64(const double *b, double *x, double *r, size_t n, double rtol2, double *c, double *part,
+                       void *stream) {
+    if (!cg_vectors(n, b, x, r)) return UST_EINVAL;
+    hipLaunchKernelGGL(kv_cg_begin<double>, dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), b, 1.0, x, r, n, rtol2, c,
+                       part);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
-int ust_k_cg_beta(const double *rz, double *rz_old, double *ctl, void *stream) {
-    hipLaunchKernelGGL(kv_cg_beta, dim3(1), dim3(1), 0, ust_stream(stream), rz, rz_old, ctl);
+int ust_k_cg_begin_f32(const double *b, double s, float *x, float *r, size_t n, double rtol2, double *c, double *part,
+                       void *stream) {
+    if (!cg_vectors(n, b, x, r)) return UST_EINVAL;
+    hipLaunchKernelGGL(kv_cg_begin<float>, dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), b, s, x, r, n, rtol2, c,
+                       part);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
-int ust_k_cg_p_guarded_f64(const double *z, double *p, const double *ctl, size_t n, void *stream) {
-    LV(kv_cg_p_guarded, n, z, p, ctl, n);
+int ust_k_cg_dot_rz_f64(const double *r, const double *z, size_t n, double *part, void *stream) {
+    return cg_dot(r, z, n, part + CG_RZ, stream);
 }
-int ust_k_cg_xr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
-                            const double *pq, const double *ctl, size_t n, void *stream) {
-    LV(kv_cg_xr_guarded, n, x, r, p, q, rz, pq, ctl, n);
+int ust_k_cg_dot_rz_zf(const double *r, const float *z, size_t n, double *part, void *stream) {
+    return cg_dot(r, z, n, part + CG_RZ, stream);
 }
-int ust_k_dot_mixed_beta(const double *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
-                         double *ctl, void *stream) {
-    const unsigned g = rgrid(n);
-    hipLaunchKernelGGL(kv_dot_mixed_stage1, dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
-    hipLaunchKernelGGL(kv_reduce_beta, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rz, rz_old, ctl);
+int ust_k_cg_dot_rz_f32(const float *r, const float *z, size_t n, double *part, void *stream) {
+    return cg_dot(r, z, n, part + CG_RZ, stream);
+}
+int ust_k_cg_dot_pq_f64(const double *p, const double *q, size_t n, double *part, void *stream) {
+    return cg_dot(p, q, n, part + CG_PQ, stream);
+}
+int ust_k_cg_dot_pq_f32(const float *p, const float *q, size_t n, double *part, void *stream) {
+    return cg_dot(p, q, n, part + CG_PQ, stream);
+}
+int ust_k_cg_dir_f64(const double *z, double *p, double *c, double *part, int nrz, size_t n, void *stream) {
+    return cg_dir(z, p, c, part, nrz, n, stream);
+}
+int ust_k_cg_dir_zf(const float *z, double *p, double *c, double *part, int nrz, size_t n, void *stream) {
+    return cg_dir(z, p, c, part, nrz, n, stream);
+}
+int ust_k_cg_dir_f32(const float *z, float *p, double *c, double *part, int nrz, size_t n, void *stream) {
+    return cg_dir(z, p, c, part, nrz, n, stream);
+}
+int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, double *c, double *part, int npq, size_t n,
+                      void *stream) {
+    return cg_step(x, r, p, q, c, part, npq, n, stream);
+}
+int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, double *c, double *part, int npq, size_t n,
+                      void *stream) {
+    return cg_step(x, r, p, q, c, part, npq, n, stream);
+}
+int ust_k_cg_state(double *c, const double *part, size_t n, double *host, void *stream) {
+    hipLaunchKernelGGL(kv_cg_state, dim3(1), dim3(256), 0, ust_stream(stream), c, part, (int)rgrid(n), host);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
-int ust_k_dot_beta_f64(const double *x, const double *y, size_t n, double *partial, double *rz, double *rz_old,
-                       double *ctl, void *stream) {
-    const unsigned g = rgrid(n);
-    hipLaunchKernelGGL((kv_dot_stage1<double, true>), dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
-    hipLaunchKernelGGL(kv_reduce_beta, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rz, rz_old, ctl);
-    UST_LAUNCH_CHECK();
-    return UST_OK;
-}
-int ust_k_dot_mixed(const double *x, const float *y, size_t n, double *partial, double *out, void *stream) {
-    const unsigned g = rgrid(n);
-    hipLaunchKernelGGL(kv_dot_mixed_stage1, dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
-    hipLaunchKernelGGL(kv_reduce_stage2, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, out);
-    UST_LAUNCH_CHECK();
-    return UST_OK;
-}
-int ust_k_cg_p_guarded_zf(const float *z, double *p, const double *ctl, size_t n, void *stream) {
-    LV(kv_cg_p_guarded_zf, n, z, p, ctl, n);
-}
-int ust_k_cg_xr_rr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
-                               const double *pq, double *ctl, size_t n, double *partial, double *rr,
-                               void *stream) {
-    const unsigned g = rgrid(n);
-    hipLaunchKernelGGL(kv_cg_xr_rr_guarded, dim3(g), dim3(256), 0, ust_stream(stream), x, r, p, q, rz, pq, ctl, n,
-                       partial);
-    hipLaunchKernelGGL(kv_reduce_check, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rr, ctl);
-    UST_LAUNCH_CHECK();
-    return UST_OK;
-}
+
 int ust_k_cheby_first_from_f64(const double *b, float *b32, const float *invd, float *d, float *x, float c2,
                                size_t n, void *stream) {
     LV(kv_cheby_first_from64, n, b, b32, invd, d, x, c2, n);
@@ -591,29 +729,9 @@ int ust_k_cg_xr_rr_guarded_f32(float *x, float *r, const float *p, const float *
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
-int ust_k_dot_beta_f32(const float *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
-                       double *ctl, void *stream) {
-    const unsigned g = rgrid(n);
-    if (al16(x) && al16(y))
-        hipLaunchKernelGGL(kv4_dot_f32, dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
-    else
-        hipLaunchKernelGGL((kv_dot_stage1<float, true>), dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
-    hipLaunchKernelGGL(kv_reduce_beta, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rz, rz_old, ctl);
-    UST_LAUNCH_CHECK();
-    return UST_OK;
-}
-int ust_k_copy_f64_to_f32_scaled(const double *x, float *y, double s, size_t n, void *stream) {
-    LV(kv_d2f_scaled, n, x, y, s, n);
-}
 int ust_k_axpy_f32_to_f64(double s, const float *x, double *y, size_t n, void *stream) {
     LV(kv_axpy_f32_to_f64, n, s, x, y, n);
 }
-int ust_k_cg_check(const double *rr, double *ctl, void *stream) {
-    hipLaunchKernelGGL(kv_cg_check, dim3(1), dim3(1), 0, ust_stream(stream), rr, ctl);
-    UST_LAUNCH_CHECK();
-    return UST_OK;
-}
-
 int ust_k_cheby_step_f64(const double *b, const double *Ax, const double *invd, double *d, double *x, double c1,
                          double c2, size_t n, void *stream) {
     LV(kv_cheby<double>, n, b, Ax, invd, d, x, c1, c2, c1 == 0.0 ? 1 : 0, n);

@@ -60,6 +60,7 @@ int ust_create(ust_context **out, int device) {
         return rc;
     }
     rc = ust_dev_malloc((void **)&ctx->partial, 2048 * sizeof(double));
+    if (rc == UST_OK) rc = ust_dev_malloc((void **)&ctx->cgpart, 3 * UST_CG_PARTS * sizeof(double));
     if (rc == UST_OK) rc = ust_dev_malloc((void **)&ctx->scal, SC_COUNT * sizeof(double));
     if (rc == UST_OK) rc = ust_host_malloc_pinned((void **)&ctx->scal_h, SC_COUNT * sizeof(double));
     if (rc == UST_OK) rc = ust_dev_malloc((void **)&ctx->mats_d, UST_MAX_MATERIALS * sizeof(ust_material));
@@ -130,6 +131,7 @@ void ust_destroy(ust_context *ctx) {
     free_swarm(ctx);
     ust_mlp_free(ctx);
     DFREE(ctx->partial);
+    DFREE(ctx->cgpart);
     DFREE(ctx->scal);
     DFREE(ctx->mats_d);
     if (ctx->scal_h) ust_host_free_pinned(ctx->scal_h);

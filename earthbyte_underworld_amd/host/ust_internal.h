@@ -9,9 +9,9 @@
 #define UST_MAX_CHEBY 24
 
 /* device scalar slots */
-enum { SC_RZ = 0, SC_RZOLD, SC_PQ, SC_RR, SC_BB, SC_SUM, SC_T0, SC_T1, SC_T2, SC_T3,
+enum { SC_SUM = 0, SC_T0, SC_T1, SC_T2, SC_T3,
        SC_O_RZ, SC_O_RZOLD, SC_O_PQ, SC_O_RR,
-       SC_CG = 16, /* 4 slots: device-controlled inner CG (threshold, state, iterations, beta) */
+       SC_CG = 16, /* 7 slots: device-controlled inner CG (ust_k_cg_begin_f64) */
        SC_COUNT = 32 };
 
 typedef struct {
@@ -106,6 +106,7 @@ struct ust_context {
     int nc;
     /* solver work */
     double *partial, *scal, *scal_h;
+    double *cgpart;                   /* inner CG: partial sums of r.z, p.q and r.r */
     double *vr, *vz, *vp, *vq, *vt;   /* FP64 velocity work (inner PCG) */
     double *vx;                       /* inner PCG iterate */
     void *pcg_exec[3];                /* captured inner PCG iteration (FP64 / FP32 V-cycle / FP32 PCG), NULL if stale */

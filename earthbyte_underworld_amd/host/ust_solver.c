@@ -474,7 +474,8 @@ static int dotv(ust_context *ctx, const double *a, const double *b, size_t n, in
  * once into a HIP graph. */
 static int pcg_iteration(ust_context *ctx, int pc32) {
     size_t n = (size_t)ctx->ndof;
-    double *r = ctx->vr, *z = ctx->vz, *p = ctx->vp, *q = ctx->vq, *sc = ctx->scal;
+    double *r = ctx->vr, *z = ctx->vz, *p = ctx->vp, *q = ctx->vq, *c = ctx->scal + SC_CG, *part = ctx->cgpart;
+    const int np = ust_k_cg_parts(n);
     int rc;
     if (pc32) {
         /* z stays FP32 (wz): the first smoothing step rounds r into b32 itself, r . z and p = z + beta p
@@ -488,18 +489,16 @@ static int pcg_iteration(ust_context *ctx, int pc32) {
         rc = vcycle(ctx, 0, 1, L0->b32, ctx->wz, 0);
         ctx->b64_src = NULL;
         if (rc) return rc;
-        CKD(ctx, ust_k_dot_mixed_beta(r, ctx->wz, n, ctx->partial, sc + SC_RZ, sc + SC_RZOLD, sc + SC_CG, S(ctx)));
-        CKD(ctx, ust_k_cg_p_guarded_zf(ctx->wz, p, sc + SC_CG, n, S(ctx)));
+        CKD(ctx, ust_k_cg_dot_rz_zf(r, ctx->wz, n, part, S(ctx)));
+        CKD(ctx, ust_k_cg_dir_zf(ctx->wz, p, c, part, np, n, S(ctx)));
     } else {
         if ((rc = vcycle(ctx, 0, 0, r, z, 0))) return rc;
-        CKD(ctx, ust_k_dot_beta_f64(r, z, n, ctx->partial, sc + SC_RZ, sc + SC_RZOLD, sc + SC_CG, S(ctx)));
-        CKD(ctx, ust_k_cg_p_guarded_f64(z, p, sc + SC_CG, n, S(ctx)));
+        CKD(ctx, ust_k_cg_dot_rz_f64(r, z, n, part, S(ctx)));
+        CKD(ctx, ust_k_cg_dir_f64(z, p, c, part, np, n, S(ctx)));
     }
     if ((rc = lev_apply(ctx, 0, 0, p, q))) return rc;
-    CKD(ctx, ust_k_dot_f64(p, q, n, ctx->partial, sc + SC_PQ, S(ctx)));
-    /* x, r update, r . r and the convergence check */
-    CKD(ctx, ust_k_cg_xr_rr_guarded_f64(ctx->vx, r, p, q, sc + SC_RZ, sc + SC_PQ, sc + SC_CG, n, ctx->partial,
-                                        sc + SC_RR, S(ctx)));
+    CKD(ctx, ust_k_cg_dot_pq_f64(p, q, n, part, S(ctx)));
+    CKD(ctx, ust_k_cg_step_f64(ctx->vx, r, p, q, c, part, np, n, S(ctx)));
     return UST_OK;
 }
 
@@ -515,18 +514,22 @@ static int pcg_graph(ust_context *ctx, int pc32) {
     return UST_OK;
 }
 
+/* state and iteration count of the running inner CG */
+static int cg_state(ust_context *ctx, double *state, double *count) {
+    CKD(ctx, ust_k_cg_state(ctx->scal + SC_CG, ctx->cgpart, (size_t)ctx->ndof, ctx->scal_h + SC_CG, S(ctx)));
+    CKD(ctx, ust_stream_sync(S(ctx)));
+    *state = ctx->scal_h[SC_CG];
+    *count = ctx->scal_h[SC_CG + 1];
+    return UST_OK;
+}
+
 /* PCG: x = K^-1 b to ||r|| <= rtol ||b|| from x = 0 (KSPSolve with KSPCG, StokesBlockKSPInterface.c:242).
  * The iterations run as graph launches; the host reads the device state after the number of iterations
  * the previous inner solve needed, then after every further one. */
 static int pcg(ust_context *ctx, int pc32, const double *b, double *x, double rtol, int maxit, int *its) {
     size_t n = (size_t)ctx->ndof;
-    double *sc = ctx->scal;
     int rc;
-    CKD(ctx, ust_k_fill_f64(ctx->vx, 0.0, n, S(ctx)));
-    CKD(ctx, ust_k_fill_f64(ctx->vp, 0.0, n, S(ctx)));
-    CKD(ctx, ust_memcpy_d2d(ctx->vr, b, n * sizeof(double), S(ctx)));
-    CKD(ctx, ust_k_dot_f64(b, b, n, ctx->partial, sc + SC_BB, S(ctx)));
-    CKD(ctx, ust_k_cg_start(sc + SC_BB, rtol * rtol, sc + SC_CG, sc + SC_RZOLD, S(ctx)));
+    CKD(ctx, ust_k_cg_begin_f64(b, ctx->vx, ctx->vr, n, rtol * rtol, ctx->scal + SC_CG, ctx->cgpart, S(ctx)));
     if (ctx->use_graphs && (rc = pcg_graph(ctx, pc32))) return rc;
     int done = 0, first = ctx->pcg_hint > 2 ? ctx->pcg_hint - 1 : 1;
     double state = 0.0, count = 0.0;
@@ -538,9 +541,7 @@ static int pcg(ust_context *ctx, int pc32, const double *b, double *x, double rt
             else if ((rc = pcg_iteration(ctx, pc32))) return rc;
         }
         done += k;
-        CKD(ctx, ust_memcpy_d2h(ctx->scal_h + SC_CG + 1, sc + SC_CG + 1, 2 * sizeof(double), S(ctx)));
-        state = ctx->scal_h[SC_CG + 1];
-        count = ctx->scal_h[SC_CG + 2];
+        if ((rc = cg_state(ctx, &state, &count))) return rc;
         if (state != 0.0) break;
     }
     *its = (int)count;
@@ -555,30 +556,26 @@ static int pcg(ust_context *ctx, int pc32, const double *b, double *x, double rt
  * accumulate in FP64 and the stopping test runs on the device, as in the FP64 PCG. */
 static int pcg32_iteration(ust_context *ctx) {
     size_t n = (size_t)ctx->ndof;
-    double *sc = ctx->scal;
+    double *c = ctx->scal + SC_CG, *part = ctx->cgpart;
+    const int np = ust_k_cg_parts(n);
     ust_level *L0 = &ctx->lev[0];
     int rc = vcycle(ctx, 0, 1, ctx->wr, ctx->wz, 0);
     if (rc) return rc;
-    CKD(ctx, ust_k_dot_beta_f32(ctx->wr, ctx->wz, n, ctx->partial, sc + SC_RZ, sc + SC_RZOLD, sc + SC_CG, S(ctx)));
-    CKD(ctx, ust_k_cg_p_guarded_f32(ctx->wz, ctx->wp, sc + SC_CG, n, S(ctx)));
+    CKD(ctx, ust_k_cg_dot_rz_f32(ctx->wr, ctx->wz, n, part, S(ctx)));
+    CKD(ctx, ust_k_cg_dir_f32(ctx->wz, ctx->wp, c, part, np, n, S(ctx)));
     CKD(ctx, ust_k_apply_K_f32(&L0->g, L0->WK32, L0->mask, ctx->wp, ctx->wq, (float *)ctx->kwork, S(ctx)));
-    CKD(ctx, ust_k_dot_f32(ctx->wp, ctx->wq, n, ctx->partial, sc + SC_PQ, S(ctx)));
-    CKD(ctx, ust_k_cg_xr_rr_guarded_f32(ctx->wx, ctx->wr, ctx->wp, ctx->wq, sc + SC_RZ, sc + SC_PQ, sc + SC_CG, n,
-                                        ctx->partial, sc + SC_RR, S(ctx)));
+    CKD(ctx, ust_k_cg_dot_pq_f32(ctx->wp, ctx->wq, n, part, S(ctx)));
+    CKD(ctx, ust_k_cg_step_f32(ctx->wx, ctx->wr, ctx->wp, ctx->wq, c, part, np, n, S(ctx)));
     return UST_OK;
 }
 
-/* FP32 PCG on K e = wr (wr at unit norm) to ||r|| <= rtol from e = 0; iterations as in pcg(), the launches
+/* FP32 PCG on K e = s r (at unit norm) to a residual <= rtol from e = 0; iterations as in pcg(), the launches
  * before the first check taken from the same refinement step of the previous solve (steps differ in length, so
  * one shared count would launch iterations past convergence) */
-static int pcg32(ust_context *ctx, int step, double rtol, int maxit, int *its) {
+static int pcg32(ust_context *ctx, int step, const double *r, double s, double rtol, int maxit, int *its) {
     size_t n = (size_t)ctx->ndof;
-    double *sc = ctx->scal;
     int rc;
-    CKD(ctx, ust_k_fill_f32(ctx->wx, 0.0f, n, S(ctx)));
-    CKD(ctx, ust_k_fill_f32(ctx->wp, 0.0f, n, S(ctx)));
-    CKD(ctx, ust_k_dot_f32(ctx->wr, ctx->wr, n, ctx->partial, sc + SC_BB, S(ctx)));
-    CKD(ctx, ust_k_cg_start(sc + SC_BB, rtol * rtol, sc + SC_CG, sc + SC_RZOLD, S(ctx)));
+    CKD(ctx, ust_k_cg_begin_f32(r, s, ctx->wx, ctx->wr, n, rtol * rtol, ctx->scal + SC_CG, ctx->cgpart, S(ctx)));
     if (ctx->use_graphs && !ctx->pcg_exec[2]) {
         CKD(ctx, ust_graph_begin(S(ctx)));
         if ((rc = pcg32_iteration(ctx))) {
@@ -598,9 +595,7 @@ static int pcg32(ust_context *ctx, int step, double rtol, int maxit, int *its) {
             else if ((rc = pcg32_iteration(ctx))) return rc;
         }
         done += k;
-        CKD(ctx, ust_memcpy_d2h(ctx->scal_h + SC_CG + 1, sc + SC_CG + 1, 2 * sizeof(double), S(ctx)));
-        state = ctx->scal_h[SC_CG + 1];
-        count = ctx->scal_h[SC_CG + 2];
+        if ((rc = cg_state(ctx, &state, &count))) return rc;
         if (state != 0.0) break;
     }
     *its = (int)count;
@@ -639,8 +634,7 @@ static int pcg_refined(ust_context *ctx, const double *b, double *x, double rtol
         const double rn = sqrt(rr), want = rtol * sqrt(bb) / rn;
         const double tau = want > IR_TAU_MIN ? want : IR_TAU_MIN;
         int it = 0;
-        CKD(ctx, ust_k_copy_f64_to_f32_scaled(r, ctx->wr, 1.0 / rn, n, S(ctx)));
-        if ((rc = pcg32(ctx, k, tau, maxit - total, &it))) return rc;
+        if ((rc = pcg32(ctx, k, r, 1.0 / rn, tau, maxit - total, &it))) return rc;
         total += it;
         CKD(ctx, ust_k_axpy_f32_to_f64(rn, ctx->wx, acc, n, S(ctx)));
         (*steps)++;

@@ -434,38 +434,40 @@ int ust_k_cg_update_xr_f64(double *x, double *r, const double *p, const double *
                            const double *den, size_t n, void *stream);
 int ust_k_cg_update_xr_f32(float *x, float *r, const float *p, const float *q, const double *num,
                            const double *den, size_t n, void *stream);
-/* Device-controlled CG (no host round trip per iteration).  ctl[4] on the device: ctl[0] = stopping
- * threshold rtol2 * b.b, ctl[1] = state (0 running, 1 converged, 2 NaN), ctl[2] = iterations, ctl[3] =
- * beta.  start: ctl from bb = b.b and rz_old = 1 (with p = 0 the first update gives p = z).  beta:
- * ctl[3] = rz/rz_old, rz_old = rz.  The guarded updates and check do nothing once ctl[1] != 0, so
- * iterations launched past convergence leave x and r unchanged (KSPSolve's loop with the rnorm test
- * of KSPConvergedDefault, evaluated on the device). */
-int ust_k_cg_start(const double *bb, double rtol2, double *ctl, double *rz_old, void *stream);
-int ust_k_cg_beta(const double *rz, double *rz_old, double *ctl, void *stream);
-int ust_k_cg_p_guarded_f64(const double *z, double *p, const double *ctl, size_t n, void *stream);
-int ust_k_cg_xr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
-                            const double *pq, const double *ctl, size_t n, void *stream);
-int ust_k_cg_check(const double *rr, double *ctl, void *stream);
-/* r . z (two-stage, into rz) fused with the beta update of ust_k_cg_beta; z in FP32 or FP64 */
-int ust_k_dot_mixed_beta(const double *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
-                         double *ctl, void *stream);
-int ust_k_dot_beta_f64(const double *x, const double *y, size_t n, double *partial, double *rz, double *rz_old,
-                       double *ctl, void *stream);
-/* fused forms for the FP64 PCG around the FP32 V-cycle: r . z with z in FP32; p = z + beta p with z in FP32;
- * x += a p, r -= a q together with r . r (two-stage, into rr) and the convergence check of ust_k_cg_check */
-int ust_k_dot_mixed(const double *x, const float *y, size_t n, double *partial, double *out, void *stream);
-int ust_k_cg_p_guarded_zf(const float *z, double *p, const double *ctl, size_t n, void *stream);
-int ust_k_cg_xr_rr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
-                               const double *pq, double *ctl, size_t n, double *partial, double *rr,
-                               void *stream);
-/* The FP32 velocity PCG of iterative refinement: the same steps on FP32 vectors (dots and r . r accumulated in
- * FP64 against the same control block), the scaled rounding of the FP64 residual and the FP64 correction. */
+/* Device-controlled CG: no host round trip and no reduction launch per iteration (KSPSolve's loop with the rnorm test of
+ * KSPConvergedDefault, evaluated on the device).  c: 7 doubles of control, part: 3 * UST_CG_PARTS doubles of partial sums
+ * (r.z, p.q, r.r), both on the device; vectors are 16-byte aligned.
+ *   begin:  x = 0, r = s b (s = 1 in FP64), c for a solve to ||r||^2 <= rtol2 ||b||^2
+ *   dot_rz, dot_pq: ust_k_cg_parts(n) partials; another kernel may leave its own count (at most UST_CG_PARTS) instead
+ *   dir:    the state after the iterations before this one, then p = z + beta p (p = z in the first)
+ *   step:   x += a p, r -= a q
+ *   state:  the state now, to host[0] (0 running, 1 converged, 2 NaN) and the iterations to host[1] (pinned memory)
+ * dir and step do nothing once the state is not 0: iterations launched past convergence leave x and r unchanged.
+ * zf: z in FP32, the other vectors in FP64. */
+#define UST_CG_PARTS 1024
+int ust_k_cg_parts(size_t n);
+int ust_k_cg_begin_f64(const double *b, double *x, double *r, size_t n, double rtol2, double *c, double *part,
+                       void *stream);
+int ust_k_cg_begin_f32(const double *b, double s, float *x, float *r, size_t n, double rtol2, double *c, double *part,
+                       void *stream);
+int ust_k_cg_dot_rz_f64(const double *r, const double *z, size_t n, double *part, void *stream);
+int ust_k_cg_dot_rz_zf(const double *r, const float *z, size_t n, double *part, void *stream);
+int ust_k_cg_dot_rz_f32(const float *r, const float *z, size_t n, double *part, void *stream);
+int ust_k_cg_dot_pq_f64(const double *p, const double *q, size_t n, double *part, void *stream);
+int ust_k_cg_dot_pq_f32(const float *p, const float *q, size_t n, double *part, void *stream);
+int ust_k_cg_dir_f64(const double *z, double *p, double *c, double *part, int nrz, size_t n, void *stream);
+int ust_k_cg_dir_zf(const float *z, double *p, double *c, double *part, int nrz, size_t n, void *stream);
+int ust_k_cg_dir_f32(const float *z, float *p, double *c, double *part, int nrz, size_t n, void *stream);
+int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, double *c, double *part, int npq, size_t n,
+                      void *stream);
+int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, double *c, double *part, int npq, size_t n,
+                      void *stream);
+int ust_k_cg_state(double *c, const double *part, size_t n, double *host, void *stream);
+/* p = z + beta p and x += a p, r -= a q with r.r on FP32 vectors against a control block of threshold, state, count and
+ * beta; nothing is done once the state is not 0 */
 int ust_k_cg_p_guarded_f32(const float *z, float *p, const double *ctl, size_t n, void *stream);
 int ust_k_cg_xr_rr_guarded_f32(float *x, float *r, const float *p, const float *q, const double *rz, const double *pq,
                                double *ctl, size_t n, double *partial, double *rr, void *stream);
-int ust_k_dot_beta_f32(const float *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
-                       double *ctl, void *stream);
-int ust_k_copy_f64_to_f32_scaled(const double *x, float *y, double s, size_t n, void *stream);
 int ust_k_axpy_f32_to_f64(double s, const float *x, double *y, size_t n, void *stream);
 
 /* Chebyshev smoother step (Jacobi-preconditioned).  r = b - y (y = A x given), then

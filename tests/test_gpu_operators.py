@@ -613,3 +613,76 @@ def test_fp32_product_of_a_field_with_a_large_mean(nel):
     assert rel_err(a, y64.get()) < 4e-6
     for x in (W32, W64, dm, d32, d64, y32, y64, work):
         x.free()
+
+
+# fewer dofs than a vector of four, vectors and a tail, more than one sweep of 1024 workgroups of 1024 dofs
+@pytest.mark.parametrize("n", [3, 1021, 1_050_003])
+@pytest.mark.parametrize("kind", ["f64", "zf", "f32"])
+def test_device_controlled_cg(kind, n):
+    """The device-controlled CG's kernels (begin, dots, direction, step, state) on K = tridiag(-1, 4, -1), applied on
+    the host, with z = r / 4, against the same recurrence in numpy FP64: iterations, state and x.  Bar: the recurrence
+    stops at a relative residual of 1e-8 (1e-4 in FP32) and the condition number is 3, so x and its residual agree to 3
+    times that; a launch past convergence changes nothing."""
+    import ctypes as C
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    T, TZ = (np.float32 if kind == "f32" else np.float64), (np.float64 if kind == "f64" else np.float32)
+    tp = "f32" if kind == "f32" else "f64"
+    rtol, s = (1e-4, 0.5) if kind == "f32" else (1e-8, 1.0)
+
+    def mul(v):
+        o = v.dtype.type(4) * v
+        o[1:] -= v[:-1]
+        o[:-1] -= v[1:]
+        return o
+
+    b = np.random.default_rng(n).normal(size=n)
+    db, z = _Dev(lib, b), _Dev(lib, np.zeros(n, TZ))
+    x, r, p, q = (_Dev(lib, np.full(n, np.nan, T)) for _ in range(4))  # begin and the first direction use none of it
+    c, part, host = _Dev(lib, np.zeros(7)), _Dev(lib, np.full(3072, np.nan)), _Dev(lib, np.zeros(2))
+    parts = lib.ust_k_cg_parts(n)
+    assert 1 <= parts <= 1024
+
+    def put(d, a):
+        assert lib.ust_memcpy_h2d(d.p, a.ctypes.data_as(C.c_void_p), a.nbytes, None) == 0
+
+    def begin(rtol2):
+        scale = () if tp == "f64" else (s,)
+        assert getattr(lib, f"ust_k_cg_begin_{tp}")(db.p, *scale, x.p, r.p, n, rtol2, c.p, part.p, None) == 0
+
+    def iterate(product):
+        put(z, (r.get() / 4).astype(TZ))
+        assert getattr(lib, f"ust_k_cg_dot_rz_{kind}")(r.p, z.p, n, part.p, None) == 0
+        assert getattr(lib, f"ust_k_cg_dir_{kind}")(z.p, p.p, c.p, part.p, parts, n, None) == 0
+        put(q, product(p.get()))
+        assert getattr(lib, f"ust_k_cg_dot_pq_{tp}")(p.p, q.p, n, part.p, None) == 0
+        assert getattr(lib, f"ust_k_cg_step_{tp}")(x.p, r.p, p.p, q.p, c.p, part.p, parts, n, None) == 0
+        assert lib.ust_k_cg_state(c.p, part.p, n, host.p, None) == 0
+        return tuple(host.get())
+
+    begin(rtol * rtol)
+    xr, rr, pr, rz_old = np.zeros(n), s * b, np.zeros(n), 1.0
+    for its in range(1, 60):
+        state, count = iterate(mul)
+        rz = float(rr @ rr) / 4
+        pr = rr / 4 + (rz / rz_old) * pr
+        qr = mul(pr)
+        a = rz / float(pr @ qr)
+        xr, rr, rz_old = xr + a * pr, rr - a * qr, rz
+        assert count == its
+        if state != 0:
+            break
+    assert state == 1
+    got = x.get()
+    assert np.linalg.norm(s * b - mul(got.astype(np.float64))) <= 3 * rtol * np.linalg.norm(s * b)
+    assert np.linalg.norm(got - xr) <= 3 * rtol * np.linalg.norm(xr)
+    assert iterate(mul) == (1.0, float(its)) and np.array_equal(x.get(), got)
+    # a zero right-hand side is converged at once; NaN in r.r is reported
+    for want, rhs in ((1.0, 0.0), (2.0, 1.0)):
+        put(db, np.full(n, rhs))
+        begin(1e-16)
+        assert iterate(lambda v: np.full(n, np.nan, T))[0] == want
+    # vectors off a 16-byte boundary are refused
+    assert getattr(lib, f"ust_k_cg_dir_{kind}")(C.c_void_p(z.p.value + 4), p.p, c.p, part.p, parts, n, None) == -1
+    for d in (db, x, r, p, q, z, c, part, host):
+        d.free()
