@@ -69,6 +69,12 @@ class Grid(C.Structure):
                 ("ymax", C.c_double), ("xmax", C.c_double * 3)]
 
 
+class Pass(C.Structure):  # ust_pass
+    _fields_ = [("mode", C.c_int), ("type", C.c_int), ("W", C.c_void_p), ("mask", C.c_void_p), ("u", C.c_void_p),
+                ("y", C.c_void_p), ("b", C.c_void_p), ("invd", C.c_void_p), ("d", C.c_void_p), ("xc", C.c_void_p),
+                ("c0", C.c_double), ("c1", C.c_double), ("c2", C.c_double), ("d_last", C.c_int), ("dot", C.c_void_p)]
+
+
 class SolveOpts(C.Structure):
     _fields_ = [("precision", C.c_int), ("schur_pc", C.c_int), ("mg_levels", C.c_int),
                 ("smoother_degree", C.c_int), ("cheby_ratio", C.c_double), ("outer_rtol", C.c_double),
@@ -209,6 +215,8 @@ _SIGS = {
     "ust_k_dot_f32": (I, [vp, vp, C.c_size_t, vp, vp, vp]),
     "ust_k_cg_p_guarded_f32": (I, [vp, vp, vp, C.c_size_t, vp]),
     "ust_k_cg_xr_rr_guarded_f32": (I, [vp, vp, vp, vp, vp, vp, vp, C.c_size_t, vp, vp, vp]),
+    "ust_k_apply_single": (I, [C.POINTER(Grid)]),
+    "ust_k_apply_pass": (I, [C.POINTER(Grid), C.POINTER(Pass), vp]),
     "ust_k_cg_parts": (I, [C.c_size_t]),
     "ust_k_cg_begin_f64": (I, [vp, vp, vp, C.c_size_t, D, vp, vp, vp]),
     "ust_k_cg_begin_f32": (I, [vp, D, vp, vp, C.c_size_t, D, vp, vp, vp]),

@@ -232,7 +232,17 @@ __device__ __forceinline__ bool on_tile_face(int gc, int T, int tn) {
 //   EPI_RES0    the first Jacobi-Chebyshev step from a zero guess, x = c2 invd b, then the residual
 //               r = b - K x (0 on Dirichlet dofs), in one pass: the staged velocities are c2 invd b (u is not
 //               read); y = r, d = x (the previous d is neither read nor written).
-enum { EPI_Y = 0, EPI_RES = 1, EPI_CHEBY = 2, EPI_CHEBY0 = 3, EPI_PCHEBY0 = 4, EPI_RES0 = 5 };
+//   EPI_CHEBY1  the first two Jacobi-Chebyshev steps from a zero guess: the staged velocities are x1 = c0 invd b (u is
+//               not read), then d = c1 x1 + c2 invd (b - K x1), y = x1 + d.  Halo kernels only.
+enum {
+    EPI_Y = UST_PASS_Y,
+    EPI_RES = UST_PASS_RES,
+    EPI_CHEBY = UST_PASS_CHEBY,
+    EPI_CHEBY0 = UST_PASS_CHEBY0,
+    EPI_PCHEBY0 = UST_PASS_PCHEBY0,
+    EPI_RES0 = UST_PASS_RES0,
+    EPI_CHEBY1 = UST_PASS_CHEBY1
+};
 template <typename T>
 struct Epi {
     T *y;  // EPI_Y / EPI_RES / EPI_RES0: output; EPI_CHEBY*: x after the step
@@ -242,6 +252,9 @@ struct Epi {
     T c1, c2;
     const T *xc;  // EPI_PCHEBY0: coarse-grid correction (nodes of the grid with half the elements per axis)
     const T *xs;  // EPI_CHEBY*: x before the step, the input u (y itself when the step runs in place)
+    T c0 = (T)0;            // EPI_CHEBY1
+    bool d_last = false;    // EPI_CHEBY: no later step reads the direction, leave d as it is
+    double *dot = nullptr;  // halo kernels: per workgroup u . y (EPI_Y) or b . x after the step (EPI_CHEBY*), or none
 };
 
 __host__ __device__ constexpr bool cheby_mode(int m) { return m == EPI_CHEBY || m == EPI_CHEBY0 || m == EPI_PCHEBY0; }
@@ -262,10 +275,20 @@ __device__ __forceinline__ T prolong_value(int i, int j, int k, F cval) {
     return wz * (wy * a0 + oy * a1) + oz * (wy * a2 + oy * a3);
 }
 
+// the same in 2D
+template <typename T, typename F>
+__device__ __forceinline__ T prolong_value2(int i, int j, F cval) {
+    const int I0 = i >> 1, J0 = j >> 1, I1 = I0 + (i & 1), J1 = J0 + (j & 1);
+    const T wx = (i & 1) ? (T)0.5 : (T)1, ox = (i & 1) ? (T)0.5 : (T)0;
+    const T wy = (j & 1) ? (T)0.5 : (T)1, oy = (j & 1) ? (T)0.5 : (T)0;
+    return wy * (wx * cval(I0, J0) + ox * cval(I1, J0)) + oy * (wx * cval(I0, J1) + ox * cval(I1, J1));
+}
+
 // the velocity a pass stages for dof i: u, or for EPI_RES0 the first Chebyshev step from zero, c2 invd b
 template <int MODE, typename T>
 __device__ __forceinline__ T stage_load(const Epi<T> &ep, const T *u, unsigned i) {
     if (MODE == EPI_RES0) return ep.c2 * ep.invd[i] * ep.b[i];
+    if (MODE == EPI_CHEBY1) return ep.c0 * ep.invd[i] * ep.b[i];
     return u[i];
 }
 
@@ -282,7 +305,7 @@ __device__ __forceinline__ EpiOps<T> epilogue_load(const Epi<T> &ep, const unsig
     o.m = mask[i];
     o.b = o.invd = o.d = o.x = (T)0;
     if (MODE != EPI_Y) o.b = ep.b[i];
-    if (MODE == EPI_RES0) o.invd = ep.invd[i];
+    if (MODE == EPI_RES0 || MODE == EPI_CHEBY1) o.invd = ep.invd[i];
     if (cheby_mode(MODE)) {
         o.invd = ep.invd[i];
         o.x = ep.xs[i];
@@ -291,20 +314,25 @@ __device__ __forceinline__ EpiOps<T> epilogue_load(const Epi<T> &ep, const unsig
     return o;
 }
 
-// v: the product (K u)_i before masking
+// v: the product (K u)_i before masking; returns what goes to y
 template <int MODE, typename T>
-__device__ __forceinline__ void epilogue_store(const Epi<T> &ep, const EpiOps<T> &o, unsigned i, T v) {
+__device__ __forceinline__ T epilogue_store(const Epi<T> &ep, const EpiOps<T> &o, unsigned i, T v) {
     v = o.m ? (T)0 : v;
+    T out;
     if (MODE == EPI_Y) {
-        ep.y[i] = v;
+        out = v;
     } else if (MODE == EPI_RES || MODE == EPI_RES0) {
-        ep.y[i] = o.m ? (T)0 : o.b - v;
+        out = o.m ? (T)0 : o.b - v;
         if (MODE == EPI_RES0) ep.d[i] = ep.c2 * o.invd * o.b;  // as staged (kv_cheby_first's rounding)
     } else {
-        const T dn = (MODE == EPI_CHEBY ? ep.c1 * o.d : (T)0) + ep.c2 * o.invd * (o.b - v);
-        if (MODE == EPI_CHEBY || ep.d) ep.d[i] = dn;  // a first step may leave d unwritten (no later step reads it)
-        ep.y[i] = o.x + dn;
+        const T x = MODE == EPI_CHEBY1 ? ep.c0 * o.invd * o.b : o.x;
+        const T d = MODE == EPI_CHEBY1 ? x : o.d;
+        const T dn = (MODE == EPI_CHEBY || MODE == EPI_CHEBY1 ? ep.c1 * d : (T)0) + ep.c2 * o.invd * (o.b - v);
+        if (ep.d && !ep.d_last) ep.d[i] = dn;  // a first step may come without a d, for the same reason
+        out = x + dn;
     }
+    ep.y[i] = out;
+    return out;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -715,31 +743,48 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, const WT *_
 }
 
 // ------------------------------------------------------------------------------------------
-// 3D halo-tile kernel (FP32, the small coarse multigrid levels): a 256-thread workgroup owns an 8x4x4 block of
-// NODES and computes every element touching them -- its 8x4x4 elements and a one-element halo on the low side
-// of each axis, 9x5x5 slots, one per thread -- so every owned node's sum is complete inside the workgroup: no
-// workspace and no gather launch.  The halo elements are computed twice (by two workgroups), which costs less
-// on the latency-bound small grids than the gather pass it replaces.  Neighbouring workgroups stage the nodes
-// a workgroup writes, so the Chebyshev modes must run out of place (ep.xs != ep.y).  Each node sums its 8
-// element contributions in a fixed order: deterministic.
+// Halo kernels: a 256-thread workgroup owns a block of NODES and computes every element touching them -- in 3D an 8x4x4
+// block and its 9x5x5 elements (a one-element halo on the low side of each axis), in 2D 15x15 nodes and 16x16 elements,
+// one element per thread -- so every owned node's sum is complete inside the workgroup: one launch, no workspace and no
+// gather.  The halo elements are computed by two workgroups, which costs less on the latency-bound grids than the gather
+// it replaces.  Neighbouring workgroups stage the nodes a workgroup writes, so the Chebyshev modes must run out of place
+// (ep.xs != ep.y).  Each node sums its element contributions in a fixed order: deterministic.  The operands of the
+// epilogue are loaded with the node block, so that only one trip to memory is exposed, and a pass can leave per-workgroup
+// partial sums of the dot product that follows it in the Krylov iteration.
+// What bounds them is the serial chain of one wavefront: launch, one trip to memory, 1200-1600 instructions, a store.  The
+// V-cycle on such levels takes 14 launches per inner iteration in 2D at 64x64 where steps of tiles + gather, separate
+// first steps, prolongation and dots took 24; solves: 2D 64x64 FP64 129.6 -> 74.7 ms, 3D 24x16x16 FP64 661 -> 455 ms.
+// Staging whole nodes (index arithmetic once per node, none of the loads behind a branch) instead of single dofs:
+// 466.8 -> 455 ms of the latter, the 64x64x32 solve with FP32 PCG 388 -> 379 ms.
 // ------------------------------------------------------------------------------------------
 constexpr int HOX = 8, HOY = 4, HOZ = 4;                    // owned nodes per axis
 constexpr int HEX = HOX + 1, HEY = HOY + 1, HEZ = HOZ + 1;  // element slots per axis
 constexpr int HNX = HOX + 2, HNY = HOY + 2, HNZ = HOZ + 2;  // staged nodes per axis
 constexpr int HNE = HEX * HEY * HEZ, HNN = HNX * HNY * HNZ;  // 225 element slots, 360 staged nodes
-constexpr int HND = HOX * HOY * HOZ * 3;                    // 384 owned dofs
-static_assert(HNE <= UST_TILE && HND <= 2 * UST_TILE, "one element and at most two owned dofs per thread");
+static_assert(HNE <= UST_TILE && HOX * HOY * HOZ * 2 == UST_TILE, "one element, at most two owned dofs per thread");
+constexpr int H2O = 15, H2N = H2O + 2, H2D = H2O * H2O * 2;  // 2D: owned nodes and staged nodes per axis, owned dofs
 
-// Grids up to this many elements take the halo-tile kernel; larger tile grids keep tiles + gather.  Measured on
-// the 128x128x64 solve (same box, graph-replayed): the halo passes on the 32x32x16 and 16x16x8 levels take it
-// from 0.431-0.434 s to 0.403-0.407 s; on the 64x64x32 level as well, 0.415-0.417 s (the duplicated halo
-// elements cost more there than the gather).  A 16x4x4-node block (two element slots per thread) was slower.
+// 3D grids up to this many elements take the halo kernel.  Measured on the 128x128x64 solve (same box, graph-replayed):
+// the halo passes on the 32x32x16 and 16x16x8 levels take it from 0.431-0.434 s to 0.403-0.407 s; on the 64x64x32 level
+// as well, 0.415-0.417 s (the duplicated halo elements cost more there than the gather).  2D grids take it whatever
+// their size: one element in seven is computed again, where the gather was half of a pass.
 #ifndef UST_HALO_MAX_NEL
 #define UST_HALO_MAX_NEL 65536
 #endif
 
 __host__ __device__ inline int halo_tiles(const GridDev &g) {
+    if (g.dim == 2) return ((g.nnx + H2O - 1) / H2O) * ((g.nny + H2O - 1) / H2O);
     return ((g.nnx + HOX - 1) / HOX) * ((g.nny + HOY - 1) / HOY) * ((g.nnz + HOZ - 1) / HOZ);
+}
+static inline bool halo_grid(const GridDev &g) { return g.dim == 2 || (!g.col && g.nel <= UST_HALO_MAX_NEL); }
+
+// the workgroup's sum of v into out[block]
+__device__ __forceinline__ void block_dot(double v, double *out) {
+    __shared__ double sh[4];
+    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+    if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
+    __syncthreads();
+    if (threadIdx.x == 0) out[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
 template <typename T, typename WT, int MODE>
@@ -751,44 +796,57 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
     const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
     const int nx0 = (tile % hnx) * HOX, ny0 = ((tile / hnx) % hny) * HOY, nz0 = (tile / (hnx * hny)) * HOZ;
     const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1;  // EPI_PCHEBY0: the coarse grid
-    // staging: value t of the block is node n = t / 3, component c = t % 3; nodes outside the grid stage 0
-    constexpr int NST = (HNN * 3 + UST_TILE - 1) / UST_TILE;
-    T stv[NST];
-    unsigned char stm[NST];
+    // staging: two nodes per thread, the three components together; nodes outside the grid stage 0 (their loads go to the
+    // nearest node of the grid, so that none of them waits for a branch)
+    constexpr int NST = (HNN + UST_TILE - 1) / UST_TILE;
+    T stv[NST][3];
+    unsigned char stm[NST][3];
     bool stok[NST];
 #pragma unroll
     for (int r = 0; r < NST; r++) {
-        const int t = tid + UST_TILE * r, c = t % 3, n = t / 3;
+        const int n = tid + UST_TILE * r;
         const int gx = nx0 - 1 + n % HNX, gy = ny0 - 1 + (n / HNX) % HNY, gz = nz0 - 1 + n / (HNX * HNY);
-        stok[r] = t < HNN * 3 && gx >= 0 && gy >= 0 && gz >= 0 && gx < g.nnx && gy < g.nny && gz < g.nnz;
-        const unsigned dof = stok[r] ? ((unsigned)gx + (unsigned)g.nnx * ((unsigned)gy + (unsigned)g.nny * gz)) * 3u + c
-                                     : 0u;
-        stm[r] = mask[dof];
-        stv[r] = stage_load<MODE, T>(ep, u, dof);
+        const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1), kz = min(max(gz, 0), g.nnz - 1);
+        stok[r] = gx == kx && gy == ky && gz == kz;
+        const unsigned dof = ((unsigned)kx + (unsigned)g.nnx * ((unsigned)ky + (unsigned)g.nny * kz)) * 3u;
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            stm[r][c] = mask[dof + c];
+            stv[r][c] = stage_load<MODE, T>(ep, u, dof + c);
+        }
+        if (MODE == EPI_PCHEBY0) {  // x + P xc on the free dofs, the coarse values read from global memory
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const T pc = prolong_value<T>(kx, ky, kz, [&](int I, int J, int K) {
+                    return ep.xc[((unsigned)I + (unsigned)cnx * ((unsigned)J + (unsigned)cny * K)) * 3u + c];
+                });
+                stv[r][c] += stm[r][c] ? (T)0 : pc;
+            }
+        }
     }
     // the thread's element slot and its weights, loaded while the block is staged
     const int lx = tid % HEX, ly = (tid / HEX) % HEY, lz = tid / (HEX * HEY);
     const int ex = nx0 - 1 + lx, ey = ny0 - 1 + ly, ez = nz0 - 1 + lz;
     const bool valid = tid < HNE && ex >= 0 && ey >= 0 && ez >= 0 && ex < g.nx && ey < g.ny && ez < g.nz;
-    const int e = valid ? ex + g.nx * (ey + g.ny * ez) : 0;
+    const size_t w0 = valid ? widx_at(g, ex, ey, ez, 0) : 0;
     T wq[27];
 #pragma unroll
-    for (int q = 0; q < 27; q++) wq[q] = wload<T, WT>(W, widx(g, e, q));
-    if (MODE == EPI_PCHEBY0) {  // x + P xc on the free dofs, the coarse values read from global memory
+    for (int q = 0; q < 27; q++) wq[q] = wload<T, WT>(W, w0 + (size_t)q * UST_TILE);
+    // the owned dofs: node tid % 128 of the block, component tid / 128 and, for the first 128 threads, component 2
+    const int on = tid % (HOX * HOY * HOZ), ox = on % HOX, oy = (on / HOX) % HOY, oz = on / (HOX * HOY);
+    const bool inside = nx0 + ox < g.nnx && ny0 + oy < g.nny && nz0 + oz < g.nnz;
+    const unsigned odof =
+        inside ? ((unsigned)(nx0 + ox) + (unsigned)g.nnx * ((unsigned)(ny0 + oy) + (unsigned)g.nny * (nz0 + oz))) * 3u
+               : 0u;
+    EpiOps<T> ops[2];
 #pragma unroll
-        for (int r = 0; r < NST; r++) {
-            const int t = tid + UST_TILE * r, c = t % 3, n = t / 3;
-            const int gx = nx0 - 1 + n % HNX, gy = ny0 - 1 + (n / HNX) % HNY, gz = nz0 - 1 + n / (HNX * HNY);
-            if (stok[r] && !stm[r])
-                stv[r] += prolong_value<T>(gx, gy, gz, [&](int I, int J, int K) {
-                    return ep.xc[((unsigned)I + (unsigned)cnx * ((unsigned)J + (unsigned)cny * K)) * 3u + c];
-                });
-        }
-    }
+    for (int r = 0; r < 2; r++) ops[r] = epilogue_load<MODE, T>(ep, mask, odof + (r ? 2 : tid / (HOX * HOY * HOZ)));
 #pragma unroll
     for (int r = 0; r < NST; r++) {
-        const int t = tid + UST_TILE * r;
-        if (t < HNN * 3) su[t] = (stok[r] && !stm[r]) ? stv[r] : (T)0;
+        const int n = tid + UST_TILE * r;
+        if (n < HNN)
+#pragma unroll
+            for (int c = 0; c < 3; c++) su[n * 3 + c] = (stok[r] && !stm[r][c]) ? stv[r][c] : (T)0;
     }
     __syncthreads();
     if (tid < HNE) {
@@ -804,24 +862,13 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
             for (int i = 0; i < 3; i++) eb[(a * 3 + i) * HNE + tid] = valid ? ye[a][i] : (T)0;
     }
     __syncthreads();
-    // the owned dofs d = tid, tid + 256 (< 384): node d / 3 of the block, component d % 3; each sums its 8
-    // elements in a fixed order, then the epilogue
-    EpiOps<T> ops[2];
-    unsigned dofs[2];
-    bool own[2];
+    // each owned dof sums its 8 elements in a fixed order, then the epilogue
+    double dot = 0.0;
 #pragma unroll
     for (int r = 0; r < 2; r++) {
-        const int d = tid + UST_TILE * r, n = d / 3, c = d % 3;
-        const int gx = nx0 + n % HOX, gy = ny0 + (n / HOX) % HOY, gz = nz0 + n / (HOX * HOY);
-        own[r] = d < HND && gx < g.nnx && gy < g.nny && gz < g.nnz;
-        dofs[r] = own[r] ? ((unsigned)gx + (unsigned)g.nnx * ((unsigned)gy + (unsigned)g.nny * gz)) * 3u + c : 0u;
-        ops[r] = epilogue_load<MODE, T>(ep, mask, dofs[r]);
-    }
-#pragma unroll
-    for (int r = 0; r < 2; r++) {
-        if (!own[r]) continue;
-        const int d = tid + UST_TILE * r, n = d / 3, c = d % 3;
-        const int ox = n % HOX, oy = (n / HOX) % HOY, oz = n / (HOX * HOY);
+        if (!inside || (r && tid >= HOX * HOY * HOZ)) continue;
+        const int c = r ? 2 : tid / (HOX * HOY * HOZ);
+        const T us = su[((ox + 1) + HNX * ((oy + 1) + HNY * (oz + 1))) * 3 + c];
         T v = (T)0;
 #pragma unroll
         for (int dz = 1; dz >= 0; dz--)
@@ -831,9 +878,108 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
                 for (int dx = 1; dx >= 0; dx--)  // element slot (ox + 1 - dx, ...) has this node as vertex (dx, dy, dz)
                     v += eb[((dx + 2 * dy + 4 * dz) * 3 + c) * HNE + (ox + 1 - dx) + HEX * ((oy + 1 - dy) + HEY * (oz + 1 - dz))];
         EpiOps<T> o = ops[r];
-        if (MODE == EPI_PCHEBY0 && !o.m) o.x = su[((ox + 1) + HNX * ((oy + 1) + HNY * (oz + 1))) * 3 + c];  // as staged
-        epilogue_store<MODE, T>(ep, o, dofs[r], v);
+        if (MODE == EPI_PCHEBY0 && !o.m) o.x = us;  // x + P xc, as staged
+        const T out = epilogue_store<MODE, T>(ep, o, odof + c, v);
+        dot += (double)out * (double)(MODE == EPI_Y ? us : o.b);
     }
+    if (ep.dot) block_dot(dot, ep.dot);
+}
+
+template <typename T, typename WT, int MODE>
+__global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__restrict__ W,
+                                                      const unsigned char *__restrict__ mask, const T *u, Epi<T> ep) {
+    __shared__ T su[H2N * H2N * 2];          // staged node block, origin (nx0 - 1, ny0 - 1)
+    __shared__ T eb[8 * (UST_TILE + 1)];     // element results: eb[(a*2 + i) * 257 + slot]
+    const int hnx = (g.nnx + H2O - 1) / H2O;
+    const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
+    const int nx0 = (tile % hnx) * H2O, ny0 = (tile / hnx) * H2O;
+    const int cnx = g.nx / 2 + 1;  // EPI_PCHEBY0: the coarse grid
+    constexpr int NSN = H2N * H2N, NST = (NSN + UST_TILE - 1) / UST_TILE;
+    T stv[NST][2];
+    unsigned char stm[NST][2];
+    bool stok[NST];
+#pragma unroll
+    for (int r = 0; r < NST; r++) {
+        const int n = tid + UST_TILE * r;
+        const int gx = nx0 - 1 + n % H2N, gy = ny0 - 1 + n / H2N;
+        const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1);
+        stok[r] = gx == kx && gy == ky;
+        const unsigned dof = ((unsigned)kx + (unsigned)g.nnx * (unsigned)ky) * 2u;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            stm[r][c] = mask[dof + c];
+            stv[r][c] = stage_load<MODE, T>(ep, u, dof + c);
+        }
+        if (MODE == EPI_PCHEBY0) {
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const T pc = prolong_value2<T>(kx, ky, [&](int I, int J) {
+                    return ep.xc[((unsigned)I + (unsigned)cnx * (unsigned)J) * 2u + c];
+                });
+                stv[r][c] += stm[r][c] ? (T)0 : pc;
+            }
+        }
+    }
+    const int lx = tid % 16, ly = tid / 16, ex = nx0 - 1 + lx, ey = ny0 - 1 + ly;
+    const bool valid = ex >= 0 && ey >= 0 && ex < g.nx && ey < g.ny;
+    const size_t w0 = valid ? widx_at(g, ex, ey, 0, 0) : 0;
+    T wq[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) wq[q] = wload<T, WT>(W, w0 + (size_t)q * UST_TILE);
+    EpiOps<T> ops[2];
+    unsigned dofs[2];
+    bool own[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int d = tid + UST_TILE * r, n = d / 2;
+        const int gx = nx0 + n % H2O, gy = ny0 + n / H2O;
+        own[r] = d < H2D && gx < g.nnx && gy < g.nny;
+        dofs[r] = own[r] ? ((unsigned)gx + (unsigned)g.nnx * (unsigned)gy) * 2u + d % 2 : 0u;
+        ops[r] = epilogue_load<MODE, T>(ep, mask, dofs[r]);
+    }
+#pragma unroll
+    for (int r = 0; r < NST; r++) {
+        const int n = tid + UST_TILE * r;
+        if (n < NSN)
+#pragma unroll
+            for (int c = 0; c < 2; c++) su[n * 2 + c] = (stok[r] && !stm[r][c]) ? stv[r][c] : (T)0;
+    }
+    __syncthreads();
+    {
+        T ue[4][2], ye[4][2];
+#pragma unroll
+        for (int a = 0; a < 4; a++) {
+            const int ln = (lx + (a & 1)) + H2N * (ly + (a >> 1));
+            ue[a][0] = su[ln * 2];
+            ue[a][1] = su[ln * 2 + 1];
+            ye[a][0] = ye[a][1] = (T)0;
+        }
+        const T s[3] = {(T)(2.0 / g.hx), (T)(2.0 / g.hy), (T)1};
+        element_apply2<T>(ue, wq, s, ye);
+#pragma unroll
+        for (int a = 0; a < 4; a++)
+#pragma unroll
+            for (int i = 0; i < 2; i++) eb[(a * 2 + i) * (UST_TILE + 1) + tid] = valid ? ye[a][i] : (T)0;
+    }
+    __syncthreads();
+    double dot = 0.0;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        if (!own[r]) continue;
+        const int d = tid + UST_TILE * r, n = d / 2, c = d % 2, ox = n % H2O, oy = n / H2O;
+        const T us = su[((ox + 1) + H2N * (oy + 1)) * 2 + c];
+        T v = (T)0;
+#pragma unroll
+        for (int dy = 1; dy >= 0; dy--)
+#pragma unroll
+            for (int dx = 1; dx >= 0; dx--)  // element slot (ox + 1 - dx, oy + 1 - dy) has this node as vertex (dx, dy)
+                v += eb[((dx + 2 * dy) * 2 + c) * (UST_TILE + 1) + (ox + 1 - dx) + 16 * (oy + 1 - dy)];
+        EpiOps<T> o = ops[r];
+        if (MODE == EPI_PCHEBY0 && !o.m) o.x = us;  // x + P xc, as staged
+        const T out = epilogue_store<MODE, T>(ep, o, dofs[r], v);
+        dot += (double)out * (double)(MODE == EPI_Y ? us : o.b);
+    }
+    if (ep.dot) block_dot(dot, ep.dot);
 }
 
 template <typename T, typename WT, int MODE>
@@ -1021,6 +1167,17 @@ static inline size_t work_len(const GridDev &g) {
 }
 
 template <typename T, typename WT, int MODE>
+static int apply_halo(const GridDev &g, const WT *W, const unsigned char *mask, const T *u, const Epi<T> &ep,
+                      hipStream_t st) {
+    if (g.dim == 3)
+        hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep);
+    else
+        hipLaunchKernelGGL((k_applyK2_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+
+template <typename T, typename WT, int MODE>
 static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mask, const T *u, Epi<T> ep, T *work,
                        void *stream) {
     GridDev g = grid_dev(gr, col_wg_target(sizeof(T), MODE));
@@ -1031,14 +1188,9 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
     if (MODE == EPI_PCHEBY0 && (g.dim != 3 || !ep.xc || g.nx % 2 || g.ny % 2 || g.nz % 2)) return UST_EINVAL;
     if ((size_t)g.nnx * g.nny * g.nnz * g.dim >= (1ull << 32)) return UST_EINVAL;  // 32-bit dof indices
     hipStream_t st = ust_stream(stream);
-    // FP32 on a small tile grid: the halo-tile kernel, unless a Chebyshev step runs in place
-    const bool halo = sizeof(T) == 4 && g.dim == 3 && !g.col && g.nel <= UST_HALO_MAX_NEL &&
-                      (!cheby_mode(MODE) || ep.y != ep.xs);
-    if (halo) {
-        if constexpr (sizeof(T) == 4)
-            hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask,
-                               u, ep);
-    } else if (g.dim == 3) {
+    // small 3D grids and 2D ones: the halo kernel, unless a Chebyshev step runs in place
+    if (halo_grid(g) && (!cheby_mode(MODE) || ep.y != ep.xs)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
+    if (g.dim == 3) {
         if (g.col)
             hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, W, mask, u, ep,
                                work);
@@ -1048,7 +1200,7 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
         const unsigned nf = face_node_count<3>(g);
         if (nf) hipLaunchKernelGGL((k_gather_tiles<T, 3, MODE>), dim3(ust_grid_size((size_t)nf * 3, 256)), dim3(256),
                                    0, st, g, mask, work, ep);
-    } else {
+    } else if constexpr (cheby_mode(MODE)) {
         hipLaunchKernelGGL((k_applyK2_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, W, mask, u, ep,
                            work);
         const unsigned nf = face_node_count<2>(g);
@@ -1100,6 +1252,54 @@ extern "C" int ust_k_apply_K_residual_first_f32(const ust_grid *g, const float *
                                                 const float *b, const float *invd, float *x, float *r, float c2,
                                                 float *work, void *stream) {
     return apply_residual_first<float, float>(g, WK, mask, b, invd, x, r, c2, work, stream);
+}
+
+// One halo pass from its description.
+template <typename T, typename WT>
+static int halo_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
+    const T *u = (const T *)p->u, *b = (const T *)p->b, *invd = (const T *)p->invd, *xc = (const T *)p->xc;
+    T *y = (T *)p->y, *d = (T *)p->d;
+    const WT *W = (const WT *)p->W;
+    Epi<T> ep = {y, b, invd, d, (T)p->c1, (T)p->c2, xc, u, (T)p->c0, p->d_last != 0, p->dot};
+    if (!W || !p->mask || !y) return UST_EINVAL;
+    const bool reads_u = p->mode != UST_PASS_RES0 && p->mode != UST_PASS_CHEBY1;
+    if (reads_u && (!u || u == y)) return UST_EINVAL;  // out of place
+    if (p->mode != UST_PASS_Y && !b) return UST_EINVAL;
+    if (p->mode >= UST_PASS_CHEBY && !invd) return UST_EINVAL;
+    if (!reads_u) u = b;  // not read
+    switch (p->mode) {
+        case UST_PASS_Y: return apply_halo<T, WT, EPI_Y>(g, W, p->mask, u, ep, st);
+        case UST_PASS_RES: return apply_halo<T, WT, EPI_RES>(g, W, p->mask, u, ep, st);
+        case UST_PASS_CHEBY:
+            if (!d) return UST_EINVAL;
+            return apply_halo<T, WT, EPI_CHEBY>(g, W, p->mask, u, ep, st);
+        case UST_PASS_CHEBY0: return apply_halo<T, WT, EPI_CHEBY0>(g, W, p->mask, u, ep, st);
+        case UST_PASS_PCHEBY0:
+            if (!xc || g.nx % 2 || g.ny % 2 || (g.dim == 3 && g.nz % 2)) return UST_EINVAL;
+            return apply_halo<T, WT, EPI_PCHEBY0>(g, W, p->mask, u, ep, st);
+        case UST_PASS_RES0:
+            if (!d) return UST_EINVAL;
+            return apply_halo<T, WT, EPI_RES0>(g, W, p->mask, u, ep, st);
+        case UST_PASS_CHEBY1: return apply_halo<T, WT, EPI_CHEBY1>(g, W, p->mask, u, ep, st);
+    }
+    return UST_EINVAL;
+}
+
+extern "C" int ust_k_apply_single(const ust_grid *gr) {
+    const GridDev g = grid_dev(gr);
+    return halo_grid(g) ? halo_tiles(g) : 0;
+}
+
+extern "C" int ust_k_apply_pass(const ust_grid *gr, const ust_pass *p, void *stream) {
+    if (!gr || !p) return UST_EINVAL;
+    const GridDev g = grid_dev(gr);
+    if (!halo_grid(g)) return UST_EINVAL;
+    if ((size_t)g.nnx * g.nny * g.nnz * g.dim >= (1ull << 32)) return UST_EINVAL;  // 32-bit dof indices
+    hipStream_t st = ust_stream(stream);
+    if (p->type == UST_PASS_F64) return halo_pass<double, double>(g, p, st);
+    if (p->type == UST_PASS_F32) return halo_pass<float, float>(g, p, st);
+    if (p->type == UST_PASS_F32_BF16W) return halo_pass<float, unsigned short>(g, p, st);
+    return UST_EINVAL;
 }
 
 // the largest workspace any pass needs (the passes' column grids differ in z-chunk length)

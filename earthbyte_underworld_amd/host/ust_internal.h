@@ -30,7 +30,7 @@ typedef struct {
     /* work vectors */
     double *x64, *b64, *ax64, *d64;
     float *x32, *b32, *ax32, *d32;
-    float *x32b;           /* coarse 3D levels: the second x of the out-of-place FP32 smoothing passes */
+    int single;            /* workgroups of a one-launch pass on this grid (ust_k_apply_single), 0: tiles + gather */
 } ust_level;
 
 typedef struct {

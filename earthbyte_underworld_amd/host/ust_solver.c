@@ -67,7 +67,7 @@ void ust_levels_free(ust_context *ctx) {
         DFREE(L->invd64);
         DFREE(L->invd32);
         DFREE(L->x64); DFREE(L->b64); DFREE(L->ax64); DFREE(L->d64);
-        DFREE(L->x32); DFREE(L->x32b); DFREE(L->b32); DFREE(L->ax32); DFREE(L->d32);
+        DFREE(L->x32); DFREE(L->b32); DFREE(L->ax32); DFREE(L->d32);
         memset(L, 0, sizeof(*L));
     }
     DFREE(ctx->Ainv);
@@ -103,26 +103,17 @@ static int lev_residual(ust_context *ctx, int l, int f32, const void *x, const v
     return UST_OK;
 }
 
-/* Jacobi-Chebyshev smoothing of A x = b (PETScMGSolver.c:674-709 smoother role).  x_zero 1: x is not read
+/* Jacobi-Chebyshev smoothing of A x = b in place (PETScMGSolver.c:674-709 smoother role).  x_zero 1: x is not read
  * (taken as zero); the first step is then d = c2 D^-1 b, x = d, without a product.  x_zero 2: that first
- * step was already applied (by the restriction).  Every other step is one fused product + update pass.
- * *xp holds x; with alt (the level's second FP32 vector) the product passes run out of place, each writing
- * the other vector, and *xp / *alt are swapped after each (the FP32 tile-grid kernel needs it). */
-static int lev_smooth(ust_context *ctx, int l, int f32, const void *b, void **xp, void **alt, int x_zero,
-                      const void *xc) {
+ * step was already applied (by the restriction).  Every other step is one fused product + update. */
+static int lev_smooth(ust_context *ctx, int l, int f32, const void *b, void *x, int x_zero, const void *xc) {
     ust_level *L = &ctx->lev[l];
     size_t n = (size_t)L->ndof;
-    const int oop = f32 && alt && *alt && L->WK32 && !L->WK16;
     for (int k = x_zero == 2 ? 1 : 0; k < L->cheb_deg; k++) {
-        void *x = *xp;
         if (k == 0 && xc) { /* prolongation of the coarse correction fused into the first step */
             /* a single post-smoothing step leaves its direction unwritten: no later step reads it */
             float *d32 = L->cheb_deg == 1 ? NULL : L->d32;
-            if (oop)
-                CKD(ctx, ust_k_apply_K_cheby_prolong_oop_f32(&L->g, L->WK32, L->mask, (const float *)x, (float *)*alt,
-                                                             (const float *)b, L->invd32, d32, (float)L->c2[0],
-                                                             (const float *)xc, (float *)ctx->kwork, S(ctx)));
-            else if (f32 && L->WK16)
+            if (f32 && L->WK16)
                 CKD(ctx, ust_k_apply_K_cheby_prolong_f32_bf16w(&L->g, L->WK16, L->mask, (float *)x, (const float *)b,
                                                                L->invd32, L->d32, (float)L->c2[0], (const float *)xc,
                                                                (float *)ctx->kwork, S(ctx)));
@@ -144,11 +135,6 @@ static int lev_smooth(ust_context *ctx, int l, int f32, const void *b, void **xp
             else
                 CKD(ctx, ust_k_cheby_first_f64((const double *)b, L->invd64, L->d64, (double *)x, L->c2[0], n,
                                                S(ctx)));
-            continue; /* elementwise: in place whatever the level */
-        } else if (oop) {
-            CKD(ctx, ust_k_apply_K_cheby_oop_f32(&L->g, L->WK32, L->mask, (const float *)x, (float *)*alt,
-                                                 (const float *)b, L->invd32, L->d32, (float)L->c1[k], (float)L->c2[k],
-                                                 k == 0, (float *)ctx->kwork, S(ctx)));
         } else if (f32 && L->WK16) {
             CKD(ctx, ust_k_apply_K_cheby_f32_bf16w(&L->g, L->WK16, L->mask, (float *)x, (const float *)b, L->invd32,
                                                    L->d32, (float)L->c1[k], (float)L->c2[k], k == 0,
@@ -160,85 +146,182 @@ static int lev_smooth(ust_context *ctx, int l, int f32, const void *b, void **xp
             CKD(ctx, ust_k_apply_K_cheby_f64(&L->g, L->WK64, L->mask, (double *)x, (const double *)b, L->invd64,
                                              L->d64, L->c1[k], L->c2[k], k == 0, (double *)ctx->kwork, S(ctx)));
         }
-        if (oop) { /* the step wrote the other vector */
-            *xp = *alt;
-            *alt = x;
-        }
     }
     return UST_OK;
 }
 
-/* one V-cycle: x = M^-1 b on level l (x is overwritten, not read).  first_done: the first smoothing step
- * from the zero guess was already applied to x (fused into the restriction that produced b).  *res: the
- * vector that holds the result -- x, or on an FP32 coarse level whose passes run out of place, possibly the
- * level's second vector x32b. */
-static int vcycle_r(ust_context *ctx, int l, int f32, const void *b, void *x, int first_done, void **res) {
+static int restrict_residual(ust_context *ctx, int l, int f32, const void *r) {
+    ust_level *L = &ctx->lev[l], *C = &ctx->lev[l + 1];
+    /* the residual is zero on the Dirichlet dofs, so the restriction need not read the fine mask */
+    if (f32) CKD(ctx, ust_k_restrict_f32(&L->g, NULL, C->mask, (const float *)r, C->b32, S(ctx)));
+    else CKD(ctx, ust_k_restrict_f64(&L->g, NULL, C->mask, (const double *)r, C->b64, S(ctx)));
+    return UST_OK;
+}
+
+static int vcycle(ust_context *ctx, int l, int f32, const void *b, void *x, int first_done, double *dot, void **res);
+
+/* The V-cycle of a level whose passes are one launch each (2D grids, small 3D ones): every smoothing step and residual
+ * runs out of place between x and the level's residual vector, which is free outside the residual's own use.  The first
+ * two smoothing steps from zero are one pass, one step and the residual another, and the prolongation of the correction
+ * rides on the first post-smoothing step.  dot: partial sums of b . x from the last pass (NULL: none). */
+static int vcycle_single(ust_context *ctx, int l, int f32, const void *b, void *x, double *dot, void **res) {
+    ust_level *L = &ctx->lev[l], *C = &ctx->lev[l + 1];
+    const int deg = L->cheb_deg, coarsest = l == ctx->nlev - 1;
+    void *cur = x, *alt = f32 ? (void *)L->ax32 : (void *)L->ax64, *d = f32 ? (void *)L->d32 : (void *)L->d64, *t;
+    ust_pass p;
+    int rc;
+    memset(&p, 0, sizeof p);
+    p.type = !f32 ? UST_PASS_F64 : L->WK16 ? UST_PASS_F32_BF16W : UST_PASS_F32;
+    p.W = !f32 ? (const void *)L->WK64 : L->WK16 ? (const void *)L->WK16 : (const void *)L->WK32;
+    p.mask = L->mask;
+    p.b = b;
+    p.invd = f32 ? (const void *)L->invd32 : (const void *)L->invd64;
+    if (coarsest && deg == 1) return lev_smooth(ctx, l, f32, b, *res = x, 1, NULL);
+    if (deg == 1) { /* alt = residual of x = the first step */
+        p.mode = UST_PASS_RES0;
+        p.c2 = L->c2[0];
+        p.y = alt;
+        p.d = x;
+        CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
+    } else {
+        for (int k = 1; k < deg; k++) {
+            p.mode = k == 1 ? UST_PASS_CHEBY1 : UST_PASS_CHEBY;
+            p.c0 = L->c2[0];
+            p.c1 = L->c1[k];
+            p.c2 = L->c2[k];
+            p.d_last = k == deg - 1;
+            p.d = k == 1 && deg == 2 ? NULL : d;
+            p.u = cur;
+            p.y = k == 1 ? cur : alt;
+            CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
+            if (k > 1) t = cur, cur = alt, alt = t;
+        }
+        *res = cur;
+        if (coarsest) return UST_OK;
+        p.mode = UST_PASS_RES;
+        p.u = cur;
+        p.y = alt;
+        CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
+    }
+    void *xc = NULL;
+    if ((rc = restrict_residual(ctx, l, f32, alt))) return rc;
+    if ((rc = vcycle(ctx, l + 1, f32, f32 ? (void *)C->b32 : (void *)C->b64, f32 ? (void *)C->x32 : (void *)C->x64, 0,
+                     NULL, &xc)))
+        return rc;
+    for (int k = 0; k < deg; k++) {
+        p.mode = k == 0 ? UST_PASS_PCHEBY0 : UST_PASS_CHEBY;
+        p.c1 = L->c1[k];
+        p.c2 = L->c2[k];
+        p.d_last = k == deg - 1;
+        p.d = deg == 1 ? NULL : d;
+        p.u = cur;
+        p.y = alt;
+        p.xc = xc;
+        p.dot = k == deg - 1 ? dot : NULL;
+        CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
+        t = cur, cur = alt, alt = t;
+    }
+    *res = cur;
+    return UST_OK;
+}
+
+/* one V-cycle: M^-1 b on level l (x is overwritten, not read).  first_done: the first smoothing step from the zero guess
+ * was already applied to x (fused into the restriction that produced b).  *res: the vector that holds the result -- x, or
+ * on a one-launch level possibly the level's residual vector. */
+static int vcycle(ust_context *ctx, int l, int f32, const void *b, void *x, int first_done, double *dot, void **res) {
     ust_level *L = &ctx->lev[l];
-    void *cur = x, *alt = (l > 0 && f32) ? (void *)L->x32b : NULL;
     int rc;
     *res = x;
-    if (l == ctx->nlev - 1) {
-        if (ctx->coarse_dense) {
-            if (f32) CKD(ctx, ust_k_dense_matvec_f32(ctx->Ainv, ctx->nc, (const float *)b, (float *)x, S(ctx)));
-            else CKD(ctx, ust_k_dense_matvec_f64(ctx->Ainv, ctx->nc, (const double *)b, (double *)x, S(ctx)));
-            return UST_OK;
-        }
-        rc = lev_smooth(ctx, l, f32, b, &cur, &alt, first_done ? 2 : 1, NULL);
-        *res = cur;
-        return rc;
+    if (l == ctx->nlev - 1 && ctx->coarse_dense) {
+        if (f32) CKD(ctx, ust_k_dense_matvec_f32(ctx->Ainv, ctx->nc, (const float *)b, (float *)x, S(ctx)));
+        else CKD(ctx, ust_k_dense_matvec_f64(ctx->Ainv, ctx->nc, (const double *)b, (double *)x, S(ctx)));
+        return UST_OK;
     }
+    if (L->single) return vcycle_single(ctx, l, f32, b, x, dot, res);
+    if (l == ctx->nlev - 1) return lev_smooth(ctx, l, f32, b, x, first_done ? 2 : 1, NULL);
     ust_level *C = &ctx->lev[l + 1];
     /* FP32, one pre-smoothing step from zero: the step rides on the residual pass */
     const int rfuse = f32 && !first_done && L->cheb_deg == 1 && L->WK32 && !L->WK16 && !ctx->b64_src;
-    if (!rfuse && (rc = lev_smooth(ctx, l, f32, b, &cur, &alt, first_done ? 2 : 1, NULL))) return rc;
+    if (!rfuse && (rc = lev_smooth(ctx, l, f32, b, x, first_done ? 2 : 1, NULL))) return rc;
     ctx->b64_src = NULL;
-    /* the coarse level starts with a smoothing step from zero unless it is the dense coarse solve */
-    int fuse = C->cheb_deg > 0 && !(l + 1 == ctx->nlev - 1 && ctx->coarse_dense);
-    /* 3D FP32: the prolongation of the correction rides on the first post-smoothing pass (FP64 keeps the
-     * separate prolongation: the fused FP64 pass needs more registers than two waves per SIMD allow) */
-    int pfuse = L->g.dim == 3 && L->cheb_deg > 0 && f32;
+    /* a coarse level of several launches per pass starts with its first smoothing step done by the restriction */
+    const int fuse = !C->single && !(l + 1 == ctx->nlev - 1 && ctx->coarse_dense);
     void *xcr = NULL; /* the coarse level's result */
     if (f32) {
-        /* the residual is zero on the Dirichlet dofs, so the restriction need not read the fine mask */
         if (rfuse)
             CKD(ctx, ust_k_apply_K_residual_first_f32(&L->g, L->WK32, L->mask, (const float *)b, L->invd32,
-                                                      (float *)cur, L->ax32, (float)L->c2[0], (float *)ctx->kwork,
+                                                      (float *)x, L->ax32, (float)L->c2[0], (float *)ctx->kwork,
                                                       S(ctx)));
-        else if ((rc = lev_residual(ctx, l, 1, cur, b, L->ax32)))
+        else if ((rc = lev_residual(ctx, l, 1, x, b, L->ax32)))
             return rc;
         if (fuse)
             CKD(ctx, ust_k_restrict_cheby_first_f32(&L->g, NULL, C->mask, L->ax32, C->b32, C->invd32, C->d32,
                                                     C->x32, (float)C->c2[0], S(ctx)));
-        else
-            CKD(ctx, ust_k_restrict_f32(&L->g, NULL, C->mask, L->ax32, C->b32, S(ctx)));
-        if ((rc = vcycle_r(ctx, l + 1, 1, C->b32, C->x32, fuse, &xcr))) return rc;
-        if (pfuse) {
-            rc = lev_smooth(ctx, l, 1, b, &cur, &alt, 0, xcr);
-            *res = cur;
+        else if ((rc = restrict_residual(ctx, l, 1, L->ax32)))
             return rc;
-        }
-        CKD(ctx, ust_k_prolong_add_f32(&L->g, L->mask, (const float *)xcr, (float *)cur, S(ctx)));
-    } else {
-        if ((rc = lev_residual(ctx, l, 0, cur, b, L->ax64))) return rc;
-        if (fuse)
-            CKD(ctx, ust_k_restrict_cheby_first_f64(&L->g, NULL, C->mask, L->ax64, C->b64, C->invd64, C->d64,
-                                                    C->x64, C->c2[0], S(ctx)));
-        else
-            CKD(ctx, ust_k_restrict_f64(&L->g, NULL, C->mask, L->ax64, C->b64, S(ctx)));
-        if ((rc = vcycle_r(ctx, l + 1, 0, C->b64, C->x64, fuse, &xcr))) return rc;
-        CKD(ctx, ust_k_prolong_add_f64(&L->g, L->mask, (const double *)xcr, (double *)cur, S(ctx)));
+        if ((rc = vcycle(ctx, l + 1, 1, C->b32, C->x32, fuse, NULL, &xcr))) return rc;
+        /* the prolongation of the correction rides on the first post-smoothing pass (FP64 keeps the separate
+         * prolongation: the fused FP64 pass needs more registers than two waves per SIMD allow) */
+        return lev_smooth(ctx, l, 1, b, x, 0, xcr);
     }
-    rc = lev_smooth(ctx, l, f32, b, &cur, &alt, 0, NULL);
-    *res = cur;
-    return rc;
+    if ((rc = lev_residual(ctx, l, 0, x, b, L->ax64))) return rc;
+    if (fuse)
+        CKD(ctx, ust_k_restrict_cheby_first_f64(&L->g, NULL, C->mask, L->ax64, C->b64, C->invd64, C->d64,
+                                                C->x64, C->c2[0], S(ctx)));
+    else if ((rc = restrict_residual(ctx, l, 0, L->ax64)))
+        return rc;
+    if ((rc = vcycle(ctx, l + 1, 0, C->b64, C->x64, fuse, NULL, &xcr))) return rc;
+    CKD(ctx, ust_k_prolong_add_f64(&L->g, L->mask, (const double *)xcr, (double *)x, S(ctx)));
+    return lev_smooth(ctx, l, 0, b, x, 0, NULL);
 }
 
-/* the V-cycle on the finest level, whose passes run in place: the result is in x */
-static int vcycle(ust_context *ctx, int l, int f32, const void *b, void *x, int first_done) {
-    void *res = NULL;
-    int rc = vcycle_r(ctx, l, f32, b, x, first_done, &res);
-    if (rc == UST_OK && res != x) UST_FAIL(ctx, UST_EINVAL, "V-cycle result left in the level's second vector");
-    return rc;
+/* whether level 0's last V-cycle pass and its product leave the partial sums of r.z and p.q themselves */
+static int cg_parts_of_passes(const ust_context *ctx) {
+    return ctx->lev[0].single > 0 && ctx->lev[0].single <= UST_CG_PARTS;
+}
+
+/* z = M^-1 r on the finest level and the partial sums of r . z; *np: their number */
+static int precondition(ust_context *ctx, int f32, const void *r, void *z, void **res, int *np) {
+    size_t n = (size_t)ctx->ndof;
+    double *dot = ctx->nlev > 1 && cg_parts_of_passes(ctx) ? ctx->cgpart : NULL;
+    int rc = vcycle(ctx, 0, f32, r, z, 0, dot, res);
+    if (rc) return rc;
+    *np = dot ? ctx->lev[0].single : ust_k_cg_parts(n);
+    if (dot) return UST_OK;
+    if (f32) CKD(ctx, ust_k_cg_dot_rz_f32((const float *)r, (const float *)*res, n, ctx->cgpart, S(ctx)));
+    else CKD(ctx, ust_k_cg_dot_rz_f64((const double *)r, (const double *)*res, n, ctx->cgpart, S(ctx)));
+    return UST_OK;
+}
+
+/* q = K p on the finest level (FP32: its FP32 weights) and the partial sums of p . q; *np: their number */
+static int product_dot(ust_context *ctx, int f32, const void *p, void *q, int *np) {
+    ust_level *L0 = &ctx->lev[0];
+    size_t n = (size_t)ctx->ndof;
+    double *part = ctx->cgpart;
+    if (cg_parts_of_passes(ctx)) {
+        ust_pass a;
+        memset(&a, 0, sizeof a);
+        a.mode = UST_PASS_Y;
+        a.type = f32 ? UST_PASS_F32 : UST_PASS_F64;
+        a.W = f32 ? (const void *)L0->WK32 : (const void *)L0->WK64;
+        a.mask = L0->mask;
+        a.u = p;
+        a.y = q;
+        a.dot = part + UST_CG_PARTS;
+        CKD(ctx, ust_k_apply_pass(&L0->g, &a, S(ctx)));
+        *np = L0->single;
+        return UST_OK;
+    }
+    *np = ust_k_cg_parts(n);
+    if (f32) {
+        CKD(ctx, ust_k_apply_K_f32(&L0->g, L0->WK32, L0->mask, (const float *)p, (float *)q, (float *)ctx->kwork, S(ctx)));
+        CKD(ctx, ust_k_cg_dot_pq_f32((const float *)p, (const float *)q, n, part, S(ctx)));
+    } else {
+        CKD(ctx, ust_k_apply_K_f64(&L0->g, L0->WK64, L0->mask, (const double *)p, (double *)q, (double *)ctx->kwork,
+                                   S(ctx)));
+        CKD(ctx, ust_k_cg_dot_pq_f64((const double *)p, (const double *)q, n, part, S(ctx)));
+    }
+    return UST_OK;
 }
 
 /* lambda_max of D^-1 A by power iteration (FP64) */
@@ -317,6 +400,7 @@ static int levels_structure(ust_context *ctx, const ust_solve_opts *o, int need3
         L->ndof = grid_ndof(&g);
         L->nel = grid_nel(&g);
         L->nnodes = L->ndof / dim;
+        L->single = ust_k_apply_single(&g);
         if (l == 0) {
             L->WK64 = ctx->WK;
             L->mask = ctx->mask_d;
@@ -347,8 +431,6 @@ static int levels_structure(ust_context *ctx, const ust_solve_opts *o, int need3
             if (o->vcycle_bf16) DALLOC(ctx, L->WK16, ust_k_weights_len(&L->g) * sizeof(unsigned short));
             else DALLOC(ctx, L->WK32, ust_k_weights_len(&L->g) * sizeof(float));
             DALLOC(ctx, L->x32, n * sizeof(float));
-            /* coarse 3D levels smooth out of place with FP32 weights (the tile-grid kernel needs it) */
-            if (l > 0 && dim == 3 && !o->vcycle_bf16) DALLOC(ctx, L->x32b, n * sizeof(float));
             DALLOC(ctx, L->b32, n * sizeof(float));
             DALLOC(ctx, L->ax32, n * sizeof(float));
             DALLOC(ctx, L->d32, n * sizeof(float));
@@ -474,31 +556,27 @@ static int dotv(ust_context *ctx, const double *a, const double *b, size_t n, in
  * once into a HIP graph. */
 static int pcg_iteration(ust_context *ctx, int pc32) {
     size_t n = (size_t)ctx->ndof;
-    double *r = ctx->vr, *z = ctx->vz, *p = ctx->vp, *q = ctx->vq, *c = ctx->scal + SC_CG, *part = ctx->cgpart;
-    const int np = ust_k_cg_parts(n);
-    int rc;
+    double *r = ctx->vr, *p = ctx->vp, *q = ctx->vq, *c = ctx->scal + SC_CG, *part = ctx->cgpart;
+    void *z = NULL;
+    int rc, nrz, npq;
     if (pc32) {
-        /* z stays FP32 (wz): the first smoothing step rounds r into b32 itself, r . z and p = z + beta p
-         * read z as FP32 and widen it per element */
+        /* z stays FP32: r . z and p = z + beta p widen it per element.  A level of several launches per pass rounds r
+         * into b32 in its first smoothing step */
         ust_level *L0 = &ctx->lev[0];
-        if (ctx->nlev > 1 && L0->cheb_deg > 0) {
-            ctx->b64_src = r;
-        } else {
-            CKD(ctx, ust_k_copy_f64_to_f32(r, L0->b32, n, S(ctx)));
-        }
-        rc = vcycle(ctx, 0, 1, L0->b32, ctx->wz, 0);
+        if (ctx->nlev > 1 && !L0->single) ctx->b64_src = r;
+        else CKD(ctx, ust_k_copy_f64_to_f32(r, L0->b32, n, S(ctx)));
+        rc = vcycle(ctx, 0, 1, L0->b32, ctx->wz, 0, NULL, &z);
         ctx->b64_src = NULL;
         if (rc) return rc;
-        CKD(ctx, ust_k_cg_dot_rz_zf(r, ctx->wz, n, part, S(ctx)));
-        CKD(ctx, ust_k_cg_dir_zf(ctx->wz, p, c, part, np, n, S(ctx)));
+        nrz = ust_k_cg_parts(n);
+        CKD(ctx, ust_k_cg_dot_rz_zf(r, (const float *)z, n, part, S(ctx)));
+        CKD(ctx, ust_k_cg_dir_zf((const float *)z, p, c, part, nrz, n, S(ctx)));
     } else {
-        if ((rc = vcycle(ctx, 0, 0, r, z, 0))) return rc;
-        CKD(ctx, ust_k_cg_dot_rz_f64(r, z, n, part, S(ctx)));
-        CKD(ctx, ust_k_cg_dir_f64(z, p, c, part, np, n, S(ctx)));
+        if ((rc = precondition(ctx, 0, r, ctx->vz, &z, &nrz))) return rc;
+        CKD(ctx, ust_k_cg_dir_f64((const double *)z, p, c, part, nrz, n, S(ctx)));
     }
-    if ((rc = lev_apply(ctx, 0, 0, p, q))) return rc;
-    CKD(ctx, ust_k_cg_dot_pq_f64(p, q, n, part, S(ctx)));
-    CKD(ctx, ust_k_cg_step_f64(ctx->vx, r, p, q, c, part, np, n, S(ctx)));
+    if ((rc = product_dot(ctx, 0, p, q, &npq))) return rc;
+    CKD(ctx, ust_k_cg_step_f64(ctx->vx, r, p, q, c, part, npq, n, S(ctx)));
     return UST_OK;
 }
 
@@ -557,15 +635,12 @@ static int pcg(ust_context *ctx, int pc32, const double *b, double *x, double rt
 static int pcg32_iteration(ust_context *ctx) {
     size_t n = (size_t)ctx->ndof;
     double *c = ctx->scal + SC_CG, *part = ctx->cgpart;
-    const int np = ust_k_cg_parts(n);
-    ust_level *L0 = &ctx->lev[0];
-    int rc = vcycle(ctx, 0, 1, ctx->wr, ctx->wz, 0);
-    if (rc) return rc;
-    CKD(ctx, ust_k_cg_dot_rz_f32(ctx->wr, ctx->wz, n, part, S(ctx)));
-    CKD(ctx, ust_k_cg_dir_f32(ctx->wz, ctx->wp, c, part, np, n, S(ctx)));
-    CKD(ctx, ust_k_apply_K_f32(&L0->g, L0->WK32, L0->mask, ctx->wp, ctx->wq, (float *)ctx->kwork, S(ctx)));
-    CKD(ctx, ust_k_cg_dot_pq_f32(ctx->wp, ctx->wq, n, part, S(ctx)));
-    CKD(ctx, ust_k_cg_step_f32(ctx->wx, ctx->wr, ctx->wp, ctx->wq, c, part, np, n, S(ctx)));
+    void *z = NULL;
+    int rc, nrz, npq;
+    if ((rc = precondition(ctx, 1, ctx->wr, ctx->wz, &z, &nrz))) return rc;
+    CKD(ctx, ust_k_cg_dir_f32((const float *)z, ctx->wp, c, part, nrz, n, S(ctx)));
+    if ((rc = product_dot(ctx, 1, ctx->wp, ctx->wq, &npq))) return rc;
+    CKD(ctx, ust_k_cg_step_f32(ctx->wx, ctx->wr, ctx->wp, ctx->wq, c, part, npq, n, S(ctx)));
     return UST_OK;
 }
 

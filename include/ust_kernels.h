@@ -267,6 +267,35 @@ size_t ust_k_dvc_lds_bytes(int dim, const int *res, int max_np);
 int ust_k_dvc_weights(int dim, const int *res, int nel, const int *cell_off, int max_np, double *xi0, double *xi1,
                       double *xi2, double *w, int set_centroids, int *flag, void *stream);
 
+/* --- passes of K in one launch, out of place (2D grids and small 3D ones) --- */
+#define UST_PASS_Y 0       /* y = K u */
+#define UST_PASS_RES 1     /* y = b - K u, 0 on the Dirichlet dofs */
+#define UST_PASS_CHEBY 2   /* d = c1 d + c2 invd (b - K u), y = u + d */
+#define UST_PASS_CHEBY0 3  /* the same with c1 = 0, d not read */
+#define UST_PASS_PCHEBY0 4 /* v = u + P xc (xc on the grid of half the elements), then CHEBY0 from v */
+#define UST_PASS_RES0 5    /* d = c2 invd b, y = b - K d, 0 on the Dirichlet dofs */
+#define UST_PASS_CHEBY1 6  /* v = c0 invd b, d = c1 v + c2 invd (b - K v), y = v + d */
+#define UST_PASS_F64 0
+#define UST_PASS_F32 1
+#define UST_PASS_F32_BF16W 2 /* FP32 with bfloat16 weights */
+typedef struct {
+    int mode, type;            /* UST_PASS_* */
+    const void *W;             /* weights of the type */
+    const unsigned char *mask;
+    const void *u;             /* input of modes 0-4 (distinct from y) */
+    void *y;
+    const void *b, *invd;      /* modes 1-6; modes 2-6 */
+    void *d;                   /* modes 2, 5; written in modes 3, 4, 6 when given */
+    const void *xc;            /* mode 4 */
+    double c0, c1, c2;
+    int d_last;                /* mode 2: do not write d */
+    double *dot;               /* when given, one partial sum per workgroup: of u . y (mode 0), of b . y (modes 2-4, 6) */
+} ust_pass;
+/* workgroups (partial sums) of a pass on this grid, 0 when the grid is not one of ust_k_apply_pass's */
+int ust_k_apply_single(const ust_grid *g);
+int ust_k_apply_pass(const ust_grid *g, const ust_pass *p, void *stream);
+
+
 /* --- operators.  mask: per dof (n_nodes*dim), 1 = Dirichlet.  y is overwritten. --- */
 /* y = K u on the free dofs (input and output BC dofs treated as zero).  work: device workspace of
  * ust_k_apply_work_len(g) elements of the operator's type (per-tile node partial sums); one

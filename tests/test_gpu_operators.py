@@ -686,3 +686,127 @@ def test_device_controlled_cg(kind, n):
     assert getattr(lib, f"ust_k_cg_dir_{kind}")(C.c_void_p(z.p.value + 4), p.p, c.p, part.p, parts, n, None) == -1
     for d in (db, x, r, p, q, z, c, part, host):
         d.free()
+
+
+# 2D blocks of 15x15 nodes: one block to the last node, one node more, several ragged; 3D blocks of 8x4x4 nodes likewise;
+# even sizes take the prolongation too
+@pytest.mark.parametrize("dim,nel", [(2, (14, 14)), (2, (15, 29)), (2, (46, 30)), (3, (7, 3, 3)), (3, (8, 4, 4)),
+                                     (3, (17, 9, 5)), (3, (18, 8, 12))])
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16w"])
+def test_single_launch_passes(oracle, dim, nel, prec):
+    """Every mode of the one-launch passes against the oracle's assembled K (FP64 weights; the FP64 pass on the rounded
+    weights for the other types, so that only the arithmetic differs) and the vector formulas in numpy, with the partial
+    sums of the dots.  Bar: 1e-13 of max(|K| |u|) in FP64, where sums of at most 24 x 27 products are rounded; 1e-5 of
+    the same in FP32; the dots to 1e-12 of the sum of magnitudes of what was written."""
+    import ctypes as C
+    from earthbyte_underworld_amd import _lib as L
+    s = _build(dim, nel, 6, 4)
+    lib = s.lib
+    g = L.Grid()
+    WK, WG, WF, mask = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert lib.ust_get_device_views(s.ctx, C.byref(g), C.byref(WK), C.byref(WG), C.byref(WF), C.byref(mask)) == 0
+    nw, n = lib.ust_k_weights_len(C.byref(g)), s.ndof
+    groups = lib.ust_k_apply_single(C.byref(g))
+    block = (15, 15) if dim == 2 else (8, 4, 4)
+    assert groups == np.prod([-(-(e + 1) // b) for e, b in zip(nel, block)])
+    T = np.float64 if prec == "f64" else np.float32
+    K, _ = OracleProblem(s).system(s.bc_mask).scipy()
+    free = s.bc_mask.reshape(-1) == 0
+    scale_of = lambda v: np.abs(K) @ np.abs(v[free])
+    W = WK
+    hold = []
+    if prec != "f64":
+        w = np.zeros(nw)
+        assert lib.ust_memcpy_d2h(w.ctypes.data_as(C.c_void_p), WK, w.nbytes, None) == 0
+        if prec == "f32":
+            d = _Dev(lib, w.astype(np.float32))
+            w = w.astype(np.float32).astype(np.float64)
+        else:
+            d = _Dev(lib, np.zeros(nw, np.uint16))
+            assert lib.ust_k_copy_f64_to_bf16(WK, d.p, nw, None) == 0
+            w = (d.get().astype(np.uint32) << 16).view(np.float32).astype(np.float64)
+        hold += [d, _Dev(lib, w)]
+        W = d.p
+    code = {"f64": 0, "f32": 1, "bf16w": 2}[prec]
+    rng = np.random.default_rng(17)
+    u, b, d0 = (rng.normal(size=n).astype(T) for _ in range(3))
+    invd = (rng.uniform(0.5, 1.5, n) / np.abs(K).max()).astype(T)
+    even = all(e % 2 == 0 for e in nel)
+    xc = rng.normal(size=int(np.prod([e // 2 + 1 for e in nel])) * dim).astype(T)
+    c0, c1, c2 = 0.7, 0.37, 1.9
+    dev = {k: _Dev(lib, v) for k, v in dict(u=u, b=b, invd=invd, xc=xc).items()}
+    hold += list(dev.values())
+
+    def run(mode, y0=None, with_d=True, d_last=0):
+        y, d, dot = _Dev(lib, np.full(n, np.nan, T)), _Dev(lib, d0), _Dev(lib, np.full(groups, np.nan))
+        p = L.Pass(mode=mode, type=code, W=W, mask=mask, u=dev["u"].p, y=y.p, b=dev["b"].p, invd=dev["invd"].p,
+                   d=d.p if with_d else None, xc=dev["xc"].p, c0=c0, c1=c1, c2=c2, d_last=d_last, dot=dot.p)
+        rc = lib.ust_k_apply_pass(C.byref(g), C.byref(p), None)
+        out = rc, y.get(), d.get(), dot.get()
+        for a in (y, d, dot):
+            a.free()
+        return out
+
+    def product(v):  # the reference K v, in FP64
+        v = np.asarray(v, np.float64)
+        if prec == "f64":
+            y = np.zeros(n)
+            y[free] = K @ v[free]
+            return y
+        dv, dy = _Dev(lib, v), _Dev(lib, np.zeros(n))
+        p = L.Pass(mode=0, type=0, W=hold[1].p, mask=mask, u=dv.p, y=dy.p)
+        assert lib.ust_k_apply_pass(C.byref(g), C.byref(p), None) == 0
+        y = dy.get()
+        dv.free()
+        dy.free()
+        return y
+
+    tol = 1e-13 if prec == "f64" else 1e-5
+
+    def close(got, ref, v, factor=1.0):
+        bound = tol * (factor * scale_of(np.asarray(v, np.float64)).max() + np.abs(ref).max())
+        assert np.abs(got - ref).max() <= bound, (np.abs(got - ref).max(), bound)
+
+    u64, b64, i64, d64 = (a.astype(np.float64) for a in (u, b, invd, d0))
+    ku = product(u)
+    sc = c2 * np.abs(i64).max()
+    rc, y, _, dot = run(0)
+    assert rc == 0 and np.all(y[~free] == 0.0)
+    close(y, ku, u)
+    um = np.where(free, u64, 0.0) * y
+    assert abs(dot.sum() - um.sum()) <= 1e-12 * np.abs(um).sum()
+    rc, y, _, _ = run(1)
+    assert rc == 0
+    close(y, np.where(free, b64 - ku, 0.0), u)
+    modes = [(2, u64, c1 * d64), (3, u64, 0.0), (6, c0 * i64 * b64, c1 * c0 * i64 * b64)]
+    if even:
+        dx, dxc = _Dev(lib, u64), _Dev(lib, xc.astype(np.float64))
+        assert lib.ust_k_prolong_add_f64(C.byref(g), mask, dxc.p, dx.p, None) == 0
+        modes.append((4, dx.get(), 0.0))
+        dx.free()
+        dxc.free()
+    else:
+        assert run(4)[0] == -1
+    for mode, v, dprev in modes:
+        dn = dprev + c2 * i64 * (b64 - product(v))
+        for last in (0, 1):
+            with_d = not (last and mode != 2)
+            rc, y, d, dot = run(mode, with_d=with_d, d_last=last)
+            assert rc == 0
+            close(y, v + dn, v, sc)
+            if last:
+                assert np.array_equal(d, d0)
+            else:
+                close(d, dn, v, sc)
+            by = b64 * y
+            assert abs(dot.sum() - by.sum()) <= 1e-12 * np.abs(by).sum()
+    rc, y, d, _ = run(5)
+    x = (T(c2) * invd) * b
+    assert rc == 0 and np.array_equal(d, x)
+    close(y, np.where(free, b64 - product(x), 0.0), x)
+    # in place is refused
+    p = L.Pass(mode=0, type=code, W=W, mask=mask, u=dev["u"].p, y=dev["u"].p)
+    assert lib.ust_k_apply_pass(C.byref(g), C.byref(p), None) == -1
+    for a in hold:
+        a.free()
+    s.close()
