@@ -76,6 +76,7 @@ struct GridDev {
     int tnx, tny, tnz;    // tiles per axis (3D: tnz = z-chunks per column)
     int ntiles;
     double hx, hy, hz;
+    double sx, sy, sz;    // 2 / h per axis: no division in the kernels
     double xmin, ymin, zmin;
     double ymax;
 };
@@ -148,6 +149,9 @@ static inline GridDev grid_dev(const ust_grid *g, long long wg_target = UST_COL_
     }
     d.ntiles = d.tnx * d.tny * d.tnz;
     d.hx = g->h[0];
+    d.sx = 2.0 / g->h[0];
+    d.sy = 2.0 / g->h[1];
+    d.sz = g->dim == 3 ? 2.0 / g->h[2] : 1.0;
     d.hy = g->h[1];
     d.hz = g->dim == 3 ? g->h[2] : 1.0;
     d.xmin = g->xmin[0];

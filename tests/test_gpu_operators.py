@@ -588,6 +588,14 @@ def test_column_kernel_against_element_reference(nel):
         a.free()
 
 
+@pytest.mark.parametrize("nel", [(512, 512, 1), (34, 20, 300)])
+def test_column_chunk_edges(nel):
+    """The column kernel and its gather against the element reference where a chunk is one layer thick (a single one, so
+    that no z coordinate but the first lies off a face) and where chunks start on odd planes, so that the prolongation
+    pass starts between two coarse planes.  Bars of test_column_kernel_against_element_reference."""
+    test_column_kernel_against_element_reference(nel)
+
+
 @pytest.mark.parametrize("nel", [(17, 9, 5), (40, 30, 20), (80, 70, 60)])
 def test_fp32_product_of_a_field_with_a_large_mean(nel):
     """The FP32 product (halo, tile and column kernels) of u = 1000 + N(0, 1) against FP64 on the same floats.  Velocity
