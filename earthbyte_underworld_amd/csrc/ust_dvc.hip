@@ -250,14 +250,15 @@ __device__ void dvc_element_words(const DvcShape &s, unsigned char *dvc_lds, int
 // a wave looks at `per` elements and redoes the marked ones.  per = 1: every element, where particles so many that
 // k_dvc_grow's LDS does not fit share one.
 template <int DIM, typename OT>
-__global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, int nel, double *xi0,
+__global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, const int *elems, int nel, double *xi0,
                                                          double *xi1, double *xi2, double *w, int set_centroids,
                                                          int *flag, int per) {
     extern __shared__ __align__(16) unsigned char dvc_lds[];
-    const int el = blockIdx.x * per + (int)threadIdx.x;
+    int el = blockIdx.x * per + (int)threadIdx.x;
     const bool mine = (int)threadIdx.x < per && el < nel;
     int off = 0, np = 0;
     if (mine) {
+        if (elems) el = elems[el];
         off = cell_off[el];
         np = cell_off[el + 1] - off;
     }
@@ -291,8 +292,8 @@ constexpr int GROW_WAVES = 2;
 constexpr int DVC_WIDE_2D = 16384;  // 2D swarms of fewer elements give an element 32 lanes
 
 template <int DIM, int G, typename OT>
-__global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const int *__restrict__ cell_off, int nel,
-                                                              double *xi0, double *xi1, double *xi2, double *w,
+__global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const int *__restrict__ cell_off,
+                                                              const int *__restrict__ elems, int nel, double *xi0, double *xi1, double *xi2, double *w,
                                                               int set_centroids, int *flag) {
     static_assert(G == 16 || G == 32, "group votes are 32-bit");
     extern __shared__ __align__(16) unsigned char dvc_lds[];
@@ -323,9 +324,10 @@ __global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const 
         }
     }
     const int lane = threadIdx.x & 63, gl = lane % G, grp = threadIdx.x / G;
-    const int e = blockIdx.x * (64 * GROW_WAVES / G) + grp;
+    int e = blockIdx.x * (64 * GROW_WAVES / G) + grp;
     int off = 0, np = 0;
     if (e < nel) {
+        if (elems) e = elems[e];  // the elements of a list
         off = cell_off[e];
         np = cell_off[e + 1] - off;
         if ((np <= 0 || np > s.max_np) && gl == 0) atomicOr(flag, np <= 0 ? 1 : 2);
@@ -540,17 +542,17 @@ __global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const 
 }
 
 template <int DIM, int G, typename OT>
-static int launch_dvc(const DvcShape &s, size_t lds_words, const int *cell_off, int nel, double *xi0, double *xi1,
+static int launch_dvc(const DvcShape &s, size_t lds_words, const int *cell_off, const int *elems, int nel, double *xi0, double *xi1,
                       double *xi2, double *w, int set_centroids, int *flag, hipStream_t st) {
     constexpr int EPB = 64 * GROW_WAVES / G;
     const size_t lds = grow_lds_shared(s) + EPB * grow_lds_element(s, sizeof(OT));
     const bool grow = lds <= 65536;
     if (grow)
         hipLaunchKernelGGL((k_dvc_grow<DIM, G, OT>), dim3((nel + EPB - 1) / EPB), dim3(64 * GROW_WAVES), lds, st, s,
-                           cell_off, nel, xi0, xi1, xi2, w, set_centroids, flag);
+                           cell_off, elems, nel, xi0, xi1, xi2, w, set_centroids, flag);
     const int per = grow ? DVC_LANES : 1;
     hipLaunchKernelGGL((k_dvc_spill<DIM, OT>), dim3((nel + per - 1) / per), dim3(DVC_LANES), lds_words, st, s, cell_off,
-                       nel, xi0, xi1, xi2, w, set_centroids, flag, per);
+                       elems, nel, xi0, xi1, xi2, w, set_centroids, flag, per);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
@@ -569,6 +571,11 @@ size_t ust_k_dvc_lds_bytes(int dim, const int *res, int max_np) {
 
 int ust_k_dvc_weights(int dim, const int *res, int nel, const int *cell_off, int max_np, double *xi0, double *xi1,
                       double *xi2, double *w, int set_centroids, int *flag, void *stream) {
+    return ust_k_dvc_weights_of(dim, res, nel, nullptr, cell_off, max_np, xi0, xi1, xi2, w, set_centroids, flag, stream);
+}
+
+int ust_k_dvc_weights_of(int dim, const int *res, int nel, const int *elems, const int *cell_off, int max_np, double *xi0,
+                         double *xi1, double *xi2, double *w, int set_centroids, int *flag, void *stream) {
     if ((dim != 2 && dim != 3) || !res || nel < 0 || !cell_off || !xi0 || !xi1 || !w || !flag || max_np < 1 ||
         max_np > 32767)
         return UST_EINVAL;
@@ -596,7 +603,7 @@ int ust_k_dvc_weights(int dim, const int *res, int nel, const int *cell_off, int
     // 14.9 ms with 1,210, 12.8 ms with 1,016.
     const int by_cell = s.ncell + 7 * max_np, by_np = 5 * s.ncell / 8 + 13 * max_np;
     s.ring = ((by_cell < by_np ? by_cell : by_np) + 1) & ~1;
-#define DVC(D, G, OT) return launch_dvc<D, G, OT>(s, lds, cell_off, nel, xi0, xi1, xi2, w, set_centroids, flag, st)
+#define DVC(D, G, OT) return launch_dvc<D, G, OT>(s, lds, cell_off, elems, nel, xi0, xi1, xi2, w, set_centroids, flag, st)
     // 3D boundaries hold 10 to 20 sub-cells on average: 32 lanes (64^3 x 30 particles: 12.8 ms, with 16 lanes 20.1 ms).
     // 2D ones hold 4: 16 lanes (512^2 x 20: 1.33 ms, with 32 lanes 2.05 ms), unless the elements are too few to fill
     // the GPU, where the shorter turns count (64^2 x 20: 0.126 ms with 32 lanes, 0.144 ms with 16).

@@ -273,6 +273,63 @@ int ust_rheology_from_xml(const char *type_name, int nkeys, const char *const *k
     return UST_OK;
 }
 
+/* a swarm on its way into the context, in its own device arrays (unset ones NULL) */
+typedef struct {
+    int *off;
+    double *x[3], *c[3], *w;
+    unsigned char *mat;
+    float *coh;
+    double *pfw, *inc;
+} new_swarm;
+
+static void new_swarm_free(new_swarm *s) {
+    void **p[] = {(void **)&s->off,  (void **)&s->x[0], (void **)&s->x[1], (void **)&s->x[2],
+                  (void **)&s->c[0], (void **)&s->c[1], (void **)&s->c[2], (void **)&s->w,
+                  (void **)&s->mat,  (void **)&s->coh,  (void **)&s->pfw,  (void **)&s->inc};
+    for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); i++) dfree(p[i]);
+}
+
+/* the arrays of a swarm of n particles with the attributes of the current one (off comes from the caller) */
+static int new_swarm_alloc(const ust_context *ctx, new_swarm *s, size_t n, int centroids) {
+    int rc = UST_OK;
+    for (int d = 0; d < ctx->grid.dim && !rc; d++) {
+        rc = ust_dev_malloc((void **)&s->x[d], n * sizeof(double) + 8);
+        if (!rc && centroids) rc = ust_dev_malloc((void **)&s->c[d], n * sizeof(double) + 8);
+    }
+    if (!rc) rc = ust_dev_malloc((void **)&s->w, n * sizeof(double) + 8);
+    if (!rc && ctx->mat) rc = ust_dev_malloc((void **)&s->mat, n + 8);
+    if (!rc && ctx->coh) rc = ust_dev_malloc((void **)&s->coh, n * sizeof(float) + 8);
+    if (!rc && ctx->pfw) rc = ust_dev_malloc((void **)&s->pfw, n * sizeof(double) + 8);
+    if (!rc && ctx->pfw) rc = ust_dev_malloc((void **)&s->inc, n * sizeof(double) + 8);
+    return rc;
+}
+
+/* the context's swarm becomes s (whose arrays it takes over), as by ust_swarm_upload_dev with its arrays */
+static int swarm_adopt(ust_context *ctx, new_swarm *s, int np, int max_ppc) {
+    free_swarm(ctx);
+    const size_t n = (size_t)np;
+    ctx->np = np;
+    ctx->max_ppc = max_ppc;
+    ctx->cell_off = s->off;
+    ctx->xi0 = s->x[0];
+    ctx->xi1 = s->x[1];
+    ctx->xi2 = s->x[2];
+    ctx->ixi0 = s->c[0];
+    ctx->ixi1 = s->c[1];
+    ctx->ixi2 = s->c[2];
+    ctx->w = s->w;
+    ctx->mat = s->mat;
+    ctx->coh = s->coh;
+    ctx->pfw = s->pfw;
+    ctx->pfw_inc = s->inc;
+    memset(s, 0, sizeof(*s));
+    ctx->assembled = 0;
+    DALLOC(ctx, ctx->eta, n * sizeof(double));
+    DALLOC(ctx, ctx->yielded, n);
+    DALLOC(ctx, ctx->tensile, n);
+    return UST_OK;
+}
+
 int ust_swarm_upload_dev(ust_context *ctx, int np, const int *cell_off_dev, const double *xi0_dev,
                          const double *xi1_dev, const double *xi2_dev, const double *w_dev,
                          const unsigned char *material_dev, const float *coh_scale_dev, int max_ppc) {
@@ -1055,79 +1112,53 @@ int ust_swarm_advect(ust_context *ctx, double dt, int order, int allow_fallback,
     const int np = ctx->np, nel = ctx->nel, dim = ctx->grid.dim;
     const size_t n = (size_t)np;
     size_t wb = ust_k_sort_by_cell_work_bytes(np, nel);
-    void *key = NULL, *key_s = NULL, *perm = NULL, *perm_t = NULL, *nxi = NULL, *flag = NULL, *work = NULL;
-    void *off = NULL, *oxi = NULL, *ow = NULL, *omat = NULL, *ocoh = NULL;
-    int rc = UST_OK, hflag = 0;
+    void *key = NULL, *key_s = NULL, *perm = NULL, *perm_t = NULL, *nxi = NULL, *work = NULL, *cwork = NULL;
+    new_swarm s = {0};
+    int rc = UST_OK, *flag = (int *)(ctx->scal + SC_T0); /* 3 ints */
+    long long *host = (long long *)(ctx->scal_h + SC_T0); /* particles, -, largest count, empty elements, flags */
     if (!rc) rc = ust_dev_malloc(&key, n * sizeof(unsigned) + 8);
     if (!rc) rc = ust_dev_malloc(&key_s, n * sizeof(unsigned) + 8);
     if (!rc) rc = ust_dev_malloc(&perm, n * sizeof(unsigned) + 8);
     if (!rc) rc = ust_dev_malloc(&perm_t, n * sizeof(unsigned) + 8);
     if (!rc) rc = ust_dev_malloc(&nxi, 3 * n * sizeof(double) + 8);
-    if (!rc) rc = ust_dev_malloc(&flag, sizeof(double));
     if (!rc) rc = ust_dev_malloc(&work, wb + 8);
-    if (!rc) rc = ust_dev_malloc(&off, (size_t)(nel + 1) * sizeof(int));
+    if (!rc) rc = ust_dev_malloc(&cwork, ust_k_count_work_len(nel) * sizeof(int));
+    if (!rc) rc = ust_dev_malloc((void **)&s.off, (size_t)(nel + 1) * sizeof(int));
     double *n0 = (double *)nxi, *n1 = n0 + n, *n2 = n0 + 2 * n;
-    if (!rc) rc = ust_k_fill_f64((double *)flag, 0.0, 1, ctx->stream); /* all-zero bits: the int flag reads 0 */
+    if (!rc) rc = ust_k_fill_f64((double *)flag, 0.0, 2, ctx->stream); /* all-zero bits: the ints read 0 */
     if (!rc)
         rc = ust_k_advect(&ctx->grid, ctx->cell_off, np, ctx->xi0, ctx->xi1, ctx->xi2, ctx->u, dt, order,
-                          allow_fallback, (unsigned *)key, n0, n1, n2, (int *)flag, ctx->stream);
-    if (!rc) rc = ust_memcpy_d2h(&hflag, flag, sizeof(int), ctx->stream);
-    if (!rc && hflag) {
+                          allow_fallback, (unsigned *)key, n0, n1, n2, flag, ctx->stream);
+    /* the flag is looked at with the new offsets' totals, in one wait: a flagged particle's key is valid too */
+    if (!rc)
+        rc = ust_k_sort_by_cell((const unsigned *)key, (unsigned *)key_s, (unsigned *)perm, (unsigned *)perm_t, np,
+                                nel, work, wb, ctx->stream);
+    if (!rc) rc = ust_k_cell_offsets((const unsigned *)key_s, np, nel, s.off, ctx->stream);
+    if (!rc) rc = ust_k_offset_stats(nel, s.off, flag, host, (int *)cwork, ctx->stream);
+    if (!rc) rc = ust_stream_sync(ctx->stream);
+    if (!rc && host[4]) {
         snprintf(ctx->err, sizeof(ctx->err),
                  "a corrector step found no velocity (point outside the box) and allow_fallback is off "
                  "(TimeIntegrand.c:324-327)");
         rc = UST_ENOTCONV;
     }
+    const int kept = rc ? 0 : (int)host[0], max_ppc = rc ? 0 : (int)host[2], empty = rc ? 0 : (int)host[3];
+    if (!rc) rc = new_swarm_alloc(ctx, &s, (size_t)kept, 0);
     if (!rc)
-        rc = ust_k_sort_by_cell((const unsigned *)key, (unsigned *)key_s, (unsigned *)perm, (unsigned *)perm_t, np,
-                                nel, work, wb, ctx->stream);
-    if (!rc) rc = ust_k_cell_offsets((const unsigned *)key_s, np, nel, (int *)off, ctx->stream);
-    int *off_h = (int *)malloc((size_t)(nel + 1) * sizeof(int));
-    if (!off_h && !rc) rc = UST_ENOMEM;
-    if (!rc) rc = ust_memcpy_d2h(off_h, off, (size_t)(nel + 1) * sizeof(int), ctx->stream);
-    int kept = 0, empty = 0, max_ppc = 0;
-    if (!rc) {
-        kept = off_h[nel];
-        for (int e = 0; e < nel; e++) {
-            const int c = off_h[e + 1] - off_h[e];
-            if (c == 0) empty++;
-            if (c > max_ppc) max_ppc = c;
-        }
-    }
-    free(off_h);
-    const size_t k = (size_t)kept;
-    if (!rc) rc = ust_dev_malloc(&oxi, 3 * k * sizeof(double) + 8);
-    if (!rc) rc = ust_dev_malloc(&ow, k * sizeof(double) + 8);
-    if (!rc && ctx->mat) rc = ust_dev_malloc(&omat, k + 8);
-    if (!rc && ctx->coh) rc = ust_dev_malloc(&ocoh, k * sizeof(float) + 8);
-    double *o0 = (double *)oxi, *o1 = o0 + k, *o2 = o0 + 2 * k;
-    if (!rc)
-        rc = ust_k_swarm_gather(dim, kept, (const unsigned *)perm, (const unsigned *)key_s, (const int *)off, n0, n1,
-                                n2, ctx->mat, ctx->coh, o0, o1, o2, (double *)ow, (unsigned char *)omat,
-                                (float *)ocoh, ctx->stream);
+        rc = ust_k_swarm_gather(dim, kept, (const unsigned *)perm, (const unsigned *)key_s, s.off, n0, n1, n2, ctx->mat,
+                                ctx->coh, s.x[0], s.x[1], s.x[2], s.w, s.mat, s.coh, ctx->stream);
     /* the strain-weakening state travels with its particles */
-    void *opfw = NULL, *oinc = NULL;
     if (!rc && ctx->pfw) {
-        rc = ust_dev_malloc(&opfw, k * sizeof(double) + 8);
-        if (!rc) rc = ust_dev_malloc(&oinc, k * sizeof(double) + 8);
-        if (!rc) rc = ust_k_permute_f64((const unsigned *)perm, ctx->pfw, (double *)opfw, kept, ctx->stream);
-        if (!rc) rc = ust_k_permute_f64((const unsigned *)perm, ctx->pfw_inc, (double *)oinc, kept, ctx->stream);
+        rc = ust_k_permute_f64((const unsigned *)perm, ctx->pfw, s.pfw, kept, ctx->stream);
+        if (!rc) rc = ust_k_permute_f64((const unsigned *)perm, ctx->pfw_inc, s.inc, kept, ctx->stream);
     }
-    if (!rc) {
-        rc = ust_swarm_upload_dev(ctx, kept, (const int *)off, o0, o1, dim == 3 ? o2 : NULL, (const double *)ow,
-                                  (const unsigned char *)omat, (const float *)ocoh, max_ppc);
-        if (!rc && opfw) { /* upload_dev released the old state: the permuted arrays become the state */
-            ctx->pfw = (double *)opfw;
-            ctx->pfw_inc = (double *)oinc;
-            opfw = oinc = NULL;
-        }
-    } else if (!ctx->err[0] || rc != UST_ENOTCONV) {
+    if (!rc) rc = ust_stream_sync(ctx->stream);
+    if (!rc) rc = swarm_adopt(ctx, &s, kept, max_ppc);
+    else if (!ctx->err[0] || rc != UST_ENOTCONV)
         snprintf(ctx->err, sizeof(ctx->err), "swarm advection failed (%d): %s", rc, ust_dev_error_string());
-    }
-    ust_dev_free(opfw);
-    ust_dev_free(oinc);
-    void *tmp[] = {key, key_s, perm, perm_t, nxi, flag, work, off, oxi, ow, omat, ocoh};
+    void *tmp[] = {key, key_s, perm, perm_t, nxi, work, cwork};
     for (size_t i = 0; i < sizeof(tmp) / sizeof(tmp[0]); i++) ust_dev_free(tmp[i]);
+    new_swarm_free(&s);
     if (rc) return rc;
     if (n_removed) *n_removed = np - kept;
     if (n_empty) *n_empty = empty;
@@ -1141,6 +1172,50 @@ void ust_pcdvc_default(ust_pcdvc *o) {
     o->lower_t = 0.6;
     o->max_deletions = 2;
     o->max_splits = 3;
+}
+
+static int dvc_check(ust_context *ctx, const int *res) {
+    if (!ctx->np) UST_FAIL(ctx, UST_ESTATE, "no swarm");
+    if (!res) UST_FAIL(ctx, UST_EINVAL, "resolution missing");
+    const int dim = ctx->grid.dim;
+    int ncell = 1;
+    for (int a = 0; a < dim; a++) {
+        if (res[a] < 1 || res[a] > 64) UST_FAIL(ctx, UST_EINVAL, "DVC resolution %d out of 1..64", res[a]);
+        ncell *= res[a];
+    }
+    if (ncell > 4096) UST_FAIL(ctx, UST_EINVAL, "DVC sub-grid of %d cells exceeds 4096", ncell);
+    if (ctx->max_ppc < 1 || ctx->max_ppc > 32767)
+        UST_FAIL(ctx, UST_EINVAL, "%d particles per element: DVC holds 1..32767", ctx->max_ppc);
+    const size_t lds = ust_k_dvc_lds_bytes(dim, res, ctx->max_ppc);
+    if (lds > 65536)
+        UST_FAIL(ctx, UST_EINVAL, "DVC needs %zu bytes of LDS per element (%d particles, %d sub-cells): limit 65536",
+                 lds, ctx->max_ppc, ncell);
+    return UST_OK;
+}
+
+/* the regions of n elements (elems, or all of them when NULL) whose seeds are in the integration points (in the material
+ * points without set_centroids) */
+static int dvc_regions(ust_context *ctx, const int *res, int set_centroids, const int *elems, int n) {
+    int *flag = (int *)(ctx->scal + SC_T0);
+    double *d0 = set_centroids ? ctx->ixi0 : ctx->xi0, *d1 = set_centroids ? ctx->ixi1 : ctx->xi1;
+    double *d2 = set_centroids ? ctx->ixi2 : ctx->xi2;
+    int rc = ust_k_fill_f64((double *)flag, 0.0, 1, ctx->stream); /* all-zero bits: the int flag reads 0 */
+    if (!rc)
+        rc = ust_k_dvc_weights_of(ctx->grid.dim, res, n, elems, ctx->cell_off, ctx->max_ppc, d0, d1, d2, ctx->w,
+                                  set_centroids, flag, ctx->stream);
+    if (!rc) rc = ust_memcpy_d2h(ctx->scal_h + SC_T0, flag, sizeof(double), ctx->stream);
+    if (rc) UST_FAIL(ctx, rc, "DVC weights failed (%d): %s", rc, ust_dev_error_string());
+    int hflag = 0;
+    memcpy(&hflag, ctx->scal_h + SC_T0, sizeof(int));
+    /* the weights and points changed even when an element failed: nothing assembled stays valid */
+    ctx->assembled = 0;
+    ctx->cache_valid = 0;
+    if (hflag & 1)
+        UST_FAIL(ctx, UST_EINVAL, "under resolved cell: an element has no particles, add more particles "
+                                  "(DVCWeights.c:787)");
+    if (hflag & 2) UST_FAIL(ctx, UST_EINVAL, "an element holds more particles than the swarm's maximum per cell");
+    if (hflag & 4) UST_FAIL(ctx, UST_ENOTCONV, "DVC region growth did not settle within its round limit");
+    return UST_OK;
 }
 
 int ust_swarm_pcdvc(ust_context *ctx, const ust_pcdvc *opts, int *n_split, int *n_deleted) {
@@ -1167,81 +1242,55 @@ int ust_swarm_pcdvc(ust_context *ctx, const ust_pcdvc *opts, int *n_split, int *
     /* 1. the regions of the current particles (weights and centroids in the integration points) */
     int rc = ust_swarm_dvc_weights(ctx, opts->res, 1);
     if (rc) return rc;
-    /* 2. the per-element plans */
-    void *cnt = NULL, *list = NULL, *flag = NULL, *noff = NULL, *o = NULL, *ow = NULL, *omat = NULL, *ocoh = NULL;
-    void *os0 = NULL, *os1 = NULL;
-    int hflag[4] = {0, 0, 0, 0};
-    int *cnt_h = NULL, *off_h = NULL;
+    /* 2. the per-element plans, the new offsets and the elements that change */
+    void *cnt = NULL, *list = NULL, *elems = NULL, *cwork = NULL;
+    new_swarm s = {0};
+    int *flag = (int *)(ctx->scal + SC_T0); /* 3 ints */
+    long long *host = (long long *)(ctx->scal_h + SC_T0); /* particles, changed, largest count, empty, flag[0..2] */
     const size_t lcap = (size_t)np + (size_t)nel * (size_t)ko.max_splits;
     if (!rc) rc = ust_dev_malloc(&cnt, (size_t)nel * sizeof(int) + 8);
     if (!rc) rc = ust_dev_malloc(&list, lcap * sizeof(int) + 8);
-    if (!rc) rc = ust_dev_malloc(&flag, 2 * sizeof(double));
+    if (!rc) rc = ust_dev_malloc(&elems, (size_t)nel * sizeof(int) + 8);
+    if (!rc) rc = ust_dev_malloc(&cwork, ust_k_count_work_len(nel) * sizeof(int));
+    if (!rc) rc = ust_dev_malloc((void **)&s.off, (size_t)(nel + 1) * sizeof(int));
     if (!rc) rc = ust_k_fill_f64((double *)flag, 0.0, 2, ctx->stream); /* all-zero bits: the ints read 0 */
-    if (!rc) rc = ust_k_pcdvc_plan(&ctx->grid, ctx->cell_off, ctx->w, ctx->mat, &ko, (int *)cnt, (int *)list,
-                                   (int *)flag, ctx->stream);
-    if (!rc) rc = ust_memcpy_d2h(hflag, flag, 3 * sizeof(int), ctx->stream);
-    cnt_h = (int *)malloc((size_t)nel * sizeof(int));
-    off_h = (int *)malloc((size_t)(nel + 1) * sizeof(int));
-    if (!rc && (!cnt_h || !off_h)) rc = UST_ENOMEM;
-    if (!rc) rc = ust_memcpy_d2h(cnt_h, cnt, (size_t)nel * sizeof(int), ctx->stream);
-    long long total = 0;
-    int max_ppc = 0;
-    if (!rc) {
-        off_h[0] = 0;
-        for (int e = 0; e < nel; e++) {
-            total += cnt_h[e];
-            if (cnt_h[e] > max_ppc) max_ppc = cnt_h[e];
-            off_h[e + 1] = total > 2147483647LL ? 0 : (int)total;
+    if (!rc) rc = ust_k_pcdvc_plan(&ctx->grid, ctx->cell_off, ctx->w, ctx->mat, &ko, (int *)cnt, (int *)list, flag,
+                                   ctx->stream);
+    if (!rc) rc = ust_k_count_offsets(nel, (const int *)cnt, s.off, (int *)elems, flag, host, (int *)cwork, ctx->stream);
+    if (!rc) rc = ust_stream_sync(ctx->stream);
+    const long long total = rc ? 0 : host[0];
+    const int changed = rc ? 0 : (int)host[1], max_ppc = rc ? 0 : (int)host[2];
+    const int under = rc ? 0 : (int)host[4] & 1, nspl = rc ? 0 : (int)host[5], ndel = rc ? 0 : (int)host[6];
+    if (!rc && total > 2147483647LL) rc = UST_EINVAL;
+    if (!rc && under) {
+        snprintf(ctx->err, sizeof(ctx->err), "under resolved cell after population control: a changed element keeps "
+                                             "fewer than 3 particles (PCDVC.c:1418-1421)");
+        rc = UST_EINVAL;
+    } else {
+        /* 3. the new swarm; the elements that keep their particles keep their regions */
+        if (!rc) rc = new_swarm_alloc(ctx, &s, (size_t)total, 1);
+        if (!rc) {
+            const ust_pcdvc_swarm from = {{ctx->xi0, ctx->xi1, ctx->xi2}, {ctx->ixi0, ctx->ixi1, ctx->ixi2}, ctx->w,
+                                          ctx->mat, ctx->coh, ctx->pfw, ctx->pfw_inc};
+            const ust_pcdvc_swarm to = {{s.x[0], s.x[1], s.x[2]}, {s.c[0], s.c[1], s.c[2]}, s.w, s.mat, s.coh, s.pfw,
+                                        s.inc};
+            rc = ust_k_pcdvc_build(dim, nel, ko.max_splits, ctx->cell_off, s.off, (const int *)cnt, (const int *)list,
+                                   &from, &to, ctx->stream);
         }
-        if (total > 2147483647LL) rc = UST_EINVAL;
+        if (!rc) rc = ust_stream_sync(ctx->stream);
+        if (!rc) rc = swarm_adopt(ctx, &s, (int)total, max_ppc);
+        else if (!ctx->err[0])
+            snprintf(ctx->err, sizeof(ctx->err), "PCDVC population control failed (%d): %s", rc, ust_dev_error_string());
+        /* 4. the regions of the changed elements: integration points at the centroids, weights the volumes */
+        if (!rc) rc = dvc_check(ctx, opts->res);
+        if (!rc) rc = dvc_regions(ctx, opts->res, 1, (const int *)elems, changed);
     }
-    if (!rc && (hflag[0] & 1)) {
-        free(cnt_h);
-        free(off_h);
-        ust_dev_free(cnt);
-        ust_dev_free(list);
-        ust_dev_free(flag);
-        UST_FAIL(ctx, UST_EINVAL, "under resolved cell after population control: a changed element keeps fewer than 3 "
-                                  "particles (PCDVC.c:1418-1421)");
-    }
-    /* 3. the new swarm */
-    const size_t k = (size_t)total;
-    if (!rc) rc = ust_dev_malloc(&noff, (size_t)(nel + 1) * sizeof(int));
-    if (!rc) rc = ust_memcpy_h2d(noff, off_h, (size_t)(nel + 1) * sizeof(int), ctx->stream);
-    if (!rc) rc = ust_dev_malloc(&o, 3 * k * sizeof(double) + 8);
-    if (!rc) rc = ust_dev_malloc(&ow, k * sizeof(double) + 8);
-    if (!rc && ctx->mat) rc = ust_dev_malloc(&omat, k + 8);
-    if (!rc && ctx->coh) rc = ust_dev_malloc(&ocoh, k * sizeof(float) + 8);
-    if (!rc && ctx->pfw) rc = ust_dev_malloc(&os0, k * sizeof(double) + 8);
-    if (!rc && ctx->pfw) rc = ust_dev_malloc(&os1, k * sizeof(double) + 8);
-    double *o0 = (double *)o, *o1 = o0 + k, *o2 = o0 + 2 * k;
-    if (!rc)
-        rc = ust_k_pcdvc_build(dim, nel, ko.max_splits, ctx->cell_off, (const int *)noff, (const int *)list, ctx->xi0,
-                               ctx->xi1, ctx->xi2, ctx->ixi0, ctx->ixi1, ctx->ixi2, ctx->mat, ctx->coh, ctx->pfw,
-                               ctx->pfw_inc, o0, o1, dim == 3 ? o2 : NULL, (unsigned char *)omat, (float *)ocoh,
-                               (double *)os0, (double *)os1, ctx->stream);
-    if (!rc) rc = ust_k_fill_f64((double *)ow, 0.0, k, ctx->stream);
-    if (!rc) {
-        rc = ust_swarm_upload_dev(ctx, (int)k, (const int *)noff, o0, o1, dim == 3 ? o2 : NULL, (const double *)ow,
-                                  (const unsigned char *)omat, (const float *)ocoh, max_ppc);
-        if (!rc && os0) { /* upload_dev released the old state: the rebuilt arrays become the state */
-            ctx->pfw = (double *)os0;
-            ctx->pfw_inc = (double *)os1;
-            os0 = os1 = NULL;
-        }
-    } else if (!ctx->err[0]) {
-        snprintf(ctx->err, sizeof(ctx->err), "PCDVC population control failed (%d): %s", rc, ust_dev_error_string());
-    }
-    free(cnt_h);
-    free(off_h);
-    void *tmp[] = {cnt, list, flag, noff, o, ow, omat, ocoh, os0, os1};
+    void *tmp[] = {cnt, list, elems, cwork};
     for (size_t i = 0; i < sizeof(tmp) / sizeof(tmp[0]); i++) ust_dev_free(tmp[i]);
+    new_swarm_free(&s);
     if (rc) return rc;
-    /* 4. the regions of the new particles: integration points at the centroids, weights the volumes */
-    rc = ust_swarm_dvc_weights(ctx, opts->res, 1);
-    if (rc) return rc;
-    if (n_split) *n_split = hflag[1];
-    if (n_deleted) *n_deleted = hflag[2];
+    if (n_split) *n_split = nspl;
+    if (n_deleted) *n_deleted = ndel;
     return UST_OK;
 }
 
@@ -1274,26 +1323,13 @@ int ust_swarm_download_integration_points(ust_context *ctx, double *xi, double *
 }
 
 int ust_swarm_dvc_weights(ust_context *ctx, const int *res, int set_centroids) {
-    if (!ctx->np) UST_FAIL(ctx, UST_ESTATE, "no swarm");
-    if (!res) UST_FAIL(ctx, UST_EINVAL, "resolution missing");
-    const int dim = ctx->grid.dim;
-    int ncell = 1;
-    for (int a = 0; a < dim; a++) {
-        if (res[a] < 1 || res[a] > 64) UST_FAIL(ctx, UST_EINVAL, "DVC resolution %d out of 1..64", res[a]);
-        ncell *= res[a];
-    }
-    if (ncell > 4096) UST_FAIL(ctx, UST_EINVAL, "DVC sub-grid of %d cells exceeds 4096", ncell);
-    if (ctx->max_ppc < 1 || ctx->max_ppc > 32767)
-        UST_FAIL(ctx, UST_EINVAL, "%d particles per element: DVC holds 1..32767", ctx->max_ppc);
-    const size_t lds = ust_k_dvc_lds_bytes(dim, res, ctx->max_ppc);
-    if (lds > 65536)
-        UST_FAIL(ctx, UST_EINVAL, "DVC needs %zu bytes of LDS per element (%d particles, %d sub-cells): limit 65536",
-                 lds, ctx->max_ppc, ncell);
+    int rc = dvc_check(ctx, res);
+    if (rc) return rc;
     /* DVCWeights moves the integration points (DVCWeights.c:836-843), not the material points they were
      * mapped from: the centroids go to the context's integration-point coordinates, seeded from the
      * material points as CoincidentMapper maps them, and the material points stay where they are */
+    const int dim = ctx->grid.dim;
     const size_t n = (size_t)ctx->np;
-    double *d0 = ctx->xi0, *d1 = ctx->xi1, *d2 = ctx->xi2;
     if (set_centroids) {
         if (!ctx->ixi0) {
             DALLOC(ctx, ctx->ixi0, n * sizeof(double));
@@ -1303,29 +1339,8 @@ int ust_swarm_dvc_weights(ust_context *ctx, const int *res, int set_centroids) {
         CKD(ctx, ust_memcpy_d2d(ctx->ixi0, ctx->xi0, n * sizeof(double), ctx->stream));
         CKD(ctx, ust_memcpy_d2d(ctx->ixi1, ctx->xi1, n * sizeof(double), ctx->stream));
         if (dim == 3) CKD(ctx, ust_memcpy_d2d(ctx->ixi2, ctx->xi2, n * sizeof(double), ctx->stream));
-        d0 = ctx->ixi0;
-        d1 = ctx->ixi1;
-        d2 = ctx->ixi2;
     } else {
         free_integration_points(ctx); /* weights only: the integration points coincide with the material points */
     }
-    void *flag = NULL;
-    int hflag = 0;
-    CKD(ctx, ust_dev_malloc(&flag, sizeof(double)));
-    int rc = ust_k_fill_f64((double *)flag, 0.0, 1, ctx->stream); /* all-zero bits: the int flag reads 0 */
-    if (!rc)
-        rc = ust_k_dvc_weights(dim, res, ctx->nel, ctx->cell_off, ctx->max_ppc, d0, d1, d2, ctx->w, set_centroids,
-                               (int *)flag, ctx->stream);
-    if (!rc) rc = ust_memcpy_d2h(&hflag, flag, sizeof(int), ctx->stream);
-    ust_dev_free(flag);
-    if (rc) UST_FAIL(ctx, rc, "DVC weights failed (%d): %s", rc, ust_dev_error_string());
-    /* the weights and points changed even when an element failed: nothing assembled stays valid */
-    ctx->assembled = 0;
-    ctx->cache_valid = 0;
-    if (hflag & 1)
-        UST_FAIL(ctx, UST_EINVAL, "under resolved cell: an element has no particles, add more particles "
-                                  "(DVCWeights.c:787)");
-    if (hflag & 2) UST_FAIL(ctx, UST_EINVAL, "an element holds more particles than the swarm's maximum per cell");
-    if (hflag & 4) UST_FAIL(ctx, UST_ENOTCONV, "DVC region growth did not settle within its round limit");
-    return UST_OK;
+    return dvc_regions(ctx, res, set_centroids, NULL, ctx->nel);
 }

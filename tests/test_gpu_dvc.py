@@ -223,6 +223,37 @@ def test_pcdvc_matches_oracle(dim, nel, res):
     s.close()
 
 
+# element counts around the 1024 of a block of the count scan; more particles than the 32 lanes of an element's group
+@pytest.mark.parametrize("dim,nel,top", [(2, (33, 31), 30), (2, (41, 25), 70), (3, (16, 8, 8), 40)])
+def test_pcdvc_regions_of_unchanged_elements(dim, nel, top):
+    """After population control, which grows the regions of the changed elements only, the regions of all elements grown
+    anew from the same particles: weights and integration points bit for bit, with some elements changed and some not.
+    Offsets, splits and deletions against the regions before it."""
+    s = _system(dim, nel)
+    ne = int(np.prod(nel))
+    counts = np.random.default_rng(ne).integers(3, top, ne)
+    s.random_particle_layout(seed=31, cell_counts=counts)
+    s.dvc_weights(resolution=8)
+    off, _, w, _ = s.swarm()
+    limit = 2.0 ** dim * np.array([25.0, 0.6]) / 100.0
+    cell = np.repeat(np.arange(ne), counts)
+    nspl = np.minimum(np.bincount(cell[w > limit[0]], minlength=ne), 3)
+    cap = np.where(2 > counts - 4, counts // 2, 2)
+    ndel = np.minimum(np.bincount(cell[w < limit[1]], minlength=ne), cap)
+    changed = (nspl > 0) | (ndel > 0)
+    assert 0 < changed.sum() < ne
+    assert s.pcdvc(resolution=8) == (nspl.sum(), ndel.sum())
+    off2, xi2, w2, _ = s.swarm()
+    ixi2, iw2 = s.integration_points()
+    assert np.array_equal(np.diff(off2), counts + nspl - ndel)
+    s.dvc_weights(resolution=8)
+    _, xi3, w3, _ = s.swarm()
+    ixi3, iw3 = s.integration_points()
+    for a, b in ((xi2, xi3), (w2, w3), (ixi2, ixi3), (iw2, iw3)):
+        assert np.array_equal(a, b)
+    s.close()
+
+
 def test_pcdvc_suite_statistics():
     """PCDVCSuite.c:140-353 on the GPU path (testPCDVC.xml: 2x2 elements on [0,4]^2, 20 particles per cell, 10x10
     sub-grid, maxDeletions = maxSplits = 0, 1000 seeds): the suite's expected error statistics of three element-0
