@@ -7,6 +7,7 @@
 
 #define UST_MAX_LEVELS 12
 #define UST_MAX_CHEBY 24
+#define UST_POOL_BLOCKS 64
 
 /* device scalar slots */
 enum { SC_SUM = 0, SC_T0, SC_T1, SC_T2, SC_T3,
@@ -61,6 +62,14 @@ struct ust_context {
      * points coincide with the material points (CoincidentMapper) unless a weights calculator moved them:
      * then ixi0..2 hold their own local coordinates (DVCWeights' centroids), NULL otherwise. */
     int np, max_ppc;
+    /* blocks of 1 MiB or more that advection and population control took: in use (live), or idle for their next one */
+    struct {
+        void *p;
+        size_t bytes;
+        int live;
+    } pool[UST_POOL_BLOCKS];
+    int npool;
+    size_t pool_idle; /* bytes of the idle ones */
     int *cell_off;
     double *xi0, *xi1, *xi2, *w;
     double *ixi0, *ixi1, *ixi2;

@@ -254,6 +254,57 @@ def test_pcdvc_regions_of_unchanged_elements(dim, nel, top):
     s.close()
 
 
+def test_particle_buffers_across_steps_and_contexts():
+    """Advection and population control hand large blocks on from step to step (240k particles: arrays of 1.9 MB).  Two
+    contexts stepped in turns, with the strain-weakening state dropped and the swarm laid out anew in between, against
+    contexts that take the same steps from the start without the other: swarms, weights and points bit for bit."""
+    import earthbyte_underworld_amd as ust
+    nel = (100, 80)
+
+    def system(seed):
+        s = _system(2, nel)
+        s.random_particle_layout(seed=seed, particlesPerCell=30)
+        s.assign_materials([ust.Everywhere(0), ust.Sphere(1, (0.5, 0.5), 0.3)])
+        xyz = s.node_coords()
+        u = np.zeros(s.ndof)
+        u[0::2] = np.sin(np.pi * xyz[:, 0]) * np.cos(np.pi * xyz[:, 1])
+        u[1::2] = -np.cos(np.pi * xyz[:, 0]) * np.sin(np.pi * xyz[:, 1])
+        s.set_solution(u, None)
+        return s
+
+    def step(s):
+        s.advect(0.3 / max(nel), order=2, allowFallbackToFirstOrder=True)
+        s.pcdvc(resolution=6)
+
+    def state(s):
+        return s.swarm() + s.integration_points()
+
+    a, b = system(1), system(2)
+    a.set_strain_weakening(ust.StrainWeakening(softeningStrain=1.0))
+    for s in (a, b, a, b):
+        step(s)
+    a.set_strain_weakening(None)
+    for s in (b, a, b, a):
+        step(s)
+    for s, seed, n in ((a, 1, 4), (b, 2, 4)):
+        ref = system(seed)
+        for _ in range(n):
+            step(ref)
+        for x, y in zip(state(s), state(ref)):
+            assert np.array_equal(x, y)
+        ref.close()
+    a.random_particle_layout(seed=5, particlesPerCell=35)
+    step(a)
+    step(b)
+    ref = system(5)
+    ref.random_particle_layout(seed=5, particlesPerCell=35)
+    step(ref)
+    for x, y in zip(state(a)[:3], state(ref)[:3]):
+        assert np.array_equal(x, y)
+    for s in (a, b, ref):
+        s.close()
+
+
 def test_pcdvc_suite_statistics():
     """PCDVCSuite.c:140-353 on the GPU path (testPCDVC.xml: 2x2 elements on [0,4]^2, 20 particles per cell, 10x10
     sub-grid, maxDeletions = maxSplits = 0, 1000 seeds): the suite's expected error statistics of three element-0
