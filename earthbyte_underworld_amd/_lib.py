@@ -72,7 +72,8 @@ class Grid(C.Structure):
 class Pass(C.Structure):  # ust_pass
     _fields_ = [("mode", C.c_int), ("type", C.c_int), ("W", C.c_void_p), ("mask", C.c_void_p), ("u", C.c_void_p),
                 ("y", C.c_void_p), ("b", C.c_void_p), ("invd", C.c_void_p), ("d", C.c_void_p), ("xc", C.c_void_p),
-                ("c0", C.c_double), ("c1", C.c_double), ("c2", C.c_double), ("d_last", C.c_int), ("dot", C.c_void_p)]
+                ("bc", C.c_void_p), ("maskc", C.c_void_p), ("c0", C.c_double), ("c1", C.c_double), ("c2", C.c_double),
+                ("d_last", C.c_int), ("dot", C.c_void_p)]
 
 
 class SolveOpts(C.Structure):
@@ -228,8 +229,10 @@ _SIGS = {
     "ust_k_cg_dir_f64": (I, [vp, vp, vp, vp, I, C.c_size_t, vp]),
     "ust_k_cg_dir_zf": (I, [vp, vp, vp, vp, I, C.c_size_t, vp]),
     "ust_k_cg_dir_f32": (I, [vp, vp, vp, vp, I, C.c_size_t, vp]),
-    "ust_k_cg_step_f64": (I, [vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
-    "ust_k_cg_step_f32": (I, [vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_step_f64": (I, [vp, vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_step_f32": (I, [vp, vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_cg_dir_apply": (I, [C.POINTER(Grid), I, vp, vp, vp, vp, vp, vp, vp, vp, I, C.c_size_t, vp]),
+    "ust_k_apply_groups": (I, [C.POINTER(Grid), I]),
     "ust_k_cg_state": (I, [vp, vp, C.c_size_t, vp, vp]),
     "ust_k_apply_K_f32_bf16w": (I, [C.POINTER(Grid), vp, vp, vp, vp, vp, vp]),
     "ust_k_apply_K_residual_f32_bf16w": (I, [C.POINTER(Grid), vp, vp, vp, vp, vp, vp, vp]),

@@ -17,6 +17,7 @@
 #include <mutex>
 #include <stdio.h>
 
+#include "ust_cg.h"
 #include "ust_common.h"
 
 // axes orthogonal to k, in increasing order
@@ -241,7 +242,8 @@ enum {
     EPI_CHEBY0 = UST_PASS_CHEBY0,
     EPI_PCHEBY0 = UST_PASS_PCHEBY0,
     EPI_RES0 = UST_PASS_RES0,
-    EPI_CHEBY1 = UST_PASS_CHEBY1
+    EPI_CHEBY1 = UST_PASS_CHEBY1,
+    EPI_P = -1  // halo kernels: u is z, staged is the CG direction z + beta p, which goes to next; y as EPI_Y
 };
 template <typename T>
 struct Epi {
@@ -304,7 +306,7 @@ __device__ __forceinline__ EpiOps<T> epilogue_load(const Epi<T> &ep, const unsig
     EpiOps<T> o;
     o.m = mask[i];
     o.b = o.invd = o.d = o.x = (T)0;
-    if (MODE != EPI_Y) o.b = ep.b[i];
+    if (MODE != EPI_Y && MODE != EPI_P) o.b = ep.b[i];
     if (MODE == EPI_RES0 || MODE == EPI_CHEBY1) o.invd = ep.invd[i];
     if (cheby_mode(MODE)) {
         o.invd = ep.invd[i];
@@ -319,7 +321,7 @@ template <int MODE, typename T>
 __device__ __forceinline__ T epilogue_store(const Epi<T> &ep, const EpiOps<T> &o, unsigned i, T v) {
     v = o.m ? (T)0 : v;
     T out;
-    if (MODE == EPI_Y) {
+    if (MODE == EPI_Y || MODE == EPI_P) {
         out = v;
     } else if (MODE == EPI_RES || MODE == EPI_RES0) {
         out = o.m ? (T)0 : o.b - v;
@@ -777,9 +779,9 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, const WT *_
 // deterministic.  The operands of the
 // epilogue are loaded with the node block, so that only one trip to memory is exposed, and a pass can leave per-workgroup
 // partial sums of the dot product that follows it in the Krylov iteration.
-// What bounds them is the serial chain of one wavefront: launch, one trip to memory, 1200-1600 instructions, a store.  The
-// V-cycle on such levels takes 14 launches per inner iteration in 2D at 64x64 where steps of tiles + gather, separate
-// first steps, prolongation and dots took 24; solves: 2D 64x64 FP64 129.6 -> 74.7 ms, 3D 24x16x16 FP64 661 -> 455 ms.
+// What bounds them is the serial chain of one wavefront: launch, one trip to memory, 1200-1600 instructions, a store.  With
+// every pass of such levels on them an inner iteration took 14 launches in 2D at 64x64 where tiles + gather, separate first
+// steps, prolongation and dots took 24; solves: 2D 64x64 FP64 129.6 -> 74.7 ms, 3D 24x16x16 FP64 661 -> 455 ms.
 // Staging whole nodes (index arithmetic once per node, none of the loads behind a branch) instead of single dofs:
 // 466.8 -> 455 ms of the latter, the 64x64x32 solve with FP32 PCG 388 -> 379 ms.
 // ------------------------------------------------------------------------------------------
@@ -789,6 +791,33 @@ constexpr int HNX = HOX + 2, HNY = HOY + 2, HNZ = HOZ + 2;  // staged nodes per 
 constexpr int HNE = HEX * HEY * HEZ, HNN = HNX * HNY * HNZ;  // 225 element slots, 360 staged nodes
 static_assert(HNE <= UST_TILE && HOX * HOY * HOZ * 2 == UST_TILE, "one element, at most two owned dofs per thread");
 constexpr int H2O = 15, H2N = H2O + 2, H2D = H2O * H2O * 2;  // 2D: owned nodes and staged nodes per axis, owned dofs
+
+// EPI_P: the previous direction p, the new one next, and the CG's control block and partial sums (ust_cg.h)
+template <typename T>
+struct CgDir {
+    const T *p;
+    T *next;
+    double *c;
+    const double *part;
+    int nrz, nrr;
+};
+// the direction's beta, or false once the CG has stopped; called by every thread of the workgroup, whose first one writes
+// the control block
+template <typename T>
+__device__ __forceinline__ bool cg_direction(const CgDir<T> &cg, bool *first, T *beta) {
+    const CgSums s = cg_sums(cg.part + CG_RZ, cg.nrz, cg.part + CG_RR, cg.nrr, cg.c);
+    double thr = 0.0;
+    const double state = cg_state(s, s.b, &thr);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && s.c[1] == 0.0) {
+        cg.c[1] = state;
+        cg.c[2] = s.c[4];
+        cg.c[3] = s.a;
+        cg.c[6] = thr;
+    }
+    *first = s.c[4] == 0.0;
+    *beta = (T)(s.a / s.c[5]);
+    return state == 0.0;
+}
 
 // 3D grids up to this many elements take the halo kernel.  Measured on the 128x128x64 solve (same box, graph-replayed):
 // the halo passes on the 32x32x16 and 16x16x8 levels take it from 0.431-0.434 s to 0.403-0.407 s; on the 64x64x32 level
@@ -815,7 +844,8 @@ __device__ __forceinline__ void block_dot(double v, double *out) {
 
 template <typename T, typename WT, int MODE>
 __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__restrict__ W,
-                                                      const unsigned char *__restrict__ mask, const T *u, Epi<T> ep) {
+                                                      const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
+                                                      CgDir<T> cg) {
     __shared__ T su[HNN * 3];   // staged node block, origin (nx0 - 1, ny0 - 1, nz0 - 1)
     __shared__ T eb[24 * HNE];  // element results: eb[(a*3 + i) * HNE + slot] (HNE odd: rows shift banks)
     const int hnx = (g.nnx + HOX - 1) / HOX, hny = (g.nny + HOY - 1) / HOY;
@@ -826,6 +856,7 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
     // nearest node of the grid, so that none of them waits for a branch)
     constexpr int NST = (HNN + UST_TILE - 1) / UST_TILE;
     T stv[NST][3];
+    T stp[MODE == EPI_P ? NST : 1][3];
     unsigned char stm[NST][3];
     bool stok[NST];
 #pragma unroll
@@ -839,6 +870,7 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
         for (int c = 0; c < 3; c++) {
             stm[r][c] = mask[dof + c];
             stv[r][c] = stage_load<MODE, T>(ep, u, dof + c);
+            if (MODE == EPI_P) stp[r][c] = cg.p[dof + c];
         }
         if (MODE == EPI_PCHEBY0) {  // x + P xc on the free dofs, the coarse values read from global memory
 #pragma unroll
@@ -867,6 +899,23 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
     EpiOps<T> ops[2];
 #pragma unroll
     for (int r = 0; r < 2; r++) ops[r] = epilogue_load<MODE, T>(ep, mask, odof + (r ? 2 : tid / (HOX * HOY * HOZ)));
+    if (MODE == EPI_P) {
+        bool first;
+        T beta;
+        if (!cg_direction(cg, &first, &beta)) return;
+#pragma unroll
+        for (int r = 0; r < NST; r++) {
+            const int n = tid + UST_TILE * r;
+            const int ax = n % HNX, ay = (n / HNX) % HNY, az = n / (HNX * HNY);
+            const bool mine = stok[r] && ax >= 1 && ax <= HOX && ay >= 1 && ay <= HOY && az >= 1 && az <= HOZ && n < HNN;
+            const unsigned dof = ((unsigned)(nx0 - 1 + ax) + (unsigned)g.nnx * ((unsigned)(ny0 - 1 + ay) + (unsigned)g.nny * (nz0 - 1 + az))) * 3u;
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                stv[r][c] = first ? stv[r][c] : stv[r][c] + beta * stp[r][c];
+                if (mine) cg.next[dof + c] = stv[r][c];
+            }
+        }
+    }
 #pragma unroll
     for (int r = 0; r < NST; r++) {
         const int n = tid + UST_TILE * r;
@@ -906,14 +955,15 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
         EpiOps<T> o = ops[r];
         if (MODE == EPI_PCHEBY0 && !o.m) o.x = us;  // x + P xc, as staged
         const T out = epilogue_store<MODE, T>(ep, o, odof + c, (T)v);
-        dot += (double)out * (double)(MODE == EPI_Y ? us : o.b);
+        dot += (double)out * (double)(MODE == EPI_Y || MODE == EPI_P ? us : o.b);
     }
     if (ep.dot) block_dot(dot, ep.dot);
 }
 
 template <typename T, typename WT, int MODE>
 __global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__restrict__ W,
-                                                      const unsigned char *__restrict__ mask, const T *u, Epi<T> ep) {
+                                                      const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
+                                                      CgDir<T> cg) {
     __shared__ T su[H2N * H2N * 2];          // staged node block, origin (nx0 - 1, ny0 - 1)
     __shared__ T eb[8 * (UST_TILE + 1)];     // element results: eb[(a*2 + i) * 257 + slot]
     const int hnx = (g.nnx + H2O - 1) / H2O;
@@ -922,6 +972,7 @@ __global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__res
     const int cnx = g.nx / 2 + 1;  // EPI_PCHEBY0: the coarse grid
     constexpr int NSN = H2N * H2N, NST = (NSN + UST_TILE - 1) / UST_TILE;
     T stv[NST][2];
+    T stp[MODE == EPI_P ? NST : 1][2];
     unsigned char stm[NST][2];
     bool stok[NST];
 #pragma unroll
@@ -935,6 +986,7 @@ __global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__res
         for (int c = 0; c < 2; c++) {
             stm[r][c] = mask[dof + c];
             stv[r][c] = stage_load<MODE, T>(ep, u, dof + c);
+            if (MODE == EPI_P) stp[r][c] = cg.p[dof + c];
         }
         if (MODE == EPI_PCHEBY0) {
 #pragma unroll
@@ -962,6 +1014,23 @@ __global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__res
         own[r] = d < H2D && gx < g.nnx && gy < g.nny;
         dofs[r] = own[r] ? ((unsigned)gx + (unsigned)g.nnx * (unsigned)gy) * 2u + d % 2 : 0u;
         ops[r] = epilogue_load<MODE, T>(ep, mask, dofs[r]);
+    }
+    if (MODE == EPI_P) {
+        bool first;
+        T beta;
+        if (!cg_direction(cg, &first, &beta)) return;
+#pragma unroll
+        for (int r = 0; r < NST; r++) {
+            const int n = tid + UST_TILE * r;
+            const int ax = n % H2N, ay = n / H2N;
+            const bool mine = stok[r] && ax >= 1 && ax <= H2O && ay >= 1 && ay <= H2O && n < NSN;
+            const unsigned dof = ((unsigned)(nx0 - 1 + ax) + (unsigned)g.nnx * (unsigned)(ny0 - 1 + ay)) * 2u;
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                stv[r][c] = first ? stv[r][c] : stv[r][c] + beta * stp[r][c];
+                if (mine) cg.next[dof + c] = stv[r][c];
+            }
+        }
     }
 #pragma unroll
     for (int r = 0; r < NST; r++) {
@@ -1003,9 +1072,420 @@ __global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__res
         EpiOps<T> o = ops[r];
         if (MODE == EPI_PCHEBY0 && !o.m) o.x = us;  // x + P xc, as staged
         const T out = epilogue_store<MODE, T>(ep, o, dofs[r], (T)v);
-        dot += (double)out * (double)(MODE == EPI_Y ? us : o.b);
+        dot += (double)out * (double)(MODE == EPI_Y || MODE == EPI_P ? us : o.b);
     }
     if (ep.dot) block_dot(dot, ep.dot);
+}
+
+// ------------------------------------------------------------------------------------------
+// Fused level passes: the pre-smoothing of a level with its residual and restriction, and in 2D both post-smoothing steps,
+// in one launch.  A workgroup owns a block of coarse nodes (of nodes, for the post-smoothing) and computes what they depend
+// on, one or two rings of elements around the block: more arithmetic, but on the grids that take the halo kernels a launch
+// and its trip to memory cost more.  With the direction formed by the product's pass, an inner iteration takes 7 launches
+// for 14 at 2D 64x64 and 11 for 14 at 3D 24x16x16.  Solves: 2D 64x64 FP64 74.2 -> 54.4 ms, 256x256 117 -> 70, 512x256
+// 181 -> 113; 3D 24x16x16 FP64 453 -> 431, 64x64x32 with FP32 PCG (two such levels) 368 -> 363.5.
+// Every value is computed by the formulas and in the order of the separate passes.
+// ------------------------------------------------------------------------------------------
+// 2D, three kinds: residual of u; of the first step from zero; of the first two steps from zero.  6x6 coarse nodes, that is
+// 13x13 residual nodes, 14x14 elements, 15x15 nodes of x, and one more ring for the kind whose x takes a product.
+constexpr int F2C = 6, F2R = 2 * F2C + 1, F2X = F2R + 2, F2S = F2X + 2, F2E = 16;
+static_assert(F2S == F2E + 1 && F2E * F2E == UST_TILE, "one element per thread");
+enum { PRE_U = 0, PRE_FIRST = 1, PRE_TWO = 2 };
+
+// the element of this thread's slot applied to the staged block su into eb; slots outside the grid leave zeros
+template <typename T>
+__device__ __forceinline__ void block_apply2(const T *su, int lx, int ly, bool valid, const T *wq, const T *s, T *eb) {
+    T ue[4][2], ye[4][2];
+#pragma unroll
+    for (int a = 0; a < 4; a++) {
+        const int ln = (lx + (a & 1)) + F2S * (ly + (a >> 1));
+        ue[a][0] = su[ln * 2];
+        ue[a][1] = su[ln * 2 + 1];
+        ye[a][0] = ye[a][1] = (T)0;
+    }
+    element_apply2<T>(ue, wq, s, ye);
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int i = 0; i < 2; i++) eb[(a * 2 + i) * (UST_TILE + 1) + lx + F2E * ly] = valid ? ye[a][i] : (T)0;
+}
+// (K x) at node (i, j) of the 15x15 ring, component c
+template <typename T>
+__device__ __forceinline__ T block_sum2(const T *eb, int i, int j, int c) {
+    double v = 0.0;
+#pragma unroll
+    for (int dy = 1; dy >= 0; dy--)
+#pragma unroll
+        for (int dx = 1; dx >= 0; dx--)
+            v += (double)eb[((dx + 2 * dy) * 2 + c) * (UST_TILE + 1) + (i + 1 - dx) + F2E * (j + 1 - dy)];
+    return (T)v;
+}
+
+template <typename T, typename WT, int KIND>
+__global__ __launch_bounds__(256) void k_pre2(GridDev g, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+                                              const unsigned char *__restrict__ maskc, const T *__restrict__ u,
+                                              const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ y,
+                                              T *__restrict__ d, T *__restrict__ bc, T c0, T c1, T c2) {
+    __shared__ T su[F2S * F2S * 2];
+    __shared__ T eb[8 * (UST_TILE + 1)];
+    __shared__ T sr[F2R * F2R * 2];
+    const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1, tbx = (cnx + F2C - 1) / F2C;
+    const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
+    const int I0 = (tile % tbx) * F2C, J0 = (tile / tbx) * F2C;
+    const int ox = 2 * I0 - 3, oy = 2 * J0 - 3;  // origin of the staged block
+    const auto dof_of = [&](int gx, int gy, bool *in) -> unsigned {
+        const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1);
+        *in = kx == gx && ky == gy;
+        return ((unsigned)kx + (unsigned)g.nnx * (unsigned)ky) * 2u;
+    };
+    // the first x at the staged nodes
+    constexpr int NST = (F2S * F2S + UST_TILE - 1) / UST_TILE;
+    T sv[NST][2];
+#pragma unroll
+    for (int r = 0; r < NST; r++) {
+        const int n = min(tid + UST_TILE * r, F2S * F2S - 1);
+        bool in;
+        const unsigned k = dof_of(ox + n % F2S, oy + n / F2S, &in);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const bool m = mask[k + c] != 0;
+            const T x = KIND == PRE_U ? u[k + c] : (KIND == PRE_FIRST ? c2 : c0) * invd[k + c] * b[k + c];
+            sv[r][c] = in && !m ? x : (T)0;
+        }
+    }
+    // the thread's element and its weights, and its node of the 15x15 ring
+    const int lx = tid % F2E, ly = tid / F2E, ex = ox + lx, ey = oy + ly;
+    const bool valid = ex >= 0 && ey >= 0 && ex < g.nx && ey < g.ny;
+    const size_t w0 = valid ? widx_at(g, ex, ey, 0, 0) : 0;
+    T wq[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) wq[q] = wload<T, WT>(W, w0 + (size_t)q * UST_TILE);
+    const bool node = tid < F2X * F2X;
+    const int i = min(tid, F2X * F2X - 1) % F2X, j = min(tid, F2X * F2X - 1) / F2X;
+    bool in;
+    const unsigned k = dof_of(ox + 1 + i, oy + 1 + j, &in);
+    const bool own = node && in && i >= 2 && j >= 2 && i < 2 + 2 * F2C && j < 2 + 2 * F2C;
+    bool m[2];
+    T bv[2], iv[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        m[c] = mask[k + c] != 0;
+        bv[c] = b[k + c];
+        iv[c] = KIND == PRE_U ? (T)0 : invd[k + c];
+    }
+    const int cn = tid / 2, cc = tid % 2, I = I0 + cn % F2C, J = J0 + cn / F2C;
+    const bool coarse = tid < F2C * F2C * 2 && I < cnx && J < cny;
+    const unsigned ck = coarse ? ((unsigned)I + (unsigned)cnx * (unsigned)J) * 2u + cc : 0u;
+    const bool mc = maskc[ck] != 0;
+#pragma unroll
+    for (int r = 0; r < NST; r++) {
+        const int n = tid + UST_TILE * r;
+        if (n < F2S * F2S) {
+            su[n * 2] = sv[r][0];
+            su[n * 2 + 1] = sv[r][1];
+        }
+    }
+    const T s[3] = {(T)g.sx, (T)g.sy, (T)1};
+    __syncthreads();
+    block_apply2(su, lx, ly, valid, wq, s, eb);
+    __syncthreads();
+    if (KIND == PRE_TWO) {
+        if (node) {
+            T x2[2];
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                const T v = m[c] ? (T)0 : block_sum2(eb, i, j, c);
+                const T x = c0 * iv[c] * bv[c];
+                const T dn = c1 * x + c2 * iv[c] * (bv[c] - v);
+                x2[c] = x + dn;
+                if (own) {
+                    y[k + c] = x2[c];
+                    if (d) d[k + c] = dn;
+                }
+            }
+#pragma unroll
+            for (int c = 0; c < 2; c++) su[((i + 1) + F2S * (j + 1)) * 2 + c] = in && !m[c] ? x2[c] : (T)0;
+        }
+        __syncthreads();
+        block_apply2(su, lx, ly, valid, wq, s, eb);  // the outer ring of slots is not used any more
+        __syncthreads();
+    }
+    if (KIND == PRE_FIRST && own) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) d[k + c] = c2 * iv[c] * bv[c];
+    }
+    if (node && i >= 1 && j >= 1 && i <= F2R && j <= F2R) {
+#pragma unroll
+        for (int c = 0; c < 2; c++)
+            sr[((i - 1) + F2R * (j - 1)) * 2 + c] = in && !m[c] ? bv[c] - block_sum2(eb, i, j, c) : (T)0;
+    }
+    __syncthreads();
+    if (!coarse) return;
+    const int ci = 2 * (I - I0) + 1, cj = 2 * (J - J0) + 1;
+    T acc = (T)0;
+#pragma unroll
+    for (int dy = -1; dy <= 1; dy++)
+#pragma unroll
+        for (int dx = -1; dx <= 1; dx++)
+            acc += (T)((dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0)) * sr[((ci + dx) + F2R * (cj + dy)) * 2 + cc];
+    bc[ck] = mc ? (T)0 : acc;
+}
+
+// 2D, both post-smoothing steps: 13x13 nodes
+template <typename T, typename WT>
+__global__ __launch_bounds__(256) void k_post2(GridDev g, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+                                               const T *__restrict__ u, const T *__restrict__ xc, const T *__restrict__ b,
+                                               const T *__restrict__ invd, T *__restrict__ y, T c0, T c1, T c2,
+                                               double *__restrict__ dots) {
+    __shared__ T su[F2S * F2S * 2];
+    __shared__ T eb[8 * (UST_TILE + 1)];
+    const int tbx = (g.nnx + F2R - 1) / F2R, cnx = g.nx / 2 + 1;
+    const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
+    const int ox = (tile % tbx) * F2R - 2, oy = (tile / tbx) * F2R - 2;  // origin of the staged block
+    const auto dof_of = [&](int gx, int gy, bool *in) -> unsigned {
+        const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1);
+        *in = kx == gx && ky == gy;
+        return ((unsigned)kx + (unsigned)g.nnx * (unsigned)ky) * 2u;
+    };
+    constexpr int NST = (F2S * F2S + UST_TILE - 1) / UST_TILE;
+    T sv[NST][2];
+#pragma unroll
+    for (int r = 0; r < NST; r++) {
+        const int n = min(tid + UST_TILE * r, F2S * F2S - 1);
+        const int gx = ox + n % F2S, gy = oy + n / F2S;
+        bool in;
+        const unsigned k = dof_of(gx, gy, &in);
+        const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1);
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const bool m = mask[k + c] != 0;
+            const T pc = prolong_value2<T>(kx, ky, [&](int I, int J) {
+                return xc[((unsigned)I + (unsigned)cnx * (unsigned)J) * 2u + c];
+            });
+            const T x = u[k + c] + pc;
+            sv[r][c] = in && !m ? x : (T)0;
+        }
+    }
+    const int lx = tid % F2E, ly = tid / F2E, ex = ox + lx, ey = oy + ly;
+    const bool valid = ex >= 0 && ey >= 0 && ex < g.nx && ey < g.ny;
+    const size_t w0 = valid ? widx_at(g, ex, ey, 0, 0) : 0;
+    T wq[9];
+#pragma unroll
+    for (int q = 0; q < 9; q++) wq[q] = wload<T, WT>(W, w0 + (size_t)q * UST_TILE);
+    const bool node = tid < F2X * F2X;
+    const int i = min(tid, F2X * F2X - 1) % F2X, j = min(tid, F2X * F2X - 1) / F2X;
+    bool in;
+    const unsigned k = dof_of(ox + 1 + i, oy + 1 + j, &in);
+    bool m[2];
+    T bv[2], iv[2], uv[2];
+#pragma unroll
+    for (int c = 0; c < 2; c++) {
+        m[c] = mask[k + c] != 0;
+        bv[c] = b[k + c];
+        iv[c] = invd[k + c];
+        uv[c] = u[k + c];
+    }
+#pragma unroll
+    for (int r = 0; r < NST; r++) {
+        const int n = tid + UST_TILE * r;
+        if (n < F2S * F2S) {
+            su[n * 2] = sv[r][0];
+            su[n * 2 + 1] = sv[r][1];
+        }
+    }
+    const T s[3] = {(T)g.sx, (T)g.sy, (T)1};
+    __syncthreads();
+    block_apply2(su, lx, ly, valid, wq, s, eb);
+    __syncthreads();
+    T x1[2], d1[2];
+    if (node) {
+        const int sn = ((i + 1) + F2S * (j + 1)) * 2;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const T v = m[c] ? (T)0 : block_sum2(eb, i, j, c);
+            const T x = m[c] ? uv[c] : su[sn + c];
+            d1[c] = c0 * iv[c] * (bv[c] - v);
+            x1[c] = x + d1[c];
+        }
+#pragma unroll
+        for (int c = 0; c < 2; c++) su[sn + c] = in && !m[c] ? x1[c] : (T)0;
+    }
+    __syncthreads();
+    block_apply2(su, lx, ly, valid, wq, s, eb);
+    __syncthreads();
+    double dot = 0.0;
+    if (node && in && i >= 1 && j >= 1 && i <= F2R && j <= F2R) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const T v = m[c] ? (T)0 : block_sum2(eb, i, j, c);
+            const T dn = c1 * d1[c] + c2 * iv[c] * (bv[c] - v);
+            const T out = x1[c] + dn;
+            y[k + c] = out;
+            dot += (double)out * (double)bv[c];
+        }
+    }
+    if (dots) block_dot(dot, dots);
+}
+
+// 3D, residual of u or of the first step from zero: 3x2x2 coarse nodes, that is 7x5x5 residual nodes, 8x6x6 elements (one
+// per thread of 320), 9x7x7 staged nodes.
+constexpr int F3X = 3, F3Y = 2, F3Z = 2;                                      // coarse nodes
+constexpr int F3RX = 2 * F3X + 1, F3RY = 2 * F3Y + 1, F3RZ = 2 * F3Z + 1;     // residual nodes
+constexpr int F3EX = F3RX + 1, F3EY = F3RY + 1, F3EZ = F3RZ + 1;              // elements
+constexpr int F3SX = F3EX + 1, F3SY = F3EY + 1, F3SZ = F3EZ + 1;              // staged nodes
+constexpr int F3E = F3EX * F3EY * F3EZ, F3R = F3RX * F3RY * F3RZ, F3S = F3SX * F3SY * F3SZ, F3T = 320;
+static_assert(F3E <= F3T && F3R * 3 <= 2 * F3T && F3S <= 2 * F3T, "288 elements, 525 residual dofs, 441 nodes");
+
+template <typename T, typename WT, int KIND>
+__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+                                              const unsigned char *__restrict__ maskc, const T *__restrict__ u,
+                                              const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ d,
+                                              T *__restrict__ bc, T c2) {
+    constexpr int EB = F3E + 1;
+    __shared__ T su[F3S * 3];
+    __shared__ T eb[24 * EB];
+    __shared__ T sr[F3R * 3];
+    const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1, cnz = g.nz / 2 + 1;
+    const int tbx = (cnx + F3X - 1) / F3X, tby = (cny + F3Y - 1) / F3Y;
+    const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
+    const int I0 = (tile % tbx) * F3X, J0 = ((tile / tbx) % tby) * F3Y, K0 = (tile / (tbx * tby)) * F3Z;
+    const int ox = 2 * I0 - 2, oy = 2 * J0 - 2, oz = 2 * K0 - 2;  // origin of the staged block and of the elements
+    const auto dof_of = [&](int gx, int gy, int gz, bool *in) -> unsigned {
+        const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1), kz = min(max(gz, 0), g.nnz - 1);
+        *in = kx == gx && ky == gy && kz == gz;
+        return ((unsigned)kx + (unsigned)g.nnx * ((unsigned)ky + (unsigned)g.nny * kz)) * 3u;
+    };
+    T sv[2][3];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int n = min(tid + F3T * r, F3S - 1);
+        bool in;
+        const unsigned k = dof_of(ox + n % F3SX, oy + (n / F3SX) % F3SY, oz + n / (F3SX * F3SY), &in);
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            const bool m = mask[k + c] != 0;
+            const T x = KIND == PRE_U ? u[k + c] : c2 * invd[k + c] * b[k + c];
+            sv[r][c] = in && !m ? x : (T)0;
+        }
+    }
+    const int et = min(tid, F3E - 1), lx = et % F3EX, ly = (et / F3EX) % F3EY, lz = et / (F3EX * F3EY);
+    const int ex = ox + lx, ey = oy + ly, ez = oz + lz;
+    const bool valid = ex >= 0 && ey >= 0 && ez >= 0 && ex < g.nx && ey < g.ny && ez < g.nz;
+    const size_t w0 = valid ? widx_at(g, ex, ey, ez, 0) : 0;
+    T wq[27];
+#pragma unroll
+    for (int q = 0; q < 27; q++) wq[q] = wload<T, WT>(W, w0 + (size_t)q * UST_TILE);
+    // the residual dofs t = tid, tid + 320: component t / 175 of node t % 175
+    bool rin[2], rm[2];
+    T rb[2], ri[2];
+    unsigned rk[2];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int t = min(tid + F3T * r, F3R * 3 - 1), c = t / F3R, n = t % F3R;
+        rk[r] = dof_of(ox + 1 + n % F3RX, oy + 1 + (n / F3RX) % F3RY, oz + 1 + n / (F3RX * F3RY), &rin[r]) + c;
+        rm[r] = mask[rk[r]] != 0;
+        rb[r] = b[rk[r]];
+        ri[r] = KIND == PRE_U ? (T)0 : invd[rk[r]];
+    }
+    const int cn = tid / 3, cc = tid % 3;
+    const int I = I0 + cn % F3X, J = J0 + (cn / F3X) % F3Y, K = K0 + cn / (F3X * F3Y);
+    const bool coarse = tid < F3X * F3Y * F3Z * 3 && I < cnx && J < cny && K < cnz;
+    const unsigned ck = coarse ? ((unsigned)I + (unsigned)cnx * ((unsigned)J + (unsigned)cny * K)) * 3u + cc : 0u;
+    const bool mc = maskc[ck] != 0;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int n = tid + F3T * r;
+        if (n < F3S)
+#pragma unroll
+            for (int c = 0; c < 3; c++) su[n * 3 + c] = sv[r][c];
+    }
+    __syncthreads();
+    if (tid < F3E) {
+        T ye[8][3];
+        const T s[3] = {(T)g.sx, (T)g.sy, (T)g.sz};
+        const T *sb = &su[(lx + F3SX * (ly + F3SY * lz)) * 3];
+        element_apply3<T>([&](int a, int q) -> T {
+            return sb[((a & 1) + F3SX * (((a >> 1) & 1) + F3SY * (a >> 2))) * 3 + q];
+        }, wq, s, ye);
+#pragma unroll
+        for (int a = 0; a < 8; a++)
+#pragma unroll
+            for (int q = 0; q < 3; q++) eb[(a * 3 + q) * EB + tid] = valid ? ye[a][q] : (T)0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        const int t = tid + F3T * r;
+        if (t >= F3R * 3) continue;
+        const int c = t / F3R, n = t % F3R, i = n % F3RX, j = (n / F3RX) % F3RY, k = n / (F3RX * F3RY);
+        double v = 0.0;
+#pragma unroll
+        for (int dz = 1; dz >= 0; dz--)
+#pragma unroll
+            for (int dy = 1; dy >= 0; dy--)
+#pragma unroll
+                for (int dx = 1; dx >= 0; dx--)
+                    v += (double)eb[((dx + 2 * dy + 4 * dz) * 3 + c) * EB + (i + 1 - dx) +
+                                    F3EX * ((j + 1 - dy) + F3EY * (k + 1 - dz))];
+        sr[n * 3 + c] = rin[r] && !rm[r] ? rb[r] - (T)v : (T)0;
+        // x = the first step, on the nodes 2 I0 .. 2 I0 + 5 and so on, each of one workgroup
+        if (KIND == PRE_FIRST && rin[r] && i >= 1 && j >= 1 && k >= 1) d[rk[r]] = c2 * ri[r] * rb[r];
+    }
+    __syncthreads();
+    if (!coarse) return;
+    const int ci = 2 * (I - I0) + 1, cj = 2 * (J - J0) + 1, cq = 2 * (K - K0) + 1;
+    T acc = (T)0;
+#pragma unroll
+    for (int dz = -1; dz <= 1; dz++)
+#pragma unroll
+        for (int dy = -1; dy <= 1; dy++)
+#pragma unroll
+            for (int dx = -1; dx <= 1; dx++)
+                acc += (T)((dx ? 0.5 : 1.0) * (dy ? 0.5 : 1.0) * (dz ? 0.5 : 1.0)) *
+                       sr[((ci + dx) + F3RX * ((cj + dy) + F3RY * (cq + dz))) * 3 + cc];
+    bc[ck] = mc ? (T)0 : acc;
+}
+
+static int fused_groups(const GridDev &g, int mode) {
+    const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1, cnz = g.nz / 2 + 1;
+    if (mode == UST_PASS_PCHEBY2) return ((g.nnx + F2R - 1) / F2R) * ((g.nny + F2R - 1) / F2R);
+    if (g.dim == 2) return ((cnx + F2C - 1) / F2C) * ((cny + F2C - 1) / F2C);
+    return ((cnx + F3X - 1) / F3X) * ((cny + F3Y - 1) / F3Y) * ((cnz + F3Z - 1) / F3Z);
+}
+
+template <typename T, typename WT>
+static int fused_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
+    const T *u = (const T *)p->u, *b = (const T *)p->b, *invd = (const T *)p->invd;
+    T *y = (T *)p->y, *d = (T *)p->d, *bc = (T *)p->bc;
+    const WT *W = (const WT *)p->W;
+    const T c0 = (T)p->c0, c1 = (T)p->c1, c2 = (T)p->c2;
+    const int mode = p->mode;
+    if (!W || !p->mask || !b) return UST_EINVAL;
+    if (g.nx % 2 || g.ny % 2 || (g.dim == 3 && g.nz % 2)) return UST_EINVAL;
+    if (g.dim == 3 && mode != UST_PASS_RESR && mode != UST_PASS_RES0R) return UST_EINVAL;
+    if (mode != UST_PASS_RESR && !invd) return UST_EINVAL;
+    if (mode != UST_PASS_PCHEBY2 && (!bc || !p->maskc)) return UST_EINVAL;
+    if ((mode == UST_PASS_RESR || mode == UST_PASS_PCHEBY2) && !u) return UST_EINVAL;
+    if (mode == UST_PASS_RES0R && (!d || d == b)) return UST_EINVAL;
+    if (mode == UST_PASS_CHEBY1R && (!y || y == b)) return UST_EINVAL;
+    if (mode == UST_PASS_PCHEBY2 && (!y || y == u || !p->xc)) return UST_EINVAL;
+    const dim3 grid(fused_groups(g, mode));
+#define PRE2(KIND) hipLaunchKernelGGL((k_pre2<T, WT, KIND>), grid, dim3(UST_TILE), 0, st, g, W, p->mask, p->maskc, u, b, \
+                                      invd, y, d, bc, c0, c1, c2)
+#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, W, p->mask, p->maskc, u, b, invd, \
+                                      d, bc, c2)
+    if (mode == UST_PASS_PCHEBY2)
+        hipLaunchKernelGGL((k_post2<T, WT>), grid, dim3(UST_TILE), 0, st, g, W, p->mask, u, (const T *)p->xc, b, invd, y,
+                           c0, c1, c2, p->dot);
+    else if (g.dim == 3 && mode == UST_PASS_RESR) PRE3(PRE_U);
+    else if (g.dim == 3) PRE3(PRE_FIRST);
+    else if (mode == UST_PASS_RESR) PRE2(PRE_U);
+    else if (mode == UST_PASS_RES0R) PRE2(PRE_FIRST);
+    else PRE2(PRE_TWO);
+#undef PRE2
+#undef PRE3
+    UST_LAUNCH_CHECK();
+    return UST_OK;
 }
 
 template <typename T, typename WT, int MODE>
@@ -1221,11 +1701,11 @@ static inline size_t work_len(const GridDev &g) {
 
 template <typename T, typename WT, int MODE>
 static int apply_halo(const GridDev &g, const WT *W, const unsigned char *mask, const T *u, const Epi<T> &ep,
-                      hipStream_t st) {
+                      hipStream_t st, const CgDir<T> &cg = {}) {
     if (g.dim == 3)
-        hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep);
+        hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep, cg);
     else
-        hipLaunchKernelGGL((k_applyK2_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep);
+        hipLaunchKernelGGL((k_applyK2_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep, cg);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
@@ -1311,6 +1791,7 @@ static int halo_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
     const T *u = (const T *)p->u, *b = (const T *)p->b, *invd = (const T *)p->invd, *xc = (const T *)p->xc;
     T *y = (T *)p->y, *d = (T *)p->d;
     const WT *W = (const WT *)p->W;
+    if (p->mode >= UST_PASS_RESR && p->mode <= UST_PASS_PCHEBY2) return fused_pass<T, WT>(g, p, st);
     Epi<T> ep = {y, b, invd, d, (T)p->c1, (T)p->c2, xc, u, (T)p->c0, p->d_last != 0, p->dot};
     if (!W || !p->mask || !y) return UST_EINVAL;
     const bool reads_u = p->mode != UST_PASS_RES0 && p->mode != UST_PASS_CHEBY1;
@@ -1339,6 +1820,36 @@ static int halo_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
 extern "C" int ust_k_apply_single(const ust_grid *gr) {
     const GridDev g = grid_dev(gr);
     return halo_grid(g) ? halo_tiles(g) : 0;
+}
+
+extern "C" int ust_k_apply_groups(const ust_grid *gr, int mode) {
+    const GridDev g = grid_dev(gr);
+    if (!halo_grid(g)) return 0;
+    return mode >= UST_PASS_RESR && mode <= UST_PASS_PCHEBY2 ? fused_groups(g, mode) : halo_tiles(g);
+}
+
+extern "C" int ust_k_cg_dir_apply(const ust_grid *gr, int type, const void *W, const unsigned char *mask, const void *z,
+                                  const void *p, void *next, void *q, double *c, double *part, int nrz, size_t n,
+                                  void *stream) {
+    if (!gr || !W || !mask || !z || !p || !next || !q || !c || !part || nrz < 1 || nrz > UST_CG_PARTS) return UST_EINVAL;
+    if (next == z || next == p || q == z || q == p || q == next) return UST_EINVAL;
+    const GridDev g = grid_dev(gr);
+    if (!halo_grid(g) || halo_tiles(g) > UST_CG_PARTS) return UST_EINVAL;
+    if (n != (size_t)g.nnx * g.nny * g.nnz * g.dim || n >= (1ull << 32)) return UST_EINVAL;
+    hipStream_t st = ust_stream(stream);
+    const int nrr = ust_k_cg_parts(n);
+    if (type == UST_PASS_F64) {
+        const CgDir<double> cg = {(const double *)p, (double *)next, c, part, nrz, nrr};
+        const Epi<double> ep = {(double *)q, nullptr, nullptr, nullptr, 0.0, 0.0, nullptr, nullptr, 0.0, false, part + CG_PQ};
+        return apply_halo<double, double, EPI_P>(g, (const double *)W, mask, (const double *)z, ep, st, cg);
+    }
+    if (type == UST_PASS_F32) {
+        const CgDir<float> cg = {(const float *)p, (float *)next, c, part, nrz, nrr};
+        const Epi<float> ep = {(float *)q, nullptr, nullptr, nullptr, 0.0f, 0.0f, nullptr, nullptr, 0.0f, false,
+                               part + CG_PQ};
+        return apply_halo<float, float, EPI_P>(g, (const float *)W, mask, (const float *)z, ep, st, cg);
+    }
+    return UST_EINVAL;
 }
 
 extern "C" int ust_k_apply_pass(const ust_grid *gr, const ust_pass *p, void *stream) {

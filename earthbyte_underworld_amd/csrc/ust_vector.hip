@@ -1,6 +1,7 @@
 // Krylov / smoother vector kernels (the PETSc Vec operations inside the BSSCR CG and the
 // multigrid smoothers).  Scalars that the device computes (dots, CG ratios) stay in device
 // memory, so a Krylov iteration issues no host round-trip except its convergence check.
+#include "ust_cg.h"
 #include "ust_common.h"
 
 #define GRID_STRIDE(i, n) \
@@ -278,26 +279,6 @@ __global__ __launch_bounds__(256) void kv4_cg_p_guarded_f32(const float *__restr
     for (size_t i = 4 * n4 + gid(); i < n; i += gstride()) p[i] = z[i] + beta * p[i];
 }
 
-// ------------------------------------------------------------------------------------------
-// The inner CG with its scalars on the device, three vector kernels per iteration and no reduction kernels between them:
-// every dot product leaves one partial sum per workgroup (at most UST_CG_PARTS), and the kernel that needs the scalar
-// sums them in each of its workgroups, in one fixed order, so all of them hold the same value.  A separate one-workgroup
-// reduction cost a launch of 4-5 us in a chain where most kernels take 3-6 us; reading 8 KB of partials from L2 in every
-// workgroup costs about 1 us, and starting a solve takes one kernel instead of six.  Whole solves with reduction kernels
-// and now: 2D 64x64 FP64 136.0 -> 129.6 ms, 3D 24x16x16 FP64 699 -> 661 ms, 64x64x32 with FP32 PCG 371 -> 351 ms.
-//
-// Control block c: c[0] = rtol^2, c[1] = state (0 running, 1 converged, 2 NaN), c[2] = iterations taken when the state
-// was last decided, c[3] = r.z of this iteration, c[4] = iterations done, c[5] = r.z of the previous one, c[6] = the
-// threshold on r.r.  The direction kernel decides the state of the iterations before it: its workgroup 0 writes c[1],
-// c[2], c[3] and c[6] while the others may still read them, which is safe since each workgroup decides from the same
-// sums, and c[1] only changes to the state that they all find (a workgroup reading the new state stops as it would have
-// done by itself).  c[4] and c[5] are written by the step kernel, which reads neither.  Once the state has left 0 both
-// kernels return, so iterations launched past convergence change nothing.
-// ------------------------------------------------------------------------------------------
-#define CG_RZ 0
-#define CG_PQ UST_CG_PARTS
-#define CG_RR (2 * UST_CG_PARTS)
-
 // four consecutive values, one or two 16-byte accesses
 template <typename T>
 struct alignas(16) V4 {
@@ -310,47 +291,6 @@ __device__ __forceinline__ void block_partial(double s, double *out) {
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) out[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-}
-
-// sums of na partials at a and nb at b, and the control block, the same in every thread of every workgroup
-struct CgSums {
-    double a, b, c[7];
-};
-__device__ __forceinline__ CgSums cg_sums(const double *a, int na, const double *b, int nb, const double *c) {
-    __shared__ double sh[8 + 7];
-    double sa = 0.0, sb = 0.0;
-    if (threadIdx.x < 7) sh[8 + threadIdx.x] = c[threadIdx.x];
-#pragma unroll
-    for (int r = 0; r < UST_CG_PARTS / 256; r++) {
-        const int i = threadIdx.x + 256 * r;
-        if (i < na) sa += a[i];
-        if (i < nb) sb += b[i];
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        sa += __shfl_xor(sa, off, 64);
-        sb += __shfl_xor(sb, off, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sh[threadIdx.x >> 6] = sa;
-        sh[4 + (threadIdx.x >> 6)] = sb;
-    }
-    __syncthreads();
-    CgSums o;
-    o.a = (sh[0] + sh[1]) + (sh[2] + sh[3]);
-    o.b = (sh[4] + sh[5]) + (sh[6] + sh[7]);
-    for (int k = 0; k < 7; k++) o.c[k] = sh[8 + k];
-    return o;
-}
-
-// the state that the sums decide, with the threshold: before the first iteration rr is b.b
-__device__ __forceinline__ double cg_state(const CgSums &s, double rr, double *thr) {
-    if (s.c[1] != 0.0) return s.c[1];
-    if (s.c[4] == 0.0) {
-        *thr = s.c[0] * rr;
-        return rr > 0.0 ? 0.0 : 1.0;
-    }
-    *thr = s.c[6];
-    return !(rr == rr) ? 2.0 : rr <= s.c[6] ? 1.0 : 0.0;
 }
 
 // x = 0, r = s b (in r's type), partials of r.r, the control block
@@ -422,10 +362,11 @@ __global__ __launch_bounds__(256) void kv_cg_dir(const TZ *__restrict__ z, TP *_
     for (size_t j = 4 * n4 + gid(); j < n; j += gstride()) p[j] = first ? (TP)z[j] : (TP)z[j] + beta * p[j];
 }
 
-// step: a = r.z / p.q, x += a p, r -= a q, partials of r.r
+// step: a = r.z / p.q, x += a p, r -= a q, partials of r.r; keep: p for the next direction, where p is not its place
 template <typename T>
 __global__ __launch_bounds__(256) void kv_cg_step(T *__restrict__ x, T *__restrict__ r, const T *__restrict__ p,
-                                                  const T *__restrict__ q, double *c, double *part, int npq, size_t n) {
+                                                  const T *__restrict__ q, T *__restrict__ keep, double *c, double *part,
+                                                  int npq, size_t n) {
     const size_t n4 = n / 4;
     size_t i = gid();
     V4<T> xv = {}, rv = {}, pv = {}, qv = {};
@@ -452,6 +393,7 @@ __global__ __launch_bounds__(256) void kv_cg_step(T *__restrict__ x, T *__restri
         }
         ((V4<T> *)x)[i] = xv;
         ((V4<T> *)r)[i] = rv;
+        if (keep) ((V4<T> *)keep)[i] = pv;
         i += gstride();
         if (i < n4) {
             xv = ((const V4<T> *)x)[i];
@@ -464,6 +406,7 @@ __global__ __launch_bounds__(256) void kv_cg_step(T *__restrict__ x, T *__restri
         x[j] += a * p[j];
         const T ri = r[j] - a * q[j];
         r[j] = ri;
+        if (keep) keep[j] = p[j];
         acc += (double)ri * (double)ri;
     }
     block_partial(acc, part + CG_RR);
@@ -555,9 +498,10 @@ static int cg_dir(const TZ *z, TP *p, double *c, double *part, int nrz, size_t n
     return UST_OK;
 }
 template <typename T>
-static int cg_step(T *x, T *r, const T *p, const T *q, double *c, double *part, int npq, size_t n, void *stream) {
-    if (!cg_vectors(n, x, r, p, q) || npq < 1 || npq > UST_CG_PARTS) return UST_EINVAL;
-    hipLaunchKernelGGL(kv_cg_step<T>, dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), x, r, p, q, c, part, npq, n);
+static int cg_step(T *x, T *r, const T *p, const T *q, T *keep, double *c, double *part, int npq, size_t n,
+                   void *stream) {
+    if (!cg_vectors(n, x, r, p, q) || !al16(keep) || npq < 1 || npq > UST_CG_PARTS) return UST_EINVAL;
+    hipLaunchKernelGGL(kv_cg_step<T>, dim3(rgrid(n)), dim3(256), 0, ust_stream(stream), x, r, p, q, keep, c, part, npq, n);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
@@ -694,13 +638,13 @@ int ust_k_cg_dir_zf(const float *z, double *p, double *c, double *part, int nrz,
 int ust_k_cg_dir_f32(const float *z, float *p, double *c, double *part, int nrz, size_t n, void *stream) {
     return cg_dir(z, p, c, part, nrz, n, stream);
 }
-int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, double *c, double *part, int npq, size_t n,
-                      void *stream) {
-    return cg_step(x, r, p, q, c, part, npq, n, stream);
+int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, double *keep, double *c, double *part, int npq,
+                      size_t n, void *stream) {
+    return cg_step(x, r, p, q, keep, c, part, npq, n, stream);
 }
-int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, double *c, double *part, int npq, size_t n,
-                      void *stream) {
-    return cg_step(x, r, p, q, c, part, npq, n, stream);
+int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, float *keep, double *c, double *part, int npq,
+                      size_t n, void *stream) {
+    return cg_step(x, r, p, q, keep, c, part, npq, n, stream);
 }
 int ust_k_cg_state(double *c, const double *part, size_t n, double *host, void *stream) {
     hipLaunchKernelGGL(kv_cg_state, dim3(1), dim3(256), 0, ust_stream(stream), c, part, (int)rgrid(n), host);

@@ -160,13 +160,14 @@ static int restrict_residual(ust_context *ctx, int l, int f32, const void *r) {
 
 static int vcycle(ust_context *ctx, int l, int f32, const void *b, void *x, int first_done, double *dot, void **res);
 
-/* The V-cycle of a level whose passes are one launch each (2D grids, small 3D ones): every smoothing step and residual
- * runs out of place between x and the level's residual vector, which is free outside the residual's own use.  The first
- * two smoothing steps from zero are one pass, one step and the residual another, and the prolongation of the correction
- * rides on the first post-smoothing step.  dot: partial sums of b . x from the last pass (NULL: none). */
+/* The V-cycle of a level whose passes are one launch each (2D grids, small 3D ones): the smoothing steps run out of place
+ * between x and the level's residual vector.  The last pass before the coarse level leaves its right-hand side: the residual
+ * never reaches memory.  The first two smoothing steps from zero are one pass (in 2D with the residual and restriction), one
+ * step goes with the residual, and the prolongation of the correction rides on the first post-smoothing step (in 2D two
+ * steps are one pass).  dot: partial sums of b . x from the last pass (NULL: none). */
 static int vcycle_single(ust_context *ctx, int l, int f32, const void *b, void *x, double *dot, void **res) {
     ust_level *L = &ctx->lev[l], *C = &ctx->lev[l + 1];
-    const int deg = L->cheb_deg, coarsest = l == ctx->nlev - 1;
+    const int deg = L->cheb_deg, coarsest = l == ctx->nlev - 1, two = deg == 2 && L->g.dim == 2 && !coarsest;
     void *cur = x, *alt = f32 ? (void *)L->ax32 : (void *)L->ax64, *d = f32 ? (void *)L->d32 : (void *)L->d64, *t;
     ust_pass p;
     int rc;
@@ -177,13 +178,11 @@ static int vcycle_single(ust_context *ctx, int l, int f32, const void *b, void *
     p.b = b;
     p.invd = f32 ? (const void *)L->invd32 : (const void *)L->invd64;
     if (coarsest && deg == 1) return lev_smooth(ctx, l, f32, b, *res = x, 1, NULL);
-    if (deg == 1) { /* alt = residual of x = the first step */
-        p.mode = UST_PASS_RES0;
-        p.c2 = L->c2[0];
-        p.y = alt;
-        p.d = x;
-        CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
-    } else {
+    if (!coarsest) {
+        p.bc = f32 ? (void *)C->b32 : (void *)C->b64;
+        p.maskc = C->mask;
+    }
+    if (deg > 1 && !two)
         for (int k = 1; k < deg; k++) {
             p.mode = k == 1 ? UST_PASS_CHEBY1 : UST_PASS_CHEBY;
             p.c0 = L->c2[0];
@@ -196,20 +195,21 @@ static int vcycle_single(ust_context *ctx, int l, int f32, const void *b, void *
             CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
             if (k > 1) t = cur, cur = alt, alt = t;
         }
-        *res = cur;
-        if (coarsest) return UST_OK;
-        p.mode = UST_PASS_RES;
-        p.u = cur;
-        p.y = alt;
-        CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
-    }
+    *res = cur;
+    if (coarsest) return UST_OK;
+    p.mode = deg == 1 ? UST_PASS_RES0R : two ? UST_PASS_CHEBY1R : UST_PASS_RESR;
+    p.c0 = L->c2[0];
+    p.c1 = deg > 1 ? L->c1[1] : 0.0;
+    p.c2 = deg == 1 ? L->c2[0] : L->c2[1];
+    p.u = cur;
+    p.y = cur;
+    p.d = deg == 1 ? cur : NULL;
+    CKD(ctx, ust_k_apply_pass(&L->g, &p, S(ctx)));
     void *xc = NULL;
-    if ((rc = restrict_residual(ctx, l, f32, alt))) return rc;
-    if ((rc = vcycle(ctx, l + 1, f32, f32 ? (void *)C->b32 : (void *)C->b64, f32 ? (void *)C->x32 : (void *)C->x64, 0,
-                     NULL, &xc)))
-        return rc;
-    for (int k = 0; k < deg; k++) {
-        p.mode = k == 0 ? UST_PASS_PCHEBY0 : UST_PASS_CHEBY;
+    if ((rc = vcycle(ctx, l + 1, f32, p.bc, f32 ? (void *)C->x32 : (void *)C->x64, 0, NULL, &xc))) return rc;
+    for (int k = two ? 1 : 0; k < deg; k++) {
+        p.mode = two ? UST_PASS_PCHEBY2 : k == 0 ? UST_PASS_PCHEBY0 : UST_PASS_CHEBY;
+        p.c0 = L->c2[0];
         p.c1 = L->c1[k];
         p.c2 = L->c2[k];
         p.d_last = k == deg - 1;
@@ -275,52 +275,69 @@ static int vcycle(ust_context *ctx, int l, int f32, const void *b, void *x, int 
     return lev_smooth(ctx, l, 0, b, x, 0, NULL);
 }
 
-/* whether level 0's last V-cycle pass and its product leave the partial sums of r.z and p.q themselves */
-static int cg_parts_of_passes(const ust_context *ctx) {
-    return ctx->lev[0].single > 0 && ctx->lev[0].single <= UST_CG_PARTS;
-}
-
 /* z = M^-1 r on the finest level and the partial sums of r . z; *np: their number */
 static int precondition(ust_context *ctx, int f32, const void *r, void *z, void **res, int *np) {
+    ust_level *L0 = &ctx->lev[0];
     size_t n = (size_t)ctx->ndof;
-    double *dot = ctx->nlev > 1 && cg_parts_of_passes(ctx) ? ctx->cgpart : NULL;
+    /* a one-launch level's last pass leaves them itself */
+    const int groups = ust_k_apply_groups(&L0->g, L0->g.dim == 2 && L0->cheb_deg == 2 ? UST_PASS_PCHEBY2 : UST_PASS_CHEBY);
+    double *dot = ctx->nlev > 1 && groups > 0 && groups <= UST_CG_PARTS ? ctx->cgpart : NULL;
     int rc = vcycle(ctx, 0, f32, r, z, 0, dot, res);
     if (rc) return rc;
-    *np = dot ? ctx->lev[0].single : ust_k_cg_parts(n);
+    *np = dot ? groups : ust_k_cg_parts(n);
     if (dot) return UST_OK;
     if (f32) CKD(ctx, ust_k_cg_dot_rz_f32((const float *)r, (const float *)*res, n, ctx->cgpart, S(ctx)));
     else CKD(ctx, ust_k_cg_dot_rz_f64((const double *)r, (const double *)*res, n, ctx->cgpart, S(ctx)));
     return UST_OK;
 }
 
-/* q = K p on the finest level (FP32: its FP32 weights) and the partial sums of p . q; *np: their number */
-static int product_dot(ust_context *ctx, int f32, const void *p, void *q, int *np) {
+/* The CG's direction from z, q = K times it on the finest level (FP32: its FP32 weights), and the x, r update.  p holds the
+ * direction from iteration to iteration; on a one-launch level the new one is formed by the product's pass, out of place,
+ * and the update puts it back. */
+static int cg_advance(ust_context *ctx, int f32, const void *z, int z32, int nrz, void *x, void *r, void *p, void *q) {
     ust_level *L0 = &ctx->lev[0];
     size_t n = (size_t)ctx->ndof;
-    double *part = ctx->cgpart;
-    if (cg_parts_of_passes(ctx)) {
-        ust_pass a;
-        memset(&a, 0, sizeof a);
-        a.mode = UST_PASS_Y;
-        a.type = f32 ? UST_PASS_F32 : UST_PASS_F64;
-        a.W = f32 ? (const void *)L0->WK32 : (const void *)L0->WK64;
-        a.mask = L0->mask;
-        a.u = p;
-        a.y = q;
-        a.dot = part + UST_CG_PARTS;
-        CKD(ctx, ust_k_apply_pass(&L0->g, &a, S(ctx)));
-        *np = L0->single;
-        return UST_OK;
-    }
-    *np = ust_k_cg_parts(n);
-    if (f32) {
-        CKD(ctx, ust_k_apply_K_f32(&L0->g, L0->WK32, L0->mask, (const float *)p, (float *)q, (float *)ctx->kwork, S(ctx)));
-        CKD(ctx, ust_k_cg_dot_pq_f32((const float *)p, (const float *)q, n, part, S(ctx)));
+    double *c = ctx->scal + SC_CG, *part = ctx->cgpart;
+    const int single = L0->single > 0 && L0->single <= UST_CG_PARTS;
+    const void *W = f32 ? (const void *)L0->WK32 : (const void *)L0->WK64;
+    void *pn = p, *keep = NULL;
+    int npq = single ? L0->single : ust_k_cg_parts(n);
+    if (single && f32 == z32) {
+        pn = f32 ? (void *)L0->x32 : (void *)L0->x64;
+        keep = p;
+        CKD(ctx, ust_k_cg_dir_apply(&L0->g, f32 ? UST_PASS_F32 : UST_PASS_F64, W, L0->mask, z, p, pn, q, c, part, nrz, n,
+                                    S(ctx)));
     } else {
-        CKD(ctx, ust_k_apply_K_f64(&L0->g, L0->WK64, L0->mask, (const double *)p, (double *)q, (double *)ctx->kwork,
-                                   S(ctx)));
-        CKD(ctx, ust_k_cg_dot_pq_f64((const double *)p, (const double *)q, n, part, S(ctx)));
+        if (f32) CKD(ctx, ust_k_cg_dir_f32((const float *)z, (float *)p, c, part, nrz, n, S(ctx)));
+        else if (z32) CKD(ctx, ust_k_cg_dir_zf((const float *)z, (double *)p, c, part, nrz, n, S(ctx)));
+        else CKD(ctx, ust_k_cg_dir_f64((const double *)z, (double *)p, c, part, nrz, n, S(ctx)));
+        if (single) {
+            ust_pass a;
+            memset(&a, 0, sizeof a);
+            a.mode = UST_PASS_Y;
+            a.type = f32 ? UST_PASS_F32 : UST_PASS_F64;
+            a.W = W;
+            a.mask = L0->mask;
+            a.u = p;
+            a.y = q;
+            a.dot = part + UST_CG_PARTS;
+            CKD(ctx, ust_k_apply_pass(&L0->g, &a, S(ctx)));
+        } else if (f32) {
+            CKD(ctx, ust_k_apply_K_f32(&L0->g, L0->WK32, L0->mask, (const float *)p, (float *)q, (float *)ctx->kwork,
+                                       S(ctx)));
+            CKD(ctx, ust_k_cg_dot_pq_f32((const float *)p, (const float *)q, n, part, S(ctx)));
+        } else {
+            CKD(ctx, ust_k_apply_K_f64(&L0->g, L0->WK64, L0->mask, (const double *)p, (double *)q, (double *)ctx->kwork,
+                                       S(ctx)));
+            CKD(ctx, ust_k_cg_dot_pq_f64((const double *)p, (const double *)q, n, part, S(ctx)));
+        }
     }
+    if (f32)
+        CKD(ctx, ust_k_cg_step_f32((float *)x, (float *)r, (const float *)pn, (const float *)q, (float *)keep, c, part, npq,
+                                   n, S(ctx)));
+    else
+        CKD(ctx, ust_k_cg_step_f64((double *)x, (double *)r, (const double *)pn, (const double *)q, (double *)keep, c, part,
+                                   npq, n, S(ctx)));
     return UST_OK;
 }
 
@@ -556,9 +573,9 @@ static int dotv(ust_context *ctx, const double *a, const double *b, size_t n, in
  * once into a HIP graph. */
 static int pcg_iteration(ust_context *ctx, int pc32) {
     size_t n = (size_t)ctx->ndof;
-    double *r = ctx->vr, *p = ctx->vp, *q = ctx->vq, *c = ctx->scal + SC_CG, *part = ctx->cgpart;
+    double *r = ctx->vr;
     void *z = NULL;
-    int rc, nrz, npq;
+    int rc, nrz;
     if (pc32) {
         /* z stays FP32: r . z and p = z + beta p widen it per element.  A level of several launches per pass rounds r
          * into b32 in its first smoothing step */
@@ -569,15 +586,11 @@ static int pcg_iteration(ust_context *ctx, int pc32) {
         ctx->b64_src = NULL;
         if (rc) return rc;
         nrz = ust_k_cg_parts(n);
-        CKD(ctx, ust_k_cg_dot_rz_zf(r, (const float *)z, n, part, S(ctx)));
-        CKD(ctx, ust_k_cg_dir_zf((const float *)z, p, c, part, nrz, n, S(ctx)));
-    } else {
-        if ((rc = precondition(ctx, 0, r, ctx->vz, &z, &nrz))) return rc;
-        CKD(ctx, ust_k_cg_dir_f64((const double *)z, p, c, part, nrz, n, S(ctx)));
+        CKD(ctx, ust_k_cg_dot_rz_zf(r, (const float *)z, n, ctx->cgpart, S(ctx)));
+    } else if ((rc = precondition(ctx, 0, r, ctx->vz, &z, &nrz))) {
+        return rc;
     }
-    if ((rc = product_dot(ctx, 0, p, q, &npq))) return rc;
-    CKD(ctx, ust_k_cg_step_f64(ctx->vx, r, p, q, c, part, npq, n, S(ctx)));
-    return UST_OK;
+    return cg_advance(ctx, 0, z, pc32, nrz, ctx->vx, r, ctx->vp, ctx->vq);
 }
 
 static int pcg_graph(ust_context *ctx, int pc32) {
@@ -633,15 +646,10 @@ static int pcg(ust_context *ctx, int pc32, const double *b, double *x, double rt
  * wr, p = z + beta p, q = K p with the FP32 weights of the finest level, and the x (wx), r update; dots and r . r
  * accumulate in FP64 and the stopping test runs on the device, as in the FP64 PCG. */
 static int pcg32_iteration(ust_context *ctx) {
-    size_t n = (size_t)ctx->ndof;
-    double *c = ctx->scal + SC_CG, *part = ctx->cgpart;
     void *z = NULL;
-    int rc, nrz, npq;
+    int rc, nrz;
     if ((rc = precondition(ctx, 1, ctx->wr, ctx->wz, &z, &nrz))) return rc;
-    CKD(ctx, ust_k_cg_dir_f32((const float *)z, ctx->wp, c, part, nrz, n, S(ctx)));
-    if ((rc = product_dot(ctx, 1, ctx->wp, ctx->wq, &npq))) return rc;
-    CKD(ctx, ust_k_cg_step_f32(ctx->wx, ctx->wr, ctx->wp, ctx->wq, c, part, npq, n, S(ctx)));
-    return UST_OK;
+    return cg_advance(ctx, 1, z, 1, nrz, ctx->wx, ctx->wr, ctx->wp, ctx->wq);
 }
 
 /* FP32 PCG on K e = s r (at unit norm) to a residual <= rtol from e = 0; iterations as in pcg(), the launches

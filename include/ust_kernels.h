@@ -289,6 +289,10 @@ int ust_k_dvc_weights_of(int dim, const int *res, int n, const int *elems, const
 #define UST_PASS_PCHEBY0 4 /* v = u + P xc (xc on the grid of half the elements), then CHEBY0 from v */
 #define UST_PASS_RES0 5    /* d = c2 invd b, y = b - K d, 0 on the Dirichlet dofs */
 #define UST_PASS_CHEBY1 6  /* v = c0 invd b, d = c1 v + c2 invd (b - K v), y = v + d */
+#define UST_PASS_RESR 7    /* the residual of RES restricted to the grid of half the elements: bc */
+#define UST_PASS_RES0R 8   /* the same of RES0 */
+#define UST_PASS_CHEBY1R 9 /* 2D: CHEBY1, then the residual of y restricted */
+#define UST_PASS_PCHEBY2 10 /* 2D: v = u + P xc, d = c0 invd (b - K v), w = v + d, y = w + c1 d + c2 invd (b - K w) */
 #define UST_PASS_F64 0
 #define UST_PASS_F32 1
 #define UST_PASS_F32_BF16W 2 /* FP32 with bfloat16 weights */
@@ -296,18 +300,26 @@ typedef struct {
     int mode, type;            /* UST_PASS_* */
     const void *W;             /* weights of the type */
     const unsigned char *mask;
-    const void *u;             /* input of modes 0-4 (distinct from y) */
-    void *y;
-    const void *b, *invd;      /* modes 1-6; modes 2-6 */
-    void *d;                   /* modes 2, 5; written in modes 3, 4, 6 when given */
-    const void *xc;            /* mode 4 */
+    const void *u;             /* input of modes 0-4, 7, 10 (distinct from y) */
+    void *y;                   /* not modes 7, 8 */
+    const void *b, *invd;      /* modes 1-10; modes 2-6, 8-10 */
+    void *d;                   /* modes 2, 5, 8; written in modes 3, 4, 6, 9 when given */
+    const void *xc;            /* modes 4, 10 */
+    void *bc;                  /* modes 7-9: the coarse right-hand side */
+    const unsigned char *maskc; /* modes 7-9: Dirichlet dofs of the coarse grid */
     double c0, c1, c2;
     int d_last;                /* mode 2: do not write d */
-    double *dot;               /* when given, one partial sum per workgroup: of u . y (mode 0), of b . y (modes 2-4, 6) */
+    double *dot;               /* when given, one partial sum per workgroup: of u . y (mode 0), of b . y (modes 2-4, 6, 10) */
 } ust_pass;
-/* workgroups (partial sums) of a pass on this grid, 0 when the grid is not one of ust_k_apply_pass's */
+/* workgroups (partial sums) of a pass of mode 0-6 on this grid, 0 when the grid is not one of ust_k_apply_pass's; of a
+ * pass of the mode */
 int ust_k_apply_single(const ust_grid *g);
+int ust_k_apply_groups(const ust_grid *g, int mode);
 int ust_k_apply_pass(const ust_grid *g, const ust_pass *p, void *stream);
+/* the direction of the device-controlled CG below (ust_k_cg_dir) and its product in one launch: next = z + beta p,
+ * q = K next, and ust_k_apply_single(g) partials of p.q; of the type's vectors, all distinct */
+int ust_k_cg_dir_apply(const ust_grid *g, int type, const void *W, const unsigned char *mask, const void *z, const void *p,
+                       void *next, void *q, double *c, double *part, int nrz, size_t n, void *stream);
 
 
 /* --- operators.  mask: per dof (n_nodes*dim), 1 = Dirichlet.  y is overwritten. --- */
@@ -483,7 +495,7 @@ int ust_k_cg_update_xr_f32(float *x, float *r, const float *p, const float *q, c
  *   begin:  x = 0, r = s b (s = 1 in FP64), c for a solve to ||r||^2 <= rtol2 ||b||^2
  *   dot_rz, dot_pq: ust_k_cg_parts(n) partials; another kernel may leave its own count (at most UST_CG_PARTS) instead
  *   dir:    the state after the iterations before this one, then p = z + beta p (p = z in the first)
- *   step:   x += a p, r -= a q
+ *   step:   x += a p, r -= a q, and keep = p unless NULL
  *   state:  the state now, to host[0] (0 running, 1 converged, 2 NaN) and the iterations to host[1] (pinned memory)
  * dir and step do nothing once the state is not 0: iterations launched past convergence leave x and r unchanged.
  * zf: z in FP32, the other vectors in FP64. */
@@ -501,10 +513,10 @@ int ust_k_cg_dot_pq_f32(const float *p, const float *q, size_t n, double *part, 
 int ust_k_cg_dir_f64(const double *z, double *p, double *c, double *part, int nrz, size_t n, void *stream);
 int ust_k_cg_dir_zf(const float *z, double *p, double *c, double *part, int nrz, size_t n, void *stream);
 int ust_k_cg_dir_f32(const float *z, float *p, double *c, double *part, int nrz, size_t n, void *stream);
-int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, double *c, double *part, int npq, size_t n,
-                      void *stream);
-int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, double *c, double *part, int npq, size_t n,
-                      void *stream);
+int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, double *keep, double *c, double *part, int npq,
+                      size_t n, void *stream);
+int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, float *keep, double *c, double *part, int npq,
+                      size_t n, void *stream);
 int ust_k_cg_state(double *c, const double *part, size_t n, double *host, void *stream);
 /* p = z + beta p and x += a p, r -= a q with r.r on FP32 vectors against a control block of threshold, state, count and
  * beta; nothing is done once the state is not 0 */

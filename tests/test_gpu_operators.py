@@ -664,7 +664,7 @@ def test_device_controlled_cg(kind, n):
         assert getattr(lib, f"ust_k_cg_dir_{kind}")(z.p, p.p, c.p, part.p, parts, n, None) == 0
         put(q, product(p.get()))
         assert getattr(lib, f"ust_k_cg_dot_pq_{tp}")(p.p, q.p, n, part.p, None) == 0
-        assert getattr(lib, f"ust_k_cg_step_{tp}")(x.p, r.p, p.p, q.p, c.p, part.p, parts, n, None) == 0
+        assert getattr(lib, f"ust_k_cg_step_{tp}")(x.p, r.p, p.p, q.p, None, c.p, part.p, parts, n, None) == 0
         assert lib.ust_k_cg_state(c.p, part.p, n, host.p, None) == 0
         return tuple(host.get())
 
@@ -815,6 +815,134 @@ def test_single_launch_passes(oracle, dim, nel, prec):
     # in place is refused
     p = L.Pass(mode=0, type=code, W=W, mask=mask, u=dev["u"].p, y=dev["u"].p)
     assert lib.ust_k_apply_pass(C.byref(g), C.byref(p), None) == -1
+    for a in hold:
+        a.free()
+    s.close()
+
+
+# blocks of 6x6 (3D: 3x2x2) coarse nodes and of 13x13 nodes: fewer than one, whole ones, one more node, several ragged
+@pytest.mark.parametrize("dim,nel", [(2, (4, 6)), (2, (22, 12)), (2, (24, 26)), (2, (50, 38)), (3, (4, 2, 2)),
+                                     (3, (10, 6, 6)), (3, (12, 8, 10))])
+@pytest.mark.parametrize("prec", ["f64", "f32", "bf16w"])
+def test_fused_level_passes(dim, nel, prec):
+    """The passes that go with the restriction, and 2D's two post-smoothing steps, against the passes they replace
+    (themselves checked against the assembled K), and the CG direction formed by the product's pass against the
+    direction kernel followed by the product.  Bar: the same sums in the same order, so FP64 to 1e-13 and FP32 to 1e-5 of
+    the largest entry times the condition of one more product (100)."""
+    import ctypes as C
+    from earthbyte_underworld_amd import _lib as L
+    s = _build(dim, nel, 6, 4)
+    lib = s.lib
+    g = L.Grid()
+    WK, WG, WF, mask = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert lib.ust_get_device_views(s.ctx, C.byref(g), C.byref(WK), C.byref(WG), C.byref(WF), C.byref(mask)) == 0
+    nw, n = lib.ust_k_weights_len(C.byref(g)), s.ndof
+    T = np.float64 if prec == "f64" else np.float32
+    code = {"f64": 0, "f32": 1, "bf16w": 2}[prec]
+    hold = []
+
+    def dev(a):
+        hold.append(_Dev(lib, a))
+        return hold[-1]
+
+    W = WK
+    if prec != "f64":
+        d = dev(np.zeros(nw, np.float32 if prec == "f32" else np.uint16))
+        copy = lib.ust_k_copy_f64_to_f32 if prec == "f32" else lib.ust_k_copy_f64_to_bf16
+        assert copy(WK, d.p, nw, None) == 0
+        W = d.p
+    nn = tuple(e + 1 for e in nel)
+    cn = tuple(e // 2 + 1 for e in nel)
+    fine = np.asarray(s.bc_mask).reshape(tuple(reversed(nn)) + (dim,))
+    maskc = np.ascontiguousarray(fine[(slice(None, None, 2),) * dim]).astype(np.uint8).reshape(-1)
+    nc = len(maskc)
+    assert nc == int(np.prod(cn)) * dim
+    mc = dev(maskc)
+    rng = np.random.default_rng(23)
+    u, b, z, pold = (dev(rng.normal(size=n).astype(T)) for _ in range(4))
+    xc = dev(rng.normal(size=nc).astype(T))
+    # a smoother's scaling: 1 / the largest row sum keeps K D^-1 at about 1
+    ones = dev(np.ones(n, T))
+    y = dev(np.zeros(n, T))
+
+    def run(mode, **kw):
+        p = L.Pass(mode=mode, type=code, W=W, mask=mask, b=b.p, c0=0.7, c1=0.37, c2=1.9)
+        for k, v in kw.items():
+            setattr(p, k, v.p if isinstance(v, _Dev) else v)
+        return lib.ust_k_apply_pass(C.byref(g), C.byref(p), None)
+
+    assert run(0, u=u, y=y) == 0
+    invd = dev(np.full(n, 0.1 / np.abs(y.get()).max(), T) * rng.uniform(0.5, 1.0, n).astype(T))
+    tol = 1e-11 if prec == "f64" else 1e-3
+
+    def close(a, r):
+        a, r = a.astype(np.float64), r.astype(np.float64)
+        assert np.abs(a - r).max() <= tol * np.abs(r).max(), np.abs(a - r).max() / np.abs(r).max()
+
+    new = lambda m: dev(np.full(m, np.nan, T))
+    x, r, rc, x2, rc2, d, d2 = new(n), new(n), new(nc), new(n), new(nc), new(n), new(n)
+    restrict = lib.ust_k_restrict_f64 if prec == "f64" else lib.ust_k_restrict_f32
+
+    def restricted():
+        assert restrict(C.byref(g), None, mc.p, r.p, rc.p, None) == 0
+        return rc.get()
+
+    # residual of u
+    assert run(1, u=u, y=r) == 0 and run(7, u=u, bc=rc2, maskc=mc) == 0
+    close(rc2.get(), restricted())
+    # of the first step
+    assert run(5, y=r, d=x, invd=invd) == 0 and run(8, d=x2, invd=invd, bc=rc2, maskc=mc) == 0
+    close(rc2.get(), restricted())
+    assert np.array_equal(x2.get(), x.get())
+    if dim == 2:
+        # of the first two steps
+        assert run(6, y=x, d=d, invd=invd) == 0 and run(1, u=x, y=r) == 0
+        assert run(9, y=x2, d=d2, invd=invd, bc=rc2, maskc=mc) == 0
+        close(rc2.get(), restricted())
+        close(x2.get(), x.get())
+        close(d2.get(), d.get())
+        # the two steps after the correction
+        groups = lib.ust_k_apply_groups(C.byref(g), 10)
+        assert groups == np.prod([-(-k // 13) for k in nn])
+        dot = dev(np.full(groups, np.nan))
+        assert run(4, u=u, y=x, d=d, xc=xc, invd=invd, c2=0.7) == 0 and run(2, u=x, y=x2, d=d, invd=invd) == 0
+        assert run(10, u=u, y=r, xc=xc, invd=invd, dot=dot) == 0
+        close(r.get(), x2.get())
+        by = b.get().astype(np.float64) * r.get()
+        assert abs(dot.get().sum() - by.sum()) <= 1e-12 * np.abs(by).sum()
+    else:
+        assert run(9, y=x2, invd=invd, bc=rc2, maskc=mc) == -1 and run(10, u=u, y=r, xc=xc, invd=invd) == -1
+    if prec != "bf16w":
+        # the CG direction, in a first and in a later iteration, and past convergence
+        groups, parts = lib.ust_k_apply_single(C.byref(g)), lib.ust_k_cg_parts(n)
+        part = np.zeros(3072)
+        part[:parts], part[2048:2048 + parts] = 0.5, 0.25
+        for c, state in (([1e-16, 0, 0, 0, 0, 1, 0], 0.0), ([1e-16, 0, 3, 0.4, 4, 0.3, 1e-20], 0.0),
+                         ([1e-16, 0, 3, 0.4, 4, 0.3, 1e20], 1.0)):
+            got = []
+            for fused in (0, 1):
+                dc, dp, p, nxt, q = dev(np.array(c, np.float64)), dev(part), dev(pold.get()), dev(np.zeros(n, T)), dev(
+                    np.zeros(n, T))
+                if fused:
+                    assert lib.ust_k_cg_dir_apply(C.byref(g), code, W, mask, z.p, p.p, nxt.p, q.p, dc.p, dp.p, parts, n,
+                                                  None) == 0
+                    assert np.array_equal(p.get(), pold.get())
+                    pq = dp.get()[1024:1024 + groups].sum()
+                    got.append((nxt.get(), q.get(), dc.get()))
+                else:
+                    f = lib.ust_k_cg_dir_f64 if prec == "f64" else lib.ust_k_cg_dir_f32
+                    assert f(z.p, p.p, dc.p, dp.p, parts, n, None) == 0
+                    assert run(0, u=p, y=q) == 0
+                    got.append((p.get(), q.get(), dc.get()))
+            assert np.array_equal(got[0][2], got[1][2]) and got[1][2][1] == state
+            if state == 0.0:
+                close(got[1][0], got[0][0])
+                close(got[1][1], got[0][1])
+                ref = got[1][0].astype(np.float64) * got[1][1]
+                assert abs(pq - ref.sum()) <= 1e-12 * np.abs(ref).sum()
+            else:  # nothing is written
+                assert not got[1][0].any() and not got[1][1].any()
+        assert lib.ust_k_cg_dir_apply(C.byref(g), code, W, mask, z.p, p.p, p.p, q.p, dc.p, dp.p, parts, n, None) == -1
     for a in hold:
         a.free()
     s.close()
