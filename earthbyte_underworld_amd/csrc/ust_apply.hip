@@ -392,7 +392,7 @@ constexpr long long col_wg_target(int tsize, int mode) {
                                                                               : UST_COL_WG_TARGET;
 }
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(GridDev g, const WT *__restrict__ W,
+__global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(GridDev g, TileDiv td, const WT *__restrict__ W,
                                                      const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
                                                      T *__restrict__ work) {
     __shared__ T su[2][CNPD];     // staged node planes k and k+1 (free dofs; Dirichlet dofs read 0)
@@ -402,11 +402,10 @@ __global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(
     constexpr int CCX = UST_TX3 / 2 + 1, CCY = UST_TY3 / 2 + 1, NCP = CCX * CCY * 3;
     static_assert(NCP <= UST_TILE, "one coarse value per thread");
     __shared__ T sc[MODE == EPI_PCHEBY0 ? 2 * NCP : 1];
-    const int ntxy = g.tnx * g.tny;
     const int tile = xcd_block(blockIdx.x, gridDim.x);
-    const int txy = tile % ntxy, chunk = tile / ntxy;
-    const int x0 = (txy % g.tnx) * UST_TX3, y0 = (txy / g.tnx) * UST_TY3;
-    const int z0 = chunk * g.tz, z1 = min(z0 + g.tz, g.nz);
+    const int3 at = tile_at(tile, td);
+    const int txy = at.x + g.tnx * at.y, x0 = at.x * UST_TX3, y0 = at.y * UST_TY3;
+    const int z0 = at.z * g.tz, z1 = min(z0 + g.tz, g.nz);
     const int tid = threadIdx.x, lx = tid % UST_TX3, ly = tid / UST_TX3;
     const bool active = x0 + lx < g.nx && y0 + ly < g.ny;
     const int es = lx + 1 + EBX * (ly + 1);  // the thread's slot in the element-result buffer
@@ -638,7 +637,7 @@ __global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(
 // through the workspace.
 // ------------------------------------------------------------------------------------------
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, const WT *__restrict__ W,
+__global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, TileDiv td, const WT *__restrict__ W,
                                                        const unsigned char *__restrict__ mask, const T *u,
                                                        Epi<T> ep, T *__restrict__ work) {
     constexpr int TX = UST_TTX3, TY = UST_TTY3, TZ = UST_TTZ3;
@@ -650,7 +649,8 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, const WT *_
     static_assert(NC <= UST_TILE, "one coarse value per thread");
     __shared__ T sc[MODE == EPI_PCHEBY0 ? NC : 1];
     const int tile = xcd_block(blockIdx.x, gridDim.x);
-    const int tx0 = (tile % g.tnx) * TX, ty0 = ((tile / g.tnx) % g.tny) * TY, tz0 = (tile / (g.tnx * g.tny)) * TZ;
+    const int3 at = tile_at(tile, td);
+    const int tx0 = at.x * TX, ty0 = at.y * TY, tz0 = at.z * TZ;
     T cv = (T)0;
     if (MODE == EPI_PCHEBY0) {
         const int t = threadIdx.x, c = t % 3, n = t / 3;
@@ -843,14 +843,14 @@ __device__ __forceinline__ void block_dot(double v, double *out) {
 }
 
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__restrict__ W,
+__global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, const WT *__restrict__ W,
                                                       const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
                                                       CgDir<T> cg) {
     __shared__ T su[HNN * 3];   // staged node block, origin (nx0 - 1, ny0 - 1, nz0 - 1)
     __shared__ T eb[24 * HNE];  // element results: eb[(a*3 + i) * HNE + slot] (HNE odd: rows shift banks)
-    const int hnx = (g.nnx + HOX - 1) / HOX, hny = (g.nny + HOY - 1) / HOY;
     const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
-    const int nx0 = (tile % hnx) * HOX, ny0 = ((tile / hnx) % hny) * HOY, nz0 = (tile / (hnx * hny)) * HOZ;
+    const int3 at = tile_at(tile, td);
+    const int nx0 = at.x * HOX, ny0 = at.y * HOY, nz0 = at.z * HOZ;
     const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1;  // EPI_PCHEBY0: the coarse grid
     // staging: two nodes per thread, the three components together; nodes outside the grid stage 0 (their loads go to the
     // nearest node of the grid, so that none of them waits for a branch)
@@ -961,14 +961,14 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, const WT *__res
 }
 
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, const WT *__restrict__ W,
+__global__ __launch_bounds__(256) void k_applyK2_halo(GridDev g, TileDiv td, const WT *__restrict__ W,
                                                       const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
                                                       CgDir<T> cg) {
     __shared__ T su[H2N * H2N * 2];          // staged node block, origin (nx0 - 1, ny0 - 1)
     __shared__ T eb[8 * (UST_TILE + 1)];     // element results: eb[(a*2 + i) * 257 + slot]
-    const int hnx = (g.nnx + H2O - 1) / H2O;
     const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
-    const int nx0 = (tile % hnx) * H2O, ny0 = (tile / hnx) * H2O;
+    const int3 at = tile_at(tile, td);
+    const int nx0 = at.x * H2O, ny0 = at.y * H2O;
     const int cnx = g.nx / 2 + 1;  // EPI_PCHEBY0: the coarse grid
     constexpr int NSN = H2N * H2N, NST = (NSN + UST_TILE - 1) / UST_TILE;
     T stv[NST][2];
@@ -1122,16 +1122,17 @@ __device__ __forceinline__ T block_sum2(const T *eb, int i, int j, int c) {
 }
 
 template <typename T, typename WT, int KIND>
-__global__ __launch_bounds__(256) void k_pre2(GridDev g, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+__global__ __launch_bounds__(256) void k_pre2(GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
                                               const unsigned char *__restrict__ maskc, const T *__restrict__ u,
                                               const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ y,
                                               T *__restrict__ d, T *__restrict__ bc, T c0, T c1, T c2) {
     __shared__ T su[F2S * F2S * 2];
     __shared__ T eb[8 * (UST_TILE + 1)];
     __shared__ T sr[F2R * F2R * 2];
-    const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1, tbx = (cnx + F2C - 1) / F2C;
+    const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1;
     const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
-    const int I0 = (tile % tbx) * F2C, J0 = (tile / tbx) * F2C;
+    const int3 at = tile_at(tile, td);
+    const int I0 = at.x * F2C, J0 = at.y * F2C;
     const int ox = 2 * I0 - 3, oy = 2 * J0 - 3;  // origin of the staged block
     const auto dof_of = [&](int gx, int gy, bool *in) -> unsigned {
         const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1);
@@ -1233,15 +1234,16 @@ __global__ __launch_bounds__(256) void k_pre2(GridDev g, const WT *__restrict__ 
 
 // 2D, both post-smoothing steps: 13x13 nodes
 template <typename T, typename WT>
-__global__ __launch_bounds__(256) void k_post2(GridDev g, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+__global__ __launch_bounds__(256) void k_post2(GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
                                                const T *__restrict__ u, const T *__restrict__ xc, const T *__restrict__ b,
                                                const T *__restrict__ invd, T *__restrict__ y, T c0, T c1, T c2,
                                                double *__restrict__ dots) {
     __shared__ T su[F2S * F2S * 2];
     __shared__ T eb[8 * (UST_TILE + 1)];
-    const int tbx = (g.nnx + F2R - 1) / F2R, cnx = g.nx / 2 + 1;
+    const int cnx = g.nx / 2 + 1;
     const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
-    const int ox = (tile % tbx) * F2R - 2, oy = (tile / tbx) * F2R - 2;  // origin of the staged block
+    const int3 at = tile_at(tile, td);
+    const int ox = at.x * F2R - 2, oy = at.y * F2R - 2;  // origin of the staged block
     const auto dof_of = [&](int gx, int gy, bool *in) -> unsigned {
         const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1);
         *in = kx == gx && ky == gy;
@@ -1337,7 +1339,7 @@ constexpr int F3E = F3EX * F3EY * F3EZ, F3R = F3RX * F3RY * F3RZ, F3S = F3SX * F
 static_assert(F3E <= F3T && F3R * 3 <= 2 * F3T && F3S <= 2 * F3T, "288 elements, 525 residual dofs, 441 nodes");
 
 template <typename T, typename WT, int KIND>
-__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
                                               const unsigned char *__restrict__ maskc, const T *__restrict__ u,
                                               const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ d,
                                               T *__restrict__ bc, T c2) {
@@ -1346,9 +1348,9 @@ __global__ __launch_bounds__(F3T) void k_pre3(GridDev g, const WT *__restrict__ 
     __shared__ T eb[24 * EB];
     __shared__ T sr[F3R * 3];
     const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1, cnz = g.nz / 2 + 1;
-    const int tbx = (cnx + F3X - 1) / F3X, tby = (cny + F3Y - 1) / F3Y;
     const int tile = xcd_block(blockIdx.x, gridDim.x), tid = threadIdx.x;
-    const int I0 = (tile % tbx) * F3X, J0 = ((tile / tbx) % tby) * F3Y, K0 = (tile / (tbx * tby)) * F3Z;
+    const int3 at = tile_at(tile, td);
+    const int I0 = at.x * F3X, J0 = at.y * F3Y, K0 = at.z * F3Z;
     const int ox = 2 * I0 - 2, oy = 2 * J0 - 2, oz = 2 * K0 - 2;  // origin of the staged block and of the elements
     const auto dof_of = [&](int gx, int gy, int gz, bool *in) -> unsigned {
         const int kx = min(max(gx, 0), g.nnx - 1), ky = min(max(gy, 0), g.nny - 1), kz = min(max(gz, 0), g.nnz - 1);
@@ -1470,12 +1472,16 @@ static int fused_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
     if (mode == UST_PASS_CHEBY1R && (!y || y == b)) return UST_EINVAL;
     if (mode == UST_PASS_PCHEBY2 && (!y || y == u || !p->xc)) return UST_EINVAL;
     const dim3 grid(fused_groups(g, mode));
-#define PRE2(KIND) hipLaunchKernelGGL((k_pre2<T, WT, KIND>), grid, dim3(UST_TILE), 0, st, g, W, p->mask, p->maskc, u, b, \
+    const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1;
+    const TileDiv td = mode == UST_PASS_PCHEBY2 ? tile_div((g.nnx + F2R - 1) / F2R, (g.nny + F2R - 1) / F2R)
+                       : g.dim == 2             ? tile_div((cnx + F2C - 1) / F2C, (cny + F2C - 1) / F2C)
+                                                : tile_div((cnx + F3X - 1) / F3X, (cny + F3Y - 1) / F3Y);
+#define PRE2(KIND) hipLaunchKernelGGL((k_pre2<T, WT, KIND>), grid, dim3(UST_TILE), 0, st, g, td, W, p->mask, p->maskc, u, b, \
                                       invd, y, d, bc, c0, c1, c2)
-#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, W, p->mask, p->maskc, u, b, invd, \
+#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, td, W, p->mask, p->maskc, u, b, invd, \
                                       d, bc, c2)
     if (mode == UST_PASS_PCHEBY2)
-        hipLaunchKernelGGL((k_post2<T, WT>), grid, dim3(UST_TILE), 0, st, g, W, p->mask, u, (const T *)p->xc, b, invd, y,
+        hipLaunchKernelGGL((k_post2<T, WT>), grid, dim3(UST_TILE), 0, st, g, td, W, p->mask, u, (const T *)p->xc, b, invd, y,
                            c0, c1, c2, p->dot);
     else if (g.dim == 3 && mode == UST_PASS_RESR) PRE3(PRE_U);
     else if (g.dim == 3) PRE3(PRE_FIRST);
@@ -1489,7 +1495,7 @@ static int fused_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
 }
 
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256) void k_applyK2_tiled(GridDev g, const WT *__restrict__ W,
+__global__ __launch_bounds__(256) void k_applyK2_tiled(GridDev g, TileDiv td, const WT *__restrict__ W,
                                                        const unsigned char *__restrict__ mask, const T *u,
                                                        Epi<T> ep, T *__restrict__ work) {
     constexpr int TX = UST_TX2, TY = UST_TY2;
@@ -1497,7 +1503,8 @@ __global__ __launch_bounds__(256) void k_applyK2_tiled(GridDev g, const WT *__re
     __shared__ T su[NN * 2];
     __shared__ double sy[NN * 2];
     const int tile = blockIdx.x;
-    const int tx0 = (tile % g.tnx) * TX, ty0 = (tile / g.tnx) * TY;
+    const int3 at = tile_at(tile, td);
+    const int tx0 = at.x * TX, ty0 = at.y * TY;
     constexpr int NST = (NN * 2 + UST_TILE - 1) / UST_TILE;
     T stv[NST];
     bool stok[NST];
@@ -1586,20 +1593,6 @@ static inline unsigned face_node_count(const GridDev &g) {
     return fz * g.nnx * g.nny + fy * g.nnx * (g.nnz - fz) + fx * (g.nny - fy) * (g.nnz - fz);
 }
 
-// Division of numbers below 2^31 by a divisor fixed for the launch, as a product (Granlund and Montgomery, "Division by
-// invariant integers using multiplication"): with 2^l >= d, m = ceil(2^(31+l) / d) < 2^32 gives n / d = n m >> (31 + l).
-struct FastDiv {
-    unsigned d, m, s;
-};
-static inline FastDiv fast_div(unsigned d) {
-    unsigned l = 0;
-    while ((1ull << l) < d) l++;
-    const unsigned long long p = 1ull << (31 + l);
-    return {d, (unsigned)((p + d - 1) / d), 31 + l};
-}
-__device__ __forceinline__ unsigned operator/(unsigned n, const FastDiv &f) {
-    return (unsigned)(((unsigned long long)n * f.m) >> f.s);
-}
 struct GatherDiv {  // divisors of the face enumeration: nodes per row and column, faces, off-face rows, z tile and z tile - 1
     FastDiv nnx, nny, fx, fy, ny, tz, tz1;
 };
@@ -1703,9 +1696,11 @@ template <typename T, typename WT, int MODE>
 static int apply_halo(const GridDev &g, const WT *W, const unsigned char *mask, const T *u, const Epi<T> &ep,
                       hipStream_t st, const CgDir<T> &cg = {}) {
     if (g.dim == 3)
-        hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep, cg);
+        hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g,
+                           tile_div((g.nnx + HOX - 1) / HOX, (g.nny + HOY - 1) / HOY), W, mask, u, ep, cg);
     else
-        hipLaunchKernelGGL((k_applyK2_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g, W, mask, u, ep, cg);
+        hipLaunchKernelGGL((k_applyK2_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g,
+                           tile_div((g.nnx + H2O - 1) / H2O, (g.nny + H2O - 1) / H2O), W, mask, u, ep, cg);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }
@@ -1714,6 +1709,7 @@ template <typename T, typename WT, int MODE>
 static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mask, const T *u, Epi<T> ep, T *work,
                        void *stream) {
     GridDev g = grid_dev(gr, col_wg_target(sizeof(T), MODE));
+    const TileDiv td = tile_div(g.tnx, g.tny);
     if (!W || !mask || !u || !ep.y || !work) return UST_EINVAL;
     if (MODE != EPI_Y && !ep.b) return UST_EINVAL;
     if (cheby_mode(MODE) && (!ep.invd || (MODE == EPI_CHEBY && !ep.d) || ep.xs != u)) return UST_EINVAL;
@@ -1725,16 +1721,16 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
     if (halo_grid(g) && (!cheby_mode(MODE) || ep.y != ep.xs)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
     if (g.dim == 3) {
         if (g.col) {
-            hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, W, mask, u, ep,
+            hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u, ep,
                                work);
             gather_tiles<T, 3, MODE, true>(g, mask, work, ep, st);
         } else {
-            hipLaunchKernelGGL((k_applyK3_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, W, mask, u,
+            hipLaunchKernelGGL((k_applyK3_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u,
                                ep, work);
             gather_tiles<T, 3, MODE, false>(g, mask, work, ep, st);
         }
     } else if constexpr (cheby_mode(MODE)) {
-        hipLaunchKernelGGL((k_applyK2_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, W, mask, u, ep,
+        hipLaunchKernelGGL((k_applyK2_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u, ep,
                            work);
         gather_tiles<T, 2, MODE, false>(g, mask, work, ep, st);
     }

@@ -169,6 +169,32 @@ __device__ __forceinline__ int xcd_block(int b, int n) {
     return x * q + (x < r ? x : r) + b / UST_XCDS;
 }
 
+// Division of numbers below 2^31 by a divisor fixed for the launch, as a product (Granlund and Montgomery, "Division by
+// invariant integers using multiplication"): with 2^l >= d, m = ceil(2^(31+l) / d) < 2^32 gives n / d = n m >> (31 + l).
+struct FastDiv {
+    unsigned d, m, s;
+};
+static inline FastDiv fast_div(unsigned d) {
+    unsigned l = 0;
+    while ((1ull << l) < d) l++;
+    const unsigned long long p = 1ull << (31 + l);
+    return {d, (unsigned)((p + d - 1) / d), 31 + l};
+}
+__device__ __forceinline__ unsigned operator/(unsigned n, const FastDiv &f) {
+    return (unsigned)(((unsigned long long)n * f.m) >> f.s);
+}
+
+// position of a tile in a grid of tiles, x fastest; the division by run-time counts would be 60 scalar instructions ahead
+// of a kernel's first load
+struct TileDiv {
+    FastDiv x, y;
+};
+static inline TileDiv tile_div(int nx, int ny) { return {fast_div((unsigned)nx), fast_div((unsigned)ny)}; }
+__device__ __forceinline__ int3 tile_at(int tile, const TileDiv &t) {
+    const unsigned r = (unsigned)tile / t.x, z = r / t.y;
+    return make_int3((int)((unsigned)tile - r * t.x.d), (int)(r - z * t.y.d), (int)z);
+}
+
 // A wavefront's own LDS: its LDS operations complete in order, so a wave-level barrier (no compiler reordering across
 // it) is all that one wave needs between its lanes' writes and reads of each other's values.
 __device__ __forceinline__ void wave_sync() {
