@@ -1860,9 +1860,20 @@ extern "C" int ust_k_apply_pass(const ust_grid *gr, const ust_pass *p, void *str
     return UST_EINVAL;
 }
 
+// the workspace of the shortest chunk that the launch considers, which no other exceeds
+static inline size_t work_len_most(const ust_grid *gr, long long wg_target) {
+    GridDev g = grid_dev(gr, wg_target);
+    if (g.col) {
+        g.tz = column_chunk_least((long long)g.tnx * g.tny, g.nz, wg_target);
+        g.tnz = (g.nz + g.tz - 1) / g.tz;
+        g.ntiles = g.tnx * g.tny * g.tnz;
+    }
+    return work_len(g);
+}
+
 // the largest workspace any pass needs (the passes' column grids differ in z-chunk length)
 extern "C" size_t ust_k_apply_work_len(const ust_grid *gr) {
-    const size_t a = work_len(grid_dev(gr, UST_COL_WG_TARGET)), b = work_len(grid_dev(gr, UST_COL_WG_TARGET_F32_YR));
+    const size_t a = work_len_most(gr, UST_COL_WG_TARGET), b = work_len_most(gr, UST_COL_WG_TARGET_F32_YR);
     return a > b ? a : b;
 }
 
@@ -2006,7 +2017,7 @@ extern "C" size_t ust_k_apply_noalloc_max_work(void) { return UST_NOALLOC_WORK; 
 extern "C" int ust_k_apply_K_f64_noalloc(const ust_grid *g, const double *WK, const unsigned char *mask,
                                          const double *u, double *y, void *stream) {
     if (!g) return UST_EINVAL;
-    const size_t need = work_len(grid_dev(g, col_wg_target(sizeof(double), EPI_Y)));
+    const size_t need = work_len_most(g, col_wg_target(sizeof(double), EPI_Y));
     if (need > UST_NOALLOC_WORK) {
         char msg[256];
         snprintf(msg, sizeof(msg),

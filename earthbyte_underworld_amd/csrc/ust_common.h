@@ -102,6 +102,28 @@ __host__ __device__ __forceinline__ size_t widx(const GridDev &g, int e, int q) 
     return widx_at(g, e % g.nx, (e / g.nx) % g.ny, e / (g.nx * g.ny), q);
 }
 
+// z-chunk of the column kernel: long enough that few node planes sit on chunk boundaries, short enough that the launch has
+// about wg_target workgroups, as many as the GPU holds at once.  A few more than that leave a second round nearly empty:
+// 525 workgroups at 101x67x45 took 33.7 us (FP64 product, with the gather), 420 take 29.8; 576 at 96^3 70.6 us (FP32
+// prolongation pass 61.3), 504 take 55.1 (49.3); 528 at 96x64x64 37.5 us (34.2), 384 take 30.1 (27.9).  So of this and the
+// longer chunks the one with the least rounds times layers is taken (and 0.7 layers for the first plane), among those
+// whose workspace is no larger.
+static inline int column_chunk_least(long long columns, int nz, long long wg_target) {
+    long long z = columns * nz / wg_target;
+    if (z < 2) z = 2;
+    if (z > UST_TZ3_MAX) z = UST_TZ3_MAX;
+    return (int)(z > nz ? nz : z);
+}
+static inline int column_chunk(long long columns, int nz, long long wg_target) {
+    const int z0 = column_chunk_least(columns, nz, wg_target);
+    const auto chunks = [&](long long z) { return (nz + z - 1) / z; };
+    const auto cost = [&](long long z) { return (columns * chunks(z) + wg_target - 1) / wg_target * (10 * z + 7); };
+    int best = z0;
+    for (int z = z0 + 1; z <= UST_TZ3_MAX && z <= nz; z++)
+        if (chunks(z) * (z + 1) <= chunks(z0) * (z0 + 1) && cost(z) < cost(best)) best = z;
+    return best;
+}
+
 // wg_target: the workgroups a column launch aims at (the z-chunk length follows)
 static inline GridDev grid_dev(const ust_grid *g, long long wg_target = UST_COL_WG_TARGET) {
     GridDev d;
@@ -123,13 +145,7 @@ static inline GridDev grid_dev(const ust_grid *g, long long wg_target = UST_COL_
             d.ty = UST_TY3;
             d.tnx = cnx;
             d.tny = cny;
-            // z-chunk: long enough that few node planes sit on chunk boundaries, short enough that the launch
-            // has about wg_target workgroups or more
-            long long zc = layers / wg_target;
-            if (zc < 2) zc = 2;
-            if (zc > UST_TZ3_MAX) zc = UST_TZ3_MAX;
-            if (zc > d.nz) zc = d.nz;
-            d.tz = (int)zc;
+            d.tz = column_chunk((long long)cnx * cny, d.nz, wg_target);
             d.tnz = (d.nz + d.tz - 1) / d.tz;
         } else {
             d.tx = UST_TTX3;
