@@ -261,3 +261,40 @@ def test_hhat_rescale():
     assert st2["stokes_residual"] < 1e-7
     assert rel_err(u2, 1e-9 * u1) < 1e-7 and rel_err(p2, 1e-9 * p1) < 1e-7
     assert abs(st2["outer_its"] - st1["outer_its"]) <= 1
+
+
+# levels whose passes are one launch (2D, small 3D) under every degree of the smoother, with a dense coarsest level, a
+# smoothed one, and one that is the finest as well; larger grids where the finest level takes tiles or columns
+@pytest.mark.parametrize("nel,opts", [
+    ((64, 32), dict(smoother_degree=1)), ((64, 32), dict(smoother_degree=2)),
+    ((64, 32), dict(smoother_degree=3, coarse_degree=1)), ((64, 32), dict(smoother_degree=1, coarse_degree=4)),
+    ((64, 64), dict(mg_levels=2)), ((64, 64), dict(mg_levels=1)), ((130, 134), dict(coarsest_degree=5)),
+    ((65, 67), dict(coarsest_degree=1)), ((65, 67), dict()), ((60, 44), dict(cheby_ratio=20.0)),
+    ((18, 14, 10), dict(smoother_degree=1)), ((18, 14, 10), dict(smoother_degree=3)), ((22, 18, 26), dict()),
+    ((16, 16, 16), dict(smoother_degree=1, coarse_degree=2)), ((48, 48, 32), dict(smoother_degree=1, coarse_degree=2)),
+    ((64, 64, 64), dict(smoother_degree=2, coarse_degree=1))])
+@pytest.mark.parametrize("kind", ["fp64", "mixed_bf16", "inner_fp32"])
+def test_smoother_paths(nel, opts, kind):
+    """One velocity block solve path per smoother option, precision and kind of level: the FP64 Stokes residual, which is
+    computed apart from the solve, meets the bar of this file, and the solution is that of a coarse-tolerance-free FP64
+    solve with the default options to 1e-6."""
+    import earthbyte_underworld_amd as ust
+    from earthbyte_underworld_amd import _lib as L
+    s = ust.StokesSystem(len(nel), nel)
+    s.random_particle_layout(particlesPerCell=6, seed=3)
+    s.set_materials([ust.RheologyMaterial([ust.MaterialViscosity(eta0=1.0)], density=1.0),
+                     ust.RheologyMaterial([ust.MaterialViscosity(eta0=20.0)], density=2.0)])
+    s.assign_materials([ust.Everywhere(0), ust.Sphere(1, (0.4,) * len(nel), 0.25)])
+    s.set_bcs(*ust.free_slip_walls(s))
+    s.assemble(gravity=1.0)
+    tight = dict(outer_rtol=1e-9, inner_rtol=1e-11)
+    assert s.solve(**tight)["stokes_residual"] < 1e-7
+    u0, p0 = s.solution()
+    kw = dict(opts, **tight)
+    if kind != "fp64":
+        kw.update(precision=L.PREC_MIXED, inner_fp32=int(kind.startswith("inner")), vcycle_bf16=int(kind.endswith("bf16")))
+    st = s.solve(**kw)
+    u, p = s.solution()
+    assert st["converged"] and st["stokes_residual"] < 1e-7, st
+    assert rel_err(u, u0) < 1e-6 and rel_err(p, p0) < 1e-6
+    s.close()
