@@ -351,50 +351,38 @@ constexpr int CNR = (CNPD + UST_TILE - 1) / UST_TILE;
 constexpr int EBX = UST_TX3 + 2, EBY = UST_TY3 + 2, EBS = 326;
 static_assert(EBX * EBY <= EBS && 24 * EBS * 4 % 16 == 0, "18x18 slots per row, cleared by 16-byte stores");
 
-// Build-time tuning of the column passes.  UST_COL_MINB_F32: workgroups per CU the register budget of the FP32
-// passes must allow.  UST_COL_PF_*: when the next layer's node plane and weights are loaded -- 1: at the start of
-// the layer, held in registers across the element apply; 2: right after the element apply, so that they are live
-// only across the reduction and the staging; 0: when they are used.  Measured on the 128x128x64 passes (MI355X,
-// 50 launches each): loads after the element apply take the FP32 residual pass from 58.2 to 55.0 us (168
-// instead of 246 VGPRs), the prolongation pass from 75.3 to 72.1 us and the FP64 product from 92.0 to 90.7 us
-// (its loads otherwise wait at the layer); 4 FP32 workgroups per CU without prefetch speed the residual pass
-// (50 us) but spill in the prolongation pass (112 us), 3 spill in both.
-#ifndef UST_COL_MINB_F32
-#define UST_COL_MINB_F32 2
-#endif
-#ifndef UST_COL_PF_F32
-#define UST_COL_PF_F32 2
-#endif
-#ifndef UST_COL_PF_F64
-#define UST_COL_PF_F64 2
-#endif
-// The FP32 product and residual passes (EPI_Y, EPI_RES) take their own values: four workgroups per CU, loads
-// when used, on a grid of ~1024 workgroups (UST_COL_WG_TARGET_F32_YR).  Measured on the 128x128x64 passes:
-// 53.5 -> 49.5 us (product) and 55.2 -> 51.8 us (residual) against the settings of the other passes; the same
-// register budget on the 512-workgroup grid was slower (61 us), and the 1024-workgroup grid slows the
-// prolongation pass (71.5 -> 77.9 us) and the FP64 product (88.8 -> 96.1 us), which keep 512.
-#ifndef UST_COL_MINB_F32_YR
-#define UST_COL_MINB_F32_YR 4
-#endif
-#ifndef UST_COL_PF_F32_YR
-#define UST_COL_PF_F32_YR 0
-#endif
-__host__ __device__ constexpr int col_minb(int tsize, int mode) {
-    return tsize == 4 ? (mode == EPI_Y || mode == EPI_RES || mode == EPI_RES0 ? UST_COL_MINB_F32_YR : UST_COL_MINB_F32)
-                      : 2;
+// The column passes' shapes: workgroups per CU the register budget must allow (minb), when the next layer's node plane and
+// weights are loaded (pf -- 1: at the start of the layer, held in registers across the element apply; 2: right after the
+// element apply, so that they are live only across the reduction and the staging; 0: when they are used), and the
+// workgroups the launch aims at, as many as the GPU then holds.  Measured at 128x128x64 (96^3), with the gather, in us:
+//   FP32 product      minb 4, pf 0, 1024: 38.9 (36.3)   2, 2, 512: 41.2 (36.7)
+//   FP32 Chebyshev    minb 2, pf 2, 1024: 49.6 (43.9)   4, 0, 1024: 49.6 (44.1; 64^3 20.7 for 19.1)   2, 2, 512: 54.7 (48.0)
+//                     (128 registers: four per CU fit)
+//   FP32 prolongation minb 3, pf 0, 768: 53.7 (46.8)    2, 2, 512: 55.0 (49.5)   2, 0, 512: 59.0 (53.1)   2, 2, 1024: 56.4
+//                     (four per CU exceed the LDS; with fewer than 768 workgroups of two layers the loads held in
+//                     registers are worth more than the third: 64^3 20.5 against 21.9)
+//   FP64 product      minb 2, pf 2, 512: 67.5 (55.3)    2, 0, 512: 81.6 (64.0)   2, 1, 512: 66.0 (54.6; the Chebyshev pass
+//                     109.2 for 97.2)   2, 2, 1024: 73.8 (64.7)
+struct ColShape {
+    int minb, pf, target;
+};
+__host__ __device__ constexpr ColShape col_shape(int tsize, int mode, bool many = false) {
+    return tsize == 8                                ? ColShape{2, 2, UST_COL_WG_TARGET}
+           : mode == EPI_PCHEBY0 && many             ? ColShape{3, 0, UST_COL_WG_TARGET_P}
+           : mode == EPI_PCHEBY0                     ? ColShape{2, 2, UST_COL_WG_TARGET}
+           : mode == EPI_CHEBY || mode == EPI_CHEBY0 ? ColShape{2, 2, UST_COL_WG_TARGET_F32_YR}
+                                                     : ColShape{4, 0, UST_COL_WG_TARGET_F32_YR};
 }
-__host__ __device__ constexpr int col_pf(int tsize, int mode) {
-    return tsize == 4 ? (mode == EPI_Y || mode == EPI_RES || mode == EPI_RES0 ? UST_COL_PF_F32_YR : UST_COL_PF_F32)
-                      : UST_COL_PF_F64;
+// whether the FP32 prolongation pass has workgroups for three per CU
+static inline bool col_many(const ust_grid *gr, int tsize, int mode) {
+    if (tsize != 4 || mode != EPI_PCHEBY0 || gr->dim != 3) return false;
+    const long long cx = (gr->nel[0] + UST_TX3 - 1) / UST_TX3, cy = (gr->nel[1] + UST_TY3 - 1) / UST_TY3;
+    return cx * cy * gr->nel[2] >= 2 * UST_COL_WG_TARGET_P;
 }
-constexpr long long col_wg_target(int tsize, int mode) {
-    return tsize == 4 && (mode == EPI_Y || mode == EPI_RES || mode == EPI_RES0) ? UST_COL_WG_TARGET_F32_YR
-                                                                              : UST_COL_WG_TARGET;
-}
-template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(GridDev g, TileDiv td, const WT *__restrict__ W,
-                                                     const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
-                                                     T *__restrict__ work) {
+template <typename T, typename WT, int MODE, bool MANY = false>
+__global__ __launch_bounds__(256, col_shape(sizeof(T), MODE, MANY).minb) void k_applyK3_col(
+    GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
+    T *__restrict__ work) {
     __shared__ T su[2][CNPD];     // staged node planes k and k+1 (free dofs; Dirichlet dofs read 0)
     __shared__ __attribute__((aligned(16))) T eb[24 * EBS];  // the layer's results: eb[(a*3 + i)*EBS + slot]
     // EPI_PCHEBY0: a ring of two coarse node planes under the column (9x9 coarse nodes; the column's origin is
@@ -501,9 +489,9 @@ __global__ __launch_bounds__(256, col_minb(sizeof(T), MODE)) void k_applyK3_col(
 #pragma unroll
         for (int q = 0; q < 27; q++) w[q] = W[wbase + ((size_t)k * 27 + q) * UST_TILE];
     };
-    // when the next layer's node plane and weights are loaded (UST_COL_PF_*): wpre at the start of this layer,
+    // when the next layer's node plane and weights are loaded (col_shape): wpre at the start of this layer,
     // wlate after its element apply; held: in registers (xr, mr, wr) until the next layer uses them
-    constexpr int pf = col_pf(sizeof(T), MODE);
+    constexpr int pf = col_shape(sizeof(T), MODE, MANY).pf;
     constexpr bool wpre = pf == 1, wlate = pf == 2, held = pf != 0;
     // ---- prologue: the coarse ring (planes z0/2 and z0/2 + 1), plane z0, and the loads for layer z0 ----
     if (MODE == EPI_PCHEBY0) {
@@ -1708,7 +1696,8 @@ static int apply_halo(const GridDev &g, const WT *W, const unsigned char *mask, 
 template <typename T, typename WT, int MODE>
 static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mask, const T *u, Epi<T> ep, T *work,
                        void *stream) {
-    GridDev g = grid_dev(gr, col_wg_target(sizeof(T), MODE));
+    const bool many = col_many(gr, sizeof(T), MODE);
+    GridDev g = grid_dev(gr, col_shape(sizeof(T), MODE, many).target);
     const TileDiv td = tile_div(g.tnx, g.tny);
     if (!W || !mask || !u || !ep.y || !work) return UST_EINVAL;
     if (MODE != EPI_Y && !ep.b) return UST_EINVAL;
@@ -1721,8 +1710,13 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
     if (halo_grid(g) && (!cheby_mode(MODE) || ep.y != ep.xs)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
     if (g.dim == 3) {
         if (g.col) {
-            hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u, ep,
-                               work);
+            if constexpr (sizeof(T) == 4 && MODE == EPI_PCHEBY0)
+                if (many)
+                    hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE, true>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W,
+                                       mask, u, ep, work);
+            if (!many)
+                hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u,
+                                   ep, work);
             gather_tiles<T, 3, MODE, true>(g, mask, work, ep, st);
         } else {
             hipLaunchKernelGGL((k_applyK3_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u,
@@ -2017,7 +2011,7 @@ extern "C" size_t ust_k_apply_noalloc_max_work(void) { return UST_NOALLOC_WORK; 
 extern "C" int ust_k_apply_K_f64_noalloc(const ust_grid *g, const double *WK, const unsigned char *mask,
                                          const double *u, double *y, void *stream) {
     if (!g) return UST_EINVAL;
-    const size_t need = work_len_most(g, col_wg_target(sizeof(double), EPI_Y));
+    const size_t need = work_len_most(g, col_shape(sizeof(double), EPI_Y).target);
     if (need > UST_NOALLOC_WORK) {
         char msg[256];
         snprintf(msg, sizeof(msg),

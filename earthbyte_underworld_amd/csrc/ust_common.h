@@ -56,15 +56,10 @@ __host__ __device__ constexpr int sgn(int a) { return 2 * a - 1; }
 #define UST_TILE 256
 #define UST_TZ3_MAX 16
 #define UST_COL_MIN 1024
-// workgroups a column launch aims at (the z-chunk length follows): two per CU; 1024 (four per CU, shorter
-// chunks) measured slower on the 128x128x64 solve (FP64 product 93 -> 100 us).  The FP32 product and residual
-// passes, which fit four workgroups per CU, aim at 1024 (UST_COL_WG_TARGET_F32_YR).
-#ifndef UST_COL_WG_TARGET
+// workgroups a column launch aims at (the z-chunk length follows): what the GPU holds of them at two, three and four per CU
 #define UST_COL_WG_TARGET 512
-#endif
-#ifndef UST_COL_WG_TARGET_F32_YR
+#define UST_COL_WG_TARGET_P 768
 #define UST_COL_WG_TARGET_F32_YR 1024
-#endif
 
 struct GridDev {
     int dim;
@@ -107,7 +102,7 @@ __host__ __device__ __forceinline__ size_t widx(const GridDev &g, int e, int q) 
 // 525 workgroups at 101x67x45 took 33.7 us (FP64 product, with the gather), 420 take 29.8; 576 at 96^3 70.6 us (FP32
 // prolongation pass 61.3), 504 take 55.1 (49.3); 528 at 96x64x64 37.5 us (34.2), 384 take 30.1 (27.9).  So of this and the
 // longer chunks the one with the least rounds times layers is taken (and 0.7 layers for the first plane), among those
-// whose workspace is no larger.
+// whose workspace is no larger (for 768 workgroups: than that of 512 or of 1024).
 static inline int column_chunk_least(long long columns, int nz, long long wg_target) {
     long long z = columns * nz / wg_target;
     if (z < 2) z = 2;
@@ -115,13 +110,18 @@ static inline int column_chunk_least(long long columns, int nz, long long wg_tar
     return (int)(z > nz ? nz : z);
 }
 static inline int column_chunk(long long columns, int nz, long long wg_target) {
-    const int z0 = column_chunk_least(columns, nz, wg_target);
     const auto chunks = [&](long long z) { return (nz + z - 1) / z; };
+    const auto work = [&](long long t) {
+        const int z = column_chunk_least(columns, nz, t);
+        return chunks(z) * (z + 1);
+    };
     const auto cost = [&](long long z) { return (columns * chunks(z) + wg_target - 1) / wg_target * (10 * z + 7); };
-    int best = z0;
-    for (int z = z0 + 1; z <= UST_TZ3_MAX && z <= nz; z++)
-        if (chunks(z) * (z + 1) <= chunks(z0) * (z0 + 1) && cost(z) < cost(best)) best = z;
-    return best;
+    const long long w = work(UST_COL_WG_TARGET), v = work(UST_COL_WG_TARGET_F32_YR);
+    const long long most = wg_target == UST_COL_WG_TARGET ? w : wg_target == UST_COL_WG_TARGET_F32_YR ? v : w > v ? w : v;
+    int best = 0;
+    for (int z = column_chunk_least(columns, nz, wg_target); z <= UST_TZ3_MAX && z <= nz; z++)
+        if (chunks(z) * (z + 1) <= most && (!best || cost(z) < cost(best))) best = z;
+    return best ? best : column_chunk_least(columns, nz, UST_COL_WG_TARGET);
 }
 
 // wg_target: the workgroups a column launch aims at (the z-chunk length follows)
