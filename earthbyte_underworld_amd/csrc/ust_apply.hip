@@ -1706,8 +1706,9 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
     if (MODE == EPI_PCHEBY0 && (g.dim != 3 || !ep.xc || g.nx % 2 || g.ny % 2 || g.nz % 2)) return UST_EINVAL;
     if ((size_t)g.nnx * g.nny * g.nnz * g.dim >= (1ull << 32)) return UST_EINVAL;  // 32-bit dof indices
     hipStream_t st = ust_stream(stream);
-    // small 3D grids and 2D ones: the halo kernel, unless a Chebyshev step runs in place
-    if (halo_grid(g) && (!cheby_mode(MODE) || ep.y != ep.xs)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
+    // small 3D grids and 2D ones: the halo kernel, unless the pass overwrites what its neighbours stage (a Chebyshev step, a
+    // product or a residual in place, a first step over its right-hand side), which tiles + gather allow
+    if (halo_grid(g) && ep.y != u && (MODE != EPI_RES0 || ep.d != ep.b)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
     if (g.dim == 3) {
         if (g.col) {
             if constexpr (sizeof(T) == 4 && MODE == EPI_PCHEBY0)
@@ -1723,7 +1724,7 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
                                ep, work);
             gather_tiles<T, 3, MODE, false>(g, mask, work, ep, st);
         }
-    } else if constexpr (cheby_mode(MODE)) {
+    } else {
         hipLaunchKernelGGL((k_applyK2_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u, ep,
                            work);
         gather_tiles<T, 2, MODE, false>(g, mask, work, ep, st);

@@ -946,3 +946,54 @@ def test_fused_level_passes(dim, nel, prec):
     for a in hold:
         a.free()
     s.close()
+
+
+@pytest.mark.parametrize("dim,nel", [(2, (33, 17)), (2, (40, 24)), (3, (17, 9, 5)), (3, (16, 16, 8))])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_passes_in_place(dim, nel, prec):
+    """Product, residual and the first step with its residual where the output overwrites the input, on grids whose passes
+    are otherwise one launch each (a workgroup there stages nodes that others write): what the calls out of place give,
+    to the rounding of another order of the same sums."""
+    import ctypes as C
+    from earthbyte_underworld_amd import _lib as L
+    s = _build(dim, nel, 6, 4)
+    lib = s.lib
+    g = L.Grid()
+    WK, WG, WF, mask = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_void_p()
+    assert lib.ust_get_device_views(s.ctx, C.byref(g), C.byref(WK), C.byref(WG), C.byref(WF), C.byref(mask)) == 0
+    T, n, nw = (np.float64 if prec == "f64" else np.float32), s.ndof, lib.ust_k_weights_len(C.byref(g))
+    w32 = _Dev(lib, np.zeros(nw, np.float32))
+    assert lib.ust_k_copy_f64_to_f32(WK, w32.p, nw, None) == 0
+    W = WK if prec == "f64" else w32.p
+    rng = np.random.default_rng(3)
+    u, b = rng.normal(size=n).astype(T), rng.normal(size=n).astype(T)
+    invd = np.full(n, 1e-5, T)
+    ws = _Dev(lib, np.zeros(lib.ust_k_apply_work_len(C.byref(g)), T))
+    fn = lambda name: getattr(lib, f"ust_k_apply_K_{name}")
+    tol = 1e-13 if prec == "f64" else 1e-5
+
+    def run(f):
+        dev = [_Dev(lib, a) for a in (u, b, invd, np.zeros(n, T), np.zeros(n, T))]
+        assert f(*[d.p for d in dev]) == 0
+        out = [d.get() for d in dev]
+        for d in dev:
+            d.free()
+        return out
+
+    product = fn(prec)
+    ref = run(lambda u_, b_, i_, y_, x_: product(C.byref(g), W, mask, u_, y_, ws.p, None))[3]
+    got = run(lambda u_, b_, i_, y_, x_: product(C.byref(g), W, mask, u_, u_, ws.p, None))[0]
+    assert rel_err(got, ref) < tol
+    res = fn(f"residual_{prec}")
+    ref = run(lambda u_, b_, i_, y_, x_: res(C.byref(g), W, mask, u_, b_, y_, ws.p, None))[3]
+    for k in (0, 1):  # over u, over b
+        got = run(lambda u_, b_, i_, y_, x_: res(C.byref(g), W, mask, u_, b_, (u_, b_)[k], ws.p, None))[k]
+        assert rel_err(got, ref) < tol
+    if prec == "f32":
+        first = lib.ust_k_apply_K_residual_first_f32
+        r = run(lambda u_, b_, i_, y_, x_: first(C.byref(g), W, mask, b_, i_, x_, y_, 0.5, ws.p, None))
+        over_r = run(lambda u_, b_, i_, y_, x_: first(C.byref(g), W, mask, b_, i_, x_, b_, 0.5, ws.p, None))
+        assert rel_err(over_r[1], r[3]) < tol and np.array_equal(over_r[4], r[4])
+    w32.free()
+    ws.free()
+    s.close()
