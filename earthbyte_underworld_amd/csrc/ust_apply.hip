@@ -896,7 +896,8 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, con
             const int n = tid + UST_TILE * r;
             const int ax = n % HNX, ay = (n / HNX) % HNY, az = n / (HNX * HNY);
             const bool mine = stok[r] && ax >= 1 && ax <= HOX && ay >= 1 && ay <= HOY && az >= 1 && az <= HOZ && n < HNN;
-            const unsigned dof = ((unsigned)(nx0 - 1 + ax) + (unsigned)g.nnx * ((unsigned)(ny0 - 1 + ay) + (unsigned)g.nny * (nz0 - 1 + az))) * 3u;
+            const unsigned row = (unsigned)(ny0 - 1 + ay) + (unsigned)g.nny * (nz0 - 1 + az);
+            const unsigned dof = ((unsigned)(nx0 - 1 + ax) + (unsigned)g.nnx * row) * 3u;
 #pragma unroll
             for (int c = 0; c < 3; c++) {
                 stv[r][c] = first ? stv[r][c] : stv[r][c] + beta * stp[r][c];
@@ -939,7 +940,8 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, con
             for (int dy = 1; dy >= 0; dy--)
 #pragma unroll
                 for (int dx = 1; dx >= 0; dx--)  // element slot (ox + 1 - dx, ...) has this node as vertex (dx, dy, dz)
-                    v += (double)eb[((dx + 2 * dy + 4 * dz) * 3 + c) * HNE + (ox + 1 - dx) + HEX * ((oy + 1 - dy) + HEY * (oz + 1 - dz))];
+                    v += (double)eb[((dx + 2 * dy + 4 * dz) * 3 + c) * HNE + (ox + 1 - dx) +
+                                    HEX * ((oy + 1 - dy) + HEY * (oz + 1 - dz))];
         EpiOps<T> o = ops[r];
         if (MODE == EPI_PCHEBY0 && !o.m) o.x = us;  // x + P xc, as staged
         const T out = epilogue_store<MODE, T>(ep, o, odof + c, (T)v);
@@ -1110,7 +1112,8 @@ __device__ __forceinline__ T block_sum2(const T *eb, int i, int j, int c) {
 }
 
 template <typename T, typename WT, int KIND>
-__global__ __launch_bounds__(256) void k_pre2(GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+__global__ __launch_bounds__(256) void k_pre2(GridDev g, TileDiv td, const WT *__restrict__ W,
+                                              const unsigned char *__restrict__ mask,
                                               const unsigned char *__restrict__ maskc, const T *__restrict__ u,
                                               const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ y,
                                               T *__restrict__ d, T *__restrict__ bc, T c0, T c1, T c2) {
@@ -1222,7 +1225,8 @@ __global__ __launch_bounds__(256) void k_pre2(GridDev g, TileDiv td, const WT *_
 
 // 2D, both post-smoothing steps: 13x13 nodes
 template <typename T, typename WT>
-__global__ __launch_bounds__(256) void k_post2(GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+__global__ __launch_bounds__(256) void k_post2(GridDev g, TileDiv td, const WT *__restrict__ W,
+                                              const unsigned char *__restrict__ mask,
                                                const T *__restrict__ u, const T *__restrict__ xc, const T *__restrict__ b,
                                                const T *__restrict__ invd, T *__restrict__ y, T c0, T c1, T c2,
                                                double *__restrict__ dots) {
@@ -1327,7 +1331,8 @@ constexpr int F3E = F3EX * F3EY * F3EZ, F3R = F3RX * F3RY * F3RZ, F3S = F3SX * F
 static_assert(F3E <= F3T && F3R * 3 <= 2 * F3T && F3S <= 2 * F3T, "288 elements, 525 residual dofs, 441 nodes");
 
 template <typename T, typename WT, int KIND>
-__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask,
+__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, const WT *__restrict__ W,
+                                              const unsigned char *__restrict__ mask,
                                               const unsigned char *__restrict__ maskc, const T *__restrict__ u,
                                               const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ d,
                                               T *__restrict__ bc, T c2) {

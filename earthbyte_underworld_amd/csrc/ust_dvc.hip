@@ -250,9 +250,9 @@ __device__ void dvc_element_words(const DvcShape &s, unsigned char *dvc_lds, int
 // a wave looks at `per` elements and redoes the marked ones.  per = 1: every element, where particles so many that
 // k_dvc_grow's LDS does not fit share one.
 template <int DIM, typename OT>
-__global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, const int *elems, int nel, double *xi0,
-                                                         double *xi1, double *xi2, double *w, int set_centroids,
-                                                         int *flag, int per) {
+__global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, const int *elems,
+                                                         int nel, double *xi0, double *xi1, double *xi2, double *w,
+                                                         int set_centroids, int *flag, int per) {
     extern __shared__ __align__(16) unsigned char dvc_lds[];
     int el = blockIdx.x * per + (int)threadIdx.x;
     const bool mine = (int)threadIdx.x < per && el < nel;
@@ -293,7 +293,8 @@ constexpr int DVC_WIDE_2D = 16384;  // 2D swarms of fewer elements give an eleme
 
 template <int DIM, int G, typename OT>
 __global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const int *__restrict__ cell_off,
-                                                              const int *__restrict__ elems, int nel, double *xi0, double *xi1, double *xi2, double *w,
+                                                              const int *__restrict__ elems, int nel, double *xi0,
+                                                              double *xi1, double *xi2, double *w,
                                                               int set_centroids, int *flag) {
     static_assert(G == 16 || G == 32, "group votes are 32-bit");
     extern __shared__ __align__(16) unsigned char dvc_lds[];
@@ -542,8 +543,8 @@ __global__ __launch_bounds__(64 * GROW_WAVES) void k_dvc_grow(DvcShape s, const 
 }
 
 template <int DIM, int G, typename OT>
-static int launch_dvc(const DvcShape &s, size_t lds_words, const int *cell_off, const int *elems, int nel, double *xi0, double *xi1,
-                      double *xi2, double *w, int set_centroids, int *flag, hipStream_t st) {
+static int launch_dvc(const DvcShape &s, size_t lds_words, const int *cell_off, const int *elems, int nel, double *xi0,
+                      double *xi1, double *xi2, double *w, int set_centroids, int *flag, hipStream_t st) {
     constexpr int EPB = 64 * GROW_WAVES / G;
     const size_t lds = grow_lds_shared(s) + EPB * grow_lds_element(s, sizeof(OT));
     const bool grow = lds <= 65536;
