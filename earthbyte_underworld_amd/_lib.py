@@ -166,6 +166,7 @@ _SIGS = {
     "ust_k_apply_K_ref_f32": (I, [C.POINTER(Grid), vp, vp, vp, vp, vp]),
     "ust_k_copy_f64_to_f32": (I, [vp, vp, C.c_size_t, vp]),
     "ust_k_weights_len": (C.c_size_t, [C.POINTER(Grid)]),
+    "ust_k_weights_index": (C.c_size_t, [C.POINTER(Grid), I, I]),
     "ust_apply_K": (I, [vp, vp, vp]),
     "ust_apply_K_dev": (I, [vp, vp, vp]),
     "ust_apply_K_f32_dev": (I, [vp, vp, vp]),

@@ -4,7 +4,7 @@
 //
 // 3D: one 256-thread workgroup owns a 16x16 column of elements, one element per thread, and streams a
 // chunk of element layers along z.  Node planes are staged in LDS once each; per layer every thread applies
-// its element (element_apply3 below, about 460 operations) and leaves its 8 vertex
+// its element (element_apply3 below, about 600 operations) and leaves its 8 vertex
 // results in LDS; each node of the plane below the layer then sums, in a fixed order, the contributions of
 // the (up to) four elements above it and the four below it (carried in registers from the previous layer),
 // and is finished: written to y through the epilogue, unless it lies on the ring of the column (shared with
@@ -26,129 +26,182 @@ __host__ __device__ constexpr int P2(int k) { return k == 2 ? 1 : 2; }
 __host__ __device__ constexpr int pow3(int k) { return k == 0 ? 1 : (k == 1 ? 3 : 9); }
 
 // ------------------------------------------------------------------------------------------
-// Element action y = K_e u in 3D, in monomials.  A velocity component is trilinear, u_i = sum c_i[m] xi^m over the
-// 8 exponents m in {0,1}^3 (a bit mask, bit 0 for x); its gradients are bilinear with the same coefficients,
-//   d u_i / d x_k = s_k sum_{m has bit k} c_i[m] xi^(m without k),
-// and the vertex functions tested with are trilinear in the same way.  The particle sums therefore enter through the 27
-// moments M[a,b,c] = sum_q W_q xi_q^a eta_q^b zeta_q^c, a, b, c <= 2, which three passes of sums and differences make from
-// the weights at {-1,0,1}^3: a normal strain meets its 4 test functions in a symmetric 4 x 4 product of moments, a shear
-// strain (6 monomials, shared by its two test functions) in a symmetric 6 x 6 one.  Per element 81 operations for the
-// moments, 81 and 66 to and from the coefficients, 72 scalings, 156 multiply-adds: 456, where interpolating gradients to
-// and stresses from the 27 points took about 750.
+// Element action y = K_e u in 3D, in edge differences.  A velocity component is trilinear, so d u_i / d x_k is constant
+// along k and, over the other two axes, interpolates the differences of u_i along the element's four edges in direction
+// k with products of hat functions; the test functions' gradients are the same.  The weights W at {-1,0,1}^3 therefore
+// enter through their sums against products of two hats per axis -- N0 N0, N0 N1, N1 N1, at a line of three weights
+// W0 + W1 / 4, W1 / 4, W2 + W1 / 4, or against one hat or none where only one or none varies along it:
+//   S_k  (9, per direction k): the 4 x 4 products of the differences along k with themselves, one component at a time,
+//   L_ik (12, per pair): the 4 x 4 products of the differences of u_i along k with those of u_k along i.
+// Per element 120 operations for S (four times) and 114 for L, 36 differences, 240 multiply-adds, 24 scalings and 72 to the
+// vertices: 606.  Interpolating gradients to and stresses from the 27 points takes about 750; monomials around the
+// element's centre, whose products share terms, 456.  But those round sums and differences of all eight vertices on the
+// way in and out, each vertex's result by the element's largest, where here a difference is rounded once before it is
+// used and, of weights of one sign, every sum is of one sign.  Error of the product of a random field, relative 2-norm,
+// and time at 128x128x64 with the gather -- points: FP32 5.39e-8, FP64 1.57e-16, 49.0 and 86.6 us; monomials: 6.45e-8,
+// 1.68e-16, 38.4 and 67.1 us; edges: 5.35e-8, 1.55e-16, 42.3 and 71.1 us.  Other grids: FP32 101x67x45 5.49, 6.73, 5.34e-8;
+// 60x44x40 (tiles) 4.87, 6.10, 4.85e-8; 64x64x32, where powers of two scale the points without rounding, 4.70, 5.83,
+// 4.91e-8; FP64 40x36x30 (halo) 1.69, 1.88, 1.57e-16.
 // ------------------------------------------------------------------------------------------
-// weights at {-1, 0, 1}^3 -> moments, in place
+// lower end of edge b in direction k: bit 0 of b on axis P1(k), bit 1 on P2(k)
+__host__ __device__ constexpr int edge3(int k, int b) { return (b & 1) << P1(k) | (b >> 1) << P2(k); }
+// the edge of direction k at bits (bi, bj) of the axes i and j
+__host__ __device__ constexpr int edge_at(int k, int i, int bi, int bj) { return P1(k) == i ? bi | bj << 1 : bj | bi << 1; }
+
+// factors of the gradients' products: w[k] = (1 / (4 h_k))^2 and r[i][k] = h_k / h_i
 template <typename T>
-__device__ __forceinline__ void moments3(T M[27]) {
+struct GradScale {
+    T w[3], r[3][3];
+};
+template <typename T>
+static inline GradScale<T> grad_scale(const GridDev &g) {
+    const double d[3] = {g.sx, g.sy, g.sz};  // 2 / h
+    GradScale<T> s;
+    for (int k = 0; k < 3; k++) {
+        s.w[k] = (T)(0.125 * d[k] * (0.125 * d[k]));
+        for (int i = 0; i < 3; i++) s.r[i][k] = (T)(d[i] / d[k]);
+    }
+    return s;
+}
+
+template <typename T, int I, int K, typename U>
+__device__ __forceinline__ void differences3(const U &u, T d[4]) {
 #pragma unroll
-    for (int k = 0; k < 3; k++)
+    for (int b = 0; b < 4; b++) d[b] = u(edge3(K, b) | 1 << K, I) - u(edge3(K, b), I);
+}
+
+// 16 S_K, index q1 + 3 q2 with q the number of upper hats on P1(K) and P2(K)
+template <typename T, int K>
+__device__ __forceinline__ void edge_weights3(const T W[27], T S[9]) {
+    constexpr int k = pow3(K), p = pow3(P1(K)), q = pow3(P2(K));
 #pragma unroll
-        for (int l = 0; l < 9; l++) {
-            const int i = (l % 3) * pow3(P1(k)) + (l / 3) * pow3(P2(k)), d = pow3(k);
-            const T t = M[i] + M[i + 2 * d], df = M[i + 2 * d] - M[i];
-            M[i] = t + M[i + d];
-            M[i + d] = df;
-            M[i + 2 * d] = t;
+    for (int j = 0; j < 3; j++) {
+        T l[3];
+#pragma unroll
+        for (int i = 0; i < 3; i++) l[i] = (W[i * p + j * q] + W[i * p + j * q + 2 * k]) + W[i * p + j * q + k];
+        S[3 * j] = (T)4 * l[0] + l[1];
+        S[3 * j + 1] = l[1];
+        S[3 * j + 2] = (T)4 * l[2] + l[1];
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+        S[i] = (T)4 * S[i] + S[3 + i];
+        S[6 + i] = (T)4 * S[6 + i] + S[3 + i];
+    }
+}
+
+// 16 L_IK: one hat on I (first index) and on K, two on the third axis (last index: the number of upper ones)
+template <typename T, int I, int K>
+__device__ __forceinline__ void cross_weights3(const T W[27], T L[2][2][3]) {
+    constexpr int i = pow3(I), k = pow3(K), j = pow3(3 - I - K);
+#pragma unroll
+    for (int a = 0; a < 2; a++) {
+        T m[3][3];
+#pragma unroll
+        for (int n = 0; n < 9; n++) {
+            const int o = (n % 3) * k + (n / 3) * j;
+            m[n % 3][n / 3] = (T)2 * W[o + 2 * a * i] + W[o + i];
+        }
+#pragma unroll
+        for (int b = 0; b < 2; b++) {
+            T l[3];
+#pragma unroll
+            for (int n = 0; n < 3; n++) l[n] = (T)2 * m[2 * b][n] + m[1][n];
+            L[a][b][0] = (T)4 * l[0] + l[1];
+            L[a][b][1] = l[1];
+            L[a][b][2] = (T)4 * l[2] + l[1];
+        }
+    }
+}
+
+// r += S d, the product with the largest weight last
+template <typename T>
+__device__ __forceinline__ void edge_product3(const T S[9], const T d[4], T r[4]) {
+#pragma unroll
+    for (int a = 0; a < 4; a++)
+#pragma unroll
+        for (int n = 1; n < 5; n++) {
+            const int b = a ^ (n & 3);
+            r[a] += S[(a & 1) + (b & 1) + 3 * ((a >> 1) + (b >> 1))] * d[b];
         }
 }
 
-// 8 times the coefficients of component I (index: the bit mask; [0] is not needed).  Differences are taken before sums,
-// so a smooth field loses no digits to its mean.
-template <typename T, int I, typename U>
-__device__ __forceinline__ void coefficients3(const U &u, T c[8]) {
-    T v[8];
-#pragma unroll
-    for (int a = 0; a < 8; a++) v[a] = u(a, I);
-    const T x0 = v[1] - v[0], x1 = v[3] - v[2], x2 = v[5] - v[4], x3 = v[7] - v[6];  // along x at (y, z)
-    const T p0 = x0 + x1, p1 = x2 + x3, m0 = x1 - x0, m1 = x3 - x2;
-    c[1] = p0 + p1;
-    c[5] = p1 - p0;
-    c[3] = m0 + m1;
-    c[7] = m1 - m0;
-    const T y0 = (v[2] - v[0]) + (v[3] - v[1]), y1 = (v[6] - v[4]) + (v[7] - v[5]);  // along y, summed over x
-    c[2] = y0 + y1;
-    c[6] = y1 - y0;
-    c[4] = ((v[4] - v[0]) + (v[5] - v[1])) + ((v[6] - v[2]) + (v[7] - v[3]));
-}
-
-// the transpose: y[a][I] = sum over the masks of z times the vertex's signs
-template <typename T, int I>
-__device__ __forceinline__ void vertices3(const T z[8], T y[8][3]) {
-    const T p0 = z[1] + z[3], m0 = z[1] - z[3], p1 = z[5] + z[7], m1 = z[5] - z[7];
-    const T f0 = z[2] - z[6], f1 = z[2] + z[6];
-    // x part e and the rest h at (y, z)
-    const T e[4] = {m0 - m1, p0 - p1, m0 + m1, p0 + p1};
-    const T h[4] = {-f0 - z[4], f0 - z[4], z[4] - f1, f1 + z[4]};
+// the edges' w r to the vertices
+template <typename T, int I, int K, bool FIRST>
+__device__ __forceinline__ void edges_to_vertices3(const T r[4], T w, T y[8][3]) {
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-        y[2 * b][I] = h[b] - e[b];
-        y[2 * b + 1][I] = h[b] + e[b];
+        const int a = edge3(K, b);
+        y[a | 1 << K][I] = FIRST ? w * r[b] : y[a | 1 << K][I] + w * r[b];
+        y[a][I] = FIRST ? -(w * r[b]) : y[a][I] - w * r[b];
     }
 }
 
-// stress of the normal strain I against its test functions
-template <typename T, int I>
-__device__ __forceinline__ void normal3(const T c[3][8], const T M[27], const T s[3], T z[3][8]) {
-    T g[4];
-#pragma unroll
-    for (int m = 0; m < 4; m++) g[m] = (T)2 * s[I] * c[I][(1 << I) | (m & 1) << P1(I) | (m >> 1) << P2(I)];
-#pragma unroll
-    for (int n = 0; n < 4; n++) {
-        T r = (T)0;
-#pragma unroll
-        for (int m = 0; m < 4; m++)
-            r += M[((m & 1) + (n & 1)) * pow3(P1(I)) + ((m >> 1) + (n >> 1)) * pow3(P2(I))] * g[m];
-        z[I][(1 << I) | (n & 1) << P1(I) | (n >> 1) << P2(I)] += s[I] * r;
-    }
+// between the parts of an element's action, kept APART: instructions of one are not moved among those of another.
+// Interleaved, several parts' sums are held at once: the FP64 column kernel (256 registers) then spills 10 of them, the FP32
+// product's (128) 12.  The kernels of small grids have registers to spare and hide the latency of one part behind another:
+// 24x16x16 FP64 product 5.1 us, with the parts apart 5.6; 64x64x32 (tiles) 13.2, 13.6.
+template <bool APART>
+__device__ __forceinline__ void part_end() {
+    if (APART) __builtin_amdgcn_sched_barrier(0);
 }
 
-// stress of the shear strain d u_I / d x_K + d u_K / d x_I: monomials {1, xi_I, xi_K} x {1, xi_J}
-template <typename T, int I, int K>
-__device__ __forceinline__ void shear3(const T c[3][8], const T M[27], const T s[3], T z[3][8]) {
-    constexpr int J = 3 - I - K;
-    T t[3][2];
+// d u_I / d x_K with itself (S_K) and with d u_K / d x_I (L_IK), and the same with I and K exchanged.  SI, SK: the edge
+// weights, made here (NEW) or by a part before
+template <bool APART, typename T, int I, int K, bool FIRST_I, bool FIRST_K, bool NEW_I, bool NEW_K, typename U>
+__device__ __forceinline__ void pair3(const U &u, const T W[27], T SI[9], T SK[9], const GradScale<T> &s, T y[8][3]) {
+    T di[4], dk[4], ri[4], rk[4];
+    {
+        T L[2][2][3];
+        cross_weights3<T, I, K>(W, L);
+        differences3<T, I, K>(u, di);
+        differences3<T, K, I>(u, dk);
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        t[0][j] = s[K] * c[I][(1 << K) | j << J] + s[I] * c[K][(1 << I) | j << J];
-        t[1][j] = s[K] * c[I][(1 << K) | (1 << I) | j << J];
-        t[2][j] = s[I] * c[K][(1 << I) | (1 << K) | j << J];
+        for (int a = 0; a < 2; a++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) {
+                T vi = (T)0, vk = (T)0;
+#pragma unroll
+                for (int n = 0; n < 4; n++) {
+                    const int b = n & 1, e = n >> 1;
+                    vi += L[a][b][c + e] * dk[edge_at(I, K, b, e)];
+                    vk += L[b][a][c + e] * di[edge_at(K, I, b, e)];
+                }
+                ri[edge_at(K, I, a, c)] = s.r[I][K] * vi;
+                rk[edge_at(I, K, a, c)] = s.r[K][I] * vk;
+            }
     }
-#pragma unroll
-    for (int n = 0; n < 3; n++)
-#pragma unroll
-        for (int l = 0; l < 2; l++) {
-            T r = (T)0;
-#pragma unroll
-            for (int m = 0; m < 3; m++)
-#pragma unroll
-                for (int j = 0; j < 2; j++)
-                    r += M[((m == 1) + (n == 1)) * pow3(I) + ((m == 2) + (n == 2)) * pow3(K) + (j + l) * pow3(J)] * t[m][j];
-            if (n != 2) z[I][(1 << K) | (n == 1) << I | l << J] += s[K] * r;
-            if (n != 1) z[K][(1 << I) | (n == 2) << K | l << J] += s[I] * r;
-        }
+    part_end<APART>();
+    if (NEW_K) edge_weights3<T, K>(W, SK);
+    edge_product3<T>(SK, di, ri);
+    edges_to_vertices3<T, I, K, FIRST_I>(ri, s.w[K], y);
+    part_end<APART>();
+    if (NEW_I) edge_weights3<T, I>(W, SI);
+    edge_product3<T>(SI, dk, rk);
+    edges_to_vertices3<T, K, I, FIRST_K>(rk, s.w[I], y);
+    part_end<APART>();
 }
 
-// u(a, i): component i of the element's vertex a; W: the element's weights (made into its moments); s: 2 / h
-template <typename T, typename U>
-__device__ __forceinline__ void element_apply3(const U &u, T W[27], const T h2[3], T y[8][3]) {
-    T c[3][8], z[3][8];
-    const T s[3] = {(T)0.125 * h2[0], (T)0.125 * h2[1], (T)0.125 * h2[2]};
-    coefficients3<T, 0>(u, c[0]);
-    coefficients3<T, 1>(u, c[1]);
-    coefficients3<T, 2>(u, c[2]);
-    moments3<T>(W);
-#pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int m = 0; m < 8; m++) z[i][m] = (T)0;
-    normal3<T, 0>(c, W, s, z);
-    normal3<T, 1>(c, W, s, z);
-    normal3<T, 2>(c, W, s, z);
-    shear3<T, 0, 1>(c, W, s, z);
-    shear3<T, 0, 2>(c, W, s, z);
-    shear3<T, 1, 2>(c, W, s, z);
-    vertices3<T, 0>(z[0], y);
-    vertices3<T, 1>(z[1], y);
-    vertices3<T, 2>(z[2], y);
+// d u_K / d x_K with itself, which its strain holds twice
+template <bool APART, typename T, int K, typename U>
+__device__ __forceinline__ void normal3(const U &u, const T S[9], const GradScale<T> &s, T y[8][3]) {
+    T d[4], r[4] = {(T)0, (T)0, (T)0, (T)0};
+    differences3<T, K, K>(u, d);
+    edge_product3<T>(S, d, r);
+    edges_to_vertices3<T, K, K, false>(r, (T)2 * s.w[K], y);
+    part_end<APART>();
+}
+
+// u(a, i): component i of the element's vertex a
+template <bool APART, typename T, typename U>
+__device__ __forceinline__ void element_apply3(const U &u, const T W[27], const GradScale<T> &s, T y[8][3]) {
+    T S0[9], S1[9], S2[9];
+    pair3<APART, T, 0, 1, true, true, true, true>(u, W, S0, S1, s, y);
+    pair3<APART, T, 0, 2, false, true, false, true>(u, W, S0, S2, s, y);
+    normal3<APART, T, 0>(u, S0, s, y);
+    pair3<APART, T, 1, 2, false, false, true, false>(u, W, S1, S2, s, y);
+    normal3<APART, T, 1>(u, S1, s, y);
+    normal3<APART, T, 2>(u, S2, s, y);
 }
 
 // ---------------------------------------- 2D ----------------------------------------------
@@ -345,9 +398,9 @@ constexpr int CNR = (CNPD + UST_TILE - 1) / UST_TILE;
 // The element-result buffer holds a layer's results with a border of zero elements (18x18 slots per row), so that every
 // node sums its four elements per layer at fixed offsets, without a test for the column's edge (row strides of 326 to 342
 // measured alike).  With the quotients 2/h taken out of the kernel and the coarse planes of the prolongation interpolated
-// once (staged below), a layer takes 990 instead of 1400 instructions per thread in the FP32 product and 1200 instead of
-// 3150 in the prolongation pass.  128x128x64 passes, with the gather: FP32 product 42.8 -> 38 us, residual with the first
-// step 47.9 -> 44.5, prolongation pass 62.0 -> 54.8, FP64 product 73.3 -> 67.3; the column kernels now move 4.5-5.4 TB/s.
+// once (staged below), a layer took 990 instead of 1400 instructions per thread in the FP32 product and 1200 instead of
+// 3150 in the prolongation pass (with an element action of 456 operations; now 606).  128x128x64 passes then, with the
+// gather: FP32 product 42.8 -> 38 us, residual with the first step 47.9 -> 44.5, prolongation pass 62.0 -> 54.8, FP64 product 73.3 -> 67.3; the column kernels now move 4.5-5.4 TB/s.
 constexpr int EBX = UST_TX3 + 2, EBY = UST_TY3 + 2, EBS = 326;
 static_assert(EBX * EBY <= EBS && 24 * EBS * 4 % 16 == 0, "18x18 slots per row, cleared by 16-byte stores");
 
@@ -355,14 +408,13 @@ static_assert(EBX * EBY <= EBS && 24 * EBS * 4 % 16 == 0, "18x18 slots per row, 
 // weights are loaded (pf -- 1: at the start of the layer, held in registers across the element apply; 2: right after the
 // element apply, so that they are live only across the reduction and the staging; 0: when they are used), and the
 // workgroups the launch aims at, as many as the GPU then holds.  Measured at 128x128x64 (96^3), with the gather, in us:
-//   FP32 product      minb 4, pf 0, 1024: 38.9 (36.3)   2, 2, 512: 41.2 (36.7)
-//   FP32 Chebyshev    minb 2, pf 2, 1024: 49.6 (43.9)   4, 0, 1024: 49.6 (44.1; 64^3 20.7 for 19.1)   2, 2, 512: 54.7 (48.0)
+//   FP32 product      minb 4, pf 0, 1024: 42.0 (39.0)   2, 2, 512: 44.9 (39.1)   3, 2, 768: 44.0 (38.7)
+//   FP32 Chebyshev    minb 2, pf 2, 1024: 50.9 (45.2)   4, 0, 1024: 50.7 (46.0; 64^3 21.6 for 20.3)   3, 2, 768: 54.3 (47.3)
 //                     (128 registers: four per CU fit)
-//   FP32 prolongation minb 3, pf 0, 768: 53.7 (46.8)    2, 2, 512: 55.0 (49.5)   2, 0, 512: 59.0 (53.1)   2, 2, 1024: 56.4
+//   FP32 prolongation minb 3, pf 0, 768: 57.0 (49.6)    2, 2, 512: 59.3 (52.6)   3, 2, 768: 60.8 (53.6)
 //                     (four per CU exceed the LDS; with fewer than 768 workgroups of two layers the loads held in
-//                     registers are worth more than the third: 64^3 20.5 against 21.9)
-//   FP64 product      minb 2, pf 2, 512: 67.5 (55.3)    2, 0, 512: 81.6 (64.0)   2, 1, 512: 66.0 (54.6; the Chebyshev pass
-//                     109.2 for 97.2)   2, 2, 1024: 73.8 (64.7)
+//                     registers are worth more than the third: 64^3 20.5 against 21.9 with an action of 456 operations)
+//   FP64 product      minb 2, pf 2, 512: 71.6 (58.0)    2, 0, 512: 85.5 (65.9)   2, 1, 512: 143 (119; spills)
 struct ColShape {
     int minb, pf, target;
 };
@@ -381,8 +433,8 @@ static inline bool col_many(const ust_grid *gr, int tsize, int mode) {
 }
 template <typename T, typename WT, int MODE, bool MANY = false>
 __global__ __launch_bounds__(256, col_shape(sizeof(T), MODE, MANY).minb) void k_applyK3_col(
-    GridDev g, TileDiv td, const WT *__restrict__ W, const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
-    T *__restrict__ work) {
+    GridDev g, TileDiv td, GradScale<T> gs, const WT *__restrict__ W, const unsigned char *__restrict__ mask, const T *u,
+    Epi<T> ep, T *__restrict__ work) {
     __shared__ T su[2][CNPD];     // staged node planes k and k+1 (free dofs; Dirichlet dofs read 0)
     __shared__ __attribute__((aligned(16))) T eb[24 * EBS];  // the layer's results: eb[(a*3 + i)*EBS + slot]
     // EPI_PCHEBY0: a ring of two coarse node planes under the column (9x9 coarse nodes; the column's origin is
@@ -524,7 +576,6 @@ __global__ __launch_bounds__(256, col_shape(sizeof(T), MODE, MANY).minb) void k_
     // it); its value is loaded one layer ahead
     T cv = (T)0;
     if (MODE == EPI_PCHEBY0 && wpre && ((z0 + 1) & 1) == 0) cv = coarse_load(((z0 + 1) >> 1) + 1);
-    const T s[3] = {(T)g.sx, (T)g.sy, (T)g.sz};
     // two layers per turn where the next layer's operands are held in registers (FP32 product, loads when used: 38.5 us
     // against 37.9)
 #pragma unroll(held ? 2 : 1)
@@ -578,7 +629,7 @@ __global__ __launch_bounds__(256, col_shape(sizeof(T), MODE, MANY).minb) void k_
             auto ue = [&](int a, int i) -> T {
                 return (a >> 2 ? st : sb)[((a & 1) + CPX * ((a >> 1) & 1)) * 3 + i];
             };
-            element_apply3<T>(ue, wq, s, ye);
+            element_apply3<true, T>(ue, wq, gs, ye);
 #pragma unroll
             for (int a = 0; a < 8; a++)
 #pragma unroll
@@ -589,23 +640,19 @@ __global__ __launch_bounds__(256, col_shape(sizeof(T), MODE, MANY).minb) void k_
         if (!wpre) load_ops(k, zsh, ops);
         __syncthreads();
         // plane k: the carried contributions of layer k-1 plus those of layer k below the plane; the
-        // contributions of layer k above plane k+1 become the new carry.  Fixed order: elements (i-1, j-1),
-        // (i, j-1), (i-1, j), (i, j).
+        // contributions of layer k above plane k+1 become the new carry.  Fixed order, in pairs along x, then y.
         T v[CNR];
 #pragma unroll
         for (int r = 0; r < CNR; r++) {
-            T lo = (T)0, hi = (T)0;
+            T lo[4], hi[4];
 #pragma unroll
-            for (int dy = 1; dy >= 0; dy--)
-#pragma unroll
-                for (int dx = 1; dx >= 0; dx--) {
-                    const int a = dx + 2 * dy;
-                    const T *e = eb + rofs[r] - dx - EBX * dy;
-                    lo += e[a * 3 * EBS];
-                    hi += e[(a + 4) * 3 * EBS];
-                }
-            v[r] = carry[r] + lo;
-            carry[r] = hi;
+            for (int a = 0; a < 4; a++) {
+                const T *e = eb + rofs[r] - (a & 1) - EBX * (a >> 1);
+                lo[a] = e[a * 3 * EBS];
+                hi[a] = e[(a + 4) * 3 * EBS];
+            }
+            v[r] = carry[r] + ((lo[3] + lo[2]) + (lo[1] + lo[0]));
+            carry[r] = (hi[3] + hi[2]) + (hi[1] + hi[0]);
         }
         finish(k, k - z0, zsh, su[cur], ops, v);
     }
@@ -625,7 +672,8 @@ __global__ __launch_bounds__(256, col_shape(sizeof(T), MODE, MANY).minb) void k_
 // through the workspace.
 // ------------------------------------------------------------------------------------------
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, TileDiv td, const WT *__restrict__ W,
+__global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, TileDiv td, GradScale<T> gs,
+                                                       const WT *__restrict__ W,
                                                        const unsigned char *__restrict__ mask, const T *u,
                                                        Epi<T> ep, T *__restrict__ work) {
     constexpr int TX = UST_TTX3, TY = UST_TTY3, TZ = UST_TTZ3;
@@ -707,15 +755,10 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, TileDiv td,
 #pragma unroll
             for (int q = 0; q < 27; q++) wq[q] = wload<T, WT>(W, ((size_t)tile * 27 + q) * UST_TILE + threadIdx.x);
         }
-        T ue[8][3];
-#pragma unroll
-        for (int a = 0; a < 8; a++) {
-            const int ln = (lx + (a & 1)) + NX * ((ly + ((a >> 1) & 1)) + NY * (lz + (a >> 2)));
-#pragma unroll
-            for (int i = 0; i < 3; i++) ue[a][i] = su[ln * 3 + i];
-        }
-        const T s[3] = {(T)g.sx, (T)g.sy, (T)g.sz};
-        element_apply3<T>([&](int a, int i) -> T { return ue[a][i]; }, wq, s, ye);
+        const T *sb = &su[(lx + NX * (ly + NY * lz)) * 3];
+        element_apply3<false, T>([&](int a, int i) -> T {
+            return sb[((a & 1) + NX * (((a >> 1) & 1) + NY * (a >> 2))) * 3 + i];
+        }, wq, gs, ye);
     }
     // Wave w holds the element layer lz = w, whose nodes are layers w and w+1: even waves never share a
     // node, nor do odd waves, and within one LDS add the 64 lanes hit 64 distinct nodes.  Adding in two
@@ -830,8 +873,17 @@ __device__ __forceinline__ void block_dot(double v, double *out) {
     if (threadIdx.x == 0) out[blockIdx.x] = (sh[0] + sh[1]) + (sh[2] + sh[3]);
 }
 
+// the contributions v(a) of the elements that have a node as vertex a, in pairs along x, then y, then z: fewer roundings than
+// one after the other, and no more operations
+template <typename V>
+__device__ __forceinline__ double vertex_sum3(V v) {
+    const double lo = (v(3) + v(2)) + (v(1) + v(0)), hi = (v(7) + v(6)) + (v(5) + v(4));
+    return hi + lo;
+}
+
 template <typename T, typename WT, int MODE>
-__global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, const WT *__restrict__ W,
+__global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, GradScale<T> gs,
+                                                      const WT *__restrict__ W,
                                                       const unsigned char *__restrict__ mask, const T *u, Epi<T> ep,
                                                       CgDir<T> cg) {
     __shared__ T su[HNN * 3];   // staged node block, origin (nx0 - 1, ny0 - 1, nz0 - 1)
@@ -915,11 +967,10 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, con
     __syncthreads();
     if (tid < HNE) {
         T ye[8][3];
-        const T s[3] = {(T)g.sx, (T)g.sy, (T)g.sz};
         const T *sb = &su[(lx + HNX * (ly + HNY * lz)) * 3];
-        element_apply3<T>([&](int a, int i) -> T {
+        element_apply3<false, T>([&](int a, int i) -> T {
             return sb[((a & 1) + HNX * (((a >> 1) & 1) + HNY * (a >> 2))) * 3 + i];
-        }, wq, s, ye);
+        }, wq, gs, ye);
 #pragma unroll
         for (int a = 0; a < 8; a++)
 #pragma unroll
@@ -933,15 +984,10 @@ __global__ __launch_bounds__(256) void k_applyK3_halo(GridDev g, TileDiv td, con
         if (!inside || (r && tid >= HOX * HOY * HOZ)) continue;
         const int c = r ? 2 : tid / (HOX * HOY * HOZ);
         const T us = su[((ox + 1) + HNX * ((oy + 1) + HNY * (oz + 1))) * 3 + c];
-        double v = 0.0;
-#pragma unroll
-        for (int dz = 1; dz >= 0; dz--)
-#pragma unroll
-            for (int dy = 1; dy >= 0; dy--)
-#pragma unroll
-                for (int dx = 1; dx >= 0; dx--)  // element slot (ox + 1 - dx, ...) has this node as vertex (dx, dy, dz)
-                    v += (double)eb[((dx + 2 * dy + 4 * dz) * 3 + c) * HNE + (ox + 1 - dx) +
-                                    HEX * ((oy + 1 - dy) + HEY * (oz + 1 - dz))];
+        const double v = vertex_sum3([&](int a) {  // element slot (ox + 1 - dx, ...) has this node as vertex (dx, dy, dz)
+            return (double)eb[(a * 3 + c) * HNE + (ox + 1 - (a & 1)) + HEX * ((oy + 1 - ((a >> 1) & 1)) +
+                                                                              HEY * (oz + 1 - (a >> 2)))];
+        });
         EpiOps<T> o = ops[r];
         if (MODE == EPI_PCHEBY0 && !o.m) o.x = us;  // x + P xc, as staged
         const T out = epilogue_store<MODE, T>(ep, o, odof + c, (T)v);
@@ -1331,7 +1377,7 @@ constexpr int F3E = F3EX * F3EY * F3EZ, F3R = F3RX * F3RY * F3RZ, F3S = F3SX * F
 static_assert(F3E <= F3T && F3R * 3 <= 2 * F3T && F3S <= 2 * F3T, "288 elements, 525 residual dofs, 441 nodes");
 
 template <typename T, typename WT, int KIND>
-__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, const WT *__restrict__ W,
+__global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, GradScale<T> gs, const WT *__restrict__ W,
                                               const unsigned char *__restrict__ mask,
                                               const unsigned char *__restrict__ maskc, const T *__restrict__ u,
                                               const T *__restrict__ b, const T *__restrict__ invd, T *__restrict__ d,
@@ -1397,11 +1443,10 @@ __global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, const WT *_
     __syncthreads();
     if (tid < F3E) {
         T ye[8][3];
-        const T s[3] = {(T)g.sx, (T)g.sy, (T)g.sz};
         const T *sb = &su[(lx + F3SX * (ly + F3SY * lz)) * 3];
-        element_apply3<T>([&](int a, int q) -> T {
+        element_apply3<false, T>([&](int a, int q) -> T {
             return sb[((a & 1) + F3SX * (((a >> 1) & 1) + F3SY * (a >> 2))) * 3 + q];
-        }, wq, s, ye);
+        }, wq, gs, ye);
 #pragma unroll
         for (int a = 0; a < 8; a++)
 #pragma unroll
@@ -1413,15 +1458,10 @@ __global__ __launch_bounds__(F3T) void k_pre3(GridDev g, TileDiv td, const WT *_
         const int t = tid + F3T * r;
         if (t >= F3R * 3) continue;
         const int c = t / F3R, n = t % F3R, i = n % F3RX, j = (n / F3RX) % F3RY, k = n / (F3RX * F3RY);
-        double v = 0.0;
-#pragma unroll
-        for (int dz = 1; dz >= 0; dz--)
-#pragma unroll
-            for (int dy = 1; dy >= 0; dy--)
-#pragma unroll
-                for (int dx = 1; dx >= 0; dx--)
-                    v += (double)eb[((dx + 2 * dy + 4 * dz) * 3 + c) * EB + (i + 1 - dx) +
-                                    F3EX * ((j + 1 - dy) + F3EY * (k + 1 - dz))];
+        const double v = vertex_sum3([&](int a) {
+            return (double)eb[(a * 3 + c) * EB + (i + 1 - (a & 1)) + F3EX * ((j + 1 - ((a >> 1) & 1)) +
+                                                                           F3EY * (k + 1 - (a >> 2)))];
+        });
         sr[n * 3 + c] = rin[r] && !rm[r] ? rb[r] - (T)v : (T)0;
         // x = the first step, on the nodes 2 I0 .. 2 I0 + 5 and so on, each of one workgroup
         if (KIND == PRE_FIRST && rin[r] && i >= 1 && j >= 1 && k >= 1) d[rk[r]] = c2 * ri[r] * rb[r];
@@ -1471,7 +1511,7 @@ static int fused_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
                                                 : tile_div((cnx + F3X - 1) / F3X, (cny + F3Y - 1) / F3Y);
 #define PRE2(KIND) hipLaunchKernelGGL((k_pre2<T, WT, KIND>), grid, dim3(UST_TILE), 0, st, g, td, W, p->mask, p->maskc, u, b, \
                                       invd, y, d, bc, c0, c1, c2)
-#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, td, W, p->mask, p->maskc, u, b, invd, \
+#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, td, grad_scale<T>(g), W, p->mask, p->maskc, u, b, invd, \
                                       d, bc, c2)
     if (mode == UST_PASS_PCHEBY2)
         hipLaunchKernelGGL((k_post2<T, WT>), grid, dim3(UST_TILE), 0, st, g, td, W, p->mask, u, (const T *)p->xc, b, invd, y,
@@ -1690,7 +1730,7 @@ static int apply_halo(const GridDev &g, const WT *W, const unsigned char *mask, 
                       hipStream_t st, const CgDir<T> &cg = {}) {
     if (g.dim == 3)
         hipLaunchKernelGGL((k_applyK3_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g,
-                           tile_div((g.nnx + HOX - 1) / HOX, (g.nny + HOY - 1) / HOY), W, mask, u, ep, cg);
+                           tile_div((g.nnx + HOX - 1) / HOX, (g.nny + HOY - 1) / HOY), grad_scale<T>(g), W, mask, u, ep, cg);
     else
         hipLaunchKernelGGL((k_applyK2_halo<T, WT, MODE>), dim3(halo_tiles(g)), dim3(UST_TILE), 0, st, g,
                            tile_div((g.nnx + H2O - 1) / H2O, (g.nny + H2O - 1) / H2O), W, mask, u, ep, cg);
@@ -1715,18 +1755,19 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
     // product or a residual in place, a first step over its right-hand side), which tiles + gather allow
     if (halo_grid(g) && ep.y != u && (MODE != EPI_RES0 || ep.d != ep.b)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
     if (g.dim == 3) {
+        const GradScale<T> gs = grad_scale<T>(g);
         if (g.col) {
             if constexpr (sizeof(T) == 4 && MODE == EPI_PCHEBY0)
                 if (many)
-                    hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE, true>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W,
-                                       mask, u, ep, work);
+                    hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE, true>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, gs,
+                                       W, mask, u, ep, work);
             if (!many)
-                hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u,
-                                   ep, work);
+                hipLaunchKernelGGL((k_applyK3_col<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, gs, W,
+                                   mask, u, ep, work);
             gather_tiles<T, 3, MODE, true>(g, mask, work, ep, st);
         } else {
-            hipLaunchKernelGGL((k_applyK3_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, W, mask, u,
-                               ep, work);
+            hipLaunchKernelGGL((k_applyK3_tiled<T, WT, MODE>), dim3(g.ntiles), dim3(UST_TILE), 0, st, g, td, gs, W, mask,
+                               u, ep, work);
             gather_tiles<T, 3, MODE, false>(g, mask, work, ep, st);
         }
     } else {

@@ -997,3 +997,46 @@ def test_passes_in_place(dim, nel, prec):
     w32.free()
     ws.free()
     s.close()
+
+
+# one element of the halo, tile and column kernels: inside, on the grid's corner, beside a tile's edge
+@pytest.mark.parametrize("nel,elements", [((17, 9, 5), [(0, 0, 0), (8, 4, 3), (16, 8, 4)]),
+                                          ((64, 40, 30), [(15, 3, 4), (16, 20, 29)]),
+                                          ((33, 33, 130), [(15, 16, 64), (32, 5, 129)])])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_rounding_of_the_product_is_local(nel, elements, prec):
+    """An element whose only weight sits on one of its corners moves that vertex and the three joined to it by edges; the
+    test functions of the other four have no gradient there.  No bar: the product rounds each vertex's result by what that
+    vertex receives, so theirs is exactly zero.  Rounded against the element's largest sums, it would be 1e-7 (1e-16) of
+    them, and the error of every product larger by what the small contributions lose."""
+    import ctypes as C
+    import earthbyte_underworld_amd as ust  # noqa: F401  (loads the library)
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    g = _grid(3, nel)
+    T = np.float64 if prec == "f64" else np.float32
+    nn = [k + 1 for k in nel]
+    n, wl = int(np.prod(nn)) * 3, lib.ust_k_weights_len(C.byref(g))
+    u = np.random.default_rng(8).normal(size=n).astype(T)
+    du, dy, dm, dw = _Dev(lib, u), _Dev(lib, u), _Dev(lib, np.zeros(n, np.uint8)), _Dev(lib, np.zeros(wl, T))
+    work = _Dev(lib, np.zeros(lib.ust_k_apply_work_len(C.byref(g)), T))
+    apply_K = getattr(lib, f"ust_k_apply_K_{prec}")
+    value = np.array([0.7], T)
+    for e in elements:
+        eid = e[0] + nel[0] * (e[1] + nel[1] * e[2])
+        for corner in range(8):
+            bits = [(corner >> k) & 1 for k in range(3)]
+            slot = lib.ust_k_weights_index(C.byref(g), eid, 2 * bits[0] + 6 * bits[1] + 18 * bits[2])
+            at = C.c_void_p(dw.p.value + slot * value.itemsize)
+            assert lib.ust_memcpy_h2d(at, value.ctypes.data_as(C.c_void_p), value.nbytes, None) == 0
+            assert apply_K(C.byref(g), dw.p, dm.p, du.p, dy.p, work.p, None) == 0
+            zero = np.zeros(1, T)
+            assert lib.ust_memcpy_h2d(at, zero.ctypes.data_as(C.c_void_p), zero.nbytes, None) == 0
+            y = dy.get().reshape(-1, 3)
+            moved = np.zeros(len(y), bool)
+            for a in [corner] + [corner ^ (1 << k) for k in range(3)]:
+                i = [e[k] + ((a >> k) & 1) for k in range(3)]
+                moved[i[0] + nn[0] * (i[1] + nn[1] * i[2])] = True
+            assert np.all(np.any(y[moved] != 0, axis=1)) and not y[~moved].any()
+    for d in (du, dy, dm, dw, work):
+        d.free()
