@@ -15,10 +15,37 @@ static void dfree(void **p) {
 }
 #define DFREE(x) dfree((void **)&(x))
 
+/* Blocks kept for the particle half of the next time step.  A step at 96^3 elements x 30 particles allocates and frees 30
+ * arrays of 27 to 640 MB, of which hipFree took 6.8 ms and hipMalloc 2 ms of 67 (57.5 with the blocks kept).  A freed block
+ * of 1 MiB or more stays with its context, for the next request of up to its size and no less than four fifths of it
+ * (swarm_malloc, swarm_free); the idle ones are held to 256 bytes per particle (about what a step takes beside the swarm
+ * itself), the oldest given back first.  All of them are given back with the swarm, and when any device allocation of the
+ * context fails, which is then tried again (ctx_malloc).  All work on them is on the context's one stream, so a block handed
+ * on is in order behind its last use. */
+static void pool_trim(ust_context *ctx, size_t keep) {
+    for (int i = 0; i < ctx->npool && ctx->pool_idle > keep;) {
+        if (ctx->pool[i].live) {
+            i++;
+            continue;
+        }
+        ctx->pool_idle -= ctx->pool[i].bytes;
+        ust_dev_free(ctx->pool[i].p);
+        memmove(&ctx->pool[i], &ctx->pool[i + 1], (size_t)(ctx->npool - i - 1) * sizeof(ctx->pool[0]));
+        ctx->npool--;
+    }
+}
+
+static int ctx_malloc(ust_context *ctx, void **p, size_t bytes) {
+    int rc = ust_dev_malloc(p, bytes);
+    if (rc == UST_OK || !ctx->pool_idle) return rc;
+    pool_trim(ctx, 0);
+    return ust_dev_malloc(p, bytes);
+}
+
 int ust_dev_alloc_zero(ust_context *ctx, void **p, size_t bytes) {
     /* round up to whole doubles so that the zero fill stays inside the allocation */
     const size_t ab = (bytes + 7) & ~(size_t)7;
-    int rc = ust_dev_malloc(p, ab);
+    int rc = ctx_malloc(ctx, p, ab);
     if (rc != UST_OK) UST_FAIL(ctx, rc, "device allocation of %zu bytes failed: %s", ab, ust_dev_error_string());
     CKD(ctx, ust_k_fill_f64((double *)*p, 0.0, ab / 8, ctx->stream));
     return UST_OK;
@@ -111,28 +138,9 @@ static void free_mesh_data(ust_context *ctx) {
     ctx->assembled = 0;
 }
 
-/* Blocks kept for the particle half of the next time step.  A step at 96^3 elements x 30 particles allocates and frees 30
- * arrays of 27 to 640 MB, of which hipFree took 6.8 ms and hipMalloc 2 ms of 67 (57.5 with the blocks kept).  A freed block of 1 MiB or more stays with
- * its context, for the next request of up to its size and no less than four fifths of it; the idle ones are held to 256
- * bytes per particle (about what a step takes beside the swarm itself), the oldest given back first, and all of them are
- * given back with the swarm, or when an allocation fails.  All work on them is on the context's one stream, so a block
- * handed on is in order behind its last use. */
-static void pool_trim(ust_context *ctx, size_t keep) {
-    for (int i = 0; i < ctx->npool && ctx->pool_idle > keep;) {
-        if (ctx->pool[i].live) {
-            i++;
-            continue;
-        }
-        ctx->pool_idle -= ctx->pool[i].bytes;
-        ust_dev_free(ctx->pool[i].p);
-        memmove(&ctx->pool[i], &ctx->pool[i + 1], (size_t)(ctx->npool - i - 1) * sizeof(ctx->pool[0]));
-        ctx->npool--;
-    }
-}
-
 static int swarm_malloc(ust_context *ctx, void **p, size_t bytes) {
     *p = NULL;
-    if (bytes < ((size_t)1 << 20)) return ust_dev_malloc(p, bytes);
+    if (bytes < ((size_t)1 << 20)) return ctx_malloc(ctx, p, bytes);
     int best = -1;
     for (int i = 0; i < ctx->npool; i++)
         if (!ctx->pool[i].live && ctx->pool[i].bytes >= bytes && ctx->pool[i].bytes / 5 * 4 <= bytes &&
@@ -145,12 +153,7 @@ static int swarm_malloc(ust_context *ctx, void **p, size_t bytes) {
         return UST_OK;
     }
     const size_t take = bytes + bytes / 16; /* the particle count moves a little from step to step */
-    int rc = ust_dev_malloc(p, take);
-    if (rc) {
-        pool_trim(ctx, 0);
-        rc = ust_dev_malloc(p, take);
-    }
-    if (rc) return ust_dev_malloc(p, bytes);
+    if (ctx_malloc(ctx, p, take)) return ctx_malloc(ctx, p, bytes);
     if (ctx->npool == UST_POOL_BLOCKS) pool_trim(ctx, 0);
     if (ctx->npool < UST_POOL_BLOCKS) { /* else: freed as any other block */
         ctx->pool[ctx->npool].p = *p;
@@ -473,11 +476,11 @@ int ust_swarm_upload(ust_context *ctx, int np, const int *cell_off, const double
     }
     void *d_off = NULL, *d_xi = NULL, *d_w = NULL, *d_m = NULL, *d_c = NULL;
     int rc = UST_OK;
-    rc = ust_dev_malloc(&d_off, (size_t)(ctx->nel + 1) * sizeof(int));
-    if (!rc) rc = ust_dev_malloc(&d_xi, 3 * n * sizeof(double) + 8);
-    if (!rc) rc = ust_dev_malloc(&d_w, n * sizeof(double) + 8);
-    if (!rc && material) rc = ust_dev_malloc(&d_m, n + 8);
-    if (!rc && coh_scale) rc = ust_dev_malloc(&d_c, n * sizeof(float) + 8);
+    rc = ctx_malloc(ctx, &d_off, (size_t)(ctx->nel + 1) * sizeof(int));
+    if (!rc) rc = ctx_malloc(ctx, &d_xi, 3 * n * sizeof(double) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &d_w, n * sizeof(double) + 8);
+    if (!rc && material) rc = ctx_malloc(ctx, &d_m, n + 8);
+    if (!rc && coh_scale) rc = ctx_malloc(ctx, &d_c, n * sizeof(float) + 8);
     if (!rc) rc = ust_memcpy_h2d(d_off, cell_off, (size_t)(ctx->nel + 1) * sizeof(int), ctx->stream);
     if (!rc) rc = ust_memcpy_h2d(d_xi, soa, 3 * n * sizeof(double), ctx->stream);
     if (!rc) rc = ust_memcpy_h2d(d_w, w, n * sizeof(double), ctx->stream);
@@ -794,7 +797,7 @@ int ust_get_element_matrices(ust_context *ctx, int first, int count, double *Ke)
     double *buf = NULL;
     int bs = count < UST_BATCH ? count : UST_BATCH;
     if (bs == 0) return UST_OK;
-    CKD(ctx, ust_dev_malloc((void **)&buf, (size_t)bs * nd * nd * sizeof(double)));
+    CKD(ctx, ctx_malloc(ctx, (void **)&buf, (size_t)bs * nd * nd * sizeof(double)));
     for (int s = 0; s < count; s += bs) {
         int c = count - s < bs ? count - s : bs;
         rc = ust_k_element_matrices(&ctx->grid, ctx->WK, first + s, c, buf, ctx->stream);
@@ -813,7 +816,7 @@ static int get_elem_vec(ust_context *ctx, int first, int count, double *out, int
     if (count == 0) return UST_OK;
     int nd = (1 << ctx->grid.dim) * ctx->grid.dim;
     double *buf = NULL;
-    CKD(ctx, ust_dev_malloc((void **)&buf, (size_t)count * nd * sizeof(double)));
+    CKD(ctx, ctx_malloc(ctx, (void **)&buf, (size_t)count * nd * sizeof(double)));
     if (which == 0) rc = ust_k_element_G(&ctx->grid, ctx->WG, first, count, buf, ctx->stream);
     else {
         double dir[3];
@@ -910,8 +913,8 @@ int ust_apply_K_f32_dev(ust_context *ctx, const float *u, float *y) {
 int ust_apply_K_f32(ust_context *ctx, const float *u, float *y) {
     size_t n = (size_t)ctx->ndof;
     float *a = NULL, *b = NULL;
-    CKD(ctx, ust_dev_malloc((void **)&a, n * sizeof(float)));
-    int rc = ust_dev_malloc((void **)&b, n * sizeof(float));
+    CKD(ctx, ctx_malloc(ctx, (void **)&a, n * sizeof(float)));
+    int rc = ctx_malloc(ctx, (void **)&b, n * sizeof(float));
     if (!rc) rc = ust_memcpy_h2d(a, u, n * sizeof(float), ctx->stream);
     if (!rc) rc = ust_apply_K_f32_dev(ctx, a, b);
     if (!rc) rc = ust_memcpy_d2h(y, b, n * sizeof(float), ctx->stream);
@@ -934,8 +937,8 @@ static int host_op(ust_context *ctx, const double *in, size_t nin, double *out, 
     int rc = need_assembled(ctx);
     if (rc) return rc;
     double *a = NULL, *b = NULL;
-    CKD(ctx, ust_dev_malloc((void **)&a, nin * sizeof(double)));
-    rc = ust_dev_malloc((void **)&b, nout * sizeof(double));
+    CKD(ctx, ctx_malloc(ctx, (void **)&a, nin * sizeof(double)));
+    rc = ctx_malloc(ctx, (void **)&b, nout * sizeof(double));
     if (!rc) rc = ust_memcpy_h2d(a, in, nin * sizeof(double), ctx->stream);
     if (!rc) {
         if (which == 0) rc = ust_k_apply_K_f64(&ctx->grid, ctx->WK, ctx->mask_d, a, b, (double *)ctx->kwork, ctx->stream);
@@ -1053,15 +1056,15 @@ int ust_swarm_spacefiller(ust_context *ctx, double avg_ppc) {
     void *key = NULL, *key_s = NULL, *perm = NULL, *perm_t = NULL, *nxi = NULL, *work = NULL, *off = NULL;
     void *oxi = NULL, *ow = NULL;
     int rc = UST_OK, max_ppc = 0;
-    if (!rc) rc = ust_dev_malloc(&key, n * sizeof(unsigned) + 8);
-    if (!rc) rc = ust_dev_malloc(&key_s, n * sizeof(unsigned) + 8);
-    if (!rc) rc = ust_dev_malloc(&perm, n * sizeof(unsigned) + 8);
-    if (!rc) rc = ust_dev_malloc(&perm_t, n * sizeof(unsigned) + 8);
-    if (!rc) rc = ust_dev_malloc(&nxi, 3 * n * sizeof(double) + 8);
-    if (!rc) rc = ust_dev_malloc(&work, wb + 8);
-    if (!rc) rc = ust_dev_malloc(&off, (size_t)(nel + 1) * sizeof(int));
-    if (!rc) rc = ust_dev_malloc(&oxi, 3 * n * sizeof(double) + 8);
-    if (!rc) rc = ust_dev_malloc(&ow, n * sizeof(double) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &key, n * sizeof(unsigned) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &key_s, n * sizeof(unsigned) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &perm, n * sizeof(unsigned) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &perm_t, n * sizeof(unsigned) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &nxi, 3 * n * sizeof(double) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &work, wb + 8);
+    if (!rc) rc = ctx_malloc(ctx, &off, (size_t)(nel + 1) * sizeof(int));
+    if (!rc) rc = ctx_malloc(ctx, &oxi, 3 * n * sizeof(double) + 8);
+    if (!rc) rc = ctx_malloc(ctx, &ow, n * sizeof(double) + 8);
     double *n0 = (double *)nxi, *n1 = n0 + n, *n2 = n0 + 2 * n;
     double *o0 = (double *)oxi, *o1 = o0 + n, *o2 = o0 + 2 * n;
     if (!rc) rc = ust_k_spacefiller_layout(&ctx->grid, np, &dirs[0][0], (unsigned *)key, n0, n1, n2, ctx->stream);
@@ -1101,7 +1104,7 @@ int ust_swarm_assign_materials(ust_context *ctx, int nshape, const ust_shape *sh
     void *d_sh = NULL, *d_cm = NULL;
     int rc = UST_OK;
     if (nshape) {
-        rc = ust_dev_malloc(&d_sh, sizeof(ust_shape) * (size_t)nshape);
+        rc = ctx_malloc(ctx, &d_sh, sizeof(ust_shape) * (size_t)nshape);
         if (!rc) rc = ust_memcpy_h2d(d_sh, shapes, sizeof(ust_shape) * (size_t)nshape, ctx->stream);
     }
     if (!rc && cell_material) {
@@ -1110,7 +1113,7 @@ int ust_swarm_assign_materials(ust_context *ctx, int nshape, const ust_shape *sh
                 ust_dev_free(d_sh);
                 UST_FAIL(ctx, UST_EINVAL, "cell %d names material %d (only %d defined)", e, cell_material[e], ctx->nmat);
             }
-        rc = ust_dev_malloc(&d_cm, (size_t)ctx->nel);
+        rc = ctx_malloc(ctx, &d_cm, (size_t)ctx->nel);
         if (!rc) rc = ust_memcpy_h2d(d_cm, cell_material, (size_t)ctx->nel, ctx->stream);
     }
     if (!rc)
@@ -1134,7 +1137,7 @@ int ust_swarm_assign_materials_field(ust_context *ctx, const float *field_nodal,
     if (!ctx->mat) DALLOC(ctx, ctx->mat, (size_t)ctx->np);
     void *d_f = NULL;
     const size_t nb = (size_t)ctx->nnodes * sizeof(float);
-    int rc = ust_dev_malloc(&d_f, nb);
+    int rc = ctx_malloc(ctx, &d_f, nb);
     if (!rc) rc = ust_memcpy_h2d(d_f, field_nodal, nb, ctx->stream);
     if (!rc)
         rc = ust_k_assign_materials_field(&ctx->grid, ctx->cell_off, ctx->np, ctx->xi0, ctx->xi1, ctx->xi2,
