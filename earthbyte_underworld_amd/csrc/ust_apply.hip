@@ -864,6 +864,17 @@ __host__ __device__ inline int halo_tiles(const GridDev &g) {
 }
 static inline bool halo_grid(const GridDev &g) { return g.dim == 2 || (!g.col && g.nel <= UST_HALO_MAX_NEL); }
 
+// whether a pass writes a vector that it stages, at nodes that other workgroups own: u, or for the steps from zero b and
+// invd, and the coarse correction.  (Those an owned node alone reads may be written over.)
+template <int MODE, typename T>
+static inline bool writes_staged(const Epi<T> &ep, const T *u) {
+    const bool zero = MODE == EPI_RES0 || MODE == EPI_CHEBY1;
+    const T *staged[3] = {zero ? ep.b : u, zero ? ep.invd : nullptr, MODE == EPI_PCHEBY0 ? ep.xc : nullptr};
+    for (const T *v : staged)
+        if (v && (ep.y == v || ep.d == v)) return true;
+    return false;
+}
+
 // the workgroup's sum of v into out[block]
 __device__ __forceinline__ void block_dot(double v, double *out) {
     __shared__ double sh[4];
@@ -1501,9 +1512,19 @@ static int fused_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
     if (mode != UST_PASS_RESR && !invd) return UST_EINVAL;
     if (mode != UST_PASS_PCHEBY2 && (!bc || !p->maskc)) return UST_EINVAL;
     if ((mode == UST_PASS_RESR || mode == UST_PASS_PCHEBY2) && !u) return UST_EINVAL;
-    if (mode == UST_PASS_RES0R && (!d || d == b)) return UST_EINVAL;
-    if (mode == UST_PASS_CHEBY1R && (!y || y == b)) return UST_EINVAL;
-    if (mode == UST_PASS_PCHEBY2 && (!y || y == u || !p->xc)) return UST_EINVAL;
+    if (mode == UST_PASS_RES0R && !d) return UST_EINVAL;
+    if (mode == UST_PASS_CHEBY1R && !y) return UST_EINVAL;
+    if (mode == UST_PASS_PCHEBY2 && (!y || !p->xc)) return UST_EINVAL;
+    // every vector read is read at nodes that other workgroups own, and what is written is written once
+    const bool from_u = mode == UST_PASS_RESR || mode == UST_PASS_PCHEBY2, post = mode == UST_PASS_PCHEBY2;
+    const void *in[4] = {b, from_u ? u : nullptr, mode == UST_PASS_RESR ? nullptr : invd, post ? p->xc : nullptr};
+    const void *out[3] = {post || mode == UST_PASS_CHEBY1R ? y : nullptr,
+                          mode == UST_PASS_RES0R || mode == UST_PASS_CHEBY1R ? d : nullptr, post ? nullptr : bc};
+    for (int i = 0; i < 3; i++) {
+        for (int k = 0; k < 4; k++)
+            if (out[i] && out[i] == in[k]) return UST_EINVAL;
+        if (out[i] && out[i] == out[(i + 1) % 3]) return UST_EINVAL;
+    }
     const dim3 grid(fused_groups(g, mode));
     const int cnx = g.nx / 2 + 1, cny = g.ny / 2 + 1;
     const TileDiv td = mode == UST_PASS_PCHEBY2 ? tile_div((g.nnx + F2R - 1) / F2R, (g.nny + F2R - 1) / F2R)
@@ -1753,7 +1774,7 @@ static int apply_tiled(const ust_grid *gr, const WT *W, const unsigned char *mas
     hipStream_t st = ust_stream(stream);
     // small 3D grids and 2D ones: the halo kernel, unless the pass overwrites what its neighbours stage (a Chebyshev step, a
     // product or a residual in place, a first step over its right-hand side), which tiles + gather allow
-    if (halo_grid(g) && ep.y != u && (MODE != EPI_RES0 || ep.d != ep.b)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
+    if (halo_grid(g) && !writes_staged<MODE>(ep, u)) return apply_halo<T, WT, MODE>(g, W, mask, u, ep, st);
     if (g.dim == 3) {
         const GradScale<T> gs = grad_scale<T>(g);
         if (g.col) {
@@ -1832,25 +1853,29 @@ static int halo_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
     Epi<T> ep = {y, b, invd, d, (T)p->c1, (T)p->c2, xc, u, (T)p->c0, p->d_last != 0, p->dot};
     if (!W || !p->mask || !y) return UST_EINVAL;
     const bool reads_u = p->mode != UST_PASS_RES0 && p->mode != UST_PASS_CHEBY1;
-    if (reads_u && (!u || u == y)) return UST_EINVAL;  // out of place
+    if (reads_u && !u) return UST_EINVAL;
     if (p->mode != UST_PASS_Y && !b) return UST_EINVAL;
     if (p->mode >= UST_PASS_CHEBY && !invd) return UST_EINVAL;
     if (!reads_u) u = b;  // not read
+    if (p->mode <= UST_PASS_RES) ep.d = nullptr;  // not written
+    // out of place
+#define HALO(MODE) return writes_staged<MODE>(ep, u) ? UST_EINVAL : apply_halo<T, WT, MODE>(g, W, p->mask, u, ep, st)
     switch (p->mode) {
-        case UST_PASS_Y: return apply_halo<T, WT, EPI_Y>(g, W, p->mask, u, ep, st);
-        case UST_PASS_RES: return apply_halo<T, WT, EPI_RES>(g, W, p->mask, u, ep, st);
+        case UST_PASS_Y: HALO(EPI_Y);
+        case UST_PASS_RES: HALO(EPI_RES);
         case UST_PASS_CHEBY:
             if (!d) return UST_EINVAL;
-            return apply_halo<T, WT, EPI_CHEBY>(g, W, p->mask, u, ep, st);
-        case UST_PASS_CHEBY0: return apply_halo<T, WT, EPI_CHEBY0>(g, W, p->mask, u, ep, st);
+            HALO(EPI_CHEBY);
+        case UST_PASS_CHEBY0: HALO(EPI_CHEBY0);
         case UST_PASS_PCHEBY0:
             if (!xc || g.nx % 2 || g.ny % 2 || (g.dim == 3 && g.nz % 2)) return UST_EINVAL;
-            return apply_halo<T, WT, EPI_PCHEBY0>(g, W, p->mask, u, ep, st);
+            HALO(EPI_PCHEBY0);
         case UST_PASS_RES0:
             if (!d) return UST_EINVAL;
-            return apply_halo<T, WT, EPI_RES0>(g, W, p->mask, u, ep, st);
-        case UST_PASS_CHEBY1: return apply_halo<T, WT, EPI_CHEBY1>(g, W, p->mask, u, ep, st);
+            HALO(EPI_RES0);
+        case UST_PASS_CHEBY1: HALO(EPI_CHEBY1);
     }
+#undef HALO
     return UST_EINVAL;
 }
 

@@ -281,7 +281,10 @@ int ust_k_dvc_weights(int dim, const int *res, int nel, const int *cell_off, int
 int ust_k_dvc_weights_of(int dim, const int *res, int n, const int *elems, const int *cell_off, int max_np, double *xi0,
                          double *xi1, double *xi2, double *w, int set_centroids, int *flag, void *stream);
 
-/* --- passes of K in one launch, out of place (2D grids and small 3D ones) --- */
+/* --- passes of K in one launch, out of place (2D grids and small 3D ones) ---
+ * A workgroup reads nodes that others own, so a vector that is written there may not be one that is read: y and d not u
+ * (modes 0-4), not b or invd (modes 5, 6), not xc (mode 4); in modes 7-10 y, d and bc none of the vectors read, nor each
+ * other.  Such a call is refused. */
 #define UST_PASS_Y 0       /* y = K u */
 #define UST_PASS_RES 1     /* y = b - K u, 0 on the Dirichlet dofs */
 #define UST_PASS_CHEBY 2   /* d = c1 d + c2 invd (b - K u), y = u + d */

@@ -119,3 +119,31 @@ def test_undeclared_entry_points_are_refused():
     for n in undeclared[:5]:
         with pytest.raises(AttributeError, match="no signature declared"):
             getattr(lib, n)
+
+
+def test_one_launch_passes_refuse_what_they_would_overwrite():
+    """Workgroups of a one-launch pass read nodes that others own, so each mode refuses an output that is a vector it reads
+    there (the call returns before it looks at a pointer's target: the addresses here are not memory)."""
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    names = ["W", "mask", "u", "y", "b", "invd", "d", "xc", "bc", "maskc"]
+    at = {k: 4096 * (i + 1) for i, k in enumerate(names)}
+    refused = {0: ["y=u"], 1: ["y=u"], 2: ["y=u", "d=u"], 3: ["y=u", "d=u"], 4: ["y=u", "d=u", "y=xc", "d=xc"],
+               5: ["y=b", "y=invd", "d=b", "d=invd"], 6: ["y=b", "y=invd", "d=b", "d=invd"], 7: ["bc=u", "bc=b"],
+               8: ["d=b", "d=invd", "bc=b", "bc=invd", "bc=d"],
+               9: ["y=b", "y=invd", "d=b", "d=invd", "bc=b", "bc=invd", "bc=d", "bc=y", "d=y"],
+               10: ["y=u", "y=b", "y=invd", "y=xc"]}
+    for dim in (2, 3):
+        g = L.Grid()
+        g.dim = dim
+        for k in range(3):
+            g.nel[k] = 8 if k < dim else 1
+            g.h[k] = 0.125
+        for mode, cases in refused.items():
+            if dim == 3 and mode > 8:
+                continue
+            for code in (0, 1, 2):
+                for case in cases:
+                    a, b = case.split("=")
+                    p = L.Pass(mode=mode, type=code, c0=0.5, c1=0.5, c2=0.5, **dict(at, **{a: at[b]}))
+                    assert lib.ust_k_apply_pass(C.byref(g), C.byref(p), None) == -1, (dim, mode, code, case)

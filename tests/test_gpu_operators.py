@@ -1040,3 +1040,43 @@ def test_rounding_of_the_product_is_local(nel, elements, prec):
             assert np.all(np.any(y[moved] != 0, axis=1)) and not y[~moved].any()
     for d in (du, dy, dm, dw, work):
         d.free()
+
+
+@pytest.mark.parametrize("nel", [(17, 9, 5), (16, 16, 8)])
+def test_passes_over_other_staged_vectors(nel):
+    """A Chebyshev step whose direction goes over its input, and the first step with its residual where either goes over the
+    scaling, on small 3D grids: what the calls with vectors of their own give, to FP32 rounding of another order of the
+    same sums (the one-launch kernels, which read those vectors at nodes that others write, are not taken)."""
+    import ctypes as C
+    import earthbyte_underworld_amd as ust  # noqa: F401  (loads the library)
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    g = _grid(3, nel)
+    n, wl = int(np.prod([k + 1 for k in nel])) * 3, lib.ust_k_weights_len(C.byref(g))
+    rng = np.random.default_rng(6)
+    x, b = rng.normal(size=n).astype(np.float32), rng.normal(size=n).astype(np.float32)
+    invd = rng.uniform(0.05, 0.1, n).astype(np.float32)
+    W, dm = _Dev(lib, rng.uniform(0.1, 1.0, wl).astype(np.float32)), _Dev(lib, np.zeros(n, np.uint8))
+    work = _Dev(lib, np.zeros(lib.ust_k_apply_work_len(C.byref(g)), np.float32))
+    G = C.byref(g)
+
+    def run(f):
+        dev = [_Dev(lib, a) for a in (x, b, invd, np.zeros(n, np.float32), np.zeros(n, np.float32))]
+        assert f(*[d.p for d in dev]) == 0
+        out = [d.get() for d in dev]
+        for d in dev:
+            d.free()
+        return out
+
+    step = lib.ust_k_apply_K_cheby_oop_f32
+    ref = run(lambda x_, b_, i_, y_, d_: step(G, W.p, dm.p, x_, y_, b_, i_, d_, 0.0, 0.5, 1, work.p, None))
+    got = run(lambda x_, b_, i_, y_, d_: step(G, W.p, dm.p, x_, y_, b_, i_, x_, 0.0, 0.5, 1, work.p, None))
+    assert rel_err(got[3], ref[3]) < 1e-5 and rel_err(got[0], ref[4]) < 1e-5
+    first = lib.ust_k_apply_K_residual_first_f32
+    ref = run(lambda x_, b_, i_, y_, d_: first(G, W.p, dm.p, b_, i_, x_, y_, 0.5, work.p, None))
+    over_x = run(lambda x_, b_, i_, y_, d_: first(G, W.p, dm.p, b_, i_, i_, y_, 0.5, work.p, None))
+    over_r = run(lambda x_, b_, i_, y_, d_: first(G, W.p, dm.p, b_, i_, x_, i_, 0.5, work.p, None))
+    assert rel_err(over_x[3], ref[3]) < 1e-5 and np.array_equal(over_x[2], ref[0])
+    assert rel_err(over_r[2], ref[3]) < 1e-5 and np.array_equal(over_r[0], ref[0])
+    for a in (W, dm, work):
+        a.free()
