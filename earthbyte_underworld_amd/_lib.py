@@ -219,6 +219,18 @@ _SIGS = {
     "ust_k_cg_xr_rr_guarded_f32": (I, [vp, vp, vp, vp, vp, vp, vp, C.c_size_t, vp, vp, vp]),
     "ust_k_apply_single": (I, [C.POINTER(Grid)]),
     "ust_k_apply_pass": (I, [C.POINTER(Grid), C.POINTER(Pass), vp]),
+    "ust_k_cg_start": (I, [vp, D, vp, vp, vp]),
+    "ust_k_cg_beta": (I, [vp, vp, vp, vp]),
+    "ust_k_cg_check": (I, [vp, vp, vp]),
+    "ust_k_cg_p_guarded_f64": (I, [vp, vp, vp, C.c_size_t, vp]),
+    "ust_k_cg_p_guarded_zf": (I, [vp, vp, vp, C.c_size_t, vp]),
+    "ust_k_cg_xr_guarded_f64": (I, [vp, vp, vp, vp, vp, vp, vp, C.c_size_t, vp]),
+    "ust_k_cg_xr_rr_guarded_f64": (I, [vp, vp, vp, vp, vp, vp, vp, C.c_size_t, vp, vp, vp]),
+    "ust_k_dot_mixed": (I, [vp, vp, C.c_size_t, vp, vp, vp]),
+    "ust_k_dot_mixed_beta": (I, [vp, vp, C.c_size_t, vp, vp, vp, vp, vp]),
+    "ust_k_dot_beta_f64": (I, [vp, vp, C.c_size_t, vp, vp, vp, vp, vp]),
+    "ust_k_dot_beta_f32": (I, [vp, vp, C.c_size_t, vp, vp, vp, vp, vp]),
+    "ust_k_copy_f64_to_f32_scaled": (I, [vp, vp, D, C.c_size_t, vp]),
     "ust_k_cg_parts": (I, [C.c_size_t]),
     "ust_k_cg_begin_f64": (I, [vp, vp, vp, C.c_size_t, D, vp, vp, vp]),
     "ust_k_cg_begin_f32": (I, [vp, D, vp, vp, C.c_size_t, D, vp, vp, vp]),

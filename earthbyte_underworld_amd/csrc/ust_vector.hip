@@ -71,8 +71,8 @@ __global__ void kv_div(const double *a, const double *b, double *y, size_t n) {
 }
 
 // two-stage deterministic reductions: stage 1 writes one partial per block (<= 1024 blocks)
-template <typename T, bool SQ>
-__global__ __launch_bounds__(256) void kv_dot_stage1(const T *x, const T *y, size_t n, double *partial) {
+template <typename TX, bool SQ, typename TY = TX>
+__global__ __launch_bounds__(256) void kv_dot_stage1(const TX *x, const TY *y, size_t n, double *partial) {
     __shared__ double sh[256 / 64];
     double s = 0.0;
     GRID_STRIDE(i, n) s += SQ ? (double)x[i] * (double)y[i] : (double)x[i];
@@ -102,15 +102,30 @@ __global__ __launch_bounds__(256) void kv_reduce_stage2(const double *partial, i
     if (threadIdx.x == 0) out[0] = s;
 }
 
-// stage 2 of r . r fused with the CG convergence check
+// stage 2 of r . z fused with the CG's beta, of r . r with its convergence check
+__device__ __forceinline__ void cg_beta(double rz, double *rz_old, double *c) {
+    if (c[1] != 0.0) return;
+    c[3] = rz / rz_old[0];
+    rz_old[0] = rz;
+}
+__device__ __forceinline__ void cg_check(double rr, double *c) {
+    if (c[1] != 0.0) return;
+    c[2] += 1.0;
+    if (!(rr == rr)) c[1] = 2.0;
+    else if (rr <= c[0]) c[1] = 1.0;
+}
+__global__ __launch_bounds__(256) void kv_reduce_beta(const double *partial, int np, double *rz, double *rz_old,
+                                                      double *c) {
+    const double s = block_sum_partials(partial, np);
+    if (threadIdx.x != 0) return;
+    rz[0] = s;
+    cg_beta(s, rz_old, c);
+}
 __global__ __launch_bounds__(256) void kv_reduce_check(const double *partial, int np, double *rr, double *c) {
     const double s = block_sum_partials(partial, np);
     if (threadIdx.x != 0) return;
     rr[0] = s;
-    if (c[1] != 0.0) return;
-    c[2] += 1.0;
-    if (!(s == s)) c[1] = 2.0;
-    else if (s <= c[0]) c[1] = 1.0;
+    cg_check(s, c);
 }
 
 __global__ __launch_bounds__(256) void kv_absmax_stage1(const double *x, size_t n, double *partial) {
@@ -163,24 +178,48 @@ __global__ void kv_cg_xr(T *x, T *r, const T *p, const T *q, const double *num, 
     }
 }
 
-// p = z + beta p, and x += a p, r -= a q with the block partials of r . r accumulated in FP64, as separate kernels
-// guarded by a control block c (c[0] threshold on r.r, c[1] state, c[2] iterations, c[3] beta)
-__global__ void kv_cg_p_guarded_f32(const float *z, float *p, const double *c, size_t n) {
+// The CG step by step, for callers that launch its parts themselves (the solves use the kernels of ust_cg.h), guarded by a
+// control block c: c[0] threshold on r.r, c[1] state (0 running, 1 converged, 2 NaN), c[2] iterations, c[3] beta.  Once the
+// state has left 0 the updates return at once.
+__global__ void kv_cg_start(const double *bb, double rtol2, double *c, double *rz_old) {
+    c[0] = rtol2 * bb[0];
+    c[1] = bb[0] > 0.0 ? 0.0 : 1.0;
+    c[2] = 0.0;
+    c[3] = 0.0;
+    rz_old[0] = 1.0;
+}
+__global__ void kv_cg_beta(const double *rz, double *rz_old, double *c) { cg_beta(rz[0], rz_old, c); }
+__global__ void kv_cg_check(const double *rr, double *c) { cg_check(rr[0], c); }
+
+template <typename TZ, typename TP>
+__global__ void kv_cg_p_guarded(const TZ *z, TP *p, const double *c, size_t n) {
     if (c[1] != 0.0) return;
-    const float beta = (float)c[3];
-    GRID_STRIDE(i, n) p[i] = z[i] + beta * p[i];
+    const TP beta = (TP)c[3];
+    GRID_STRIDE(i, n) p[i] = (TP)z[i] + beta * p[i];
 }
 
-__global__ __launch_bounds__(256) void kv_cg_xr_rr_guarded_f32(float *x, float *r, const float *p, const float *q,
-                                                               const double *rz, const double *pq, const double *c,
-                                                               size_t n, double *partial) {
+__global__ void kv_cg_xr_guarded(double *x, double *r, const double *p, const double *q, const double *rz,
+                                 const double *pq, const double *c, size_t n) {
+    if (c[1] != 0.0) return;
+    const double a = rz[0] / pq[0];
+    GRID_STRIDE(i, n) {
+        x[i] += a * p[i];
+        r[i] -= a * q[i];
+    }
+}
+
+// x += a p, r -= a q and the block partials of r . r (zero once converged)
+template <typename T>
+__global__ __launch_bounds__(256) void kv_cg_xr_rr_guarded(T *x, T *r, const T *p, const T *q, const double *rz,
+                                                           const double *pq, const double *c, size_t n,
+                                                           double *partial) {
     __shared__ double sh[256 / 64];
     double s = 0.0;
     if (c[1] == 0.0) {
-        const float a = (float)(rz[0] / pq[0]);
+        const T a = (T)(rz[0] / pq[0]);
         GRID_STRIDE(i, n) {
             x[i] += a * p[i];
-            const float ri = r[i] - a * q[i];
+            const T ri = r[i] - a * q[i];
             r[i] = ri;
             s += (double)ri * (double)ri;
         }
@@ -189,6 +228,11 @@ __global__ __launch_bounds__(256) void kv_cg_xr_rr_guarded_f32(float *x, float *
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = s;
     __syncthreads();
     if (threadIdx.x == 0) partial[blockIdx.x] = sh[0] + sh[1] + sh[2] + sh[3];
+}
+
+// y = (float)(s x)
+__global__ void kv_d2f_scaled(const double *x, float *y, double s, size_t n) {
+    GRID_STRIDE(i, n) y[i] = (float)(s * x[i]);
 }
 
 // The FP32 PCG's streaming kernels on 16-byte aligned vectors: four dofs per thread and step (one 16-byte load
@@ -656,9 +700,81 @@ int ust_k_cheby_first_from_f64(const double *b, float *b32, const float *invd, f
                                size_t n, void *stream) {
     LV(kv_cheby_first_from64, n, b, b32, invd, d, x, c2, n);
 }
+int ust_k_cg_start(const double *bb, double rtol2, double *ctl, double *rz_old, void *stream) {
+    hipLaunchKernelGGL(kv_cg_start, dim3(1), dim3(1), 0, ust_stream(stream), bb, rtol2, ctl, rz_old);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_cg_beta(const double *rz, double *rz_old, double *ctl, void *stream) {
+    hipLaunchKernelGGL(kv_cg_beta, dim3(1), dim3(1), 0, ust_stream(stream), rz, rz_old, ctl);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_cg_check(const double *rr, double *ctl, void *stream) {
+    hipLaunchKernelGGL(kv_cg_check, dim3(1), dim3(1), 0, ust_stream(stream), rr, ctl);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_cg_p_guarded_f64(const double *z, double *p, const double *ctl, size_t n, void *stream) {
+    LV((kv_cg_p_guarded<double, double>), n, z, p, ctl, n);
+}
+int ust_k_cg_p_guarded_zf(const float *z, double *p, const double *ctl, size_t n, void *stream) {
+    LV((kv_cg_p_guarded<float, double>), n, z, p, ctl, n);
+}
+int ust_k_cg_xr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
+                            const double *pq, const double *ctl, size_t n, void *stream) {
+    LV(kv_cg_xr_guarded, n, x, r, p, q, rz, pq, ctl, n);
+}
+int ust_k_cg_xr_rr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
+                               const double *pq, double *ctl, size_t n, double *partial, double *rr,
+                               void *stream) {
+    const unsigned g = rgrid(n);
+    hipLaunchKernelGGL(kv_cg_xr_rr_guarded<double>, dim3(g), dim3(256), 0, ust_stream(stream), x, r, p, q, rz, pq, ctl, n,
+                       partial);
+    hipLaunchKernelGGL(kv_reduce_check, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rr, ctl);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_dot_mixed(const double *x, const float *y, size_t n, double *partial, double *out, void *stream) {
+    const unsigned g = rgrid(n);
+    hipLaunchKernelGGL((kv_dot_stage1<double, true, float>), dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
+    hipLaunchKernelGGL(kv_reduce_stage2, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, out);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_dot_mixed_beta(const double *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
+                         double *ctl, void *stream) {
+    const unsigned g = rgrid(n);
+    hipLaunchKernelGGL((kv_dot_stage1<double, true, float>), dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
+    hipLaunchKernelGGL(kv_reduce_beta, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rz, rz_old, ctl);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_dot_beta_f64(const double *x, const double *y, size_t n, double *partial, double *rz, double *rz_old,
+                       double *ctl, void *stream) {
+    const unsigned g = rgrid(n);
+    hipLaunchKernelGGL((kv_dot_stage1<double, true>), dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
+    hipLaunchKernelGGL(kv_reduce_beta, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rz, rz_old, ctl);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_dot_beta_f32(const float *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
+                       double *ctl, void *stream) {
+    const unsigned g = rgrid(n);
+    if (al16(x) && al16(y))
+        hipLaunchKernelGGL(kv4_dot_f32, dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
+    else
+        hipLaunchKernelGGL((kv_dot_stage1<float, true>), dim3(g), dim3(256), 0, ust_stream(stream), x, y, n, partial);
+    hipLaunchKernelGGL(kv_reduce_beta, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rz, rz_old, ctl);
+    UST_LAUNCH_CHECK();
+    return UST_OK;
+}
+int ust_k_copy_f64_to_f32_scaled(const double *x, float *y, double s, size_t n, void *stream) {
+    LV(kv_d2f_scaled, n, x, y, s, n);
+}
 int ust_k_cg_p_guarded_f32(const float *z, float *p, const double *ctl, size_t n, void *stream) {
     if (al16(z) && al16(p)) LV(kv4_cg_p_guarded_f32, (n + 3) / 4, z, p, ctl, n);
-    LV(kv_cg_p_guarded_f32, n, z, p, ctl, n);
+    LV((kv_cg_p_guarded<float, float>), n, z, p, ctl, n);
 }
 int ust_k_cg_xr_rr_guarded_f32(float *x, float *r, const float *p, const float *q, const double *rz, const double *pq,
                                double *ctl, size_t n, double *partial, double *rr, void *stream) {
@@ -667,7 +783,7 @@ int ust_k_cg_xr_rr_guarded_f32(float *x, float *r, const float *p, const float *
         hipLaunchKernelGGL(kv4_cg_xr_rr_guarded_f32, dim3(g), dim3(256), 0, ust_stream(stream), x, r, p, q, rz, pq, ctl,
                            n, partial);
     else
-        hipLaunchKernelGGL(kv_cg_xr_rr_guarded_f32, dim3(g), dim3(256), 0, ust_stream(stream), x, r, p, q, rz, pq, ctl,
+        hipLaunchKernelGGL(kv_cg_xr_rr_guarded<float>, dim3(g), dim3(256), 0, ust_stream(stream), x, r, p, q, rz, pq, ctl,
                            n, partial);
     hipLaunchKernelGGL(kv_reduce_check, dim3(1), dim3(256), 0, ust_stream(stream), partial, (int)g, rr, ctl);
     UST_LAUNCH_CHECK();

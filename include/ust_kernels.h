@@ -521,8 +521,31 @@ int ust_k_cg_step_f64(double *x, double *r, const double *p, const double *q, do
 int ust_k_cg_step_f32(float *x, float *r, const float *p, const float *q, float *keep, double *c, double *part, int npq,
                       size_t n, void *stream);
 int ust_k_cg_state(double *c, const double *part, size_t n, double *host, void *stream);
-/* p = z + beta p and x += a p, r -= a q with r.r on FP32 vectors against a control block of threshold, state, count and
- * beta; nothing is done once the state is not 0 */
+/* The same iteration step by step, for callers that launch its parts themselves (the solves use the kernels above), on
+ * vectors of any alignment.  ctl[4] on the device: ctl[0] = stopping threshold rtol2 * b.b, ctl[1] = state (0 running, 1
+ * converged, 2 NaN), ctl[2] = iterations, ctl[3] = beta.  start: ctl from bb = b.b and rz_old = 1 (with p = 0 the first
+ * update gives p = z).  beta: ctl[3] = rz/rz_old, rz_old = rz.  The guarded updates and check do nothing once ctl[1] != 0.
+ * zf: z in FP32, p in FP64. */
+int ust_k_cg_start(const double *bb, double rtol2, double *ctl, double *rz_old, void *stream);
+int ust_k_cg_beta(const double *rz, double *rz_old, double *ctl, void *stream);
+int ust_k_cg_check(const double *rr, double *ctl, void *stream);
+int ust_k_cg_p_guarded_f64(const double *z, double *p, const double *ctl, size_t n, void *stream);
+int ust_k_cg_p_guarded_zf(const float *z, double *p, const double *ctl, size_t n, void *stream);
+int ust_k_cg_xr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
+                            const double *pq, const double *ctl, size_t n, void *stream);
+/* x . y (two-stage) with y in FP32; r . z (two-stage, into rz) fused with the beta update */
+int ust_k_dot_mixed(const double *x, const float *y, size_t n, double *partial, double *out, void *stream);
+int ust_k_dot_mixed_beta(const double *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
+                         double *ctl, void *stream);
+int ust_k_dot_beta_f64(const double *x, const double *y, size_t n, double *partial, double *rz, double *rz_old,
+                       double *ctl, void *stream);
+int ust_k_dot_beta_f32(const float *x, const float *y, size_t n, double *partial, double *rz, double *rz_old,
+                       double *ctl, void *stream);
+/* x += a p, r -= a q with r . r (two-stage, into rr) and the check; the FP32 forms' sums are in FP64 */
+int ust_k_cg_xr_rr_guarded_f64(double *x, double *r, const double *p, const double *q, const double *rz,
+                               const double *pq, double *ctl, size_t n, double *partial, double *rr,
+                               void *stream);
+int ust_k_copy_f64_to_f32_scaled(const double *x, float *y, double s, size_t n, void *stream);
 int ust_k_cg_p_guarded_f32(const float *z, float *p, const double *ctl, size_t n, void *stream);
 int ust_k_cg_xr_rr_guarded_f32(float *x, float *r, const float *p, const float *q, const double *rz, const double *pq,
                                double *ctl, size_t n, double *partial, double *rr, void *stream);

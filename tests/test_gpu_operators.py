@@ -1080,3 +1080,97 @@ def test_passes_over_other_staged_vectors(nel):
     assert rel_err(over_r[2], ref[3]) < 1e-5 and np.array_equal(over_r[0], ref[0])
     for a in (W, dm, work):
         a.free()
+
+
+@pytest.mark.parametrize("n", [5, 100_003])
+@pytest.mark.parametrize("kind", ["f64", "zf", "f32"])
+@pytest.mark.parametrize("off", [0, 1])
+def test_step_by_step_cg(kind, n, off):
+    """The CG's parts as launches of their own on K = tridiag(-1, 4, -1) with z = r / 4, each iteration started and checked
+    on the device, on aligned vectors and on ones an element past a 16-byte boundary: numpy's recurrence.  Bar: as in
+    test_device_controlled_cg, 3 times the stopping tolerance (condition number 3)."""
+    import ctypes as C
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    T, TZ = (np.float32 if kind == "f32" else np.float64), (np.float64 if kind == "f64" else np.float32)
+    tp = "f32" if kind == "f32" else "f64"
+    rtol = 1e-4 if kind == "f32" else 1e-8
+
+    def mul(v):
+        o = v.dtype.type(4) * v
+        o[1:] -= v[:-1]
+        o[:-1] -= v[1:]
+        return o
+
+    class Vec:  # n values, `off` values past the start of the allocation
+        def __init__(self, a):
+            self.d = _Dev(lib, np.concatenate([np.zeros(off, a.dtype), a]))
+            self.p = C.c_void_p(self.d.p.value + off * a.itemsize)
+
+        def get(self):
+            return self.d.get()[off:]
+
+        def put(self, a):
+            assert lib.ust_memcpy_h2d(self.p, a.ctypes.data_as(C.c_void_p), a.nbytes, None) == 0
+
+    b = np.random.default_rng(n).normal(size=n)
+    db, x, p, q, z = Vec(b), Vec(np.zeros(n, T)), Vec(np.zeros(n, T)), Vec(np.zeros(n, T)), Vec(np.zeros(n, TZ))
+    r, half = Vec(np.zeros(n, T)), 0.5
+    if kind == "f32":
+        assert lib.ust_k_copy_f64_to_f32_scaled(db.p, r.p, half, n, None) == 0
+        assert np.array_equal(r.get(), (half * b).astype(T))
+    else:
+        r.put(b)
+    rhs = r.get().astype(np.float64)
+    part, ctl = _Dev(lib, np.zeros(1024)), _Dev(lib, np.zeros(4))
+    s = _Dev(lib, np.array([rhs @ rhs, 0.0, 0.0, 0.0, 0.0]))  # b.b, rz, rz_old, pq, rr
+    bb, rz, rz_old, pq, rr = (C.c_void_p(s.p.value + 8 * k) for k in range(5))
+    assert lib.ust_k_cg_start(bb, rtol * rtol, ctl.p, rz_old, None) == 0
+    assert list(ctl.get()) == [rtol * rtol * (rhs @ rhs), 0.0, 0.0, 0.0] and s.get()[2] == 1.0
+
+    def iterate():
+        z.put((r.get() / 4).astype(TZ))
+        ref = r.get().astype(np.float64) @ z.get().astype(np.float64)
+        if kind == "zf" and off:  # the separate launches
+            assert lib.ust_k_dot_mixed(r.p, z.p, n, part.p, rz, None) == 0
+            assert lib.ust_k_cg_beta(rz, rz_old, ctl.p, None) == 0
+        else:
+            f = getattr(lib, {"f64": "ust_k_dot_beta_f64", "zf": "ust_k_dot_mixed_beta", "f32": "ust_k_dot_beta_f32"}[kind])
+            assert f(r.p, z.p, n, part.p, rz, rz_old, ctl.p, None) == 0
+        assert abs(s.get()[1] - ref) <= 1e-12 * ref
+        assert getattr(lib, f"ust_k_cg_p_guarded_{kind}")(z.p, p.p, ctl.p, n, None) == 0
+        q.put(mul(p.get()))
+        h = s.get()
+        h[3] = p.get().astype(np.float64) @ q.get().astype(np.float64)
+        assert lib.ust_memcpy_h2d(s.p, h.ctypes.data_as(C.c_void_p), h.nbytes, None) == 0
+        if kind == "f64" and off:
+            assert lib.ust_k_cg_xr_guarded_f64(x.p, r.p, p.p, q.p, rz, pq, ctl.p, n, None) == 0
+            h[4] = r.get() @ r.get()
+            assert lib.ust_memcpy_h2d(s.p, h.ctypes.data_as(C.c_void_p), h.nbytes, None) == 0
+            assert lib.ust_k_cg_check(rr, ctl.p, None) == 0
+        else:
+            f = getattr(lib, f"ust_k_cg_xr_rr_guarded_{tp}")
+            assert f(x.p, r.p, p.p, q.p, rz, pq, ctl.p, n, part.p, rr, None) == 0
+        return tuple(ctl.get()[1:3])
+
+    xr, rr_, pr, old = np.zeros(n), rhs.copy(), np.zeros(n), 1.0
+    for its in range(1, 60):
+        state, count = iterate()
+        new = float(rr_ @ rr_) / 4
+        pr = rr_ / 4 + (new / old) * pr
+        qr = mul(pr)
+        a = new / float(pr @ qr)
+        xr, rr_, old = xr + a * pr, rr_ - a * qr, new
+        assert count == its
+        if state != 0:
+            break
+    assert state == 1
+    got = x.get()
+    assert np.linalg.norm(rhs - mul(got.astype(np.float64))) <= 3 * rtol * np.linalg.norm(rhs)
+    assert np.linalg.norm(got - xr) <= 3 * rtol * np.linalg.norm(xr)
+    before = p.get()
+    assert iterate() == (1.0, float(its)) and np.array_equal(x.get(), got) and np.array_equal(p.get(), before)
+    for v in (db, x, p, q, z, r):
+        v.d.free()
+    for d in (part, ctl, s):
+        d.free()
