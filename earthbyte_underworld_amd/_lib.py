@@ -266,6 +266,8 @@ _SIGS = {
     "ust_k_strain_weakening_step": (I, [vp, vp, I, C.c_double, vp]),
     "ust_k_permute_f64": (I, [vp, vp, vp, I, vp]),
     "ust_k_pcdvc_plan": (I, [C.POINTER(Grid), vp, vp, vp, C.POINTER(PcdvcOpts), vp, vp, vp, vp]),
+    "ust_k_pcdvc_build": (I, [I, I, I, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp, vp,
+                              vp, vp]),
     "ust_k_count_work_len": (C.c_size_t, [I]),
     "ust_k_count_offsets": (I, [I, vp, vp, vp, vp, vp, vp, vp]),
     "ust_k_offset_stats": (I, [I, vp, vp, vp, vp, vp]),

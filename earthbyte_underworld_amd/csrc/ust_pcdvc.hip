@@ -26,7 +26,8 @@ __device__ __forceinline__ int group_sum(int v) {
 // A thread per element read the weights uncoalesced and wrote every element's list: 634 us at 96^3 elements x 30 particles;
 // a group of lanes per element, with lists for the changed ones only, 458-527 us, most of it the serial lists (2D 64x64 x
 // 20: 30 -> 11 us).
-template <int DIM>
+// ALL: every element's list is written and the count is the count alone (ust_k_pcdvc_plan).
+template <int DIM, bool ALL>
 __global__ __launch_bounds__(256) void k_pcdvc_plan(GridDev g, const int *__restrict__ cell_off,
                                                     const double *__restrict__ w, const unsigned char *__restrict__ mat,
                                                     ust_pcdvc_opts o, int *__restrict__ new_count,
@@ -62,11 +63,11 @@ __global__ __launch_bounds__(256) void k_pcdvc_plan(GridDev g, const int *__rest
             if (!o.split_in_interface_cells && !boundary) mspl = 0;
         }
         if (mdel > n - 4) mdel = n / 2;  // :1373
-        const int nspl = min(big, mspl), ndel = min(small, mdel), len = n + nspl - ndel;
+        const int nspl = min(big, mspl), ndel = max(min(small, mdel), 0), len = n + nspl - ndel;
         const bool changed = nspl > 0 || ndel > 0;
         if (gl != 0) continue;
-        new_count[e] = len | (changed ? PCDVC_CHANGED : 0);
-        if (!changed) continue;
+        new_count[e] = len | (changed && !ALL ? PCDVC_CHANGED : 0);
+        if (!changed && !ALL) continue;
         int *L = list + p0 + (size_t)e * o.max_splits;
         for (int i = 0; i < n; i++) L[i] = i;
         // splits: the first mspl particles (in element order) whose region exceeds max_w (:1351, :1378-1392)
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(256) void k_pcdvc_plan(GridDev g, const int *__rest
             while (L[pos] != i) pos++;  // i is in the list: only earlier (larger) candidates were removed
             L[pos] = L[--k];
         }
-        if (len < 3) atomicOr(tot, 1);  // :1418-1421
+        if (changed && len < 3) atomicOr(tot, 1);  // :1418-1421
         if (nspl) atomicAdd(tot + 1, nspl);
         if (ndel) atomicAdd(tot + 2, ndel);
     }
@@ -233,7 +234,8 @@ __global__ __launch_bounds__(256) void k_count_offsets(const int *__restrict__ c
 
 // Bound by memory: 96^3 elements x 30 particles read and write 3.1 GB.  A thread per element, uncoalesced, took 2934 us (and
 // the weights and centroids were computed again); a group of lanes per element takes 920 us, 3.4 TB/s.
-template <int DIM>
+// ALL: every element's particles are its list's, and only they are written (ust_k_pcdvc_build).
+template <int DIM, bool ALL>
 __global__ __launch_bounds__(256) void k_pcdvc_build(int nel, int max_splits, const int *__restrict__ cell_off,
                                                      const int *__restrict__ new_off, const int *__restrict__ new_count,
                                                      const int *__restrict__ list, ust_pcdvc_swarm a,
@@ -242,7 +244,7 @@ __global__ __launch_bounds__(256) void k_pcdvc_build(int nel, int max_splits, co
     for (long long e64 = (long long)blockIdx.x * PC_EPB + threadIdx.x / PC_LANES; e64 < nel;
          e64 += (long long)gridDim.x * PC_EPB) {
         const int e = (int)e64, p0 = cell_off[e], q0 = new_off[e], len = new_off[e + 1] - q0;
-        const bool changed = (new_count[e] & PCDVC_CHANGED) != 0;
+        const bool changed = ALL || (new_count[e] & PCDVC_CHANGED) != 0;
         const int *L = list + p0 + (size_t)e * max_splits;
         for (int k = gl; k < len; k += PC_LANES) {
             const int v = changed ? L[k] : k;
@@ -254,9 +256,9 @@ __global__ __launch_bounds__(256) void k_pcdvc_build(int nel, int max_splits, co
                 // a changed element's regions grow from its particles, the others keep theirs
                 const double c = a.c[d][src], x = split ? c : a.x[d][src];
                 b.x[d][dst] = x;
-                b.c[d][dst] = changed ? x : c;
+                if (!ALL) b.c[d][dst] = changed ? x : c;
             }
-            b.w[dst] = changed ? 0.0 : a.w[src];
+            if (!ALL) b.w[dst] = changed ? 0.0 : a.w[src];
             if (a.mat) b.mat[dst] = a.mat[src];
             if (a.coh) b.coh[dst] = a.coh[src];
             if (a.s0) b.s0[dst] = a.s0[src];
@@ -270,20 +272,31 @@ static inline unsigned element_groups(int nel) {
     return (unsigned)(b < 8192 ? b : 8192);
 }
 
-extern "C" int ust_k_pcdvc_plan(const ust_grid *gr, const int *cell_off, const double *w, const unsigned char *mat,
-                                const ust_pcdvc_opts *o, int *new_count, int *list, int *flag, void *stream) {
+template <bool ALL>
+static int pcdvc_plan(const ust_grid *gr, const int *cell_off, const double *w, const unsigned char *mat,
+                      const ust_pcdvc_opts *o, int *new_count, int *list, int *flag, void *stream) {
     if (!gr || !cell_off || !w || !o || !new_count || !list || !flag) return UST_EINVAL;
     if (o->max_splits < 0) return UST_EINVAL;
     GridDev g = grid_dev(gr);
     if (g.nel <= 0) return UST_OK;
     if (g.dim == 3)
-        hipLaunchKernelGGL(k_pcdvc_plan<3>, dim3(element_groups(g.nel)), dim3(256), 0, ust_stream(stream), g, cell_off, w,
-                           mat, *o, new_count, list, flag);
+        hipLaunchKernelGGL((k_pcdvc_plan<3, ALL>), dim3(element_groups(g.nel)), dim3(256), 0, ust_stream(stream), g,
+                           cell_off, w, mat, *o, new_count, list, flag);
     else
-        hipLaunchKernelGGL(k_pcdvc_plan<2>, dim3(element_groups(g.nel)), dim3(256), 0, ust_stream(stream), g, cell_off, w,
-                           mat, *o, new_count, list, flag);
+        hipLaunchKernelGGL((k_pcdvc_plan<2, ALL>), dim3(element_groups(g.nel)), dim3(256), 0, ust_stream(stream), g,
+                           cell_off, w, mat, *o, new_count, list, flag);
     UST_LAUNCH_CHECK();
     return UST_OK;
+}
+
+extern "C" int ust_k_pcdvc_plan(const ust_grid *gr, const int *cell_off, const double *w, const unsigned char *mat,
+                                const ust_pcdvc_opts *o, int *new_count, int *list, int *flag, void *stream) {
+    return pcdvc_plan<true>(gr, cell_off, w, mat, o, new_count, list, flag, stream);
+}
+
+extern "C" int ust_k_pcdvc_plan_changed(const ust_grid *gr, const int *cell_off, const double *w, const unsigned char *mat,
+                                        const ust_pcdvc_opts *o, int *new_count, int *list, int *flag, void *stream) {
+    return pcdvc_plan<false>(gr, cell_off, w, mat, o, new_count, list, flag, stream);
 }
 
 extern "C" size_t ust_k_count_work_len(int nel) { return 4 * (((size_t)nel + CNT_BLOCK - 1) / CNT_BLOCK); }
@@ -312,24 +325,42 @@ extern "C" int ust_k_offset_stats(int nel, const int *off, const int *flag, long
     return UST_OK;
 }
 
-extern "C" int ust_k_pcdvc_build(int dim, int nel, int max_splits, const int *cell_off, const int *new_off,
-                                 const int *new_count, const int *list, const ust_pcdvc_swarm *from,
-                                 const ust_pcdvc_swarm *to, void *stream) {
-    if ((dim != 2 && dim != 3) || nel < 0 || max_splits < 0 || !cell_off || !new_off || !new_count || !list || !from ||
-        !to)
-        return UST_EINVAL;
+template <bool ALL>
+static int pcdvc_build(int dim, int nel, int max_splits, const int *cell_off, const int *new_off, const int *new_count,
+                       const int *list, const ust_pcdvc_swarm &from, const ust_pcdvc_swarm &to, void *stream) {
+    if (nel < 0 || max_splits < 0 || !cell_off || !new_off || !list) return UST_EINVAL;
     for (int d = 0; d < dim; d++)
-        if (!from->x[d] || !from->c[d] || !to->x[d] || !to->c[d]) return UST_EINVAL;
-    if (!from->w || !to->w || (from->mat && !to->mat) || (from->coh && !to->coh) || (from->s0 && !to->s0) ||
-        (from->s1 && !to->s1))
-        return UST_EINVAL;
+        if (!from.x[d] || !from.c[d] || !to.x[d]) return UST_EINVAL;
+    if ((from.mat && !to.mat) || (from.coh && !to.coh) || (from.s0 && !to.s0) || (from.s1 && !to.s1)) return UST_EINVAL;
     if (nel == 0) return UST_OK;
     if (dim == 3)
-        hipLaunchKernelGGL(k_pcdvc_build<3>, dim3(element_groups(nel)), dim3(256), 0, ust_stream(stream), nel, max_splits,
-                           cell_off, new_off, new_count, list, *from, *to);
+        hipLaunchKernelGGL((k_pcdvc_build<3, ALL>), dim3(element_groups(nel)), dim3(256), 0, ust_stream(stream), nel,
+                           max_splits, cell_off, new_off, new_count, list, from, to);
     else
-        hipLaunchKernelGGL(k_pcdvc_build<2>, dim3(element_groups(nel)), dim3(256), 0, ust_stream(stream), nel, max_splits,
-                           cell_off, new_off, new_count, list, *from, *to);
+        hipLaunchKernelGGL((k_pcdvc_build<2, ALL>), dim3(element_groups(nel)), dim3(256), 0, ust_stream(stream), nel,
+                           max_splits, cell_off, new_off, new_count, list, from, to);
     UST_LAUNCH_CHECK();
     return UST_OK;
+}
+
+extern "C" int ust_k_pcdvc_build(int dim, int nel, int max_splits, const int *cell_off, const int *new_off,
+                                 const int *list, const double *xi0, const double *xi1, const double *xi2,
+                                 const double *c0, const double *c1, const double *c2, const unsigned char *mat,
+                                 const float *coh, const double *state0, const double *state1, double *o0, double *o1,
+                                 double *o2, unsigned char *omat, float *ocoh, double *ostate0, double *ostate1,
+                                 void *stream) {
+    // read only
+    const ust_pcdvc_swarm from = {{(double *)xi0, (double *)xi1, (double *)xi2}, {(double *)c0, (double *)c1, (double *)c2},
+                                  nullptr, (unsigned char *)mat, (float *)coh, (double *)state0, (double *)state1};
+    const ust_pcdvc_swarm to = {{o0, o1, o2}, {}, nullptr, omat, ocoh, ostate0, ostate1};
+    return pcdvc_build<true>(dim == 3 ? 3 : 2, nel, max_splits, cell_off, new_off, nullptr, list, from, to, stream);
+}
+
+extern "C" int ust_k_pcdvc_build_changed(int dim, int nel, int max_splits, const int *cell_off, const int *new_off,
+                                         const int *new_count, const int *list, const ust_pcdvc_swarm *from,
+                                         const ust_pcdvc_swarm *to, void *stream) {
+    if ((dim != 2 && dim != 3) || !new_count || !from || !to || !from->w || !to->w) return UST_EINVAL;
+    for (int d = 0; d < dim; d++)
+        if (!to->c[d]) return UST_EINVAL;
+    return pcdvc_build<false>(dim, nel, max_splits, cell_off, new_off, new_count, list, *from, *to, stream);
 }

@@ -1336,8 +1336,8 @@ int ust_swarm_pcdvc(ust_context *ctx, const ust_pcdvc *opts, int *n_split, int *
     if (!rc) rc = swarm_malloc(ctx, &cwork, ust_k_count_work_len(nel) * sizeof(int));
     if (!rc) rc = swarm_malloc(ctx, (void **)&s.off, (size_t)(nel + 1) * sizeof(int));
     if (!rc) rc = ust_k_fill_f64((double *)flag, 0.0, 2, ctx->stream); /* all-zero bits: the ints read 0 */
-    if (!rc) rc = ust_k_pcdvc_plan(&ctx->grid, ctx->cell_off, ctx->w, ctx->mat, &ko, (int *)cnt, (int *)list, flag,
-                                   ctx->stream);
+    if (!rc) rc = ust_k_pcdvc_plan_changed(&ctx->grid, ctx->cell_off, ctx->w, ctx->mat, &ko, (int *)cnt, (int *)list,
+                                           flag, ctx->stream);
     if (!rc) rc = ust_k_count_offsets(nel, (const int *)cnt, s.off, (int *)elems, flag, host, (int *)cwork, ctx->stream);
     if (!rc) rc = ust_stream_sync(ctx->stream);
     const long long total = rc ? 0 : host[0];
@@ -1356,8 +1356,8 @@ int ust_swarm_pcdvc(ust_context *ctx, const ust_pcdvc *opts, int *n_split, int *
                                           ctx->mat, ctx->coh, ctx->pfw, ctx->pfw_inc};
             const ust_pcdvc_swarm to = {{s.x[0], s.x[1], s.x[2]}, {s.c[0], s.c[1], s.c[2]}, s.w, s.mat, s.coh, s.pfw,
                                         s.inc};
-            rc = ust_k_pcdvc_build(dim, nel, ko.max_splits, ctx->cell_off, s.off, (const int *)cnt, (const int *)list,
-                                   &from, &to, ctx->stream);
+            rc = ust_k_pcdvc_build_changed(dim, nel, ko.max_splits, ctx->cell_off, s.off, (const int *)cnt,
+                                           (const int *)list, &from, &to, ctx->stream);
         }
         if (!rc) rc = ust_stream_sync(ctx->stream);
         if (!rc) rc = swarm_adopt(ctx, &s, (int)total, max_ppc);

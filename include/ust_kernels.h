@@ -191,31 +191,42 @@ int ust_k_particle_weights(const ust_grid *g, const int *cell_off, int ppc_hint,
                            const double *velocity, const double *pressure, int prev_solution,
                            const ust_yield_state *yield_state, const ust_buoyancy *buoyancy, double *eta_out,
                            unsigned char *yield_out, double *WK, double *WG, double *WF, void *stream);
-/* PCDVC population control (PCDVC.c:1338-1432 2D, :880-990 3D, non-Inflow branch), around a scan of the counts.
- * plan: reads the DVC region volumes w of an element's particles and writes its new particle count, with bit 30 set where
- * its particles change, and then its new particle list (entries s: original particle s of the element; s | 2^30: a split
- * copy of s) at list[cell_off[e] + e * max_splits], capacity n_e + max_splits; flag[0] gets 1 where a changed element
- * keeps fewer than 3 particles, flag[1] and flag[2] count the splits and deletions.
+/* PCDVC population control (PCDVC.c:1338-1432 2D, :880-990 3D, non-Inflow branch), in two passes around a scan of the
+ * counts.  plan: reads the DVC region volumes w of an element's particles and writes its new particle count and its new
+ * particle list (entries s: original particle s of the element; s | 2^30: a split copy of s) at
+ * list[cell_off[e] + e * max_splits], capacity n_e + max_splits; flag[0] gets 1 where a changed element keeps fewer than 3
+ * particles, flag[1] and flag[2] count the splits and deletions.
+ * build: writes the new swarm from the lists (split copies at the parent's region centroid c0/c1/c2, the parent's material,
+ * cohesion factor and two optional per-particle states). */
+int ust_k_pcdvc_plan(const ust_grid *g, const int *cell_off, const double *w, const unsigned char *mat,
+                     const ust_pcdvc_opts *opts, int *new_count, int *list, int *flag, void *stream);
+int ust_k_pcdvc_build(int dim, int nel, int max_splits, const int *cell_off, const int *new_off, const int *list,
+                      const double *xi0, const double *xi1, const double *xi2, const double *c0, const double *c1,
+                      const double *c2, const unsigned char *mat, const float *coh, const double *state0,
+                      const double *state1, double *o0, double *o1, double *o2, unsigned char *omat, float *ocoh,
+                      double *ostate0, double *ostate1, void *stream);
+/* The same for a swarm whose weights and centroids are kept where an element's particles do not change.
+ * plan_changed: bit 30 of the new count is set where they change, and only then is the element's list written.
  * count_offsets: exclusive sums of the counts to off (nel + 1) and the changed elements to elems, both in order; host
  * (pinned, 7 entries): particles, changed elements, largest count, elements without particles, flag[0..2].  offset_stats:
  * the same entries from offsets that are there.  work: ust_k_count_work_len ints.
- * build: writes the new swarm: a changed element's from its list (split copies at the parent's region centroid c, the
- * parent's material, cohesion factor and two optional per-particle states; c = x, w = 0, for its regions to be grown
- * anew), the others' as they are, with their weights and centroids. */
+ * build_changed: writes the new swarm: a changed element's from its list (c = x, w = 0, for its regions to be grown anew),
+ * the others' as they are, with their weights and centroids. */
 typedef struct {
     double *x[3], *c[3], *w;
     unsigned char *mat;
     float *coh;
     double *s0, *s1;
 } ust_pcdvc_swarm;
-int ust_k_pcdvc_plan(const ust_grid *g, const int *cell_off, const double *w, const unsigned char *mat,
-                     const ust_pcdvc_opts *opts, int *new_count, int *list, int *flag, void *stream);
+int ust_k_pcdvc_plan_changed(const ust_grid *g, const int *cell_off, const double *w, const unsigned char *mat,
+                             const ust_pcdvc_opts *opts, int *new_count, int *list, int *flag, void *stream);
 size_t ust_k_count_work_len(int nel);
 int ust_k_count_offsets(int nel, const int *count, int *off, int *elems, const int *flag, long long *host, int *work,
                         void *stream);
 int ust_k_offset_stats(int nel, const int *off, const int *flag, long long *host, int *work, void *stream);
-int ust_k_pcdvc_build(int dim, int nel, int max_splits, const int *cell_off, const int *new_off, const int *new_count,
-                      const int *list, const ust_pcdvc_swarm *from, const ust_pcdvc_swarm *to, void *stream);
+int ust_k_pcdvc_build_changed(int dim, int nel, int max_splits, const int *cell_off, const int *new_off,
+                              const int *new_count, const int *list, const ust_pcdvc_swarm *from,
+                              const ust_pcdvc_swarm *to, void *stream);
 /* StrainWeakening time step: pfw += dt * pfw_inc, then negative values to 0 (the TimeIntegrand update of
  * postFailureWeakening, whose time derivative is the stored increment, StrainWeakening.c:401-407, and
  * _StrainWeakening_MakeValuesPositive, :411-426) */

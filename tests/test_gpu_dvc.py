@@ -449,3 +449,85 @@ def test_dvc_2d_lane_groups_agree(oracle):
         xi_ref, w_ref = oracle.dvc_swarm(2, (10, 10), off, xi)
         assert np.array_equal(w1, w_ref) and np.array_equal(xi1[:, :2], xi_ref[:, :2])
         s.close()
+
+
+def _plan(dim, nel, off, w, mat, o):
+    """The reference's lists (PCDVC.c:1338-1432), element by element: entries s, or s | 2^30 for a split copy."""
+    lists, flag = [], [0, 0, 0]
+    vol = float(1 << dim)
+    max_w, min_w = o.upper_t * vol / 100.0, o.lower_t * vol / 100.0
+    for e in range(int(np.prod(nel))):
+        n, we, me = off[e + 1] - off[e], w[off[e]:off[e + 1]], mat[off[e]:off[e + 1]]
+        i = [e % nel[0], (e // nel[0]) % nel[1], e // (nel[0] * nel[1])][:dim]
+        boundary = any(i[k] in (0, nel[k] - 1) for k in range(dim))
+        mdel, mspl = o.max_deletions, o.max_splits
+        if n and np.any(me != me[0]):
+            mdel = mdel if o.delete_in_interface_cells else 0
+            mspl = mspl if o.split_in_interface_cells or boundary else 0
+        mdel = n // 2 if mdel > n - 4 else mdel
+        big = [k | 1 << 30 for k in range(n) if we[k] > max_w][:max(mspl, 0)]
+        lst = list(range(n)) + big
+        small = [k for k in range(n - 1, -1, -1) if we[k] < min_w][:max(mdel, 0)]
+        for k in small:
+            lst[lst.index(k)] = lst[-1]
+            lst.pop()
+        if (big or small) and len(lst) < 3:
+            flag[0] = 1
+        flag[1] += len(big)
+        flag[2] += len(small)
+        lists.append(lst)
+    return lists, flag
+
+
+@pytest.mark.parametrize("dim,nel", [(2, (7, 5)), (3, (5, 4, 3))])
+@pytest.mark.parametrize("max_deletions,max_splits", [(3, 2), (0, 0), (-1, 4), (100, 7)])
+def test_pcdvc_kernels_with_a_host_scan(dim, nel, max_deletions, max_splits):
+    """The plan and build kernels around a scan on the host: every element's new count and list as the reference walks
+    them, and the new swarm from those lists, with and without the optional arrays.  No bar: integers and copies."""
+    import ctypes as C
+    from earthbyte_underworld_amd import _lib as L
+    from tests.test_gpu_operators import _Dev, _grid
+    lib = L.load()
+    g, ne = _grid(dim, nel), int(np.prod(nel))
+    rng = np.random.default_rng(max_splits + dim)
+    cnt = rng.integers(0, 40, ne)
+    off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    n = int(off[-1])
+    w = rng.exponential(0.08 * (1 << dim), n)
+    mat = (rng.random(n) < 0.02).astype(np.uint8)
+    o = L.PcdvcOpts(upper_t=10.0, lower_t=1.0, max_deletions=max_deletions, max_splits=max_splits,
+                    split_in_interface_cells=0, delete_in_interface_cells=1)
+    lists, flag = _plan(dim, nel, off, w, mat, o)
+    x, c = rng.uniform(-1, 1, (3, n)), rng.uniform(-1, 1, (3, n))
+    coh, s0, s1 = rng.random(n).astype(np.float32), rng.random(n), rng.random(n)
+    dev = [_Dev(lib, a) for a in (off, w, mat, np.full(ne, -1, np.int32), np.full(n + ne * max_splits + 1, -1, np.int32),
+                                  np.zeros(4, np.int32))]
+    doff, dw, dmat, dcnt, dlist, dflag = dev
+    assert lib.ust_k_pcdvc_plan(C.byref(g), doff.p, dw.p, dmat.p, C.byref(o), dcnt.p, dlist.p, dflag.p, None) == 0
+    assert np.array_equal(dcnt.get(), [len(v) for v in lists]) and list(dflag.get()[:3]) == flag
+    got = dlist.get()
+    for e, v in enumerate(lists):
+        assert np.array_equal(got[off[e] + e * max_splits:][:len(v)], v), e
+    new_off = np.concatenate([[0], np.cumsum([len(v) for v in lists])]).astype(np.int32)
+    m = int(new_off[-1])
+    flat = np.array([k for v in lists for k in v], np.int64)
+    src = (flat & ((1 << 30) - 1)) + np.repeat(off[:-1], np.diff(new_off))
+    split = (flat >> 30) != 0
+    dnew = _Dev(lib, new_off)
+    din = [_Dev(lib, a) for a in (*x, *c, coh, s0, s1)]
+    for optional in (True, False):
+        out = [_Dev(lib, np.zeros(m, t)) for t in (np.float64,) * 3 + (np.uint8, np.float32, np.float64, np.float64)]
+        pick = lambda d: d.p if optional else None
+        third = lambda d: d.p if dim == 3 else None
+        assert lib.ust_k_pcdvc_build(dim, ne, max_splits, doff.p, dnew.p, dlist.p, din[0].p, din[1].p, third(din[2]),
+                                     din[3].p, din[4].p, third(din[5]), pick(dmat), pick(din[6]), pick(din[7]),
+                                     pick(din[8]), out[0].p, out[1].p, third(out[2]), pick(out[3]), pick(out[4]),
+                                     pick(out[5]), pick(out[6]), None) == 0
+        for d in range(dim):
+            assert np.array_equal(out[d].get(), np.where(split, c[d][src], x[d][src]))
+        for k, a in ((3, mat), (4, coh), (5, s0), (6, s1)):
+            assert np.array_equal(out[k].get(), a[src] if optional else np.zeros(m, a.dtype))
+        for d in out:
+            d.free()
+    for d in dev + din + [dnew]:
+        d.free()
