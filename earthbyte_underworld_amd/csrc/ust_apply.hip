@@ -850,19 +850,28 @@ __device__ __forceinline__ bool cg_direction(const CgDir<T> &cg, bool *first, T 
     return state == 0.0;
 }
 
-// 3D grids up to this many elements take the halo kernel.  Measured on the 128x128x64 solve (same box, graph-replayed):
-// the halo passes on the 32x32x16 and 16x16x8 levels take it from 0.431-0.434 s to 0.403-0.407 s; on the 64x64x32 level
-// as well, 0.415-0.417 s (the duplicated halo elements cost more there than the gather).  2D grids take it whatever
-// their size: one element in seven is computed again, where the gather was half of a pass.
+// 3D grids up to this many elements may take the halo kernel: the 128x128x64 solve takes 0.403-0.407 s with the halo passes
+// on its 32x32x16 and 16x16x8 levels (0.431-0.434 without) and 0.415-0.417 s with them on the 64x64x32 level as well.
 #ifndef UST_HALO_MAX_NEL
 #define UST_HALO_MAX_NEL 65536
 #endif
+// A CU works through its halo workgroups one after the other (FP64 product: 5.2 us with up to 256 of them, 7.3 up to 512, 10.5
+// beyond), through a tile and the gather in about 9.3, two tiles in 10.9.  So beyond 512 workgroups grids of at most one tile
+// per CU take tiles.  FP64 product, halo / tiles: 36^3 7.4 / 9.1 us, 48x36x36 10.4 / 9.3, 64x32x32 10.6 / 9.5, 40^3 (300 tiles)
+// 10.6 / 10.8, 65x33x30 (360) 10.5 / 11.0; FP32 prolongation pass 36^3 10.4 / 10.7, 64x32x32 14.5 / 11.0.  Solves of 64x32x32
+// in FP64 837 / 814 ms, with FP32 PCG 300 / 281; 128x64x64 539 / 526.
+// 2D grids take it whatever their size: one element in seven is computed again, where the gather was half of a pass.  FP64
+// product 256^2 3.9 / 6.8 us, 512x256 4.2 / 7.3, 1000^2 17.1 / 25.8, 1500^2 34.2 / 53; FP32 1000^2 12.4 / 19.8.
+constexpr int HALO_FULL = 512, HALO_CUS = 256;
 
 __host__ __device__ inline int halo_tiles(const GridDev &g) {
     if (g.dim == 2) return ((g.nnx + H2O - 1) / H2O) * ((g.nny + H2O - 1) / H2O);
     return ((g.nnx + HOX - 1) / HOX) * ((g.nny + HOY - 1) / HOY) * ((g.nnz + HOZ - 1) / HOZ);
 }
-static inline bool halo_grid(const GridDev &g) { return g.dim == 2 || (!g.col && g.nel <= UST_HALO_MAX_NEL); }
+static inline bool halo_grid(const GridDev &g) {
+    if (g.dim == 2) return true;
+    return !g.col && g.nel <= UST_HALO_MAX_NEL && (halo_tiles(g) <= HALO_FULL || g.ntiles > HALO_CUS);
+}
 
 // whether a pass writes a vector that it stages, at nodes that other workgroups own: u, or for the steps from zero b and
 // invd, and the coarse correction.  (Those an owned node alone reads may be written over.)

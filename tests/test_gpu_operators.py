@@ -1174,3 +1174,29 @@ def test_step_by_step_cg(kind, n, off):
         v.d.free()
     for d in (part, ctl, s):
         d.free()
+
+
+# the halo kernel's workgroups, 0 where tiles are taken: up to 512 and past them, one tile per CU and more, most elements
+@pytest.mark.parametrize("nel,groups", [((36, 36, 36), 500), ((48, 36, 36), 0), ((64, 32, 32), 0), ((40, 40, 40), 726),
+                                        ((65, 33, 30), 648), ((66, 33, 31), 0), ((15, 63, 63), 512)])
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+def test_kernel_choice_of_small_3d_grids(nel, groups, prec):
+    """Either side of the lines between halo and tile kernels: the choice, and the product against the one-element-per-thread
+    reference operator.  Bar: that of test_column_kernel_against_element_reference."""
+    import ctypes as C
+    import earthbyte_underworld_amd as ust  # noqa: F401  (loads the library)
+    from earthbyte_underworld_amd import _lib as L
+    lib = L.load()
+    g = _grid(3, nel)
+    assert lib.ust_k_apply_single(C.byref(g)) == groups
+    T = np.float64 if prec == "f64" else np.float32
+    n, wl = int(np.prod([k + 1 for k in nel])) * 3, lib.ust_k_weights_len(C.byref(g))
+    rng = np.random.default_rng(2)
+    W, dm = _Dev(lib, rng.uniform(0.1, 1.0, wl).astype(T)), _Dev(lib, (rng.random(n) < 0.1).astype(np.uint8))
+    du, y, ref = _Dev(lib, rng.normal(size=n).astype(T)), _Dev(lib, np.zeros(n, T)), _Dev(lib, np.zeros(n, T))
+    work = _Dev(lib, np.zeros(lib.ust_k_apply_work_len(C.byref(g)), T))
+    assert getattr(lib, f"ust_k_apply_K_{prec}")(C.byref(g), W.p, dm.p, du.p, y.p, work.p, None) == 0
+    assert getattr(lib, f"ust_k_apply_K_ref_{prec}")(C.byref(g), W.p, dm.p, du.p, ref.p, None) == 0
+    assert rel_err(y.get().astype(np.float64), ref.get().astype(np.float64)) < (1e-13 if prec == "f64" else 1e-5)
+    for a in (W, dm, du, y, ref, work):
+        a.free()
