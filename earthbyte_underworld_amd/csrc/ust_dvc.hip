@@ -246,13 +246,17 @@ __device__ void dvc_element_words(const DvcShape &s, unsigned char *dvc_lds, int
     }
 }
 
-// per > 1: the elements whose boundary sets outgrew k_dvc_grow's ring (it left a negative weight on their first particle);
-// a wave looks at `per` elements and redoes the marked ones.  per = 1: every element, where particles so many that
-// k_dvc_grow's LDS does not fit share one.
+// The elements whose boundary sets outgrew k_dvc_grow's ring (it left a negative weight on their first particle): a wave looks
+// at `per` elements and redoes the marked ones.  all: every element, where particles so many that k_dvc_grow's LDS does not
+// fit share one.
+// per: one as long as that makes few waves, since a wave redoes its elements one after the other while the GPU runs empty (24^3
+// x 100 particles with 64 to a wave 34 ms, 5.2 now; 125 on a jittered lattice, where most spill, 66 and 9.4); up to 8 on larger
+// swarms, where a wave without work costs more than the balance (96^3: 110,000 waves).
+constexpr int DVC_SPILL_WAVES = 16384, DVC_SPILL_PER = 8;
 template <int DIM, typename OT>
 __global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, const int *elems,
                                                          int nel, double *xi0, double *xi1, double *xi2, double *w,
-                                                         int set_centroids, int *flag, int per) {
+                                                         int set_centroids, int *flag, int per, bool all) {
     extern __shared__ __align__(16) unsigned char dvc_lds[];
     int el = blockIdx.x * per + (int)threadIdx.x;
     const bool mine = (int)threadIdx.x < per && el < nel;
@@ -263,8 +267,8 @@ __global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *
         np = cell_off[el + 1] - off;
     }
     const bool holds = mine && np > 0 && np <= s.max_np;
-    if (per == 1 && mine && !holds) atomicOr(flag, np <= 0 ? 1 : 2);
-    unsigned long long todo = __ballot(holds && (per == 1 || w[off] < 0.0));
+    if (all && mine && !holds) atomicOr(flag, np <= 0 ? 1 : 2);
+    unsigned long long todo = __ballot(holds && (all || w[off] < 0.0));
     while (todo) {
         const int j = __builtin_ctzll(todo);
         todo &= todo - 1ull;
@@ -551,9 +555,10 @@ static int launch_dvc(const DvcShape &s, size_t lds_words, const int *cell_off, 
     if (grow)
         hipLaunchKernelGGL((k_dvc_grow<DIM, G, OT>), dim3((nel + EPB - 1) / EPB), dim3(64 * GROW_WAVES), lds, st, s,
                            cell_off, elems, nel, xi0, xi1, xi2, w, set_centroids, flag);
-    const int per = grow ? DVC_LANES : 1;
+    const int fill = (nel + DVC_SPILL_WAVES - 1) / DVC_SPILL_WAVES;
+    const int per = !grow ? 1 : fill < DVC_SPILL_PER ? fill : DVC_SPILL_PER;
     hipLaunchKernelGGL((k_dvc_spill<DIM, OT>), dim3((nel + per - 1) / per), dim3(DVC_LANES), lds_words, st, s, cell_off,
-                       elems, nel, xi0, xi1, xi2, w, set_centroids, flag, per);
+                       elems, nel, xi0, xi1, xi2, w, set_centroids, flag, per, !grow);
     UST_LAUNCH_CHECK();
     return UST_OK;
 }

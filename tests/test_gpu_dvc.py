@@ -531,3 +531,26 @@ def test_pcdvc_kernels_with_a_host_scan(dim, nel, max_deletions, max_splits):
             d.free()
     for d in dev + din + [dnew]:
         d.free()
+
+
+@pytest.mark.parametrize("nel", [(25, 25, 25), (26, 26, 26), (51, 51, 51)])
+def test_dvc_spilled_elements_of_large_swarms(oracle, nel):
+    """Elements whose boundary sets outgrow the ring (the crosses of test_dvc_growth_edges) among ones that fit, in swarms
+    where a wave looks at one, two and eight elements to redo, alone in their group, beside each other and last: bit-equal
+    to the oracle."""
+    cross = _dvc_edge_points("spill", np.random.default_rng(1))[2][1]
+    ne = int(np.prod(nel))
+    crowded = np.zeros(ne, bool)
+    crowded[::611] = crowded[1::1222] = crowded[-1] = True
+    cnt = np.where(crowded, len(cross), 1)
+    off = np.concatenate([[0], np.cumsum(cnt)]).astype(np.int32)
+    xi = np.random.default_rng(9).uniform(-1, 1, (off[-1], 3))
+    for e in np.flatnonzero(crowded):
+        xi[off[e]:off[e + 1]] = cross
+    s = _system(3, nel)
+    s.upload_swarm(off, xi, np.ones(off[-1]))
+    s.dvc_weights(9)
+    xi1, w1 = s.integration_points()
+    xi_ref, w_ref = oracle.dvc_swarm(3, (9, 9, 9), off, xi)
+    assert np.array_equal(w1, w_ref) and np.array_equal(xi1, xi_ref)
+    s.close()
