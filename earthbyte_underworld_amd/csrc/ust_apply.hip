@@ -4,16 +4,16 @@
 //
 // 3D: one 256-thread workgroup owns a 16x16 column of elements, one element per thread, and streams a
 // chunk of element layers along z.  Node planes are staged in LDS once each; per layer every thread applies
-// its element (element_apply3 below, about 600 operations) and leaves its 8 vertex
-// results in LDS; each node of the plane below the layer then sums, in a fixed order, the contributions of
-// the (up to) four elements above it and the four below it (carried in registers from the previous layer),
+// its element (element_apply3 below, about 600 operations) and leaves its 8 vertex results in LDS; each
+// node of the plane below the layer then sums, in a fixed order, the contributions of the (up to) four elements above it and the four below it (carried in registers from the previous layer),
 // and is finished: written to y through the epilogue, unless it lies on the ring of the column (shared with
 // a neighbouring column) or on a chunk-boundary plane (shared with the next chunk).  Those nodes go to the
 // workgroup's slot of a workspace, and a second, node-ordered pass sums the two to eight slots covering each
 // of them.  No atomics touch memory and the summation order is fixed, so K u is bitwise reproducible.
 // Grids with fewer than 1024 column layers (the coarse multigrid levels) use 16x4x4 tiles instead, one per
-// workgroup, which gives small grids more workgroups.
-// 2D: one workgroup per 16x16 tile, node block reduced in LDS, the same workspace scheme on the tile faces.
+// workgroup, which gives small grids more workgroups, and the smaller of those (halo_grid below) and all 2D grids the halo
+// kernels: a workgroup owns a block of nodes and computes every element that touches it, without a workspace.  Passes that
+// overwrite what neighbouring workgroups stage take tiles there too (2D: 16x16 elements, the same workspace scheme).
 #include <mutex>
 #include <stdio.h>
 
@@ -280,9 +280,9 @@ __device__ __forceinline__ bool on_tile_face(int gc, int T, int tn) {
 //               staged only by that tile, before its update, and tile-face nodes are updated in
 //               phase 2, after every tile has staged them.
 //   EPI_CHEBY0  the same with c1 = 0 (the previous d is not read)
-//   EPI_PCHEBY0 (3D) the multigrid prolongation x += P xc of the coarse-grid correction xc, then the
+//   EPI_PCHEBY0 the multigrid prolongation x += P xc of the coarse-grid correction xc, then the
 //               EPI_CHEBY0 step on the corrected x, in one pass: the staged velocities are x + P xc,
-//               interpolated from the tile's coarse node block held in LDS.
+//               interpolated from the tile's coarse node block held in LDS (halo kernels: from memory; 2D: halo only).
 //   EPI_RES0    the first Jacobi-Chebyshev step from a zero guess, x = c2 invd b, then the residual
 //               r = b - K x (0 on Dirichlet dofs), in one pass: the staged velocities are c2 invd b (u is not
 //               read); y = r, d = x (the previous d is neither read nor written).
@@ -400,7 +400,8 @@ constexpr int CNR = (CNPD + UST_TILE - 1) / UST_TILE;
 // measured alike).  With the quotients 2/h taken out of the kernel and the coarse planes of the prolongation interpolated
 // once (staged below), a layer took 990 instead of 1400 instructions per thread in the FP32 product and 1200 instead of
 // 3150 in the prolongation pass (with an element action of 456 operations; now 606).  128x128x64 passes then, with the
-// gather: FP32 product 42.8 -> 38 us, residual with the first step 47.9 -> 44.5, prolongation pass 62.0 -> 54.8, FP64 product 73.3 -> 67.3; the column kernels now move 4.5-5.4 TB/s.
+// gather: FP32 product 42.8 -> 38 us, residual with the first step 47.9 -> 44.5, prolongation pass 62.0 -> 54.8, FP64 product
+// 73.3 -> 67.3.
 constexpr int EBX = UST_TX3 + 2, EBY = UST_TY3 + 2, EBS = 326;
 static_assert(EBX * EBY <= EBS && 24 * EBS * 4 % 16 == 0, "18x18 slots per row, cleared by 16-byte stores");
 
@@ -806,11 +807,10 @@ __global__ __launch_bounds__(256, 2) void k_applyK3_tiled(GridDev g, TileDiv td,
 // one element per thread -- so every owned node's sum is complete inside the workgroup: one launch, no workspace and no
 // gather.  The halo elements are computed by two workgroups, which costs less on the latency-bound grids than the gather
 // it replaces.  Neighbouring workgroups stage the nodes a workgroup writes, so the Chebyshev modes must run out of place
-// (ep.xs != ep.y).  Each node sums its element contributions in a fixed order, in FP64:
-// deterministic.  The operands of the
+// (ep.xs != ep.y).  Each node sums its element contributions in a fixed order, in FP64: deterministic.  The operands of the
 // epilogue are loaded with the node block, so that only one trip to memory is exposed, and a pass can leave per-workgroup
 // partial sums of the dot product that follows it in the Krylov iteration.
-// What bounds them is the serial chain of one wavefront: launch, one trip to memory, 1200-1600 instructions, a store.  With
+// What bounds them is the serial chain of one wavefront: launch, one trip to memory, 1300-1800 instructions, a store.  With
 // every pass of such levels on them an inner iteration took 14 launches in 2D at 64x64 where tiles + gather, separate first
 // steps, prolongation and dots took 24; solves: 2D 64x64 FP64 129.6 -> 74.7 ms, 3D 24x16x16 FP64 661 -> 455 ms.
 // Staging whole nodes (index arithmetic once per node, none of the loads behind a branch) instead of single dofs:
@@ -855,11 +855,11 @@ __device__ __forceinline__ bool cg_direction(const CgDir<T> &cg, bool *first, T 
 #ifndef UST_HALO_MAX_NEL
 #define UST_HALO_MAX_NEL 65536
 #endif
-// A CU works through its halo workgroups one after the other (FP64 product: 5.2 us with up to 256 of them, 7.3 up to 512, 10.5
-// beyond), through a tile and the gather in about 9.3, two tiles in 10.9.  So beyond 512 workgroups grids of at most one tile
-// per CU take tiles.  FP64 product, halo / tiles: 36^3 7.4 / 9.1 us, 48x36x36 10.4 / 9.3, 64x32x32 10.6 / 9.5, 40^3 (300 tiles)
-// 10.6 / 10.8, 65x33x30 (360) 10.5 / 11.0; FP32 prolongation pass 36^3 10.4 / 10.7, 64x32x32 14.5 / 11.0.  Solves of 64x32x32
-// in FP64 837 / 814 ms, with FP32 PCG 300 / 281; 128x64x64 539 / 526.
+// A CU works through its halo workgroups one after the other (FP64 product: 5.2 us with up to 256 of them, 7.3 up to 512,
+// 10.5 beyond), through a tile and the gather in about 9.3, two tiles in 10.9.  So beyond 512 workgroups grids of at most one
+// tile per CU take tiles.  FP64 product, halo / tiles: 36^3 7.4 / 9.1 us, 48x36x36 10.4 / 9.3, 64x32x32 10.6 / 9.5, 40^3 (300
+// tiles) 10.6 / 10.8, 65x33x30 (360) 10.5 / 11.0; FP32 prolongation pass 36^3 10.4 / 10.7, 64x32x32 14.5 / 11.0.  Solves of
+// 64x32x32 in FP64 837 / 814 ms, with FP32 PCG 300 / 281; 128x64x64 539 / 526.
 // 2D grids take it whatever their size: one element in seven is computed again, where the gather was half of a pass.  FP64
 // product 256^2 3.9 / 6.8 us, 512x256 4.2 / 7.3, 1000^2 17.1 / 25.8, 1500^2 34.2 / 53; FP32 1000^2 12.4 / 19.8.
 constexpr int HALO_FULL = 512, HALO_CUS = 256;
@@ -1541,8 +1541,8 @@ static int fused_pass(const GridDev &g, const ust_pass *p, hipStream_t st) {
                                                 : tile_div((cnx + F3X - 1) / F3X, (cny + F3Y - 1) / F3Y);
 #define PRE2(KIND) hipLaunchKernelGGL((k_pre2<T, WT, KIND>), grid, dim3(UST_TILE), 0, st, g, td, W, p->mask, p->maskc, u, b, \
                                       invd, y, d, bc, c0, c1, c2)
-#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, td, grad_scale<T>(g), W, p->mask, p->maskc, u, b, invd, \
-                                      d, bc, c2)
+#define PRE3(KIND) hipLaunchKernelGGL((k_pre3<T, WT, KIND>), grid, dim3(F3T), 0, st, g, td, grad_scale<T>(g), W, p->mask, \
+                                      p->maskc, u, b, invd, d, bc, c2)
     if (mode == UST_PASS_PCHEBY2)
         hipLaunchKernelGGL((k_post2<T, WT>), grid, dim3(UST_TILE), 0, st, g, td, W, p->mask, u, (const T *)p->xc, b, invd, y,
                            c0, c1, c2, p->dot);
@@ -1964,8 +1964,7 @@ extern "C" int ust_k_apply_K_cheby_prolong_f32(const ust_grid *g, const float *W
     return apply_cheby_prolong<float, float>(g, WK, mask, x, x, b, invd, d, c2, xc, work, stream);
 }
 
-// out of place: x before the step, xo after it (distinct vectors); on FP32 tile grids this runs the halo-tile
-// kernel (one pass, no gather)
+// out of place: x before the step, xo after it (distinct vectors); on halo grids one launch, no gather
 extern "C" int ust_k_apply_K_cheby_oop_f32(const ust_grid *g, const float *WK, const unsigned char *mask, const float *x,
                                            float *xo, const float *b, const float *invd, float *d, float c1, float c2,
                                            int first, float *work, void *stream) {

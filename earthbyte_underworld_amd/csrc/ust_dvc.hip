@@ -246,12 +246,12 @@ __device__ void dvc_element_words(const DvcShape &s, unsigned char *dvc_lds, int
     }
 }
 
-// The elements whose boundary sets outgrew k_dvc_grow's ring (it left a negative weight on their first particle): a wave looks
-// at `per` elements and redoes the marked ones.  all: every element, where particles so many that k_dvc_grow's LDS does not
-// fit share one.
-// per: one as long as that makes few waves, since a wave redoes its elements one after the other while the GPU runs empty (24^3
-// x 100 particles with 64 to a wave 34 ms, 5.2 now; 125 on a jittered lattice, where most spill, 66 and 9.4); up to 8 on larger
-// swarms, where a wave without work costs more than the balance (96^3: 110,000 waves).
+// The elements whose boundary sets outgrew k_dvc_grow's ring (it left a negative weight on their first particle): a wave
+// looks at `per` elements and redoes the marked ones.  all: every element, where particles so many that k_dvc_grow's LDS
+// does not fit share one.
+// per: one as long as that makes few waves, since a wave redoes its elements one after the other while the GPU runs empty
+// (24^3 x 100 particles with 64 to a wave 34 ms, 5.2 now; 125 on a jittered lattice, where most spill, 66 and 9.4); up to 8
+// on larger swarms, where a wave without work costs more than the balance (96^3: 110,000 waves).
 constexpr int DVC_SPILL_WAVES = 16384, DVC_SPILL_PER = 8;
 template <int DIM, typename OT>
 __global__ __launch_bounds__(DVC_LANES) void k_dvc_spill(DvcShape s, const int *cell_off, const int *elems,
@@ -290,8 +290,8 @@ __host__ __device__ inline size_t grow_lds_shared(const DvcShape &s) {
 // Bound: the latency of the sequential turns (about 200 in 3D at 30 particles, some 200 VALU and 14 LDS instructions
 // each), so what counts is the elements in flight, which LDS limits (40 per CU at 30 particles), and the length of a
 // turn: the claim test reads FP32 coordinates in one 16-byte access, and a lane per neighbour expands five claimed
-// cells a pass.  96^3 elements x 30 particles: 178 ms with one element to a wave and the sets as words, 43 ms here; its
-// bytes (1.5 GB) would take 0.3 ms.
+// cells a pass.  96^3 elements x 30 random particles: 151 ms with one element to a wave and the sets as words, 41 ms here
+// (46 ms after an advection step, whose fullest element sizes every ring); its bytes (1.5 GB) would take 0.3 ms.
 constexpr int GROW_WAVES = 2;
 constexpr int DVC_WIDE_2D = 16384;  // 2D swarms of fewer elements give an element 32 lanes
 

@@ -36,7 +36,8 @@ int ust_dev_malloc(void **p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         ust_set_hip_error(e, __FILE__, __LINE__);
-        (void)hipGetLastError();  // reported here: a caller that makes room and tries again must not find it at its next launch
+        // reported here: a caller that makes room and tries again must not find it at its next launch
+        (void)hipGetLastError();
         *p = NULL;
         return UST_ENOMEM;
     }

@@ -356,8 +356,8 @@ int ust_k_apply_K_residual_f64(const ust_grid *g, const double *WK, const unsign
 int ust_k_apply_K_residual_f32(const ust_grid *g, const float *WK, const unsigned char *mask, const float *u,
                                const float *b, float *r, float *work, void *stream);
 /* the same Chebyshev passes out of place: the step reads x and writes xo (distinct vectors; d is read and
- * written per dof, or left unwritten when NULL as above).  On small 3D grids (at most 65,536 elements: the coarser multigrid levels) the FP32 pass is
- * one halo-tile launch without a workspace gather (work is then not used). */
+ * written per dof, or left unwritten when NULL as above).  Where ust_k_apply_single(g) > 0 the pass is one launch
+ * without a workspace gather (work is then not used, but still has to be given). */
 int ust_k_apply_K_cheby_oop_f32(const ust_grid *g, const float *WK, const unsigned char *mask, const float *x,
                                 float *xo, const float *b, const float *invd, float *d, float c1, float c2, int first,
                                 float *work, void *stream);
