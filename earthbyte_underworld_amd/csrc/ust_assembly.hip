@@ -258,6 +258,12 @@ __device__ double particle_density(const GridDev &g, const BuoyDev &bd, const us
 // read one factor of each side per lane.  The next 64 particles are loaded while the matrix steps run.  A lane ends with
 // one of the element's 43 sums, so nothing is reduced; the sums of 8 elements are written together, in 64-byte runs.
 //
+// The steps of the 32 staged particles add to two sums in turn, which are closed into a third where an element goes on in
+// the next 32: one chain through all of an element's steps rounds once per step, which grew with the particles (rms error
+// of WK against 80-bit sums, 16^3 elements: 20 particles 1.5e-16 -> 1.0e-16, 40 1.8e-16 -> 1.0e-16, 100 2.8e-16 ->
+// 1.0e-16).  It costs 0 to 5% of the kernel (64^3, 40 particles per element, 231 -> 242 us; 8 particles, 112 -> 116 us);
+// four sums in an unrolled loop cost 8 to 10%, closing one sum at the 32 alone was 10% less exact at 25 to 36 particles.
+//
 // Bound: latency, with 16 waves per CU for plain rheology (LDS) and 8 where stresses are looked up (registers: 207 in 3D).
 // 21 M particles on 128x128x64, 61 materials: 842 -> 400 us (1.2 GB, 3 TB/s) against lanes that accumulate the 43 sums in
 // registers and reduce them through LDS, 8 waves per CU.  Arrhenius + DruckerPrager with cohesion noise, 4.6 M particles
@@ -381,12 +387,13 @@ __global__ __launch_bounds__(64 * pw_waves(NEED_T || NEED_VEL), pw_minb(NEED_T |
     // lane t: the slot of weight 0 of element e0 + t (t < ne <= 16)
     const unsigned long long slots = widx(g, e0 + (lane < ne ? lane : 0), 0);
     const double detJ = (DIM == 3) ? 0.125 * g.hx * g.hy * g.hz : 0.25 * g.hx * g.hy;
-    double D = 0.0;
+    double S0 = 0.0, S1 = 0.0, before = 0.0;
     int e = 0, elo = pbeg, ehi = __builtin_amdgcn_readlane(offs, 1);
     auto finish = [&]() {
+        double D = (S0 + S1) + before;
         if (DIM == 2) D += __shfl_xor(D, 8);  // the two halves of a step
         if (col >= 0) osum[col * (PW_OUT + 1) + e % PW_OUT] = D;
-        D = 0.0;
+        S0 = S1 = before = 0.0;
         e++;
         elo = ehi;
         ehi = __builtin_amdgcn_readlane(offs, e < ne ? e + 1 : ne);
@@ -490,13 +497,19 @@ __global__ __launch_bounds__(64 * pw_waves(NEED_T || NEED_VEL), pw_minb(NEED_T |
                     for (int st = lo + STEP; st < hi; st += STEP) {
                         row = st + sub < hi ? st + sub : PW_HALF;
                         const double an = buf[row * ROW + fa], bn = buf[row * ROW + fb];
-                        D = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, D, 0, 0, 0);
+                        const double t = S1 + __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, 0.0, 0, 0, 0);
+                        S1 = S0;
+                        S0 = t;
                         a = an;
                         b = bn;
                     }
-                    D = __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, D, 0, 0, 0);
+                    S1 += __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, 0.0, 0, 0, 0);
                 }
-                if (ehi > hend) break;  // the element goes on in the next particles
+                if (ehi > hend) {  // the element goes on in the next particles
+                    before += S0 + S1;
+                    S0 = S1 = 0.0;
+                    break;
+                }
                 finish();
             }
             wave_sync();

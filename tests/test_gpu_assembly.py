@@ -504,6 +504,50 @@ def test_particle_weights_of_empty_elements(dim, nel):
         a.free()
 
 
+@pytest.mark.parametrize("dim,nel,ppc", [(3, (8, 8, 8), 100), (3, (8, 4, 4), 300), (2, (16, 16), 300)])
+def test_rounding_of_the_particle_sums(dim, nel, ppc):
+    """The sums' error does not grow with the particles.  Spacing, weights, viscosity and density are powers of two, so only
+    the factors of a particle (independent: they average out) and the additions round.  A rounding's rms is about 0.4 u of
+    the sum at that point (u = 2^-53); m additions in a chain of like terms come to 0.4 u sqrt(m / 3).  Blocks of 32
+    particles, each of two chains of four steps: 0.4 u sqrt(8 / 3) = 0.65 u per block, independent between blocks, and the
+    blocks' chain of at most 10: 0.75 u; together below 1 u.  One chain through all steps of four particles that round at
+    each particle is 2.3 u at 100 and 4 u at 300.  Bar: 1.5 u in the 2-norm."""
+    import earthbyte_underworld_amd as ust
+    from tests.test_gpu_operators import _Dev
+    rng = np.random.default_rng(11)
+    ne = int(np.prod(nel))
+    off = (np.arange(ne + 1) * ppc).astype(np.int32)
+    xi = rng.uniform(-1, 1, (3, off[-1]))
+    w = np.full(off[-1], 2.0 ** -6)
+    s = ust.StokesSystem(dim, nel)
+    s.set_materials([ust.RheologyMaterial([ust.MaterialViscosity(eta0=4.0)], density=2.0)])
+    d = [_Dev(s.lib, a) for a in (off, xi[0], xi[1], xi[2], w)]
+    assert s.lib.ust_swarm_upload_dev(s.ctx, int(off[-1]), *[a.p for a in d], None, None, ppc) == 0
+    s.assemble()
+    got = s.weights()
+    X = xi[:dim].astype(np.longdouble)
+    detJ = float(np.prod([0.5 / k for k in nel]))
+    lag = [(x * (x - 1) / 2, 1 - x * x, x * (x + 1) / 2) for x in X]
+    lin = [((1 - x) / 2, (1 + x) / 2) for x in X]
+
+    def sums(factors, base, scale):
+        rows = []
+        for q in range(base ** dim):
+            v = np.full(off[-1], scale, np.longdouble)
+            for k in range(dim):
+                v = v * factors[k][(q // base ** k) % base]
+            rows.append(np.add.reduceat(v, off[:-1]))
+        return np.array(rows)
+
+    one = detJ * 2.0 ** -6
+    for name, g, r in zip(("WK", "WG", "WF"), got,
+                          (sums(lag, 3, 4.0 * one), sums(lin, 2, one), sums(lin, 2, 2.0 * one))):
+        err = float(np.sqrt(np.sum((g.astype(np.longdouble) - r) ** 2) / np.sum(r ** 2)))
+        assert err < 1.5 * 2.0 ** -53, (name, err * 2.0 ** 53)
+    for a in d:
+        a.free()
+
+
 # fewer elements than a block, partial blocks, and more than the passes' blocks take at once (1024 x 256)
 @pytest.mark.parametrize("dim,nel", [(2, (5, 3)), (2, (600, 500)), (3, (3, 2, 5)), (3, (70, 65, 60))])
 def test_derived_terms_of_an_assembly(dim, nel):
