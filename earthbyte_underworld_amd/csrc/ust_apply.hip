@@ -4,12 +4,13 @@
 //
 // 3D: one 256-thread workgroup owns a 16x16 column of elements, one element per thread, and streams a
 // chunk of element layers along z.  Node planes are staged in LDS once each; per layer every thread applies
-// its element (element_apply3 below, about 600 operations) and leaves its 8 vertex results in LDS; each
-// node of the plane below the layer then sums, in a fixed order, the contributions of the (up to) four elements above it and the four below it (carried in registers from the previous layer),
-// and is finished: written to y through the epilogue, unless it lies on the ring of the column (shared with
-// a neighbouring column) or on a chunk-boundary plane (shared with the next chunk).  Those nodes go to the
-// workgroup's slot of a workspace, and a second, node-ordered pass sums the two to eight slots covering each
-// of them.  No atomics touch memory and the summation order is fixed, so K u is bitwise reproducible.
+// its element (element_apply3 below, about 600 operations) and leaves its 8 vertex results in LDS; each node
+// of the plane below the layer then sums, in a fixed order, the contributions of the (up to) four elements
+// above it and the four below it (carried in registers from the previous layer), and is finished: written to
+// y through the epilogue, unless it lies on the ring of the column (shared with a neighbouring column) or on
+// a chunk-boundary plane (shared with the next chunk).  Those nodes go to the workgroup's slot of a workspace,
+// and a second, node-ordered pass sums the two to eight slots covering each of them.  No atomics touch memory
+// and the summation order is fixed, so K u is bitwise reproducible.
 // Grids with fewer than 1024 column layers (the coarse multigrid levels) use 16x4x4 tiles instead, one per
 // workgroup, which gives small grids more workgroups, and the smaller of those (halo_grid below) and all 2D grids the halo
 // kernels: a workgroup owns a block of nodes and computes every element that touches it, without a workspace.  Passes that

@@ -265,9 +265,9 @@ __device__ double particle_density(const GridDev &g, const BuoyDev &bd, const us
 // four sums in an unrolled loop cost 8 to 10%, closing one sum at the 32 alone was 10% less exact at 25 to 36 particles.
 //
 // Bound: latency, with 16 waves per CU for plain rheology (LDS) and 8 where stresses are looked up (registers: 207 in 3D).
-// 21 M particles on 128x128x64, 61 materials: 842 -> 400 us (1.2 GB, 3 TB/s) against lanes that accumulate the 43 sums in
-// registers and reduce them through LDS, 8 waves per CU.  Arrhenius + DruckerPrager with cohesion noise, 4.6 M particles
-// on 95x51x47: 685 -> 280 us; 3.3 M on 512x256: 228 -> 105 us (the friction terms once per material; 3 waves per SIMD for
+// 21 M particles on 128x128x64, 61 materials: 842 us with lanes that accumulate the 43 sums in registers and reduce them
+// through LDS, 8 waves per CU; 427 here (1.2 GB, 2.9 TB/s).  Arrhenius + DruckerPrager with cohesion noise, 4.6 M particles
+// on 95x51x47: 685 -> 283 us; 3.3 M on 512x256: 228 -> 107 us (the friction terms once per material; 3 waves per SIMD for
 // the 3D one, with 20 to 27 spilled registers, were slower: 437 against 392 us for the whole assembly).
 //
 // NEED_T / NEED_VEL / SW compile the temperature and strain-rate lookups (Arrhenius, yield) and the strain-weakening state
